@@ -68,6 +68,14 @@ F64_SPLIT = (3, 4)
 #: parts backward) by whether the channel count is a multiple of 128; the splits of the float
 #: kernels with as many channels per lane
 F16_SHAPE = {True: (2, 2, 3), False: (1, 1, 3)}
+#: second-order backward (channel counts with tiles): (channels per lane, waves per block, parts, resident
+#: waves per SIMD) of the kernel that owns the receivers' rows and of the one over tiles, which shares
+#: the schedule of the first `bwd_tile` variant.  120k edges at 128 channels / 240k at 64, l <= 3: rows at
+#: one channel per lane in 3 parts 0.71 / 0.70 ms (2 parts 0.72 / 0.78, unsplit 1.06 at 64, two channels
+#: per lane 0.78); tiles at 128 with two channels per lane 1.22 ms, with one 1.24, at 64 1.22 (8 waves per
+#: block and two resident per SIMD 1.50).
+SECOND_DM = {64: (1, 4, 3, 3), 128: (1, 4, 3, 3), 256: (1, 4, 3, 3)}
+SECOND_TILE = {64: (1, 4, 3, 3), 128: (2, 4, 3, 2), 256: (2, 8, 3, 2)}
 #: the float64 kernels take one coefficient per class of equal magnitude as a kernel argument
 F64_MAX_CLASSES = 64
 #: `bwd_tile`: variants of the backward over tiles of receivers (trailing layout, at least 64
@@ -362,8 +370,136 @@ def emit_edge_bwd(p: Part, f64: bool = False) -> list[str]:
     return lines
 
 
-def emit_part(struct_name: str, p: Part, f64: bool = False) -> list[str]:
-    """`f64`: also the float64 forms of the arithmetic (for the parts the float64 kernels use)."""
+def _second_weights(t: Table, rows):
+    """The products `p = |c| y`, `r = |c| y2` of a path, and a function that gives the declarations and
+    names of the weights w_ij(y), w_ij(y2) of a pair."""
+    ids, defs = t.path_products(rows)
+    defs = defs + [d.replace("const float p", "const float r").replace("* y[", "* y2[") for d in defs]
+
+    def weights(j, terms):
+        expr, bare = Table.weight_expr(terms, ids)
+        if bare:
+            return [], expr, expr.replace("p", "r")
+        return [f"const float w{j} = {expr}, v{j} = {expr.replace('p', 'r')};"], f"w{j}", f"v{j}"
+
+    return defs, weights
+
+
+def emit_edge_second_dm(p: Part) -> list[str]:
+    """An edge's terms of the gradient with respect to dm in the second-order backward:
+    `acc_i += s_l u_i + s2_l m_i`, `u_i = sum_j w_ij(y) x2_j + w_ij(y2) x_j`, `m_i = sum_j w_ij(y) x_j`."""
+    lines = ["    template <int C>",
+             "    __device__ static __forceinline__ void edge_second_dm(const Vec<C> *x, const float *y, const Vec<C> *s,",
+             "                                                          const Vec<C> *x2, const float *y2,",
+             "                                                          const Vec<C> *s2, Vec<C> *acc) {"]
+    for l, rows in p.paths.items():
+        defs, weights = _second_weights(p.t, rows)
+        lines.append(f"        {{  // path {l}: rows {min(rows)}..{max(rows)}")
+        lines += defs
+        for i, cols in rows.items():
+            lines.append("            {")
+            first = True
+            for j, terms in cols.items():
+                decl, w, v = weights(j, terms)
+                lines += ["                " + d for d in decl]
+                xj = p.xj[j]
+                if first:
+                    lines.append(f"                Vec<C> u = vmul(x2[{xj}], {w}), m = vmul(x[{xj}], {w});")
+                    first = False
+                else:
+                    lines.append(f"                u = vfma(x2[{xj}], {w}, u);")
+                    lines.append(f"                m = vfma(x[{xj}], {w}, m);")
+                lines.append(f"                u = vfma(x[{xj}], {v}, u);")
+            lines.append(f"                acc[{p.zi[i]}] = vfmav(s[{p.sl[l]}], u, acc[{p.zi[i]}]);")
+            lines.append(f"                acc[{p.zi[i]}] = vfmav(s2[{p.sl[l]}], m, acc[{p.zi[i]}]);")
+            lines.append("            }")
+        lines.append("        }")
+    lines.append("    }")
+    return lines
+
+
+class _rows_ahead:
+    """The reads of dm, one row ahead of their use: a row's value is requested before the arithmetic of
+    the row before it, and a scheduling barrier keeps the compiler from moving the read back down
+    to its use (where every row would wait for the latency of LDS)."""
+
+    def __init__(self, p: "Part", vec: str):
+        self.rows = [p.zi[i] for rows in p.paths.values() for i in rows]
+        self.vec, self.at = vec, 0
+        self.first = [f"        {vec} dm_next = dm[{self.rows[0]}];"] if self.rows else []
+
+    def take(self) -> list[str]:
+        self.at += 1
+        lines = [f"                const {self.vec} dmi = dm_next;"]
+        if self.at < len(self.rows):
+            lines.append(f"                dm_next = dm[{self.rows[self.at]}];")
+        return lines + [f"                __builtin_amdgcn_sched_barrier(0);"]
+
+
+def emit_edge_second(p: Part) -> list[str]:
+    """An edge's terms of the gradients with respect to x, y and s in the second-order backward.
+
+    Per path l:
+        ds_l  = sum_i dm_i u_i,                u_i = sum_j w_ij(y) x2_j + w_ij(y2) x_j
+        dx_j += w_ij(y2) (dm_i s_l) + w_ij(y) (dm_i s2_l)
+        dy_k += sum_channels c_ijk dm_i q_j,   q_j = s_l x2_j + s2_l x_j
+    The product dm_i q_j is summed over the channels of the lane before the coefficients multiply it.
+    """
+    t = p.t
+    lines = ["    // dx: running sums the edge's contributions are added to; dy: zeros on entry; ds rows go to `ds`.",
+             "    template <int C, typename Dm, typename DsSink>",
+             "    __device__ static __forceinline__ void edge_second(const Vec<C> *x, const float *y, const Vec<C> *s,",
+             "                                                       const Vec<C> *x2, const float *y2,",
+             "                                                       const Vec<C> *s2, const Dm &dm, Vec<C> *dx,",
+             "                                                       float *dy, const DsSink &ds) {"]
+    ahead = _rows_ahead(p, "Vec<C>")
+    lines += ahead.first
+    for l, rows in p.paths.items():
+        defs, weights = _second_weights(t, rows)
+        xs = sorted({j for cols in rows.values() for j in cols})
+        sl = p.sl[l]
+        lines.append(f"        {{  // path {l}: rows {min(rows)}..{max(rows)}")
+        lines += defs
+        for j in xs:
+            lines.append(f"            const Vec<C> q{j} = vfmav(s[{sl}], x2[{p.xj[j]}], vmulv(s2[{sl}], x[{p.xj[j]}]));")
+        lines.append("            Vec<C> dsl = vzero<C>();")
+        for i, cols in rows.items():
+            lines.append("            {")
+            lines += ahead.take()
+            lines.append(f"                const Vec<C> g = vmulv(dmi, s[{sl}]), g2 = vmulv(dmi, s2[{sl}]);")
+            first = True
+            for j, terms in cols.items():
+                decl, w, v = weights(j, terms)
+                xj = p.xj[j]
+                lines += ["                " + d for d in decl]
+                lines.append(f"                dx[{xj}] = vfma(g, {v}, dx[{xj}]);")
+                lines.append(f"                dx[{xj}] = vfma(g2, {w}, dx[{xj}]);")
+                if first:
+                    lines.append(f"                Vec<C> u = vmul(x2[{xj}], {w});")
+                    first = False
+                else:
+                    lines.append(f"                u = vfma(x2[{xj}], {w}, u);")
+                lines.append(f"                u = vfma(x[{xj}], {v}, u);")
+                lines.append(f"                {{ const float pr = vdot(dmi, q{j});")
+                for c, k in terms:
+                    lines.append(f"                  dy[{k}] = fmaf(pr, {t.lit(c, False)}, dy[{k}]);")
+                lines.append("                }")
+            lines.append("                dsl = vfmav(dmi, u, dsl);")
+            lines.append("            }")
+            # (as in edge_bwd: the sums of a row are computed where the row is, or its dm value and
+            # products stay in registers until the end of the edge)
+            lines.append("            " + " ".join(f"pin(dx[{p.xj[j]}]);" for j in cols) + " pin(dsl);")
+        lines.append(f"            ds.template put<{l}>(dsl);")
+        lines.append("        }")
+    for l in p.zero_paths:
+        lines.append(f"        ds.template put<{l}>(vzero<C>());")
+    lines.append("    }")
+    return lines
+
+
+def emit_part(struct_name: str, p: Part, f64: bool = False, second: bool = False) -> list[str]:
+    """`f64`: also the float64 forms of the arithmetic (for the parts the float64 kernels use); `second`:
+    also the forms of the second-order backward."""
     t = p.t
     out = [f"struct {struct_name} {{",
            f"    static constexpr int X = {t.X}, Y = {t.Y}, S = {t.S}, Z = {t.Z};",
@@ -380,6 +516,8 @@ def emit_part(struct_name: str, p: Part, f64: bool = False) -> list[str]:
         out += emit_edge_fwd(p, f64=True)
         out.append("")
         out += emit_edge_bwd(p, f64=True)
+    if second:
+        out += ["", *emit_edge_second_dm(p), "", *emit_edge_second(p)]
     out += ["};", ""]
     return out
 
@@ -438,6 +576,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         f"#include {include}",
         "#include " + include.replace("unrolled.h", "unrolled_f64.h"),
         "#include " + include.replace("unrolled.h", "unrolled_f16.h"),
+        "#include " + include.replace("unrolled.h", "unrolled_second.h"),
         "",
         "namespace e3j_amd {",
         "namespace {",
@@ -449,7 +588,11 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
     # float64 kernels: trailing layout, whole waves of channels, few enough coefficient classes
     f64 = channels % 64 == 0 and 0 < len(t.classes) <= F64_MAX_CLASSES
     f16 = channels % 64 == 0   # float16 kernels: trailing layout, whole waves of channels
-    splits = sorted({v[2] for v in launch["fwd"] + launch["bwd"] + tile} |
+    # (a run-time table at another multiple of 64 channels takes the tiles of 64 or 128 channels)
+    second_key = channels if channels in SECOND_DM else 128 if channels % 128 == 0 else 64
+    second_dm, second_tile = (SECOND_DM[second_key], SECOND_TILE[second_key]) if tile else (None, None)
+    second_splits = {second_dm[2], second_tile[2]} if tile else set()
+    splits = sorted({v[2] for v in launch["fwd"] + launch["bwd"] + tile} | second_splits |
                     ({v[1] for v in lead["fwd"] + lead["bwd"]} if lead else set()) |
                     (set(F64_SPLIT) if f64 else set()) | (set(F16_SHAPE[channels % 128 == 0][1:]) if f16 else set()))
     part_names = {}
@@ -457,7 +600,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         names = []
         for n, part in enumerate(split_parts(t, zs)):
             sname = f"Sig_{name}_z{zs}p{n}"
-            out += emit_part(sname, part, f64=f64 and zs in F64_SPLIT)
+            out += emit_part(sname, part, f64=f64 and zs in F64_SPLIT, second=zs in second_splits)
             names.append(sname)
         part_names[zs] = ", ".join(names)
     fwd_args = ["    const float *, const float *, const float *, const int32_t *, const int32_t *,",
@@ -483,6 +626,16 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         cpl, wpb, zs, minw = (*v, 1)[:4]
         out += [f"template __global__ void unrolled_bwd_tile_kernel<{channels}, {cpl}, {wpb}, {minw}, "
                 f"{part_names[zs]}>("] + tile_args
+    second_args = ["    const float *, const float *, const float *, const float *, const float *, const float *,"]
+    if tile:
+        cpl, wpb, zs, minw = second_dm
+        out += [f"template __global__ void second_dm_kernel<{channels}, {cpl}, {wpb}, {minw}, {part_names[zs]}>("]
+        out += second_args + ["    const int32_t *, const int32_t *, const int32_t *, const int32_t *, float *, int, float,",
+                              "    unsigned, int, int, const int32_t *, int, float *);"]
+        cpl, wpb, zs, minw = second_tile
+        out += [f"template __global__ void second_tile_kernel<{channels}, {cpl}, {wpb}, {minw}, {part_names[zs]}>("]
+        out += second_args + ["    const float *, const int32_t *, const int32_t *, const int32_t *, const int32_t *,",
+                              "    const int32_t *, float *, float *, float *, int, int, int, float, unsigned);"]
     # sender-grouped backward: the finest split of the paths (parts run one after another in a wave)
     sender_split = max(v[2] for v in launch["bwd"] + tile)
     sender_minw = 2
@@ -575,6 +728,18 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         out += ["static int run_tile_rows_default() {"]
         out += [ln.replace("VARIANT", "tuning().bwd_variant.load(std::memory_order_relaxed)") for ln in switch(
             tile, lambda v: f"{v[4] if len(v) > 4 else 8};")]
+    if tile:
+        out += ["static int run_second_dm(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,",
+                "                         const int32_t *row_ptr, const int32_t *perm, float *ddm, hipStream_t stream) {"]
+        cpl, wpb, zs, minw = second_dm
+        out += [f"    return launch_second_dm<{channels}, {cpl}, {wpb}, {minw}, {part_names[zs]}>("
+                "p, a, sender, row_ptr, perm, ddm, stream);", "}"]
+        out += ["static int run_second_tile(const e3j_amd_conv_params &p, const SecondOperands &a,",
+                "                           const e3j_amd_tile_schedule &schedule, float *dx, float *dy, float *ds,",
+                "                           hipStream_t stream) {"]
+        cpl, wpb, zs, minw = second_tile
+        out += [f"    return launch_second_tile<{channels}, {cpl}, {wpb}, {minw}, {t.Y}, {t.X}, {part_names[zs]}>("
+                "p, a, schedule, dx, dy, ds, stream);", "}", ""]
     out += ["static int run_bwd_sender(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,",
             "                          const float *dm, const int32_t *receiver_t, const int32_t *row_ptr,",
             "                          const int32_t *perm, float *dx, float *dy, float *ds, hipStream_t stream) {",
@@ -588,6 +753,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
             f"    &run_fwd, &run_bwd, {tiled}, &run_bwd_sender,",
             f"    {len(t.classes)}, kClass, &run_fwd_f64, &run_bwd_f64," if f64 else "    0, nullptr, nullptr, nullptr,",
             "    &run_fwd_f16, &run_bwd_f16," if f16 else "    nullptr, nullptr,",
+            "    &run_second_dm, &run_second_tile," if tile else "    nullptr, nullptr,",
             "};", ""]
     if lead:
         out += ["static int run_fwd_leading" + fwd_sig[0]] + fwd_sig[1:]

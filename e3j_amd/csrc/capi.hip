@@ -568,6 +568,55 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
     return finish(p, stream, rc, op);
 }
 
+int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s,
+                                const void *dm, const void *ddx, const void *ddy, const void *dds,
+                                const int32_t *sender, const int32_t *receiver_ptr,
+                                const int32_t *edge_perm, const e3j_amd_tile_schedule *schedule,
+                                void *grad_x, void *grad_y, void *grad_s, void *grad_dm, void *stream_) {
+    const char *op = "convolution_bwd_bwd";
+    int rc = validate(p, op);
+    if (rc) return rc;
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    if (p->num_nodes == 0 && p->num_edges == 0) return E3J_AMD_OK;
+    for (const void *node : {x, dm, ddx, static_cast<const void *>(grad_x), static_cast<const void *>(grad_dm)})
+        if (missing(node, p->num_nodes)) return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": null operand");
+    for (const void *edge : {y, s, ddy, dds, static_cast<const void *>(sender), static_cast<const void *>(grad_y),
+                             static_cast<const void *>(grad_s)})
+        if (missing(edge, p->num_edges)) return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": null operand");
+    if (receiver_ptr == nullptr || schedule == nullptr)
+        return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": null operand");
+    if (p->num_nodes == 0) return E3J_AMD_OK;
+    if (p->signature < 0 || p->val_dtype != E3J_AMD_F32 || signature(p->signature).second_dm == nullptr)
+        return set_error(E3J_AMD_UNIMPLEMENTED,
+                         std::string(op) + ": needs a float32 compile-time-unrolled kernel of the trailing layout "
+                                           "with at least 64 channels");
+    if (!aligned16({x, s, dm, ddx, dds, grad_x, grad_s, grad_dm}))
+        return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": operands must be 16-byte aligned");
+    if (schedule->num_work < 0 || (schedule->num_work > 0 && schedule->work == nullptr) ||
+        missing(schedule->sender, p->num_edges) || missing(schedule->edge, p->num_edges) ||
+        missing(schedule->local, p->num_edges))
+        return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": incomplete schedule");
+    if (p->row_cap < 0 || p->max_segments < 0 || p->row_piece < 0 || p->row_piece > p->row_cap ||
+        (p->segments != nullptr && (p->row_cap == 0 || p->partials == nullptr ||
+                                    reinterpret_cast<uintptr_t>(p->partials) % 16 != 0)))
+        return set_error(E3J_AMD_INVALID_ARGUMENT,
+                         std::string(op) + ": row_cap / row_piece / max_segments / segments / partials");
+    const Signature &sg = signature(p->signature);
+    const SecondOperands a{static_cast<const float *>(x),   static_cast<const float *>(y),
+                           static_cast<const float *>(s),   static_cast<const float *>(dm),
+                           static_cast<const float *>(ddx), static_cast<const float *>(ddy),
+                           static_cast<const float *>(dds)};
+    float *gy = static_cast<float *>(grad_y), *gs = static_cast<float *>(grad_s), *gdm = static_cast<float *>(grad_dm);
+    rc = sg.second_dm(*p, a, sender, receiver_ptr, edge_perm, gdm, stream);
+    if (rc == E3J_AMD_OK && p->segments != nullptr)
+        rc = launch_combine_pieces(p->segments, receiver_ptr, p->max_segments,
+                                   p->row_piece > 0 ? p->row_piece : p->row_cap,
+                                   (int64_t)p->num_out * p->channels, p->partials, gdm, stream);
+    if (rc == E3J_AMD_OK) rc = sg.second_tile(*p, a, *schedule, static_cast<float *>(grad_x), gy, gs, stream);
+    if (rc == E3J_AMD_OK) rc = launch_zero_padding(*p, sender, receiver_ptr, edge_perm, gy, gs, stream);
+    return finish(p, stream, rc, op);
+}
+
 int e3j_amd_find_signature(const void *coef_host, int32_t coef_idx_bytes, int32_t val_dtype,
                            int32_t num_coef, int32_t num_x, int32_t num_y, int32_t num_out,
                            int32_t num_scalars, int32_t channels, int32_t layout,

@@ -154,6 +154,11 @@ int reduce_ordered_dx(const e3j_amd_conv_params &p, const float *u, const int32_
 int reduce_ordered_dy(const e3j_amd_conv_params &p, const float *dy_slots, int slots,
                       const int32_t *perm, float *dy, hipStream_t stream);
 
+// Operands of the second-order backward: the convolution's, dm, and the cotangents of dx, dy, ds.
+struct SecondOperands {
+    const float *x, *y, *s, *dm, *x2, *y2, *s2;
+};
+
 // Compile-time-unrolled kernels (generated, sig_*.hip) ----------------------
 struct Signature {
     const char *name;
@@ -199,6 +204,12 @@ struct Signature {
     int (*bwd_f16)(const e3j_amd_conv_params &p, const half_t *x, const half_t *y, const half_t *s,
                    const half_t *dm, const int32_t *sender, const int32_t *receiver_ptr,
                    const int32_t *edge_perm, half_t *dx, half_t *dy, half_t *ds, hipStream_t stream);
+    // second-order backward (unrolled_second.h; float32, trailing layout, the schedule of the tiled
+    // backward; nullptr: none): the gradient with respect to dm, and those with respect to x, y, s
+    int (*second_dm)(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,
+                     const int32_t *receiver_ptr, const int32_t *edge_perm, float *ddm, hipStream_t stream);
+    int (*second_tile)(const e3j_amd_conv_params &p, const SecondOperands &a, const e3j_amd_tile_schedule &schedule,
+                       float *dx, float *dy, float *ds, hipStream_t stream);
 };
 // the coefficient classes of a float64 launch, passed to the kernel by value
 constexpr int kF64Classes = E3J_AMD_F64_CLASSES;

@@ -244,6 +244,70 @@ __device__ __forceinline__ float to_vgpr(float v) {
     return v;
 }
 
+// The y row of an edge.  Lane t holds components t % 16 (+ 16, + 32, ...): one 64-byte vector load per
+// sixteen components, handed out as values of all lanes by DPP row broadcasts.  (Loaded through the
+// scalar path the row shares its wait counter with LDS accesses, and scalar loads return in any
+// order: the first LDS read behind the prefetch of the next edge's y would wait for that row's
+// memory latency, in every turn of the loop.)
+template <int Y>
+struct YRow {
+    static constexpr int N = (Y + 15) / 16;
+    float v[N];
+    __device__ __forceinline__ void load(const float *row, int lane) {
+#pragma unroll
+        for (int b = 0; b < N; b++) v[b] = row[min(16 * b + lane % 16, Y - 1)];
+    }
+    // sign bits of this lane's components (bit k of `flip`: see flip_sign)
+    __device__ static __forceinline__ void signs(unsigned flip, int lane, unsigned (&bits)[N]) {
+#pragma unroll
+        for (int b = 0; b < N; b++) bits[b] = b < 2 ? ((flip >> (16 * b + lane % 16)) & 1u) << 31 : 0u;
+    }
+    template <int K>
+    __device__ __forceinline__ void spread(float *y, const unsigned (&bits)[N]) const {
+        if constexpr (K < Y) {
+            const int signed_bits = __float_as_int(v[K / 16]) ^ (int)bits[K / 16];
+            float r = __int_as_float(__builtin_amdgcn_mov_dpp(signed_bits, 0x150 + K % 16, 0xf, 0xf, true));
+            asm volatile("" : "+v"(r));  // (not folded into its uses: see to_vgpr)
+            y[K] = r;
+            spread<K + 1>(y, bits);
+        }
+    }
+};
+
+// The indices of up to 64 consecutive positions of a row's edge segment, one position per lane:
+// `at` is read by lane, so the edge loop itself holds no scalar load (each of which is a wait of
+// its own: see `load_uniform`).  Padding positions are left out of `live`.
+struct EdgeBatch {
+    int snd, ee;
+    unsigned long long live;  // positions (bit per lane) not yet taken
+    __device__ __forceinline__ void load(const int32_t *sender, const int32_t *perm, int base, int end, int num_nodes,
+                                         int lane) {
+        const int p = min(base + lane, end - 1);
+        snd = sender[p];
+        ee = perm ? perm[p] : p;
+        live = __ballot(base + lane < end && (unsigned)snd < (unsigned)num_nodes);
+    }
+    __device__ __forceinline__ int take() {
+        const int at = __builtin_ctzll(live);
+        live &= live - 1;
+        return at;
+    }
+    __device__ __forceinline__ int sender_at(int at) const { return __builtin_amdgcn_readlane(snd, at); }
+    __device__ __forceinline__ int64_t edge_at(int at) const { return __builtin_amdgcn_readlane(ee, at); }
+};
+
+// First position p of [from, end) with key[p] != key[p - 1] (from itself if it is `begin`), `end` if
+// there is none; 64 positions at a time.  All arguments are wave-uniform.
+__device__ __forceinline__ int run_start(const int32_t *key, int begin, int from, int end, int lane) {
+    if (from <= begin) return begin;
+    for (; from < end; from += kWave) {
+        const int p = min(from + lane, end - 1);
+        const unsigned long long differs = __ballot(key[p] != key[p - 1] && from + lane < end);
+        if (differs != 0) return from + __builtin_ctzll(differs);
+    }
+    return end;
+}
+
 // Sum NV (<= 16) per-lane values over the 64 lanes of a wave with about 3*NV + 4
 // VALU operations instead of 6*NV exchanges.  Halving exchange: at each of the four
 // in-row steps a lane keeps one half of its values and adds the partner's partial sums

@@ -552,6 +552,43 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
     return dx, dy, ds
 
 
+def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph=None):
+    """Gradients of `<ddx, dx> + <ddy, dy> + <dds, ds>` with respect to `(x, y, s, dm)` in one call of the
+    library, or None where it has no kernel for that (the first-order operators then compose them)."""
+    if (meta.layout != Layout.TRAILING_CHANNELS or meta.ordering == GraphOrdering.SENDER or y.shape[0] == 0
+            or x.dtype != torch.float32 or config().deterministic):
+        return None
+    tile_rows = _tile_rows(meta.table.signature(*_shape(meta, x, y, s), meta.layout)[0])
+    if tile_rows < 1:
+        return None
+    x, y, s, dm, ddx, ddy, dds = (t.contiguous() for t in (x, y, s, dm, ddx, ddy, dds))
+    grads = tuple(torch.empty_like(t) for t in (x, y, s, dm))
+    if any(t.data_ptr() % 16 for t in (x, s, dm, ddx, dds, *grads)):
+        return None
+    if graph is None:
+        graph = _forward_graph(meta, sender, receiver)
+    graph.ready()
+    other, row_ptr, perm, order = graph
+    p, table = _fill_params(meta, x, y, s, meta.table, row_order=order)
+    lib = _lib.load()
+    with torch.cuda.device(x.device):
+        schedule = graph.schedule(tile_rows)
+        want = int(config().row_cap)
+        cap = row_cap_for(x.shape[0], y.shape[0]) if want < 0 else want
+        if cap > 0:   # rows much longer than the mean are shared between waves (as in the forward pass)
+            num_out, channels = int(dm.shape[1]), int(dm.shape[2])
+            pieces = graph.segments(cap, row_piece_for(int(y.shape[0]), num_out * channels))
+            if pieces.count > 0:
+                p.row_cap, p.row_piece = pieces.row_cap, pieces.row_piece
+                p.segments, p.max_segments = pieces.buffer.data_ptr(), pieces.count
+                p.partials = pieces.partials(num_out, channels).data_ptr()
+        _lib.check(lib.e3j_amd_convolution_bwd_bwd(
+            ctypes.byref(p), x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), ddx.data_ptr(), ddy.data_ptr(),
+            dds.data_ptr(), other.data_ptr(), row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
+            ctypes.byref(schedule.struct), *(g.data_ptr() for g in grads), _stream(x.device)))
+    return grads
+
+
 def _tile_rows(signature: int) -> int:
     """Receivers per tile of the tiled backward for a compiled signature under the current
     configuration; 0: the one-wave-per-receiver backward runs."""
@@ -663,6 +700,11 @@ class _ConvolutionBwd(torch.autograd.Function):
         meta = ctx.meta
 
         graph = ctx.graph
+        if not torch.is_grad_enabled() and not _under_transform():
+            # nothing is recorded for a further derivative: all terms in one call where a kernel takes them
+            grads = _raw_second(meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph)
+            if grads is not None:
+                return *grads, None, None, None, None
 
         def conv(a, b, c):
             return _Convolution.apply(a, b, c, sender, receiver, meta, graph)

@@ -247,6 +247,21 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
                                   const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
                                   void *stream);
 
+/* Second-order backward: the VJP of the backward, for losses on its results (forces).  With
+ * L(x, y, s) = <dm, convolution(x, y, s)> and the cotangents ddx, ddy, dds of (dx, dy, ds), the gradients
+ * of <ddx, dx> + <ddy, dy> + <dds, ds> with respect to x, y, s and dm (src/e3j/ops/convolution.py:535-562
+ * composes them from three calls of each first-order operator; here two kernels compute all terms of an
+ * edge at once).  Needs a float32 signature of the trailing layout with at least 64 channels
+ * (e3j_amd_tile_rows(signature) > 0, else E3J_AMD_UNIMPLEMENTED), 16-byte aligned operands and the schedule
+ * of e3j_amd_convolution_bwd_tiled.  grad_x is summed with float atomics, grad_dm in a fixed order.
+ * Long rows: p->row_cap, row_piece, segments and partials as for the forward pass, all in this one
+ * call (segments without partials: E3J_AMD_INVALID_ARGUMENT). */
+int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s,
+                                const void *dm, const void *ddx, const void *ddy, const void *dds,
+                                const int32_t *sender, const int32_t *receiver_ptr,
+                                const int32_t *edge_perm, const e3j_amd_tile_schedule *schedule,
+                                void *grad_x, void *grad_y, void *grad_s, void *grad_dm, void *stream);
+
 /* Match a HOST copy of a packed forward table against the tables of the
  * compile-time-unrolled kernels built into the library, up to one uniform
  * positive factor (the 1/avg_num_neighbors the reference folds into the values,

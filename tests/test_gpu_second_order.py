@@ -1,0 +1,86 @@
+"""The second-order backward (`e3j_amd_convolution_bwd_bwd`) through autograd, against the float64 oracle:
+each gradient is a sum of two or three first-order results, so the reference and the magnitude of its
+terms are sums of the oracle's (the rounding allowance of `helpers.assert_parity` applies to the sum)."""
+
+import numpy as np
+import pytest
+import torch
+
+from e3j_amd import ops
+from e3j_amd.codegen.gen_conv import BUILTIN_SIGNATURES
+from e3j_amd.convolution import Convolution
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+DUMMY = int(np.iinfo(np.int32).max)
+
+
+def _graph(rng, kind):
+    """Receivers sorted (except "shuffled"); sizes at the edges of tiles, of batches of 64 positions and of
+    the pieces of long rows."""
+    if kind == "single":                       # one edge, one node
+        return 1, np.zeros(1, np.int32), np.zeros(1, np.int32)
+    if kind == "hub":                          # one row of 300 positions, past row_cap, pieces and work items
+        n = 37
+        degree = rng.integers(0, 9, size=n)    # some rows are empty
+        degree[5] = 300
+    else:                                      # rows of 63, 64, 65 positions; padding edges; the last tile is short
+        n = 13
+        degree = np.array([63, 64, 65, 0, 1, 2, 7, 8, 9, 0, 30, 31, 4])
+    rcv = np.repeat(np.arange(n), degree).astype(np.int32)
+    snd = rng.integers(0, n, size=rcv.shape[0]).astype(np.int32)
+    if kind == "padding":
+        snd[rng.random(snd.shape[0]) < 0.2] = DUMMY
+        snd[:64] = DUMMY                       # a whole batch without a live position
+    if kind == "shuffled":
+        order = rng.permutation(rcv.shape[0])
+        snd, rcv = snd[order], rcv[order]
+    return n, snd, rcv
+
+
+#: (256 channels: other tiles, the same edge loops as at 128; two graphs keep the oracle quick)
+CASES = [(sig, kind) for sig in BUILTIN_SIGNATURES if sig[4] >= 64
+         for kind in (("single", "hub") if sig[4] == 256 else ("single", "hub", "padding", "shuffled"))]
+
+
+@pytest.mark.parametrize("sig,kind", CASES, ids=[f"{s[0]}-{k}" for s, k in CASES])
+def test_second_order_matches_oracle(sig, kind, monkeypatch):
+    name, xi, yi, oi, channels = sig
+    rng = np.random.default_rng(channels + len(kind))
+    module = Convolution((xi, yi), oi, graph_ordering="NONE" if kind == "shuffled" else "RECEIVER")
+    n, snd, rcv = _graph(rng, kind)
+    num_x, num_y, num_z, num_s = (module.source[0].dim, module.source[1].dim, module.target.dim,
+                                  module.params.num_scalars)
+    x, y, s, dm = H.random_operands(rng, n, len(snd), num_x, num_y, num_s, channels, num_z)
+    x2, y2, s2, _ = H.random_operands(rng, n, len(snd), num_x, num_y, num_s, channels, num_z)
+    pad = snd == DUMMY
+    dev = {k: torch.from_numpy(v.copy()).cuda() for k, v in dict(x=x, y=y, s=s, dm=dm, x2=x2, y2=y2, s2=s2).items()}
+    for k in ("y", "s", "y2", "s2"):           # padding edges hold anything
+        dev[k][torch.from_numpy(pad)] = float("nan")
+    calls = []
+    monkeypatch.setattr(ops, "_raw_second", lambda *a, f=ops._raw_second: calls.append(1) or f(*a))
+    leaves = [dev[k].requires_grad_(True) for k in ("x", "y", "s", "dm")]
+    out = module(*leaves[:3], torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda())
+    first = torch.autograd.grad(out, leaves[:3], leaves[3], create_graph=True)
+    got = torch.autograd.grad(first, leaves, [dev["x2"], dev["y2"], dev["s2"]])
+    assert calls
+    live = ~pad
+    idx = np.asarray(module.coef.idx, dtype=np.int64)
+    val, mix = np.asarray(module.coef.val, dtype=np.float32), module._mix.mix_indices
+    args = (idx[:, :3], val, mix)
+    e = dict(snd=snd[live], rcv=rcv[live])
+    y, s, y2, s2 = y[live], s[live], y2[live], s2[live]
+    f = [H.forward_reference(*args, a, b, c, e["snd"], e["rcv"], num_z) for a, b, c in
+         ((x2, y, s), (x, y2, s), (x, y, s2))]
+    b = [H.backward_reference(*args, a, c, d, e["snd"], e["rcv"], dm) for a, c, d in
+         ((x2, y, s), (x, y2, s), (x, y, s2))]
+    g = [t.detach().cpu().numpy() for t in got]
+    pick = lambda which, grad, part: sum(b[w][part][grad] for w in which)  # noqa: E731
+    for name_, result, ref, mag in (
+            ("x", g[0], pick((1, 2), 0, 0), pick((1, 2), 0, 1)),
+            ("y", g[1][live], pick((0, 2), 1, 0), pick((0, 2), 1, 1)),
+            ("s", g[2][live], pick((0, 1), 2, 0), pick((0, 1), 2, 1)),
+            ("dm", g[3], sum(t[0] for t in f), sum(t[1] for t in f))):
+        H.assert_parity(result, ref, mag, f"{name} {kind} gradient of {name_}")
+    assert not g[1][pad].any() and not g[2][pad].any()
