@@ -125,6 +125,7 @@ SYMBOLS = {
     "e3j_amd_last_error": (ctypes.c_char_p, []),
     "e3j_amd_version": (ctypes.c_char_p, []),
     "e3j_amd_convolution_fwd": (ctypes.c_int, [_PARAMS] + [_P] * 9),
+    "e3j_amd_convolution_fwd_whole": (ctypes.c_int, [_PARAMS] + [_P] * 9),
     "e3j_amd_convolution_bwd_sender": (ctypes.c_int, [_PARAMS] + [_P] * 12),
     "e3j_amd_convolution_bwd_receiver": (ctypes.c_int, [_PARAMS] + [_P] * 12),
     "e3j_amd_convolution_bwd_ordered_workspace_bytes": (ctypes.c_size_t, [_PARAMS]),

@@ -609,7 +609,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
                 "    const int32_t *, const int32_t *, const int32_t *, float *, float *, float *, int, float,",
                 "    unsigned);"]
     out += ["}  // namespace", "", "// both passes: the device pass needs the kernels instantiated"]
-    fwd_args_trailing = [fwd_args[0], fwd_args[1].replace("unsigned);", "unsigned, int, int, const int32_t *, int);")]
+    fwd_args_trailing = [fwd_args[0], fwd_args[1].replace("unsigned);", "unsigned, int, int, int, const int32_t *, int, float *);")]
     for v in launch["fwd"]:
         cpl, wpb, zs, minw = (*v, 1)[:4]
         out += [f"template __global__ void unrolled_fwd_kernel<{channels}, {cpl}, {wpb}, {minw}, "
@@ -661,7 +661,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
 
     fwd_sig = ["(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,",
                "                   const int32_t *sender, const int32_t *row_ptr, const int32_t *perm,",
-               "                   float *out, hipStream_t stream) {"]
+               "                   float *out, hipStream_t stream, bool rows) {"]
     bwd_sig = ["(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,",
                "                   const float *dm, const int32_t *sender, const int32_t *row_ptr,",
                "                   const int32_t *perm, float *dx, float *dy, float *ds, hipStream_t stream,",
@@ -710,18 +710,20 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
     out += ["static int run_fwd" + fwd_sig[0]] + fwd_sig[1:]
     out += [ln.replace("VARIANT", "tuning().fwd_variant.load(std::memory_order_relaxed)") for ln in switch(
         launch["fwd"], lambda v: f"launch_unrolled_fwd<{channels}, {v[0]}, {v[1]}, {(*v, 1)[3]}, {part_names[v[2]]}>("
-                                 "p, x, y, s, sender, row_ptr, perm, out, stream);")]
+                                 "p, x, y, s, sender, row_ptr, perm, out, stream, rows);")]
     out += ["static int run_bwd" + bwd_sig[0]] + bwd_sig[1:]
     out += [ln.replace("VARIANT", "tuning().bwd_variant.load(std::memory_order_relaxed)") for ln in switch(
         launch["bwd"], lambda v: f"launch_unrolled_bwd<{channels}, {v[0]}, {v[1]}, {(*v, 1)[3]}, {t.Y}, {t.X}, "
                                  f"{part_names[v[2]]}>(p, x, y, s, dm, sender, row_ptr, perm, dx, dy, ds, stream, ordered);")]
     if tile:
         out += ["static int run_bwd_tiled(const e3j_amd_conv_params &p, const float *x, const float *y,",
-                "                         const float *s, const float *dm, const e3j_amd_tile_schedule &schedule,",
+                "                         const float *s, const float *dm, const int32_t *sender, const int32_t *row_ptr,",
+                "                         const int32_t *perm, const e3j_amd_tile_schedule &schedule,",
                 "                         float *dx, float *dy, float *ds, hipStream_t stream) {"]
         out += [ln.replace("VARIANT", "tuning().bwd_variant.load(std::memory_order_relaxed)") for ln in switch(
             tile, lambda v: f"launch_unrolled_bwd_tile<{channels}, {v[0]}, {v[1]}, {(*v, 1)[3]}, {t.Y}, {t.X}, "
-                            f"{part_names[v[2]]}>(p, x, y, s, dm, schedule, dx, dy, ds, stream);")]
+                            f"{part_names[v[2]]}>(p, x, y, s, dm, sender, row_ptr, perm, schedule, dx, dy, ds, "
+                            "stream);")]
         out += ["static int run_tile_row_bytes() {"]
         out += [ln.replace("VARIANT", "tuning().bwd_variant.load(std::memory_order_relaxed)") for ln in switch(
             tile, lambda v: f"tile_row_bytes<{v[0]}, {part_names[v[2]]}>();")]
@@ -735,11 +737,12 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         out += [f"    return launch_second_dm<{channels}, {cpl}, {wpb}, {minw}, {part_names[zs]}>("
                 "p, a, sender, row_ptr, perm, ddm, stream);", "}"]
         out += ["static int run_second_tile(const e3j_amd_conv_params &p, const SecondOperands &a,",
+                "                           const int32_t *sender, const int32_t *row_ptr, const int32_t *perm,",
                 "                           const e3j_amd_tile_schedule &schedule, float *dx, float *dy, float *ds,",
                 "                           hipStream_t stream) {"]
         cpl, wpb, zs, minw = second_tile
         out += [f"    return launch_second_tile<{channels}, {cpl}, {wpb}, {minw}, {t.Y}, {t.X}, {part_names[zs]}>("
-                "p, a, schedule, dx, dy, ds, stream);", "}", ""]
+                "p, a, sender, row_ptr, perm, schedule, dx, dy, ds, stream);", "}", ""]
     out += ["static int run_bwd_sender(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,",
             "                          const float *dm, const int32_t *receiver_t, const int32_t *row_ptr,",
             "                          const int32_t *perm, float *dx, float *dy, float *ds, hipStream_t stream) {",
@@ -759,7 +762,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
         out += ["static int run_fwd_leading" + fwd_sig[0]] + fwd_sig[1:]
         out += [ln.replace("VARIANT", "tuning().fwd_variant.load(std::memory_order_relaxed)") for ln in switch(
             lead["fwd"], lambda v: f"launch_unrolled_fwd_leading<{channels}, {v[0]}, {part_names[v[1]]}>("
-                                   "p, x, y, s, sender, row_ptr, perm, out, stream);")]
+                                   "p, x, y, s, sender, row_ptr, perm, out, stream, rows);")]
         out += ["static int run_bwd_leading" + bwd_sig[0]] + bwd_sig[1:]
         out += [ln.replace("VARIANT", "tuning().bwd_variant.load(std::memory_order_relaxed)") for ln in switch(
             lead["bwd"], lambda v: f"launch_unrolled_bwd_leading<{channels}, {t.Y}, {t.X}, "

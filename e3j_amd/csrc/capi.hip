@@ -177,18 +177,12 @@ int run_backward(const e3j_amd_conv_params *p, bool group_is_receiver, const voi
                                              static_cast<const double *>(s), static_cast<const double *>(dm),
                                              other, row_ptr, edge_perm, static_cast<double *>(dx),
                                              static_cast<double *>(dy), static_cast<double *>(ds), stream);
-        if (rc == E3J_AMD_OK)
-            rc = launch_zero_padding(*p, other, row_ptr, edge_perm, static_cast<double *>(dy),
-                                     static_cast<double *>(ds), stream);
     } else if (signature_fits_f16(p)) {
         if (!group_is_receiver) return f64_receiver_rows_only(op);
         rc = signature(p->signature).bwd_f16(*p, static_cast<const half_t *>(x), static_cast<const half_t *>(y),
                                              static_cast<const half_t *>(s), static_cast<const half_t *>(dm),
                                              other, row_ptr, edge_perm, static_cast<half_t *>(dx),
                                              static_cast<half_t *>(dy), static_cast<half_t *>(ds), stream);
-        if (rc == E3J_AMD_OK)
-            rc = launch_zero_padding(*p, other, row_ptr, edge_perm, static_cast<half_t *>(dy),
-                                     static_cast<half_t *>(ds), stream);
     } else if (group_is_receiver && signature_fits(p, {x, s, dm, dx, ds}) &&
         signature(p->signature).bwd != nullptr) {
         rc = signature(p->signature).bwd(*p, static_cast<const float *>(x),
@@ -196,9 +190,6 @@ int run_backward(const e3j_amd_conv_params *p, bool group_is_receiver, const voi
                                          static_cast<const float *>(dm), other, row_ptr, edge_perm,
                                          static_cast<float *>(dx), static_cast<float *>(dy),
                                          static_cast<float *>(ds), stream, nullptr);
-        if (rc == E3J_AMD_OK)
-            rc = launch_zero_padding(*p, other, row_ptr, edge_perm, static_cast<float *>(dy),
-                                     static_cast<float *>(ds), stream);
     } else if (!group_is_receiver && p->layout == E3J_AMD_LAYOUT_TRAILING && signature_fits(p, {x, s, dm, dx, ds}) &&
                signature(p->signature).bwd_sender != nullptr) {
         // the reference's grouping on the unrolled kernels: rows own their dx (no atomics)
@@ -335,13 +326,14 @@ void e3j_amd_set_launch_variant(int32_t fwd_variant, int32_t bwd_variant) {
     mutable_tuning().bwd_variant.store(bwd_variant, std::memory_order_relaxed);
 }
 
-int e3j_amd_convolution_fwd(const e3j_amd_conv_params *p, const void *coef, const void *x,
-                            const void *y, const void *s, const int32_t *sender,
-                            const int32_t *receiver_ptr, const int32_t *edge_perm, void *out,
-                            void *stream_) {
+namespace {
+// `whole`: the rows and, where listed, the pieces of long rows in one call; otherwise the pieces are
+// the second of two calls.
+int run_forward(const e3j_amd_conv_params *p, const void *coef, const void *x, const void *y, const void *s,
+                const int32_t *sender, const int32_t *receiver_ptr, const int32_t *edge_perm, void *out,
+                hipStream_t stream, bool whole) {
     int rc = validate(p, "convolution");
     if (rc) return rc;
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (p->num_nodes == 0) return E3J_AMD_OK;
     if (missing(out, p->num_nodes) || missing(x, p->num_nodes) || receiver_ptr == nullptr ||
         missing(sender, p->num_edges) || missing(y, p->num_edges) || missing(s, p->num_edges) ||
@@ -372,30 +364,22 @@ int e3j_amd_convolution_fwd(const e3j_amd_conv_params *p, const void *coef, cons
         return set_error(E3J_AMD_UNIMPLEMENTED,
                          "convolution: row_cap / segments are taken by the unrolled kernels of the "
                          "trailing layout only (16-byte aligned operands)");
-    if (signature_fits(p, {x, s, out}) && p->segments != nullptr && p->partials != nullptr) {
-        // the pieces of long rows in a fixed order: every piece sums into a scratch row of its own
-        // (the launch names the piece's number as its row), then the rows of a receiver's pieces
-        // are added to its output row one after another
-        const int64_t row_floats = (int64_t)p->num_out * p->channels;
-        if (reinterpret_cast<uintptr_t>(p->partials) % 16 != 0)
+    if (whole && p->segments != nullptr && (p->partials == nullptr || p->row_cap == 0))
+        return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution: rows and pieces in one call need row_cap and partials");
+    if (signature_fits(p, {x, s, out})) {
+        const bool fixed_order = p->segments != nullptr && p->partials != nullptr;
+        if (fixed_order && reinterpret_cast<uintptr_t>(p->partials) % 16 != 0)
             return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution: partials must be 16-byte aligned");
-        rc = launch_prepare_partials(p->segments, p->max_segments, row_floats, p->partials, stream);
-        if (rc == E3J_AMD_OK) {
-            e3j_amd_conv_params numbered = *p;
-            numbered.segments = row_partials_list(p->partials, p->max_segments, row_floats);
-            numbered.partials = nullptr;
-            rc = signature(p->signature).fwd(numbered, static_cast<const float *>(x), static_cast<const float *>(y),
-                                             static_cast<const float *>(s), sender, receiver_ptr, edge_perm,
-                                             p->partials, stream);
-        }
-        if (rc == E3J_AMD_OK)
-            rc = launch_combine_pieces(p->segments, receiver_ptr, p->max_segments,
-                                       p->row_piece > 0 ? p->row_piece : p->row_cap, row_floats, p->partials,
-                                       static_cast<float *>(out), stream);
-    } else if (signature_fits(p, {x, s, out})) {
         rc = signature(p->signature).fwd(*p, static_cast<const float *>(x), static_cast<const float *>(y),
-                                         static_cast<const float *>(s), sender, receiver_ptr,
-                                         edge_perm, static_cast<float *>(out), stream);
+                                         static_cast<const float *>(s), sender, receiver_ptr, edge_perm,
+                                         static_cast<float *>(out), stream, whole || p->segments == nullptr);
+        // pieces in a fixed order: every piece is summed into a scratch row of its own, then the rows of a
+        // receiver's pieces are added to its output row one after another
+        if (rc == E3J_AMD_OK && fixed_order)
+            rc = launch_combine_pieces(p->segments, receiver_ptr, p->max_segments,
+                                       p->row_piece > 0 ? p->row_piece : p->row_cap,
+                                       (int64_t)p->num_out * p->channels, p->partials, static_cast<float *>(out),
+                                       stream);
     } else {
         if ((rc = flip_without_kernel(p, "convolution"))) return rc;
         if (missing(coef, p->num_coef))
@@ -405,6 +389,23 @@ int e3j_amd_convolution_fwd(const e3j_amd_conv_params *p, const void *coef, cons
         rc = launch_generic_fwd(*p, coef, x, y, s, sender, receiver_ptr, edge_perm, out, stream);
     }
     return finish(p, stream, rc, "convolution");
+}
+}  // namespace
+
+int e3j_amd_convolution_fwd(const e3j_amd_conv_params *p, const void *coef, const void *x,
+                            const void *y, const void *s, const int32_t *sender,
+                            const int32_t *receiver_ptr, const int32_t *edge_perm, void *out,
+                            void *stream) {
+    return run_forward(p, coef, x, y, s, sender, receiver_ptr, edge_perm, out, static_cast<hipStream_t>(stream),
+                       false);
+}
+
+int e3j_amd_convolution_fwd_whole(const e3j_amd_conv_params *p, const void *coef, const void *x,
+                                  const void *y, const void *s, const int32_t *sender,
+                                  const int32_t *receiver_ptr, const int32_t *edge_perm, void *out,
+                                  void *stream) {
+    return run_forward(p, coef, x, y, s, sender, receiver_ptr, edge_perm, out, static_cast<hipStream_t>(stream),
+                       true);
 }
 
 int e3j_amd_convolution_bwd_sender(const e3j_amd_conv_params *p, const void *coef, const void *x,
@@ -560,11 +561,8 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
         return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": incomplete schedule");
     rc = signature(p->signature).bwd_tiled(*p, static_cast<const float *>(x), static_cast<const float *>(y),
                                            static_cast<const float *>(s), static_cast<const float *>(dm),
-                                           *schedule, static_cast<float *>(dx), static_cast<float *>(dy),
-                                           static_cast<float *>(ds), stream);
-    if (rc == E3J_AMD_OK)
-        rc = launch_zero_padding(*p, sender, receiver_ptr, edge_perm, static_cast<float *>(dy),
-                                 static_cast<float *>(ds), stream);
+                                           sender, receiver_ptr, edge_perm, *schedule, static_cast<float *>(dx),
+                                           static_cast<float *>(dy), static_cast<float *>(ds), stream);
     return finish(p, stream, rc, op);
 }
 
@@ -612,8 +610,9 @@ int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, con
         rc = launch_combine_pieces(p->segments, receiver_ptr, p->max_segments,
                                    p->row_piece > 0 ? p->row_piece : p->row_cap,
                                    (int64_t)p->num_out * p->channels, p->partials, gdm, stream);
-    if (rc == E3J_AMD_OK) rc = sg.second_tile(*p, a, *schedule, static_cast<float *>(grad_x), gy, gs, stream);
-    if (rc == E3J_AMD_OK) rc = launch_zero_padding(*p, sender, receiver_ptr, edge_perm, gy, gs, stream);
+    if (rc == E3J_AMD_OK)
+        rc = sg.second_tile(*p, a, sender, receiver_ptr, edge_perm, *schedule, static_cast<float *>(grad_x), gy, gs,
+                            stream);
     return finish(p, stream, rc, op);
 }
 

@@ -105,13 +105,17 @@ int launch_planned_bwd(const e3j_amd_conv_params &p, bool group_is_receiver, con
                        const int32_t *row_ptr, const int32_t *perm, void *dx, void *dy, void *ds,
                        hipStream_t stream);
 std::atomic<int> &table_plans();  // 1: plan the tables that can be planned (default); 0: never
-// Zero the dy/ds rows of padding edges (float32 operands).
+// Zero the dy/ds rows of padding edges (the ordered and sender-grouped backward, which own their dx).
 int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
                         const int32_t *perm, float *dy, float *ds, hipStream_t stream);
-int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
-                        const int32_t *perm, double *dy, double *ds, hipStream_t stream);
-int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
-                        const int32_t *perm, half_t *dy, half_t *ds, hipStream_t stream);
+// Before a backward that adds to dx with atomics, in one launch: dx zeroed, the dy / ds rows of padding
+// edges zeroed, and the whole of dy where several waves add to one dy row (`shared_dy`).
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, float *dx, float *dy, float *ds, bool shared_dy, hipStream_t stream);
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, double *dx, double *dy, double *ds, bool shared_dy, hipStream_t stream);
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, half_t *dx, half_t *dy, half_t *ds, bool shared_dy, hipStream_t stream);
 
 // Launch-shape variants of the unrolled kernels, from E3J_AMD_FWD_VARIANT /
 // E3J_AMD_BWD_VARIANT (read once; 0 = default).  For tuning runs.
@@ -169,14 +173,15 @@ struct Signature {
     const uint8_t *idx;    // (num_coef, 4) i, j, k, l
     int (*fwd)(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,
                const int32_t *sender, const int32_t *receiver_ptr, const int32_t *edge_perm,
-               float *out, hipStream_t stream);
+               float *out, hipStream_t stream, bool rows);  // rows off: the listed pieces alone
     int (*bwd)(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,
                const float *dm, const int32_t *sender, const int32_t *receiver_ptr,
                const int32_t *edge_perm, float *dx, float *dy, float *ds, hipStream_t stream,
                OrderedBwd *ordered);  // ordered: nullptr = dx (and shared dy) by float atomics
     // backward over tiles of receivers (nullptr: none) and the LDS bytes it needs per tile row
     int (*bwd_tiled)(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,
-                     const float *dm, const e3j_amd_tile_schedule &schedule, float *dx, float *dy,
+                     const float *dm, const int32_t *sender, const int32_t *receiver_ptr,
+                     const int32_t *edge_perm, const e3j_amd_tile_schedule &schedule, float *dx, float *dy,
                      float *ds, hipStream_t stream);
     int (*tile_row_bytes)();
     int (*tile_rows_default)();  // receivers per tile the launch variant is tuned for
@@ -208,7 +213,8 @@ struct Signature {
     // backward; nullptr: none): the gradient with respect to dm, and those with respect to x, y, s
     int (*second_dm)(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,
                      const int32_t *receiver_ptr, const int32_t *edge_perm, float *ddm, hipStream_t stream);
-    int (*second_tile)(const e3j_amd_conv_params &p, const SecondOperands &a, const e3j_amd_tile_schedule &schedule,
+    int (*second_tile)(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,
+                       const int32_t *receiver_ptr, const int32_t *edge_perm, const e3j_amd_tile_schedule &schedule,
                        float *dx, float *dy, float *ds, hipStream_t stream);
 };
 // the coefficient classes of a float64 launch, passed to the kernel by value

@@ -308,16 +308,11 @@ __global__ void generic_bwd_kernel(const Coef4D<Idx, Val> *__restrict__ coef, in
 // padding positions among them together; live graphs have few, so this is one pass over
 // the index array.
 template <typename Val>
-__global__ void zero_padding_edges_kernel(const int32_t *__restrict__ other,
-                                          const int32_t *__restrict__ row_ptr,
-                                          const int32_t *__restrict__ perm, int num_nodes,
-                                          int64_t num_edges, Val *__restrict__ dy, int num_y,
-                                          Val *__restrict__ ds, int64_t ds_row) {
-    const int lane = threadIdx.x;
+__device__ __forceinline__ void zero_padding_rows(const int32_t *other, const int32_t *row_ptr, const int32_t *perm,
+                                                  int num_nodes, int64_t num_edges, Val *dy, int num_y, Val *ds,
+                                                  int64_t ds_row, int64_t wave, int64_t waves, int lane) {
     const int64_t live_end = row_ptr[num_nodes];
-    const int64_t stride = (int64_t)gridDim.x * blockDim.y * kWave;
-    for (int64_t base = ((int64_t)blockIdx.x * blockDim.y + threadIdx.y) * kWave; base < num_edges;
-         base += stride) {
+    for (int64_t base = wave * kWave; base < num_edges; base += waves * kWave) {
         const int64_t e = base + lane;
         bool padding = false;
         if (e < num_edges) padding = e >= live_end || (unsigned)other[e] >= (unsigned)num_nodes;
@@ -331,6 +326,57 @@ __global__ void zero_padding_edges_kernel(const int32_t *__restrict__ other,
             for (int64_t t = lane; t < ds_row; t += kWave) ds[ee * ds_row + t] = Val(0);
         }
     }
+}
+
+template <typename Val>
+__global__ void zero_padding_edges_kernel(const int32_t *__restrict__ other,
+                                          const int32_t *__restrict__ row_ptr,
+                                          const int32_t *__restrict__ perm, int num_nodes,
+                                          int64_t num_edges, Val *__restrict__ dy, int num_y,
+                                          Val *__restrict__ ds, int64_t ds_row) {
+    zero_padding_rows<Val>(other, row_ptr, perm, num_nodes, num_edges, dy, num_y, ds, ds_row,
+                           (int64_t)blockIdx.x * blockDim.y + threadIdx.y, (int64_t)gridDim.x * blockDim.y,
+                           threadIdx.x);
+}
+
+// A run of bytes to clear: whole 16-byte pieces from a 16-byte aligned address on, and the two-byte
+// values before and behind them (at most 14 bytes each).
+struct ZeroRun {
+    uint16_t *head, *tail;
+    int heads, tails;
+    uint4 *body;
+    size_t pieces;
+    ZeroRun(void *ptr, size_t bytes) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(ptr);
+        const size_t before = std::min<size_t>((16 - at % 16) % 16, bytes);
+        head = static_cast<uint16_t *>(ptr);
+        heads = (int)(before / 2);
+        body = reinterpret_cast<uint4 *>(at + before);
+        pieces = (bytes - before) / 16;
+        tail = reinterpret_cast<uint16_t *>(body + pieces);
+        tails = (int)((bytes - before) % 16 / 2);
+    }
+    __device__ __forceinline__ void clear(size_t thread, size_t threads) const {
+        for (size_t i = thread; i < pieces; i += threads) body[i] = make_uint4(0u, 0u, 0u, 0u);
+        if (thread < (size_t)heads) head[thread] = 0;
+        if (thread < (size_t)tails) tail[thread] = 0;
+    }
+};
+
+// Everything a backward with atomics on dx needs cleared, in one launch (a launch of a small graph
+// costs more than its bytes: three of them, 12 us of a 16 us gap at 150k edges, became one).
+// `dy` whole where several waves add to a row (its run is then not empty and num_y is 0).
+template <typename Val>
+__global__ __launch_bounds__(256) void bwd_targets_kernel(ZeroRun dx, ZeroRun dy, const int32_t *__restrict__ other,
+                                                          const int32_t *__restrict__ row_ptr,
+                                                          const int32_t *__restrict__ perm, int num_nodes,
+                                                          int64_t num_edges, Val *__restrict__ dy_rows, int num_y,
+                                                          Val *__restrict__ ds, int64_t ds_row) {
+    const size_t thread = (size_t)blockIdx.x * blockDim.x + threadIdx.x, threads = (size_t)gridDim.x * blockDim.x;
+    dx.clear(thread, threads);
+    dy.clear(thread, threads);
+    zero_padding_rows<Val>(other, row_ptr, perm, num_nodes, num_edges, dy_rows, num_y, ds, ds_row,
+                           (int64_t)(thread / kWave), (int64_t)(threads / kWave), threadIdx.x % kWave);
 }
 
 // n_words whole words, then `tail_halves` (0 or 1) two-byte values behind them
@@ -398,6 +444,18 @@ int zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32
                        stream, other, row_ptr, perm, p.num_nodes, p.num_edges, dy, p.num_y, ds,
                        (int64_t)p.num_scalars * p.channels);
     return check_hip(hipGetLastError(), "convolution backward padding launch");
+}
+
+template <typename Val>
+int bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr, const int32_t *perm,
+                Val *dx, Val *dy, Val *ds, bool shared_dy, hipStream_t stream) {
+    const ZeroRun dx_run(dx, sizeof(Val) * (size_t)p.num_nodes * p.num_x * p.channels);
+    const ZeroRun dy_run(dy, shared_dy ? sizeof(Val) * (size_t)p.num_edges * p.num_y : 0);
+    const int64_t items = std::max<int64_t>({(int64_t)dx_run.pieces, (int64_t)dy_run.pieces, p.num_edges, 1});
+    hipLaunchKernelGGL(bwd_targets_kernel<Val>, dim3((unsigned)std::min<int64_t>((items + 255) / 256, 4096)),
+                       dim3(256), 0, stream, dx_run, dy_run, other, row_ptr, perm, p.num_nodes, p.num_edges, dy,
+                       shared_dy ? 0 : p.num_y, ds, (int64_t)p.num_scalars * p.channels);
+    return check_hip(hipGetLastError(), "convolution backward targets launch");
 }
 
 template <typename Idx, typename Val>
@@ -564,13 +622,17 @@ int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, cons
                         const int32_t *perm, float *dy, float *ds, hipStream_t stream) {
     return zero_padding<float>(p, other, row_ptr, perm, dy, ds, stream);
 }
-int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
-                        const int32_t *perm, double *dy, double *ds, hipStream_t stream) {
-    return zero_padding<double>(p, other, row_ptr, perm, dy, ds, stream);
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, float *dx, float *dy, float *ds, bool shared_dy, hipStream_t stream) {
+    return bwd_targets<float>(p, other, row_ptr, perm, dx, dy, ds, shared_dy, stream);
 }
-int launch_zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
-                        const int32_t *perm, half_t *dy, half_t *ds, hipStream_t stream) {
-    return zero_padding<half_t>(p, other, row_ptr, perm, dy, ds, stream);
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, double *dx, double *dy, double *ds, bool shared_dy, hipStream_t stream) {
+    return bwd_targets<double>(p, other, row_ptr, perm, dx, dy, ds, shared_dy, stream);
+}
+int launch_bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr,
+                       const int32_t *perm, half_t *dx, half_t *dy, half_t *ds, bool shared_dy, hipStream_t stream) {
+    return bwd_targets<half_t>(p, other, row_ptr, perm, dx, dy, ds, shared_dy, stream);
 }
 
 // The plan of a table the planned kernels can take (conv_planned.hip): in the caller's memory

@@ -1,9 +1,8 @@
 // Long rows of the forward pass, summed in a fixed order.  The pieces of a row longer than
-// row_cap are summed by waves of their own (a second launch of the forward kernel over the list of
-// pieces).  Instead of adding them to the output row with float atomics, whose order changes from
-// run to run, every piece gets a row of a scratch array (the launch names the piece's own number
-// as its "row" and adds into a zeroed row: one addition per element), and a last kernel adds the
-// rows of a receiver's pieces to its output row in the order of their positions.  No counterpart
+// row_cap are summed by waves of their own, in the launch that sums the rows.  Instead of adding them
+// to the output row with float atomics, whose order changes from run to run, every piece stores its
+// sum in a row of a scratch array, and a second kernel adds the rows of a receiver's pieces to its
+// output row in the order of their positions.  No counterpart
 // in the reference, whose forward kernel walks the edges of a receiver one after another in one
 // block (lib/e3j_ops/cuda/convolution/fwd.cuh:346-363) and is run-to-run reproducible for that
 // reason (tests/test_ops/test_convolution_op.py:322-342); this keeps that property while sharing the row.
@@ -18,23 +17,6 @@ namespace e3j_amd {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// block q: the numbered list entry of piece q and its zeroed row
-__global__ __launch_bounds__(256) void prepare_partials_kernel(const int32_t *__restrict__ segments, int max_segments,
-                                                               int64_t row_floats, float *__restrict__ partials,
-                                                               int32_t *__restrict__ list) {
-    const int count = min(segments[0], max_segments);
-    if (blockIdx.x == 0 && threadIdx.x < 4) list[threadIdx.x] = threadIdx.x == 0 ? count : 0;
-    const int q = blockIdx.x;
-    if (q >= count) return;
-    if (threadIdx.x == 0) {
-        list[4 + 3 * q] = q;
-        list[5 + 3 * q] = segments[5 + 3 * q];
-        list[6 + 3 * q] = segments[6 + 3 * q];
-    }
-    float *row = partials + (int64_t)q * row_floats;
-    for (int64_t t = threadIdx.x; t < row_floats; t += blockDim.x) row[t] = 0.f;
-}
 
 // Block (g, chunk) walks the pieces g, g + gridDim.x, ...: where a piece is the first listed piece of
 // its row, the rows of all pieces of that row are added to 64 floats of the output row.  The four
@@ -103,19 +85,7 @@ __global__ __launch_bounds__(kWave *kCombineWaves) void combine_pieces_kernel(
 
 size_t row_partials_bytes(int64_t max_segments, int64_t row_floats) {
     if (max_segments <= 0 || row_floats <= 0) return 0;
-    return sizeof(float) * (size_t)max_segments * (size_t)row_floats + sizeof(int32_t) * (4 + 3 * (size_t)max_segments);
-}
-
-int32_t *row_partials_list(float *partials, int64_t max_segments, int64_t row_floats) {
-    return reinterpret_cast<int32_t *>(partials + max_segments * row_floats);
-}
-
-int launch_prepare_partials(const int32_t *segments, int32_t max_segments, int64_t row_floats, float *partials,
-                            hipStream_t stream) {
-    if (max_segments <= 0) return E3J_AMD_OK;
-    hipLaunchKernelGGL(prepare_partials_kernel, dim3((unsigned)max_segments), dim3(256), 0, stream, segments,
-                       max_segments, row_floats, partials, row_partials_list(partials, max_segments, row_floats));
-    return check_hip(hipGetLastError(), "row pieces: prepare");
+    return sizeof(float) * (size_t)max_segments * (size_t)row_floats;
 }
 
 int launch_combine_pieces(const int32_t *segments, const int32_t *row_ptr, int32_t max_segments, int32_t row_piece,

@@ -424,6 +424,33 @@ struct FirstOfParts {
     using type = First;
 };
 
+// The work item of a wave in a launch over rows of receivers (PER items each: channel slices and
+// parts) and, in the same launch, the listed pieces of long rows.  The pieces are dealt one block
+// at a time to the fronts of the XCDs' lists (they are longer than most rows: started last they would
+// be the tail of the launch), the rows follow in contiguous eighths (see `logical_block`).
+template <int WPB, int PER>
+__device__ __forceinline__ bool row_or_piece(int num_rows, const int32_t *segments, int max_segments, int64_t &item,
+                                             bool &piece) {
+    const unsigned xcd = blockIdx.x % kXcds, t = blockIdx.x / kXcds;
+    const int64_t pieces = segments ? (int64_t)min(segments[0], max_segments) * PER : 0;
+    const int64_t piece_blocks = (pieces + WPB - 1) / WPB;
+    const int64_t mine = (piece_blocks + (kXcds - 1) - xcd) / kXcds;  // piece blocks xcd, xcd + 8, ...
+    piece = (int64_t)t < mine;
+    if (piece) {
+        item = ((int64_t)t * kXcds + xcd) * WPB + threadIdx.y;
+        return item < pieces;
+    }
+    const int64_t rows = (int64_t)num_rows * PER;
+    const int64_t per_xcd = ((rows + WPB - 1) / WPB + kXcds - 1) / kXcds;
+    const int64_t b = (int64_t)t - mine;
+    item = ((int64_t)xcd * per_xcd + b) * WPB + threadIdx.y;
+    return b < per_xcd && item < rows;
+}
+template <int WPB, int PER>
+int64_t row_or_piece_grid(int64_t num_rows, int64_t max_segments) {
+    return padded_grid((num_rows * PER + WPB - 1) / WPB) + padded_grid((max_segments * PER + WPB - 1) / WPB);
+}
+
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
@@ -536,25 +563,29 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_fwd_kernel(
     const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ s,
     const int32_t *__restrict__ sender, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ row_order,
-    float *__restrict__ out, int num_nodes, float scale, unsigned y_flip, int row_cap, int row_piece,
-    const int32_t *__restrict__ segments, int max_segments) {
-    // segments == nullptr: one item per row; a row longer than row_cap (> 0) is cut after
-    // row_piece positions.
-    // Otherwise the items are the listed pieces of long rows (count in segments[0], then
-    // (row, begin, end) from segments[4] on), whose sums are added to `out`.
+    float *__restrict__ out, int num_nodes, float scale, unsigned y_flip, int num_rows, int row_cap, int row_piece,
+    const int32_t *__restrict__ segments, int max_segments, float *__restrict__ partials) {
+    // num_rows items are rows (0: none, or all of them); a row longer than row_cap (> 0) is cut after
+    // row_piece positions.  The listed pieces of long rows (count in segments[0], then (row, begin, end)
+    // from segments[4] on) run in the same launch: the sum of piece q is stored in row q of `partials`, or,
+    // without `partials`, added to its output row.
     constexpr int NP = sizeof...(Parts);
     constexpr int CW = Slice<K, CPL>::COUNT;
-    const int64_t item = logical_block() * WPB + threadIdx.y;
-    const int rows = segments ? min(segments[0], max_segments) : num_nodes;
-    if (item >= (int64_t)rows * (CW * NP)) return;
+    int64_t item;
+    bool piece;
+    if (!row_or_piece<WPB, CW * NP>(num_rows, segments, max_segments, item, piece)) return;
     const int part = uniform((int)(item % NP));
     const int slice = uniform((int)((item / NP) % CW));
     const int q = uniform((int)(item / (NP * CW)));
     int r, e, e1;
-    if (segments) {
+    if (piece) {
         r = segments[4 + 3 * q];
         e = segments[5 + 3 * q];
         e1 = segments[6 + 3 * q];
+        if (partials != nullptr) {
+            r = q;
+            out = partials;
+        }
     } else {
         r = row_order ? row_order[q] : q;
         e = row_ptr[r];
@@ -563,7 +594,7 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_fwd_kernel(
     }
     dispatch_fwd<K, CPL, 0, Parts...>(part, x, y, s, sender, row_ptr, perm, out, num_nodes, scale, y_flip,
                                       uniform(r), slice, threadIdx.x, uniform(e), uniform(e1),
-                                      segments != nullptr);
+                                      piece && partials == nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1605,26 +1636,28 @@ void unrolled_bwd_leading_kernel(
         threadIdx.x, threadIdx.y * kWave + threadIdx.x, region);
 }
 
+// `rows` off: the listed pieces alone, of a pass whose rows an earlier call summed.
 template <int K, int CPL, int WPB, int MINW, typename... Parts>
 int launch_unrolled_fwd(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,
                         const int32_t *sender, const int32_t *row_ptr, const int32_t *perm,
-                        float *out, hipStream_t stream) {
-    constexpr int64_t PER_NODE = (int64_t)Slice<K, CPL>::COUNT * sizeof...(Parts);
-    const int64_t items = p.segments ? (int64_t)p.max_segments : (int64_t)p.num_nodes;
-    const int64_t blocks = padded_grid((items * PER_NODE + WPB - 1) / WPB);
+                        float *out, hipStream_t stream, bool rows) {
+    constexpr int PER_NODE = Slice<K, CPL>::COUNT * (int)sizeof...(Parts);
+    const int num_rows = rows ? p.num_nodes : 0;
+    const int64_t blocks = row_or_piece_grid<WPB, PER_NODE>(num_rows, p.segments ? p.max_segments : 0);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution: grid too large");
     if (blocks == 0) return E3J_AMD_OK;
     hipLaunchKernelGGL((unrolled_fwd_kernel<K, CPL, WPB, MINW, Parts...>), dim3((unsigned)blocks),
                        dim3(kWave, WPB), 0, stream, x, y, s, sender, row_ptr, perm, p.row_order, out,
-                       p.num_nodes, p.coef_scale, p.y_flip, p.row_cap,
-                       p.row_piece > 0 ? p.row_piece : p.row_cap, p.segments, p.max_segments);
+                       p.num_nodes, p.coef_scale, p.y_flip, num_rows, p.row_cap,
+                       p.row_piece > 0 ? p.row_piece : p.row_cap, p.segments, p.max_segments, p.partials);
     return check_hip(hipGetLastError(), "convolution forward launch");
 }
 
 // Where the backward kernels put dx and dy: float atomics into zero-filled results, or (ordered)
 // the per-position buffers behind `ordered`, which is then told what the variant produced.
-template <int X, int Y, int SLOTS, unsigned long long COVERED>
-int prepare_bwd_targets(const e3j_amd_conv_params &p, OrderedBwd *ordered, int K, float *&dx, float *&dy,
+template <int SLOTS, unsigned long long COVERED>
+int prepare_bwd_targets(const e3j_amd_conv_params &p, OrderedBwd *ordered, const int32_t *sender,
+                        const int32_t *row_ptr, const int32_t *perm, float *&dx, float *&dy, float *ds,
                         hipStream_t stream) {
     static_assert(SLOTS <= kMaxDySlots, "more waves per edge than dy slots");
     if (ordered != nullptr) {
@@ -1634,9 +1667,7 @@ int prepare_bwd_targets(const e3j_amd_conv_params &p, OrderedBwd *ordered, int K
         if (SLOTS > 1) dy = ordered->dy_slots;
         return E3J_AMD_OK;
     }
-    int rc = launch_fill_zero(dx, sizeof(float) * (size_t)p.num_nodes * X * K, stream);
-    if (rc == E3J_AMD_OK && SLOTS > 1) rc = launch_fill_zero(dy, sizeof(float) * (size_t)p.num_edges * Y, stream);
-    return rc;
+    return launch_bwd_targets(p, sender, row_ptr, perm, dx, dy, ds, SLOTS > 1, stream);
 }
 
 template <int K, int CPL, int WPB, int MINW, int Y, int X, typename... Parts>
@@ -1646,7 +1677,7 @@ int launch_unrolled_bwd(const e3j_amd_conv_params &p, const float *x, const floa
                         OrderedBwd *ordered) {
     constexpr int64_t PER_NODE = (int64_t)Slice<K, CPL>::COUNT * sizeof...(Parts);
     constexpr unsigned long long kCovered = (Parts::kDxMask | ...);
-    int rc = prepare_bwd_targets<X, Y, (int)PER_NODE, kCovered>(p, ordered, K, dx, dy, stream);
+    int rc = prepare_bwd_targets<(int)PER_NODE, kCovered>(p, ordered, sender, row_ptr, perm, dx, dy, ds, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid(((int64_t)p.num_nodes * PER_NODE + WPB - 1) / WPB);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd: grid too large");
@@ -1694,7 +1725,8 @@ constexpr int tile_row_bytes() {
 
 template <int K, int CPL, int WPB, int MINW, int Y, int X, typename... Parts>
 int launch_unrolled_bwd_tile(const e3j_amd_conv_params &p, const float *x, const float *y, const float *s,
-                             const float *dm, const e3j_amd_tile_schedule &sch, float *dx, float *dy,
+                             const float *dm, const int32_t *sender, const int32_t *row_ptr,
+                             const int32_t *perm, const e3j_amd_tile_schedule &sch, float *dx, float *dy,
                              float *ds, hipStream_t stream) {
     constexpr int64_t PER_WORK = (int64_t)Slice<K, CPL>::COUNT * sizeof...(Parts);
     constexpr unsigned long long kCovered = (Parts::kDxMask | ...);
@@ -1703,7 +1735,7 @@ int launch_unrolled_bwd_tile(const e3j_amd_conv_params &p, const float *x, const
         return set_error(E3J_AMD_INVALID_ARGUMENT,
                          "convolution_bwd_tiled: the schedule's tiles hold more receivers than fit the LDS "
                          "(e3j_amd_tile_rows gives the limit)");
-    int rc = prepare_bwd_targets<X, Y, (int)PER_WORK, kCovered>(p, nullptr, K, dx, dy, stream);
+    int rc = prepare_bwd_targets<(int)PER_WORK, kCovered>(p, nullptr, sender, row_ptr, perm, dx, dy, ds, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid((int64_t)sch.num_work * PER_WORK);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd_tiled: grid too large");
@@ -1722,7 +1754,7 @@ int launch_unrolled_bwd_tile(const e3j_amd_conv_params &p, const float *x, const
 template <int K, int WPB, typename Part>
 int launch_unrolled_fwd_leading(const e3j_amd_conv_params &p, const float *x, const float *y,
                                 const float *s, const int32_t *sender, const int32_t *row_ptr,
-                                const int32_t *perm, float *out, hipStream_t stream) {
+                                const int32_t *perm, float *out, hipStream_t stream, bool) {
     using G = LeadingGeometry<K, Part::X, Part::S, Part::Z>;
     const int64_t blocks = padded_grid(((int64_t)p.num_nodes * G::COUNT + WPB - 1) / WPB);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution: grid too large");
@@ -1741,7 +1773,7 @@ int launch_unrolled_bwd_leading(const e3j_amd_conv_params &p, const float *x, co
     constexpr int NP = sizeof...(Parts);
     using G = LeadingBwdGeometry<K, P0::X, P0::S, P0::Z, NP>;
     constexpr unsigned long long kCovered = (Parts::kDxMask | ...);
-    int rc = prepare_bwd_targets<X, Y, G::COUNT * NP, kCovered>(p, ordered, K, dx, dy, stream);
+    int rc = prepare_bwd_targets<G::COUNT * NP, kCovered>(p, ordered, sender, row_ptr, perm, dx, dy, ds, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid((int64_t)p.num_nodes * G::COUNT);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd: grid too large");

@@ -357,8 +357,7 @@ int launch_unrolled_bwd_f16(const e3j_amd_conv_params &p, const half_t *x, const
     if (CPL > 1 && (reinterpret_cast<uintptr_t>(x) % 4 != 0 || reinterpret_cast<uintptr_t>(s) % 4 != 0 ||
                     reinterpret_cast<uintptr_t>(dm) % 4 != 0 || reinterpret_cast<uintptr_t>(ds) % 4 != 0))
         return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd: float16 operands must be 4-byte aligned");
-    int rc = launch_fill_zero(dx, sizeof(half_t) * (size_t)p.num_nodes * X * K, stream);
-    if (rc == E3J_AMD_OK && PER_NODE > 1) rc = launch_fill_zero(dy, sizeof(half_t) * (size_t)p.num_edges * Y, stream);
+    int rc = launch_bwd_targets(p, sender, row_ptr, perm, dx, dy, ds, PER_NODE > 1, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid(((int64_t)p.num_nodes * PER_NODE + WPB - 1) / WPB);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd: grid too large");

@@ -305,8 +305,7 @@ int launch_unrolled_bwd_f64(const e3j_amd_conv_params &p, const double *x, const
     int rc = f64_coefs(p, &coefs, "convolution_bwd");
     if (rc) return rc;
     constexpr int64_t PER_NODE = (int64_t)(K / kWave) * sizeof...(Parts);
-    rc = launch_fill_zero(dx, sizeof(double) * (size_t)p.num_nodes * X * K, stream);
-    if (rc == E3J_AMD_OK && PER_NODE > 1) rc = launch_fill_zero(dy, sizeof(double) * (size_t)p.num_edges * Y, stream);
+    rc = launch_bwd_targets(p, sender, row_ptr, perm, dx, dy, ds, PER_NODE > 1, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid(((int64_t)p.num_nodes * PER_NODE + WPB - 1) / WPB);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd: grid too large");

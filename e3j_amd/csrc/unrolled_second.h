@@ -27,33 +27,6 @@
 
 namespace e3j_amd {
 
-// The work item of a wave in a launch over rows of receivers (PER items each: channel slices and
-// parts) and, in the same launch, the listed pieces of long rows.  The pieces are dealt one block
-// at a time to the fronts of the XCDs' lists (they are longer than most rows: started last they would
-// be the tail of the launch), the rows follow in contiguous eighths (see `logical_block`).
-template <int WPB, int PER>
-__device__ __forceinline__ bool row_or_piece(int num_nodes, const int32_t *segments, int max_segments, int64_t &item,
-                                             bool &piece) {
-    const unsigned xcd = blockIdx.x % kXcds, t = blockIdx.x / kXcds;
-    const int64_t pieces = segments ? (int64_t)min(segments[0], max_segments) * PER : 0;
-    const int64_t piece_blocks = (pieces + WPB - 1) / WPB;
-    const int64_t mine = (piece_blocks + (kXcds - 1) - xcd) / kXcds;  // piece blocks xcd, xcd + 8, ...
-    piece = (int64_t)t < mine;
-    if (piece) {
-        item = ((int64_t)t * kXcds + xcd) * WPB + threadIdx.y;
-        return item < pieces;
-    }
-    const int64_t rows = (int64_t)num_nodes * PER;
-    const int64_t per_xcd = ((rows + WPB - 1) / WPB + kXcds - 1) / kXcds;
-    const int64_t b = (int64_t)t - mine;
-    item = ((int64_t)xcd * per_xcd + b) * WPB + threadIdx.y;
-    return b < per_xcd && item < rows;
-}
-template <int WPB, int PER>
-int64_t row_or_piece_grid(int64_t num_nodes, int64_t max_segments) {
-    return padded_grid((num_nodes * PER + WPB - 1) / WPB) + padded_grid((max_segments * PER + WPB - 1) / WPB);
-}
-
 // ---------------------------------------------------------------------------
 // gradient with respect to dm: rows of receivers, as the forward pass
 // ---------------------------------------------------------------------------
@@ -380,17 +353,16 @@ int launch_second_dm(const e3j_amd_conv_params &p, const SecondOperands &a, cons
 }
 
 template <int K, int CPL, int WPB, int MINW, int Y, int X, typename... Parts>
-int launch_second_tile(const e3j_amd_conv_params &p, const SecondOperands &a, const e3j_amd_tile_schedule &sch,
-                       float *dx, float *dy, float *ds, hipStream_t stream) {
+int launch_second_tile(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,
+                       const int32_t *row_ptr, const int32_t *perm, const e3j_amd_tile_schedule &sch, float *dx,
+                       float *dy, float *ds, hipStream_t stream) {
     constexpr int64_t PER_WORK = (int64_t)Slice<K, CPL>::COUNT * sizeof...(Parts);
     const size_t lds = (size_t)tile_row_bytes<CPL, Parts...>() * (size_t)sch.tile_rows;
     if (sch.tile_rows < 1 || lds > kMaxTileLds)
         return set_error(E3J_AMD_INVALID_ARGUMENT,
                          "convolution_bwd_bwd: the schedule's tiles hold more receivers than fit the LDS "
                          "(e3j_amd_tile_rows gives the limit)");
-    int rc = launch_fill_zero(dx, sizeof(float) * (size_t)p.num_nodes * X * K, stream);
-    if (rc == E3J_AMD_OK && PER_WORK > 1)
-        rc = launch_fill_zero(dy, sizeof(float) * (size_t)p.num_edges * Y, stream);
+    int rc = launch_bwd_targets(p, sender, row_ptr, perm, dx, dy, ds, PER_WORK > 1, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid((int64_t)sch.num_work * PER_WORK);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "convolution_bwd_bwd: grid too large");

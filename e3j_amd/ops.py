@@ -426,10 +426,11 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
         out = torch.empty((x.shape[0], meta.params.num_out, x.shape[2]), dtype=x.dtype, device=x.device)
     else:
         out = torch.empty((x.shape[0], x.shape[1], meta.params.num_out), dtype=x.dtype, device=x.device)
-    # Rows much longer than the mean are shared between waves: the first call cuts every row at
-    # `cap` positions, a second call sums the remaining pieces, each into a scratch row, and adds
-    # them to their output rows in a fixed order (unrolled kernels of the trailing layout): the
-    # result is the same bits in every run, as for a row that one wave sums
+    # Rows much longer than the mean are shared between waves: a row's own wave stops after
+    # `row_piece` positions, the pieces listed for the rest are summed in the same launch, each into
+    # a scratch row, and a second kernel adds them to their output rows in a fixed order (unrolled
+    # kernels of the trailing layout): the result is the same bits in every run, as for a row that
+    # one wave sums.  Without the fixed order a second call adds the pieces with float atomics.
     cap = 0
     fixed_order = bool(config().fixed_order_rows)
     if (p.signature >= 0 and meta.layout == Layout.TRAILING_CHANNELS and x.dtype == torch.float32
@@ -449,12 +450,15 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
             row_floats = int(out.shape[1]) * int(out.shape[2])
             pieces = graph.segments(cap, row_piece_for(int(y.shape[0]), row_floats) if fixed_order else ROW_PIECE)
             p.row_cap, p.row_piece = pieces.row_cap, pieces.row_piece
-        _lib.check(lib.e3j_amd_convolution_fwd(ctypes.byref(p), *args))
-        if pieces is not None and pieces.count > 0:
+        if pieces is not None and pieces.count > 0 and fixed_order:
             p.segments, p.max_segments = pieces.buffer.data_ptr(), pieces.count
-            if fixed_order:
-                p.partials = pieces.partials(int(out.shape[1]), int(out.shape[2])).data_ptr()
+            p.partials = pieces.partials(int(out.shape[1]), int(out.shape[2])).data_ptr()
+            _lib.check(lib.e3j_amd_convolution_fwd_whole(ctypes.byref(p), *args))
+        else:
             _lib.check(lib.e3j_amd_convolution_fwd(ctypes.byref(p), *args))
+            if pieces is not None and pieces.count > 0:
+                p.segments, p.max_segments = pieces.buffer.data_ptr(), pieces.count
+                _lib.check(lib.e3j_amd_convolution_fwd(ctypes.byref(p), *args))
     return out
 
 

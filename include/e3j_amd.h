@@ -138,6 +138,14 @@ int e3j_amd_convolution_fwd(const e3j_amd_conv_params *p, const void *coef,
                             const int32_t *sender, const int32_t *receiver_ptr,
                             const int32_t *edge_perm, void *out, void *stream);
 
+/* The same, rows and pieces of long rows in one launch: with p->segments (which then needs row_cap
+ * and partials, else E3J_AMD_INVALID_ARGUMENT) the call does what two calls of
+ * e3j_amd_convolution_fwd do, the first without and the second with `segments` and `partials`. */
+int e3j_amd_convolution_fwd_whole(const e3j_amd_conv_params *p, const void *coef,
+                                  const void *x, const void *y, const void *s,
+                                  const int32_t *sender, const int32_t *receiver_ptr,
+                                  const int32_t *edge_perm, void *out, void *stream);
+
 /* Backward, operands of the reference: replaces the "convolution_bwd" target
  * (lib/e3j_ops/ffi/e3j_ops.h:478-594; kernel lib/e3j_ops/cuda/convolution/bwd.cuh:116-321).
  * CSR grouped by SENDER (the transposed adjacency): receiver_t = receiver per
