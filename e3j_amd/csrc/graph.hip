@@ -57,7 +57,8 @@ constexpr int kLabelRowCap = 128;
 constexpr int kLabelLanes = 4;  // lanes that share a row (its gathers then run four at a time)
 __global__ void min_label_kernel(const int32_t *__restrict__ other,
                                  const int32_t *__restrict__ row_ptr, int num_nodes,
-                                 const int32_t *__restrict__ cur, int32_t *__restrict__ next) {
+                                 const int32_t *__restrict__ cur, int32_t *__restrict__ next,
+                                 uint32_t *__restrict__ keys, int32_t *__restrict__ vals, int bits) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int n = t / kLabelLanes, part = t % kLabelLanes;
     const bool inside = n < num_nodes;  // (no early exit: the lanes of a group exchange below)
@@ -73,18 +74,15 @@ __global__ void min_label_kernel(const int32_t *__restrict__ other,
     }
 #pragma unroll
     for (int off = 1; off < kLabelLanes; off *= 2) best = min(best, __shfl_xor(best, off, kWave));
-    if (inside && part == 0) next[n] = best;
-}
-
-// key = (label after the second sweep, label after the first): one sort lists the coarse clusters
-// and, inside them, the fine ones
-__global__ void two_level_keys_kernel(const int32_t *__restrict__ coarse, const int32_t *__restrict__ fine,
-                                      int num_nodes, int bits, uint32_t *__restrict__ keys,
-                                      int32_t *__restrict__ vals) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= num_nodes) return;
-    keys[i] = ((uint32_t)coarse[i] << bits) | (uint32_t)fine[i];
-    vals[i] = i;
+    if (!inside || part != 0) return;
+    if (keys == nullptr) {
+        next[n] = best;
+    } else {
+        // the last of two sweeps: key = (label after it, label before it); one sort lists the coarse
+        // clusters and, inside them, the fine ones
+        keys[n] = ((uint32_t)best << bits) | (uint32_t)cur[n];
+        if (vals != nullptr) vals[n] = n;
+    }
 }
 
 __global__ void copy_i32_kernel(const int32_t *__restrict__ src, int32_t *__restrict__ dst, int64_t n) {
@@ -92,14 +90,38 @@ __global__ void copy_i32_kernel(const int32_t *__restrict__ src, int32_t *__rest
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = src[i];
 }
 
+// Pieces of the rows longer than `cap`, past their first `piece` positions: a row reserves its
+// pieces with one atomic on the count (the order of the rows in the list is free).
+__device__ __forceinline__ void list_row_pieces(int r, int begin, int end, int cap, int piece, int max_segments,
+                                                int32_t *__restrict__ segments) {
+    if (end - begin <= cap) return;
+    const int extra = (end - begin - 1) / piece;  // pieces after the first
+    const int at = atomicAdd(segments, extra);
+    for (int k = 0; k < extra && at + k < max_segments; k++) {
+        const int b = begin + (k + 1) * piece;
+        int32_t *seg = segments + 4 + 3 * (at + k);
+        seg[0] = r;
+        seg[1] = b;
+        seg[2] = b + piece < end ? b + piece : end;
+    }
+}
+
+__global__ void row_segments_kernel(const int32_t *__restrict__ row_ptr, int num_nodes, int cap, int piece,
+                                    int max_segments, int32_t *__restrict__ segments) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= num_nodes) return;
+    list_row_pieces(r, row_ptr[r], row_ptr[r + 1], cap, piece, max_segments, segments);
+}
+
 // Rows with more than twice the mean number of edges ("long rows"): flag per list position.
 __global__ void long_row_flags_kernel(const int32_t *__restrict__ order, const int32_t *__restrict__ row_ptr,
-                                      int num_nodes, int32_t *__restrict__ flags) {
+                                      int num_nodes, int32_t *__restrict__ flags, int row_cap, int row_piece,
+                                      int max_segments, int32_t *__restrict__ segments) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= num_nodes) return;
-    const int r = order[i];
-    const int64_t degree = row_ptr[r + 1] - row_ptr[r];
-    flags[i] = degree * num_nodes > 2 * (int64_t)row_ptr[num_nodes] ? 1 : 0;
+    const int r = order[i], begin = row_ptr[r], end = row_ptr[r + 1];
+    flags[i] = (int64_t)(end - begin) * num_nodes > 2 * (int64_t)row_ptr[num_nodes] ? 1 : 0;
+    if (segments != nullptr) list_row_pieces(r, begin, end, row_cap, row_piece, max_segments, segments);
 }
 
 // The kernels hand one contiguous eighth of the row list to each XCD and every XCD walks its
@@ -107,23 +129,76 @@ __global__ void long_row_flags_kernel(const int32_t *__restrict__ order, const i
 // the end, so they are dealt to the fronts of the eighths: eighth p takes the p-th eighth of the
 // long rows, then the p-th eighth of the others, both in list order.  `rank` is the
 // inclusive prefix sum of `flags`.  Without long rows the list is unchanged.
+constexpr int64_t kDealParts = 8;
+// `rank`: inclusive number of long rows up to list position i
+__device__ __forceinline__ int64_t dealt_position(int i, bool is_long, int64_t rank, int64_t num_long, int num_nodes) {
+    const int64_t num_short = num_nodes - num_long;
+    const int64_t mine = is_long ? rank - 1 : i - rank;  // position among the rows of its kind
+    const int64_t kind = is_long ? num_long : num_short;
+    int64_t part = 0;
+    while (part < kDealParts - 1 && (part + 1) * kind / kDealParts <= mine) part++;
+    const int64_t start = part * num_long / kDealParts + part * num_short / kDealParts;
+    const int64_t longs_here = (part + 1) * num_long / kDealParts - part * num_long / kDealParts;
+    return is_long ? start + (mine - part * num_long / kDealParts)
+                   : start + longs_here + (mine - part * num_short / kDealParts);
+}
 __global__ void deal_long_rows_kernel(const int32_t *__restrict__ order, const int32_t *__restrict__ flags,
                                       const int32_t *__restrict__ rank, int num_nodes,
                                       int32_t *__restrict__ dealt) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= num_nodes) return;
-    constexpr int64_t kParts = 8;
-    const int64_t num_long = rank[num_nodes - 1], num_short = num_nodes - num_long;
-    const bool is_long = flags[i] != 0;
-    const int64_t mine = is_long ? rank[i] - 1 : i - rank[i];  // position among the rows of its kind
-    const int64_t kind = is_long ? num_long : num_short;
-    int64_t part = 0;
-    while (part < kParts - 1 && (part + 1) * kind / kParts <= mine) part++;
-    const int64_t start = part * num_long / kParts + part * num_short / kParts;
-    const int64_t longs_here = (part + 1) * num_long / kParts - part * num_long / kParts;
-    const int64_t at = is_long ? start + (mine - part * num_long / kParts)
-                               : start + longs_here + (mine - part * num_short / kParts);
-    dealt[at] = order[i];
+    dealt[dealt_position(i, flags[i] != 0, rank[i], rank[num_nodes - 1], num_nodes)] = order[i];
+}
+
+// The end of the row order for up to kBlockThreads * ITEMS rows, by one workgroup: the sort of the
+// keys, the deal of the long rows and, with `segments`, the list of their pieces.  Nine launches of
+// the general path (sort 4-6, flags, scan 2, deal) in one: each of those takes 3-5 us here whatever
+// it moves.  5 000 rows: 32 -> 15 us.
+constexpr int kBlockThreads = 1024;
+template <int ITEMS>
+__global__ __launch_bounds__(kBlockThreads) void order_block_kernel(const uint32_t *__restrict__ keys,
+                                                                    const int32_t *__restrict__ row_ptr,
+                                                                    int num_nodes, int key_bits,
+                                                                    int32_t *__restrict__ order, int row_cap,
+                                                                    int row_piece, int max_segments,
+                                                                    int32_t *__restrict__ segments) {
+    using Sort = hipcub::BlockRadixSort<uint32_t, kBlockThreads, ITEMS, int32_t>;
+    using Scan = hipcub::BlockScan<int, kBlockThreads>;
+    __shared__ union {
+        typename Sort::TempStorage sort;
+        typename Scan::TempStorage scan;
+    } temp;
+    uint32_t key[ITEMS];
+    int32_t row[ITEMS];
+    const int first = (int)threadIdx.x * ITEMS;
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++) {
+        // (the sort is stable: the entries past the last row stay behind every row of the same key)
+        key[k] = first + k < num_nodes ? keys[first + k] : ~0u;
+        row[k] = first + k < num_nodes ? first + k : 0;
+    }
+    Sort(temp.sort).Sort(key, row, 0, key_bits);
+    __syncthreads();
+    const int64_t live = row_ptr[num_nodes];
+    int begin[ITEMS], end[ITEMS], flag[ITEMS], rank[ITEMS], num_long;
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++) {
+        begin[k] = row_ptr[row[k]];
+        end[k] = row_ptr[row[k] + 1];
+    }
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++)
+        flag[k] = first + k < num_nodes && (int64_t)(end[k] - begin[k]) * num_nodes > 2 * live ? 1 : 0;
+    Scan(temp.scan).InclusiveSum(flag, rank, num_long);
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++) {
+        if (first + k >= num_nodes) continue;
+        const int64_t at = num_long == 0 ? first + k : dealt_position(first + k, flag[k] != 0, rank[k], num_long,
+                                                                      num_nodes);
+        order[at] = row[k];
+        if (segments != nullptr)
+            list_row_pieces(row[k], begin[k], end[k], row_cap, row_piece, max_segments, segments);
+    }
 }
 
 size_t align_up(size_t v, size_t a = 256) { return (v + a - 1) / a * a; }
@@ -160,17 +235,156 @@ int row_ptr_impl(const int32_t *key, int64_t num_edges, int32_t num_nodes, int32
 }
 
 // Global node ids of a sharded graph reduced to shard-local ids; the sentinel stays.
+__device__ __forceinline__ int32_t wrap_node(int32_t v, int32_t num_nodes) {
+    if ((uint32_t)v < (uint32_t)num_nodes || v == INT32_MAX) return v;
+    const int32_t r = v % num_nodes;  // Python semantics: the result takes the divisor's sign
+    return r < 0 ? r + num_nodes : r;
+}
 __global__ void wrap_index_kernel(const int32_t *__restrict__ index, int64_t n, int32_t num_nodes,
                                   int32_t *__restrict__ out) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int32_t v = index[i];
-        int32_t r = v;
-        if (v != INT32_MAX) {
-            r = v % num_nodes;          // Python semantics: the result takes the divisor's sign
-            if (r < 0) r += num_nodes;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
+        out[i] = wrap_node(index[i], num_nodes);
+}
+
+// ---- rows of an adjacency from its endpoints, in few launches -----------------------------------
+// With the keys in order, row_ptr[r] is the position of the first key >= r: every thread compares a key
+// with the one before it and writes the rows that begin there.  No counters to clear, no atomics, no
+// scan: one launch in the place of six (two index reductions, clear, count, two of the scan).  Keys
+// out of order are noticed on the way; the counts are then made by one workgroup (as the
+// count / scan path makes them), a launch that otherwise returns at once.
+
+// rows first .. last of row_ptr = value for every lane of the wave (none where last < first); the
+// lanes with a single row write it themselves, longer runs (rows without edges) are written by the wave
+__device__ __forceinline__ void fill_rows(int32_t *row_ptr, int first, int last, int value, int lane) {
+    if (first == last) row_ptr[first] = value;
+    unsigned long long runs = __ballot(last > first);
+    while (runs) {
+        const int src = __ffsll(runs) - 1;
+        runs &= runs - 1;
+        const int f = __shfl(first, src, kWave), l = __shfl(last, src, kWave), v = __shfl(value, src, kWave);
+        for (int r = f + lane; r <= l; r += kWave) row_ptr[r] = v;
+    }
+}
+
+// positions wave * 64 .. of every waves * 64; `perm`: other[perm[pos]] belongs to pos, and the keys are
+// those of `sort_input_kernel` (padding: num_nodes).
+// Returns whether a key of this thread was smaller than the one before it.
+__device__ __forceinline__ bool rows_from_keys(const int32_t *key, const int32_t *other, const int32_t *perm,
+                                               int64_t num_edges, int num_nodes, int32_t *other_out,
+                                               int32_t *row_ptr, int64_t wave, int64_t waves, int lane) {
+    bool unsorted = false;
+    for (int64_t base = wave * kWave; base < num_edges; base += waves * kWave) {
+        const int64_t e = base + lane;
+        int first = 1, last = 0, past_first = 1, past_last = 0;
+        if (e < num_edges) {
+            other_out[e] = wrap_node(other[perm ? perm[e] : e], num_nodes);
+            int k = key[e], before = e > 0 ? key[e - 1] : -1;
+            if (perm == nullptr) {  // (sorted keys were reduced before the sort)
+                k = wrap_node(k, num_nodes);
+                if (e > 0) before = wrap_node(before, num_nodes);
+            }
+            unsorted |= k < before;
+            first = min(before, num_nodes) + 1;
+            last = min(k, num_nodes);
+            if (e == num_edges - 1 && k < num_nodes) {
+                past_first = k + 1;
+                past_last = num_nodes;
+            }
         }
-        out[i] = r;
+        fill_rows(row_ptr, first, last, (int)e, lane);
+        fill_rows(row_ptr, past_first, past_last, (int)num_edges, lane);
+    }
+    return unsorted;
+}
+
+// row_ptr = [0] + cumsum(bincount(key)) of keys in any order, by one workgroup of kBlockThreads
+__device__ __forceinline__ void rows_by_count(const int32_t *key, int64_t num_edges, int num_nodes,
+                                              int32_t *row_ptr) {
+    __shared__ int sums[kBlockThreads];
+    const int tid = threadIdx.x;
+    auto read = [&](int64_t i) { return __hip_atomic_load(row_ptr + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+    auto write = [&](int64_t i, int v) {
+        __hip_atomic_store(row_ptr + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    for (int64_t i = tid; i <= num_nodes; i += kBlockThreads) write(i, 0);
+    __threadfence();
+    __syncthreads();
+    for (int64_t e = tid; e < num_edges; e += kBlockThreads) {
+        const int k = wrap_node(key[e], num_nodes);
+        if ((unsigned)k < (unsigned)num_nodes) atomicAdd(row_ptr + k + 1, 1);
+    }
+    __threadfence();
+    __syncthreads();
+    const int64_t each = ((int64_t)num_nodes + kBlockThreads) / kBlockThreads;  // of num_nodes + 1 entries
+    const int64_t from = min((int64_t)tid * each, (int64_t)num_nodes + 1);
+    const int64_t to = min(from + each, (int64_t)num_nodes + 1);
+    int sum = 0;
+    for (int64_t i = from; i < to; i++) sum += read(i);
+    sums[tid] = sum;
+    __syncthreads();
+    for (int off = 1; off < kBlockThreads; off *= 2) {
+        const int add = tid >= off ? sums[tid - off] : 0;
+        __syncthreads();
+        sums[tid] += add;
+        __syncthreads();
+    }
+    int running = sums[tid] - sum;
+    for (int64_t i = from; i < to; i++) {
+        running += read(i);
+        write(i, running);
+    }
+}
+
+constexpr int kMaxRowsBlocks = 1024;
+// `unsorted` (one word per block; null: the keys are known to be in order)
+__global__ __launch_bounds__(256) void rows_kernel(const int32_t *__restrict__ key, const int32_t *__restrict__ other,
+                                                   const int32_t *__restrict__ perm, int64_t num_edges, int num_nodes,
+                                                   int32_t *__restrict__ other_out, int32_t *__restrict__ row_ptr,
+                                                   int32_t *__restrict__ unsorted, int32_t *__restrict__ segments) {
+    if (segments != nullptr && blockIdx.x == 0 && threadIdx.x < 4) segments[threadIdx.x] = 0;
+    const int64_t thread = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool mine = rows_from_keys(key, other, perm, num_edges, num_nodes, other_out, row_ptr, thread / kWave,
+                                     (int64_t)gridDim.x * blockDim.x / kWave, threadIdx.x % kWave);
+    if (unsorted == nullptr) return;
+    const int any = __syncthreads_or(mine ? 1 : 0);
+    if (threadIdx.x == 0) unsorted[blockIdx.x] = any;
+}
+__global__ __launch_bounds__(kBlockThreads) void recount_rows_kernel(const int32_t *__restrict__ key,
+                                                                     int64_t num_edges, int num_nodes,
+                                                                     const int32_t *__restrict__ unsorted, int blocks,
+                                                                     int32_t *__restrict__ row_ptr) {
+    if (!__syncthreads_or((int)threadIdx.x < blocks && unsorted[threadIdx.x] != 0)) return;
+    rows_by_count(key, num_edges, num_nodes, row_ptr);
+}
+// both, and the pieces of long rows, for graphs whose edges one workgroup reads in a few microseconds
+constexpr int64_t kRowsBlockEdges = 16384;
+__global__ __launch_bounds__(kBlockThreads) void rows_block_kernel(const int32_t *__restrict__ key,
+                                                                   const int32_t *__restrict__ other,
+                                                                   int64_t num_edges, int num_nodes,
+                                                                   int32_t *__restrict__ other_out, int32_t *row_ptr,
+                                                                   bool list_pieces, int row_cap, int row_piece,
+                                                                   int max_segments, int32_t *segments) {
+    if (segments != nullptr && threadIdx.x < 4) segments[threadIdx.x] = 0;
+    const bool mine = rows_from_keys(key, other, nullptr, num_edges, num_nodes, other_out, row_ptr,
+                                     threadIdx.x / kWave, kBlockThreads / kWave, threadIdx.x % kWave);
+    if (__syncthreads_or(mine ? 1 : 0)) rows_by_count(key, num_edges, num_nodes, row_ptr);
+    if (!list_pieces || segments == nullptr) return;
+    __threadfence();
+    __syncthreads();
+    for (int r = threadIdx.x; r < num_nodes; r += kBlockThreads) {
+        const int begin = __hip_atomic_load(row_ptr + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int end = __hip_atomic_load(row_ptr + r + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        list_row_pieces(r, begin, end, row_cap, row_piece, max_segments, segments);
+    }
+}
+// keys to sort by (padding: num_nodes, behind every row) and the positions they come from
+__global__ void sort_input_kernel(const int32_t *__restrict__ key, int64_t num_edges, int num_nodes,
+                                  int32_t *__restrict__ keys, int32_t *__restrict__ positions) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < num_edges; i += stride) {
+        keys[i] = min(wrap_node(key[i], num_nodes), num_nodes);
+        positions[i] = (int32_t)i;
     }
 }
 
@@ -202,20 +416,26 @@ __global__ void tile_rank_kernel(const int32_t *__restrict__ row_order, int num_
 __device__ inline int tile_start(uint64_t packed) { return (int)(packed >> 32); }
 __device__ inline int tile_first_piece(uint64_t packed) { return (int)(uint32_t)packed; }
 
-// packed[t + 1] = (positions of tile t, descriptors of tile t); packed[0] = 0
-__global__ void tile_count_kernel(const int32_t *__restrict__ row_order, const int32_t *__restrict__ row_ptr,
-                                  int num_nodes, int tile_rows, int num_tiles, int max_work_edges,
-                                  uint64_t *__restrict__ packed) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) packed[0] = 0;
-    if (t >= num_tiles) return;
+// (positions of tile t, descriptors of tile t)
+__device__ __forceinline__ uint64_t tile_count(const int32_t *row_order, const int32_t *row_ptr, int num_nodes,
+                                               int tile_rows, int max_work_edges, int t) {
     int total = 0;
     for (int q = t * tile_rows; q < (t + 1) * tile_rows && q < num_nodes; q++) {
         const int r = row_order ? row_order[q] : q;
         total += row_ptr[r + 1] - row_ptr[r];
     }
     const int pieces = total == 0 ? 1 : (total + max_work_edges - 1) / max_work_edges;
-    packed[t + 1] = ((uint64_t)total << 32) | (uint64_t)pieces;
+    return ((uint64_t)total << 32) | (uint64_t)pieces;
+}
+
+// packed[t + 1] = the counts of tile t; packed[0] = 0
+__global__ void tile_count_kernel(const int32_t *__restrict__ row_order, const int32_t *__restrict__ row_ptr,
+                                  int num_nodes, int tile_rows, int num_tiles, int max_work_edges,
+                                  uint64_t *__restrict__ packed) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) packed[0] = 0;
+    if (t >= num_tiles) return;
+    packed[t + 1] = tile_count(row_order, row_ptr, num_nodes, tile_rows, max_work_edges, t);
 }
 
 // The three lists of one tile, by one wave: the tile's positions (its rows in tile order, each
@@ -251,14 +471,44 @@ __global__ __launch_bounds__(256) void tile_lists_kernel(
     const int first = t * tile_rows;
     const int rows = num_nodes - first < tile_rows ? num_nodes - first : tile_rows;
     if (m <= kTileSortLimit) {
+        // up to 64 rows: a lane per row reads where it lies, then the positions are taken 64 at a time
+        // across the rows (row after row, each row's three dependent loads were the kernel's time)
+        if (rows <= kWave) {
+            int b = 0, d = 0;
+            if (lane < rows) {
+                const int r = row_order ? row_order[first + lane] : first + lane;
+                b = row_ptr[r];
+                d = row_ptr[r + 1] - b;
+            }
+            int after = d;  // inclusive prefix sum over the rows
+#pragma unroll
+            for (int off = 1; off < kWave; off *= 2) {
+                const int add = __shfl_up(after, off, kWave);
+                if (lane >= off) after += add;
+            }
+            for (int q0 = 0; q0 < m; q0 += kWave) {
+                const int q = q0 + lane;
+                int row = 0, pos = 0;
+                for (int i = 0; i < rows; i++) {
+                    const int stop = __builtin_amdgcn_readlane(after, i), len = __builtin_amdgcn_readlane(d, i);
+                    const int start = __builtin_amdgcn_readlane(b, i);
+                    if (q < stop && q >= stop - len) { row = i; pos = start + q - (stop - len); }
+                }
+                if (q >= m) continue;
+                const int snd = other[pos];
+                const uint64_t sk = (unsigned)snd < (unsigned)num_nodes ? (uint64_t)snd : (uint64_t)num_nodes;
+                // (sender, position) orders the list; the row the position came from travels beside it
+                keys[q] = (sk << 32) | (uint64_t)(uint32_t)pos;
+                locals[q] = (uint16_t)row;
+            }
+        }
         int filled = 0;
-        for (int i = 0; i < rows; i++) {
+        for (int i = 0; i < (rows <= kWave ? 0 : rows); i++) {
             const int r = row_order ? row_order[first + i] : first + i;
             const int b = row_ptr[r], d = row_ptr[r + 1] - b;
             for (int q = lane; q < d; q += 64) {
                 const int snd = other[b + q];
                 const uint64_t sk = (unsigned)snd < (unsigned)num_nodes ? (uint64_t)snd : (uint64_t)num_nodes;
-                // (sender, position) orders the list; the row the position came from travels beside it
                 keys[filled + q] = (sk << 32) | (uint64_t)(uint32_t)(b + q);
                 locals[filled + q] = (uint16_t)i;
             }
@@ -324,12 +574,10 @@ __global__ __launch_bounds__(256) void tile_lists_kernel(
 // descriptors (tile, begin, end, 0), the first num_used of the num_work entries (a tile without
 // positions takes one, with begin == end; the entries behind the used ones are not written),
 // num_used in the fourth field of descriptor 0; `packed`: inclusive prefix sums, entry 0 = 0
-__global__ void tile_work_kernel(const uint64_t *__restrict__ packed, int num_tiles, int max_work_edges,
-                                 int32_t *__restrict__ work) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= num_tiles) return;
-    const int begin = tile_start(packed[t]), end = tile_start(packed[t + 1]);
-    int w = tile_first_piece(packed[t]);
+__device__ __forceinline__ void write_tile_work(int t, uint64_t before, uint64_t after, int num_used,
+                                                int max_work_edges, int32_t *work) {
+    const int begin = tile_start(before), end = tile_start(after);
+    int w = tile_first_piece(before);
     if (begin == end) {
         work[4 * w] = t; work[4 * w + 1] = begin; work[4 * w + 2] = begin; work[4 * w + 3] = 0;
     }
@@ -341,7 +589,39 @@ __global__ void tile_work_kernel(const uint64_t *__restrict__ packed, int num_ti
     }
     // the number of descriptors in use, for the kernel to deal them evenly to the XCDs (the
     // thread of tile 0 wrote descriptor 0 just above)
-    if (t == 0) work[3] = tile_first_piece(packed[num_tiles]);
+    if (t == 0) work[3] = num_used;
+}
+__global__ void tile_work_kernel(const uint64_t *__restrict__ packed, int num_tiles, int max_work_edges,
+                                 int32_t *__restrict__ work) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= num_tiles) return;
+    write_tile_work(t, packed[t], packed[t + 1], tile_first_piece(packed[num_tiles]), max_work_edges, work);
+}
+
+// Counts, prefix sums and work descriptors of up to kBlockThreads * kTileItems tiles by one workgroup
+// (the four launches of the general path take 3-5 us each on a schedule of this size).
+constexpr int kTileItems = 4;
+__global__ __launch_bounds__(kBlockThreads) void tile_plan_block_kernel(
+    const int32_t *__restrict__ row_order, const int32_t *__restrict__ row_ptr, int num_nodes, int tile_rows,
+    int num_tiles, int max_work_edges, uint64_t *__restrict__ packed, int32_t *__restrict__ work) {
+    using Scan = hipcub::BlockScan<uint64_t, kBlockThreads>;
+    __shared__ typename Scan::TempStorage temp;
+    uint64_t count[kTileItems], before[kTileItems], all;
+    const int first = (int)threadIdx.x * kTileItems;
+#pragma unroll
+    for (int k = 0; k < kTileItems; k++) {
+        const int t = first + k;
+        count[k] = t < num_tiles ? tile_count(row_order, row_ptr, num_nodes, tile_rows, max_work_edges, t) : 0;
+    }
+    Scan(temp).ExclusiveSum(count, before, all);
+    if (threadIdx.x == 0) packed[0] = 0;
+#pragma unroll
+    for (int k = 0; k < kTileItems; k++) {
+        const int t = first + k;
+        if (t >= num_tiles) continue;
+        packed[t + 1] = before[k] + count[k];
+        write_tile_work(t, before[k], before[k] + count[k], tile_first_piece(all), max_work_edges, work);
+    }
 }
 
 size_t scan64_temp_bytes(int32_t n) {
@@ -386,25 +666,6 @@ __global__ void compose_perm_kernel(const int32_t *__restrict__ outer, const int
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
         out[i] = inner ? inner[outer[i]] : outer[i];
-}
-
-// Pieces of the rows longer than `cap`, past their first `cap` positions: a row reserves its
-// pieces with one atomic on the count (the order of the list is free).
-__global__ void row_segments_kernel(const int32_t *__restrict__ row_ptr, int num_nodes, int cap, int piece,
-                                    int max_segments, int32_t *__restrict__ segments) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= num_nodes) return;
-    const int begin = row_ptr[r], end = row_ptr[r + 1];
-    if (end - begin <= cap) return;
-    const int extra = (end - begin - 1) / piece;  // pieces after the first
-    const int at = atomicAdd(segments, extra);
-    for (int k = 0; k < extra && at + k < max_segments; k++) {
-        const int b = begin + (k + 1) * piece;
-        int32_t *seg = segments + 4 + 3 * (at + k);
-        seg[0] = r;
-        seg[1] = b;
-        seg[2] = b + piece < end ? b + piece : end;
-    }
 }
 
 // ---- pairing of rows for the backward over tiles of two receivers ------------------------------
@@ -644,8 +905,8 @@ int e3j_amd_row_segments_build(const int32_t *receiver_ptr, int32_t num_nodes, i
     hipStream_t stream = static_cast<hipStream_t>(stream_);
     int rc = launch_fill_zero(segments, sizeof(int32_t) * 4, stream);
     if (rc || num_nodes == 0) return rc;
-    hipLaunchKernelGGL(row_segments_kernel, dim3(grid_for(num_nodes)), dim3(256), 0, stream, receiver_ptr,
-                       num_nodes, row_cap, row_piece, max_segments, segments);
+    hipLaunchKernelGGL(row_segments_kernel, dim3((unsigned)(((int64_t)num_nodes + 255) / 256)), dim3(256), 0, stream,
+                       receiver_ptr, num_nodes, row_cap, row_piece, max_segments, segments);
     return check_hip(hipGetLastError(), "row_segments_build");
 }
 
@@ -734,14 +995,20 @@ size_t e3j_amd_order_workspace_bytes(int32_t num_nodes) {
            5 * align_up(sizeof(int32_t) * (size_t)num_nodes) + 256;
 }
 
-int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nodes,
-                           int32_t rounds, int32_t *order, void *workspace, void *stream_) {
+namespace {
+// Where the caller wants the pieces of the rows longer than `cap` listed (segments[0] is zero when the
+// order is made); segments null: nowhere.
+struct PieceList {
+    int32_t cap, piece, max_segments;
+    int32_t *segments;
+};
+int locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nodes, int32_t rounds, int32_t *order,
+                   const PieceList &pieces, void *workspace, hipStream_t stream) {
     if (num_nodes < 0 || rounds < 0 || rounds > 64)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "locality_order: bad sizes");
     if (num_nodes == 0) return E3J_AMD_OK;
     if (order == nullptr || workspace == nullptr || row_ptr == nullptr)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "locality_order: null operand");
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
     unsigned char *ws = static_cast<unsigned char *>(workspace);
     const size_t sort_bytes = std::max(sort_temp_bytes(num_nodes), scan_temp_bytes(num_nodes));
     const size_t vec = align_up(sizeof(int32_t) * (size_t)num_nodes);
@@ -767,11 +1034,19 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
     if (two_levels) {
         // the two levels in one sort: same order as the two stable sorts below, half the passes
         hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
-                           static_cast<const int32_t *>(nullptr), lab_b);
+                           static_cast<const int32_t *>(nullptr), lab_b, nullptr, nullptr, 0);
+        const bool one_block = num_nodes <= 8 * kBlockThreads;
         hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
-                           lab_b, lab_a);
-        hipLaunchKernelGGL(two_level_keys_kernel, dim3(rows_grid), dim3(256), 0, stream, lab_a, lab_b, num_nodes,
-                           label_bits, keys_in, order);
+                           lab_b, lab_a, keys_in, one_block ? nullptr : order, label_bits);
+        if (one_block) {
+            auto kernel = num_nodes <= kBlockThreads       ? order_block_kernel<1>
+                          : num_nodes <= 2 * kBlockThreads ? order_block_kernel<2>
+                          : num_nodes <= 4 * kBlockThreads ? order_block_kernel<4>
+                                                           : order_block_kernel<8>;
+            hipLaunchKernelGGL(kernel, dim3(1), dim3(kBlockThreads), 0, stream, keys_in, row_ptr, num_nodes,
+                               2 * label_bits, order, pieces.cap, pieces.piece, pieces.max_segments, pieces.segments);
+            return check_hip(hipGetLastError(), "locality_order (one workgroup)");
+        }
         rc = check_hip(hipGetLastError(), "locality_order sweeps");
         if (rc) return rc;
         size_t temp_bytes = sort_bytes;
@@ -790,7 +1065,7 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
     for (int level = 1; level <= rounds; level *= 2) {
         for (; done < level; done++) {
             hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr,
-                               num_nodes, lab_a, lab_b);
+                               num_nodes, lab_a, lab_b, nullptr, nullptr, 0);
             int32_t *t = lab_a; lab_a = lab_b; lab_b = t;
         }
         hipLaunchKernelGGL(gather_kernel, dim3(ngrid), dim3(256), 0, stream, lab_a, order,
@@ -808,7 +1083,7 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
     // long rows to the fronts of the eighths of the list
     int32_t *flags = reinterpret_cast<int32_t *>(keys_in), *rank = reinterpret_cast<int32_t *>(keys_out);
     hipLaunchKernelGGL(long_row_flags_kernel, dim3(rows_grid), dim3(256), 0, stream, listed, row_ptr, num_nodes,
-                       flags);
+                       flags, pieces.cap, pieces.piece, pieces.max_segments, pieces.segments);
     rc = check_hip(hipGetLastError(), "locality_order flags");
     if (rc) return rc;
     size_t scan_bytes = sort_bytes;
@@ -825,6 +1100,97 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
                            (int64_t)num_nodes);
     }
     return check_hip(hipGetLastError(), "locality_order");
+}
+}  // namespace
+
+int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nodes,
+                           int32_t rounds, int32_t *order, void *workspace, void *stream) {
+    return locality_order(other, row_ptr, num_nodes, rounds, order, PieceList{0, 0, 0, nullptr}, workspace,
+                          static_cast<hipStream_t>(stream));
+}
+
+namespace {
+struct PrepareWorkspace {
+    size_t order, sort_temp, sort_bytes, keys_in, keys_out, positions, unsorted, total;
+    PrepareWorkspace(int32_t num_nodes, int64_t num_edges, bool sorted) {
+        size_t at = 0;
+        auto take = [&](size_t bytes) { const size_t here = at; at += align_up(bytes); return here; };
+        order = take(e3j_amd_order_workspace_bytes(num_nodes));
+        unsorted = take(sizeof(int32_t) * kMaxRowsBlocks);
+        sort_bytes = sorted ? 0 : sort_temp_bytes(num_edges);
+        sort_temp = take(sort_bytes);
+        const size_t list = sorted ? 0 : sizeof(int32_t) * (size_t)num_edges;
+        keys_in = take(list);
+        keys_out = take(list);
+        positions = take(list);
+        total = at;
+    }
+};
+}  // namespace
+
+size_t e3j_amd_prepare_rows_workspace_bytes(int32_t num_nodes, int64_t num_edges, int32_t sorted) {
+    if (num_nodes < 1 || num_edges < 1 || num_edges > 0x7fffffffLL) return 0;
+    return PrepareWorkspace(num_nodes, num_edges, sorted != 0).total + 256;
+}
+
+int e3j_amd_prepare_rows(const int32_t *key, const int32_t *other, int64_t num_edges, int32_t num_nodes,
+                         int32_t sorted, int32_t rounds, int32_t *perm, int32_t *other_out, int32_t *row_ptr,
+                         int32_t *order, int32_t row_cap, int32_t row_piece, int32_t max_segments,
+                         int32_t *segments, void *workspace, void *stream_) {
+    if (num_nodes < 1 || num_nodes >= INT32_MAX || num_edges < 1 || num_edges > 0x7fffffffLL || rounds < 0 ||
+        rounds > 64 || (segments != nullptr && (row_piece < 1 || row_cap < row_piece || max_segments < 0)))
+        return set_error(E3J_AMD_INVALID_ARGUMENT, "prepare_rows: bad sizes");
+    if (key == nullptr || other == nullptr || other_out == nullptr || row_ptr == nullptr || workspace == nullptr ||
+        (!sorted && perm == nullptr))
+        return set_error(E3J_AMD_INVALID_ARGUMENT, "prepare_rows: null operand");
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    unsigned char *ws = static_cast<unsigned char *>(workspace);
+    ws += (256 - reinterpret_cast<uintptr_t>(ws) % 256) % 256;
+    const PrepareWorkspace w(num_nodes, num_edges, sorted != 0);
+    int32_t *unsorted = reinterpret_cast<int32_t *>(ws + w.unsorted);
+    const int blocks = (int)std::min<int64_t>((num_edges + 255) / 256, kMaxRowsBlocks);
+    bool listed = false;  // pieces listed by the launches below
+    int rc = E3J_AMD_OK;
+    if (!sorted) {
+        int32_t *keys_in = reinterpret_cast<int32_t *>(ws + w.keys_in);
+        int32_t *keys_out = reinterpret_cast<int32_t *>(ws + w.keys_out);
+        int32_t *positions = reinterpret_cast<int32_t *>(ws + w.positions);
+        hipLaunchKernelGGL(sort_input_kernel, dim3(grid_for(num_edges)), dim3(256), 0, stream, key, num_edges,
+                           num_nodes, keys_in, positions);
+        rc = check_hip(hipGetLastError(), "prepare_rows keys");
+        if (rc) return rc;
+        int bits = 1;  // the keys reach num_nodes
+        while (bits < 32 && ((int64_t)1 << bits) <= (int64_t)num_nodes) bits++;
+        size_t temp_bytes = w.sort_bytes;
+        rc = check_hip(hipcub::DeviceRadixSort::SortPairs(
+                           ws + w.sort_temp, temp_bytes, reinterpret_cast<const uint32_t *>(keys_in),
+                           reinterpret_cast<uint32_t *>(keys_out), positions, perm, (int)num_edges, 0, bits, stream),
+                       "prepare_rows sort");
+        if (rc) return rc;
+        hipLaunchKernelGGL(rows_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, keys_out, other, perm, num_edges,
+                           num_nodes, other_out, row_ptr, static_cast<int32_t *>(nullptr), segments);
+    } else if (num_edges <= kRowsBlockEdges) {
+        listed = order == nullptr;
+        hipLaunchKernelGGL(rows_block_kernel, dim3(1), dim3(kBlockThreads), 0, stream, key, other, num_edges,
+                           num_nodes, other_out, row_ptr, listed, row_cap, row_piece, max_segments, segments);
+    } else {
+        hipLaunchKernelGGL(rows_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, key, other,
+                           static_cast<const int32_t *>(nullptr), num_edges, num_nodes, other_out, row_ptr, unsorted,
+                           segments);
+        hipLaunchKernelGGL(recount_rows_kernel, dim3(1), dim3(kBlockThreads), 0, stream, key, num_edges, num_nodes,
+                           unsorted, blocks, row_ptr);
+    }
+    rc = check_hip(hipGetLastError(), "prepare_rows");
+    if (rc) return rc;
+    if (order != nullptr)
+        return locality_order(other_out, row_ptr, num_nodes, rounds, order,
+                              PieceList{row_cap, row_piece, max_segments, segments}, ws + w.order, stream);
+    if (segments != nullptr && !listed) {
+        hipLaunchKernelGGL(row_segments_kernel, dim3((unsigned)(((int64_t)num_nodes + 255) / 256)), dim3(256), 0,
+                           stream, row_ptr, num_nodes, row_cap, row_piece, max_segments, segments);
+        rc = check_hip(hipGetLastError(), "prepare_rows pieces");
+    }
+    return rc;
 }
 
 int64_t e3j_amd_tile_schedule_num_work(int32_t num_nodes, int64_t num_edges, int32_t tile_rows,
@@ -860,16 +1226,23 @@ int e3j_amd_tile_schedule_build(const int32_t *other, const int32_t *row_ptr, co
     const int num_tiles = (num_nodes + tile_rows - 1) / tile_rows;
     const unsigned tiles_grid = (unsigned)((num_tiles + 255) / 256);
 
-    hipLaunchKernelGGL(tile_count_kernel, dim3(tiles_grid), dim3(256), 0, stream, row_order, row_ptr, num_nodes,
-                       tile_rows, num_tiles, max_work_edges, packed);
-    int rc = check_hip(hipGetLastError(), "tile schedule counts");
-    if (rc) return rc;
-    size_t temp_bytes = w.temp_bytes;
-    rc = check_hip(hipcub::DeviceScan::InclusiveSum(ws + w.temp, temp_bytes, packed, packed, num_tiles + 1, stream),
-                   "tile schedule scan");
-    if (rc) return rc;
-    hipLaunchKernelGGL(tile_work_kernel, dim3(tiles_grid), dim3(256), 0, stream, packed, num_tiles, max_work_edges,
-                       work);
+    int rc = E3J_AMD_OK;
+    if (num_tiles <= kBlockThreads * kTileItems) {
+        hipLaunchKernelGGL(tile_plan_block_kernel, dim3(1), dim3(kBlockThreads), 0, stream, row_order, row_ptr,
+                           num_nodes, tile_rows, num_tiles, max_work_edges, packed, work);
+    } else {
+        hipLaunchKernelGGL(tile_count_kernel, dim3(tiles_grid), dim3(256), 0, stream, row_order, row_ptr, num_nodes,
+                           tile_rows, num_tiles, max_work_edges, packed);
+        rc = check_hip(hipGetLastError(), "tile schedule counts");
+        if (rc) return rc;
+        size_t temp_bytes = w.temp_bytes;
+        rc = check_hip(hipcub::DeviceScan::InclusiveSum(ws + w.temp, temp_bytes, packed, packed, num_tiles + 1,
+                                                        stream),
+                       "tile schedule scan");
+        if (rc) return rc;
+        hipLaunchKernelGGL(tile_work_kernel, dim3(tiles_grid), dim3(256), 0, stream, packed, num_tiles,
+                           max_work_edges, work);
+    }
     rc = check_hip(hipGetLastError(), "tile schedule work");
     if (rc || num_edges == 0) return rc;
     // the lists: one wave per tile sorts its positions by sender in LDS

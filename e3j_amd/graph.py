@@ -160,20 +160,23 @@ class RowSegments:
     surplus workgroups of the second call leave at once, which costs less than a wait).
     `partials(num_out, channels)`: the scratch of the fixed-order sums (`e3j_amd_conv_params.partials`)."""
 
-    def __init__(self, row_ptr: torch.Tensor, num_nodes: int, num_edges: int, row_cap: int,
+    def __init__(self, row_ptr: torch.Tensor | None, num_nodes: int, num_edges: int, row_cap: int,
                  row_piece: int = ROW_PIECE):
-        device = _require_device(row_ptr)
-        lib = _lib.load()
+        """Without `row_ptr` only the sizes are set: the caller builds the list in a `buffer` of its own
+        (`prepare_rows`)."""
         self.row_cap = max(int(row_cap), int(row_piece)) if row_piece > ROW_PIECE else int(row_cap)
         self.row_piece = min(int(row_piece), self.row_cap)
         self._partials = {}
-        self.max_segments = int(lib.e3j_amd_row_segments_max(int(num_edges), self.row_piece))
+        self.max_segments = int(_lib.load().e3j_amd_row_segments_max(int(num_edges), self.row_piece))
+        self.count = self.max_segments
+        if row_ptr is None:
+            return
+        device = _require_device(row_ptr)
         self.buffer = torch.empty(4 + 3 * self.max_segments, dtype=INDEX_DTYPE, device=device)
         with torch.cuda.device(device):
-            _lib.check(lib.e3j_amd_row_segments_build(
+            _lib.check(_lib.load().e3j_amd_row_segments_build(
                 row_ptr.data_ptr(), int(num_nodes), self.row_cap, self.row_piece, self.max_segments,
                 self.buffer.data_ptr(), _stream_ptr(device)))
-        self.count = self.max_segments
 
     def partials(self, num_out: int, channels: int) -> torch.Tensor:
         key = (int(num_out), int(channels))
@@ -182,6 +185,45 @@ class RowSegments:
             nbytes = int(_lib.load().e3j_amd_row_partials_bytes(self.max_segments, *key))
             hit = self._partials[key] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.buffer.device)
         return hit
+
+
+def prepare_rows(key: torch.Tensor, other: torch.Tensor, num_nodes: int, sorted_keys: bool, rounds: int,
+                 pieces=None):
+    """An adjacency from its endpoints in one call of the library: `(row_ptr, other, perm, order, segments)`.
+
+    `key`: the endpoint the rows stand for, `other`: the one they gather; both are reduced modulo
+    `num_nodes` (the sentinel stays), as `wrap_global_index` does.  `sorted_keys` off: positions are
+    sorted by key first (`perm`, else None).  `rounds`: sweeps behind the row order (0: `order` is
+    None), `pieces`: `(row_cap, row_piece)` of the list of long rows to build (`segments`, else None).
+    """
+    device = _require_device(key, other)
+    key, other = ((t if t.dtype == INDEX_DTYPE else wrap_global_index(t, num_nodes)).contiguous() for t in (key, other))
+    num_edges = key.numel()
+    rounds = int(rounds) if num_nodes > 1 else 0
+    listed = RowSegments(None, num_nodes, num_edges, *pieces) if pieces is not None else None
+    lib = _lib.load()
+    with_order = rounds > 0
+    # one allocation for what is kept, each array on a 16-byte boundary
+    counts = (num_edges, num_nodes + 1, num_nodes if with_order else 0, 0 if sorted_keys else num_edges,
+              4 + 3 * listed.max_segments if listed is not None else 0)
+    sizes = []
+    for count in counts:
+        sizes += [count, -count % 4]
+    other_out, _, row_ptr, _, order, _, perm, _, buffer, _ = torch.empty(
+        sum(sizes), dtype=INDEX_DTYPE, device=device).split(sizes)
+    workspace = torch.empty(int(lib.e3j_amd_prepare_rows_workspace_bytes(num_nodes, num_edges, int(sorted_keys))),
+                            dtype=torch.uint8, device=device)
+    if listed is not None:
+        listed.buffer = buffer
+    with torch.cuda.device(device):
+        _lib.check(lib.e3j_amd_prepare_rows(
+            key.data_ptr(), other.data_ptr(), num_edges, num_nodes, int(sorted_keys), rounds,
+            None if sorted_keys else perm.data_ptr(), other_out.data_ptr(), row_ptr.data_ptr(),
+            order.data_ptr() if with_order else None,
+            listed.row_cap if listed is not None else 0, listed.row_piece if listed is not None else 0,
+            listed.max_segments if listed is not None else 0, buffer.data_ptr() if listed is not None else None,
+            workspace.data_ptr(), _stream_ptr(device)))
+    return row_ptr, other_out, None if sorted_keys else perm, order if with_order else None, listed
 
 
 class TileSchedule:

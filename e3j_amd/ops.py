@@ -26,7 +26,7 @@ import torch
 from . import _lib
 from .coef import Coef4D
 from .graph import (RowSegments, TileSchedule, csr_row_ptr, fold_endpoints, locality_order,
-                    pair_rows, row_cap_for, row_piece_for, sort_edges, wrap_global_index, ROW_PIECE)
+                    pair_rows, prepare_rows, row_cap_for, row_piece_for, sort_edges, wrap_global_index, ROW_PIECE)
 from .options import GraphOrdering, Layout, config
 
 
@@ -377,11 +377,11 @@ def _check_graph(graph: PreparedGraph, meta: "_Meta", num_edges: int) -> None:
                          f"{meta.ordering.name}")
 
 
-def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, build: bool = True):
+def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, build: bool = True, pieces=None):
     """Adjacency used by the forward kernel.  Without the opt-in cache it is prepared on every call
-    (`build` off: None, the caller prepares what it needs)."""
+    (`build` off: None, the caller prepares what it needs); `pieces`: see `_prepare_graph`."""
     if not config().graph_cache:
-        return _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver) if build else None
+        return _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver, pieces=pieces) if build else None
     key = (id(sender), id(receiver), sender._version, receiver._version, meta.num_nodes,
            meta.ordering, config().locality_rounds)
     hit = _GRAPH_CACHE.get(key)
@@ -389,7 +389,7 @@ def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, bu
         return hit[2]
     if not build:
         return None
-    graph = _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver)
+    graph = _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver, pieces=pieces)
     if len(_GRAPH_CACHE) >= _GRAPH_CACHE_SIZE:
         _GRAPH_CACHE.pop(next(iter(_GRAPH_CACHE)))
 
@@ -400,17 +400,54 @@ def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, bu
     return graph
 
 
+#: rows up to which the index order stays: every row then has a compute unit of its own, and whatever
+#: the rows share fits one L2 (256 rows of 16 x 128 floats: 2 MB)
+UNORDERED_ROWS = 256
+
+
 def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiver: torch.Tensor,
-                   pair: bool | None = None) -> PreparedGraph:
-    sender_l, receiver_l = wrap_global_index(sender, n), wrap_global_index(receiver, n)
-    if ordering == GraphOrdering.RECEIVER:
-        other, row_ptr, perm = sender_l.contiguous(), csr_row_ptr(receiver_l, n), None
-    elif ordering == GraphOrdering.SENDER:
+                   pair: bool | None = None, pieces=None) -> PreparedGraph:
+    """`pieces`: the `(row_cap, row_piece)` of the forward pass this graph is prepared for, which then finds
+    its list of pieces already built."""
+    if ordering == GraphOrdering.SENDER:
         # aggregate over reversed edges; y parities are folded into the coefficients
-        other, row_ptr, perm = receiver_l.contiguous(), csr_row_ptr(sender_l, n), None
+        key, other = sender, receiver
     else:
-        perm, other, row_ptr = sort_edges(receiver_l, sender_l, n)
+        key, other = receiver, sender
+    if n >= 1 and 0 < key.numel() == other.numel():
+        rounds = config().locality_rounds if n > UNORDERED_ROWS else 0
+        row_ptr, other, perm, order, segments = prepare_rows(
+            key, other, n, ordering != GraphOrdering.NONE, rounds, pieces)
+        if pair is None:
+            pair = config().pair_rows is True
+        if pair and n > 1 and config().locality_rounds > 0:
+            order = pair_rows(other, row_ptr, n, order)
+        graph = PreparedGraph(other, row_ptr, perm, order, n, ordering)
+        if segments is not None:
+            graph._segments[pieces] = segments
+        return graph
+    key, other = wrap_global_index(key, n), wrap_global_index(other, n)
+    if ordering != GraphOrdering.NONE:
+        other, row_ptr, perm = other.contiguous(), csr_row_ptr(key, n), None
+    else:
+        perm, other, row_ptr = sort_edges(key, other, n)
     return PreparedGraph(other, row_ptr, perm, _row_order(other, row_ptr, n, pair), n, ordering)
+
+
+def _row_pieces(meta: _Meta, x: torch.Tensor, num_edges: int):
+    """`(row_cap, row_piece)` of a forward pass that shares its long rows between waves, None for one
+    that does not."""
+    cfg = config()
+    fixed_order = bool(cfg.fixed_order_rows)
+    if (meta.layout != Layout.TRAILING_CHANNELS or x.dtype != torch.float32 or num_edges == 0
+            or (cfg.deterministic and not fixed_order)):
+        return None
+    want = int(cfg.row_cap)
+    cap = row_cap_for(x.shape[0], num_edges) if want < 0 else want
+    if cap <= 0:
+        return None
+    row_floats = int(meta.params.num_out) * int(x.shape[2])
+    return cap, row_piece_for(num_edges, row_floats) if fixed_order else ROW_PIECE
 
 
 def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Tensor:
@@ -431,14 +468,9 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
     # a scratch row, and a second kernel adds them to their output rows in a fixed order (unrolled
     # kernels of the trailing layout): the result is the same bits in every run, as for a row that
     # one wave sums.  Without the fixed order a second call adds the pieces with float atomics.
-    cap = 0
-    fixed_order = bool(config().fixed_order_rows)
-    if (p.signature >= 0 and meta.layout == Layout.TRAILING_CHANNELS and x.dtype == torch.float32
-            and (fixed_order or not config().deterministic)
-            and isinstance(graph, PreparedGraph) and y.shape[0] > 0
-            and all(t.data_ptr() % 16 == 0 for t in (x, s, out))):
-        want = int(config().row_cap)
-        cap = row_cap_for(x.shape[0], y.shape[0]) if want < 0 else want
+    shared = None
+    if p.signature >= 0 and isinstance(graph, PreparedGraph) and all(v.data_ptr() % 16 == 0 for v in (x, s, out)):
+        shared = _row_pieces(meta, x, int(y.shape[0]))
     lib = _lib.load()
     with torch.cuda.device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
@@ -446,11 +478,10 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
                 other.data_ptr(), row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
                 out.data_ptr(), _stream(x.device))
         pieces = None
-        if cap > 0:
-            row_floats = int(out.shape[1]) * int(out.shape[2])
-            pieces = graph.segments(cap, row_piece_for(int(y.shape[0]), row_floats) if fixed_order else ROW_PIECE)
+        if shared is not None:
+            pieces = graph.segments(*shared)
             p.row_cap, p.row_piece = pieces.row_cap, pieces.row_piece
-        if pieces is not None and pieces.count > 0 and fixed_order:
+        if pieces is not None and pieces.count > 0 and config().fixed_order_rows:
             p.segments, p.max_segments = pieces.buffer.data_ptr(), pieces.count
             p.partials = pieces.partials(int(out.shape[1]), int(out.shape[2])).data_ptr()
             _lib.check(lib.e3j_amd_convolution_fwd_whole(ctypes.byref(p), *args))
@@ -653,7 +684,7 @@ class _Convolution(torch.autograd.Function):
     @staticmethod
     def forward(x, y, s, sender, receiver, meta, graph):
         if graph is None:
-            graph = _forward_graph(meta, sender, receiver)
+            graph = _forward_graph(meta, sender, receiver, pieces=_row_pieces(meta, x, int(y.shape[0])))
         return _raw_forward(meta, x, y, s, sender, receiver, graph)
 
     @staticmethod
@@ -810,7 +841,7 @@ def convolution(coef, x, y, s, sender, receiver, params: ConvolutionParams,
         # prepared here, so that the backward pass finds it in its context; under a torch.func
         # transform the operator prepares it itself, on the plain tensors the transform hands it
         # (the batching rule first folds batched index tensors into one graph)
-        graph = _forward_graph(meta, sender, receiver)
+        graph = _forward_graph(meta, sender, receiver, pieces=_row_pieces(meta, x3, int(y2.shape[0])))
     out = _Convolution.apply(x3, y2, s3, sender, receiver, meta, graph)
     if squeeze:
         out = out.squeeze(-1 if layout == Layout.TRAILING_CHANNELS else 1)

@@ -385,6 +385,20 @@ size_t e3j_amd_order_workspace_bytes(int32_t num_nodes);
 int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nodes,
                            int32_t rounds, int32_t *order, void *workspace, void *stream);
 
+/* e3j_amd_prepare_rows: an adjacency from its endpoints in one call with few launches, for callers that
+ *   prepare a new graph for every pass: what e3j_amd_wrap_index on both endpoints, then
+ *   e3j_amd_csr_row_ptr (sorted != 0) or e3j_amd_sort_edges (sorted == 0; perm (E), else NULL),
+ *   e3j_amd_locality_order (order (N), or NULL for none) and e3j_amd_row_segments_build
+ *   (segments, or NULL for none) give, without the ids in `key` / `other` having to be reduced first.
+ *   Keys out of order despite `sorted` get the row_ptr of e3j_amd_csr_row_ptr (slowly).
+ *   num_nodes and num_edges are at least 1; other_out (E), row_ptr (N+1).
+ *   workspace: >= e3j_amd_prepare_rows_workspace_bytes(). */
+size_t e3j_amd_prepare_rows_workspace_bytes(int32_t num_nodes, int64_t num_edges, int32_t sorted);
+int e3j_amd_prepare_rows(const int32_t *key, const int32_t *other, int64_t num_edges, int32_t num_nodes,
+                         int32_t sorted, int32_t rounds, int32_t *perm, int32_t *other_out,
+                         int32_t *row_ptr, int32_t *order, int32_t row_cap, int32_t row_piece,
+                         int32_t max_segments, int32_t *segments, void *workspace, void *stream);
+
 /* e3j_amd_pair_rows: reorders a processing order for the backward over tiles of two receivers.
  *   Rows that share most of their senders are put side by side (greedy matching over a few
  *   rounds: rows that pick each other as the row with the most senders in common are paired),
