@@ -11,6 +11,7 @@ helpers is plain tensor arithmetic.
 
 from __future__ import annotations
 
+import contextlib
 
 import numpy as np
 import torch
@@ -40,8 +41,18 @@ def _require_device(*tensors: torch.Tensor) -> torch.device:
     return device
 
 
-def _stream_ptr(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+def raw_stream(device: torch.device) -> int:
+    """The handle of torch's current stream on a tensor's device (without the stream object)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_stream_ptr = raw_stream
+_ON_CURRENT_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """`torch.cuda.device(device)`, at no cost where that device is current already."""
+    return _ON_CURRENT_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def _as_index(t: torch.Tensor) -> torch.Tensor:
@@ -59,7 +70,7 @@ def csr_row_ptr(key: torch.Tensor, num_nodes: int) -> torch.Tensor:
     key = _as_index(key)
     row_ptr = torch.empty(num_nodes + 1, dtype=INDEX_DTYPE, device=device)
     ws = _workspace(num_nodes, key.numel(), device)
-    with torch.cuda.device(device):
+    with on_device(device):
         _lib.check(_lib.load().e3j_amd_csr_row_ptr(
             key.data_ptr(), key.numel(), num_nodes, row_ptr.data_ptr(), ws.data_ptr(),
             _stream_ptr(device)))
@@ -75,7 +86,7 @@ def sort_edges(key: torch.Tensor, other: torch.Tensor, num_nodes: int):
     other_sorted = torch.empty(num_edges, dtype=INDEX_DTYPE, device=device)
     row_ptr = torch.empty(num_nodes + 1, dtype=INDEX_DTYPE, device=device)
     ws = _workspace(num_nodes, num_edges, device)
-    with torch.cuda.device(device):
+    with on_device(device):
         _lib.check(_lib.load().e3j_amd_sort_edges(
             key.data_ptr(), other.data_ptr(), num_edges, num_nodes, perm.data_ptr(),
             other_sorted.data_ptr(), row_ptr.data_ptr(), ws.data_ptr(), _stream_ptr(device)))
@@ -97,7 +108,7 @@ def locality_order(other: torch.Tensor, row_ptr: torch.Tensor, num_nodes: int,
     lib = _lib.load()
     ws = torch.empty(max(int(lib.e3j_amd_order_workspace_bytes(num_nodes)), 256), dtype=torch.uint8,
                      device=device)
-    with torch.cuda.device(device):
+    with on_device(device):
         _lib.check(lib.e3j_amd_locality_order(other.data_ptr(), row_ptr.data_ptr(), num_nodes,
                                               int(rounds), order.data_ptr(), ws.data_ptr(),
                                               _stream_ptr(device)))
@@ -116,7 +127,7 @@ def pair_rows(other: torch.Tensor, row_ptr: torch.Tensor, num_nodes: int,
     out = torch.empty(num_nodes, dtype=INDEX_DTYPE, device=device)
     ws = torch.empty(max(int(lib.e3j_amd_pair_rows_workspace_bytes(num_nodes, num_edges)), 256),
                      dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with on_device(device):
         _lib.check(lib.e3j_amd_pair_rows(other.data_ptr(), row_ptr.data_ptr(), num_nodes, num_edges,
                                          order.data_ptr() if order is not None else None, out.data_ptr(),
                                          ws.data_ptr(), _stream_ptr(device)))
@@ -173,7 +184,7 @@ class RowSegments:
             return
         device = _require_device(row_ptr)
         self.buffer = torch.empty(4 + 3 * self.max_segments, dtype=INDEX_DTYPE, device=device)
-        with torch.cuda.device(device):
+        with on_device(device):
             _lib.check(_lib.load().e3j_amd_row_segments_build(
                 row_ptr.data_ptr(), int(num_nodes), self.row_cap, self.row_piece, self.max_segments,
                 self.buffer.data_ptr(), _stream_ptr(device)))
@@ -215,7 +226,7 @@ def prepare_rows(key: torch.Tensor, other: torch.Tensor, num_nodes: int, sorted_
                             dtype=torch.uint8, device=device)
     if listed is not None:
         listed.buffer = buffer
-    with torch.cuda.device(device):
+    with on_device(device):
         _lib.check(lib.e3j_amd_prepare_rows(
             key.data_ptr(), other.data_ptr(), num_edges, num_nodes, int(sorted_keys), rounds,
             None if sorted_keys else perm.data_ptr(), other_out.data_ptr(), row_ptr.data_ptr(),
@@ -247,7 +258,7 @@ class TileSchedule:
         self.local = torch.empty(num_edges, dtype=INDEX_DTYPE, device=device)
         nbytes = int(lib.e3j_amd_tile_schedule_workspace_bytes(num_nodes, num_edges, tile_rows))
         ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
-        with torch.cuda.device(device):
+        with on_device(device):
             _lib.check(lib.e3j_amd_tile_schedule_build(
                 other.data_ptr(), row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
                 row_order.data_ptr() if row_order is not None else None, num_nodes, num_edges,
@@ -308,7 +319,7 @@ def wrap_global_index(index: torch.Tensor, num_nodes: int) -> torch.Tensor:
         return local.to(INDEX_DTYPE)
     index = index.contiguous()
     out = torch.empty_like(index)
-    with torch.cuda.device(index.device):
+    with on_device(index.device):
         _lib.check(_lib.load().e3j_amd_wrap_index(index.data_ptr(), index.numel(), num_nodes,
                                                   out.data_ptr(), _stream_ptr(index.device)))
     return out

@@ -26,7 +26,7 @@ import torch
 from . import _lib
 from .coef import Coef4D
 from .graph import (RowSegments, TileSchedule, csr_row_ptr, fold_endpoints, locality_order,
-                    pair_rows, prepare_rows, row_cap_for, row_piece_for, sort_edges, wrap_global_index, ROW_PIECE)
+                    on_device, pair_rows, prepare_rows, raw_stream, row_cap_for, row_piece_for, sort_edges, wrap_global_index, ROW_PIECE)
 from .options import GraphOrdering, Layout, config
 
 
@@ -182,8 +182,7 @@ class _Meta:
     y_shape: tuple
 
 
-def _stream(device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+_stream = raw_stream
 
 
 def _shape(meta: _Meta, x: torch.Tensor, y: torch.Tensor, s: torch.Tensor):
@@ -311,9 +310,9 @@ class PreparedGraph:
 
     def ready(self):
         """Order the current stream after the kernels that prepared this adjacency."""
-        current = torch.cuda.current_stream(self.row_ptr.device)
-        if current != self.stream:
-            current.wait_event(self.event)
+        device = self.row_ptr.device
+        if _stream(device) != self.stream.cuda_stream:
+            torch.cuda.current_stream(device).wait_event(self.event)
 
     @property
     def num_edges(self) -> int:
@@ -472,7 +471,7 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
     if p.signature >= 0 and isinstance(graph, PreparedGraph) and all(v.data_ptr() % 16 == 0 for v in (x, s, out)):
         shared = _row_pieces(meta, x, int(y.shape[0]))
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with on_device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
         args = (table.device(x.device).data_ptr(), x.data_ptr(), y.data_ptr(), s.data_ptr(),
                 other.data_ptr(), row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
@@ -567,7 +566,7 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
     if (group_receiver and not ordered and y.shape[0] > 0 and p.layout == _lib.LAYOUT_TRAILING and aligned
             and x.dtype == torch.float32):
         tile_rows = _tile_rows(p.signature)
-    with torch.cuda.device(x.device):
+    with on_device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
         if tile_rows >= 1:
             if prepared is None:
@@ -606,7 +605,7 @@ def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph
     other, row_ptr, perm, order = graph
     p, table = _fill_params(meta, x, y, s, meta.table, row_order=order)
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with on_device(x.device):
         schedule = graph.schedule(tile_rows)
         want = int(config().row_cap)
         cap = row_cap_for(x.shape[0], y.shape[0]) if want < 0 else want
@@ -700,7 +699,7 @@ class _Convolution(torch.autograd.Function):
     def backward(ctx, dm):
         x, y, s = ctx.saved_tensors
         sender, receiver = ctx.index
-        dx, dy, ds = _ConvolutionBwd.apply(x, y, s, dm, sender, receiver, ctx.meta, ctx.graph)
+        dx, dy, ds = _apply_bwd(x, y, s, dm, sender, receiver, ctx.meta, ctx.graph)
         return dx, dy, ds, None, None, None, None
 
     @staticmethod
@@ -742,10 +741,10 @@ class _ConvolutionBwd(torch.autograd.Function):
                 return *grads, None, None, None, None
 
         def conv(a, b, c):
-            return _Convolution.apply(a, b, c, sender, receiver, meta, graph)
+            return _apply_fwd(a, b, c, sender, receiver, meta, graph)
 
         def conv_bwd(a, b, c):
-            return _ConvolutionBwd.apply(a, b, c, dm, sender, receiver, meta, graph)
+            return _apply_bwd(a, b, c, dm, sender, receiver, meta, graph)
 
         d_dm, d_x, d_y, d_s = [], [], [], []
         if ddx is not None:
@@ -773,6 +772,36 @@ class _ConvolutionBwd(torch.autograd.Function):
             _fold_rows(_lead(x, in_dims[0], batch)), _fold_rows(_lead(y, in_dims[1], batch)),
             _fold_rows(_lead(s, in_dims[2], batch)), _fold_rows(_lead(dm, in_dims[3], batch)), snd, rcv, folded, None)
         return (_unfold_rows(dx, batch), _unfold_rows(dy, batch), _unfold_rows(ds, batch)), (0, 0, 0)
+
+
+# The same two functions for calls outside torch.func transforms.  A function with `setup_context` binds
+# its arguments to the signature of `forward` through `inspect` in every call (about 15 us each way on
+# the host, a tenth of a small graph's pass); one that takes the context in `forward` does not, but has
+# no batching rule.
+class _PlainConvolution(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *inputs):
+        _Convolution.setup_context(ctx, inputs, None)
+        return _Convolution.forward(*inputs)
+
+    backward = _Convolution.backward
+
+
+class _PlainConvolutionBwd(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, *inputs):
+        _ConvolutionBwd.setup_context(ctx, inputs, None)
+        return _ConvolutionBwd.forward(*inputs)
+
+    backward = _ConvolutionBwd.backward
+
+
+def _apply_fwd(*args):
+    return (_Convolution if _under_transform() else _PlainConvolution).apply(*args)
+
+
+def _apply_bwd(*args):
+    return (_ConvolutionBwd if _under_transform() else _PlainConvolutionBwd).apply(*args)
 
 
 def _make_meta(coef, x, y, s, params, graph_ordering, y_parity, layout) -> _Meta:
@@ -842,7 +871,7 @@ def convolution(coef, x, y, s, sender, receiver, params: ConvolutionParams,
         # transform the operator prepares it itself, on the plain tensors the transform hands it
         # (the batching rule first folds batched index tensors into one graph)
         graph = _forward_graph(meta, sender, receiver, pieces=_row_pieces(meta, x3, int(y2.shape[0])))
-    out = _Convolution.apply(x3, y2, s3, sender, receiver, meta, graph)
+    out = _apply_fwd(x3, y2, s3, sender, receiver, meta, graph)
     if squeeze:
         out = out.squeeze(-1 if layout == Layout.TRAILING_CHANNELS else 1)
     return out
@@ -860,7 +889,7 @@ def convolution_bwd(coef, x, y, s, sender, receiver, dm, params: ConvolutionPara
     meta = _make_meta(coef, x3, y2, s3, params, graph_ordering, y_parity, layout)
     if graph is not None:
         _check_graph(graph, meta, int(y2.shape[0]))
-    dx, dy, ds = _ConvolutionBwd.apply(x3, y2, s3, dm3, sender, receiver, meta, graph)
+    dx, dy, ds = _apply_bwd(x3, y2, s3, dm3, sender, receiver, meta, graph)
     if squeeze:
         axis = -1 if layout == Layout.TRAILING_CHANNELS else 1
         dx = dx.squeeze(axis)
