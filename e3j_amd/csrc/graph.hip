@@ -150,11 +150,79 @@ __global__ void deal_long_rows_kernel(const int32_t *__restrict__ order, const i
     dealt[dealt_position(i, flags[i] != 0, rank[i], rank[num_nodes - 1], num_nodes)] = order[i];
 }
 
+constexpr int kBlockThreads = 1024;
+
+// Stable sort of up to kBlockThreads * ITEMS (key, value) pairs by one workgroup, at most eight bits a
+// pass, from and to `pairs` in LDS.  A wave takes 64 * ITEMS consecutive pairs, 64 at a time; the lanes of
+// equal digits find each other with eight ballots, so a digit's count per wave needs no atomics and the
+// ranks keep the order.
+template <int ITEMS>
+struct BlockSort {
+    static constexpr int WAVES = kBlockThreads / kWave, DIGITS = 256;
+    uint2 pairs[kBlockThreads * ITEMS];
+    uint16_t counts[DIGITS][WAVES];  // pairs of a digit in a wave, then the place of the first of them
+    int sums[WAVES];
+
+    __device__ __forceinline__ void sort(int bits) {
+        const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+        const int passes = (bits + 7) / 8, step = (bits + passes - 1) / passes;
+        const unsigned mask = (1u << step) - 1;
+        for (int shift = 0; shift < bits; shift += step) {
+            uint2 pair[ITEMS];
+            int rank[ITEMS];
+            for (int i = lane; i < DIGITS; i += kWave) counts[i][wave] = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int k = 0; k < ITEMS; k++) {
+                pair[k] = pairs[(wave * ITEMS + k) * kWave + lane];
+                const unsigned digit = (pair[k].x >> shift) & mask;
+                unsigned long long same = ~0ull;
+#pragma unroll
+                for (int bit = 0; bit < 8; bit++) {
+                    if (bit == step) break;
+                    const unsigned long long set = __ballot((digit >> bit) & 1u);
+                    same &= (digit >> bit) & 1u ? set : ~set;
+                }
+                const int before = counts[digit][wave];
+                rank[k] = before + __popcll(same & ((1ull << lane) - 1ull));
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if ((same >> lane) == 1ull) counts[digit][wave] = (uint16_t)(rank[k] + 1);  // the last of its digit
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+            __syncthreads();
+            // exclusive prefix sums over (digit, wave): four consecutive counts a thread
+            uint16_t *flat = &counts[0][0] + 4 * threadIdx.x;
+            int local[4], sum = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) { local[i] = sum; sum += flat[i]; }
+            int after = sum;
+#pragma unroll
+            for (int off = 1; off < kWave; off *= 2) {
+                const int add = __shfl_up(after, off, kWave);
+                if (lane >= off) after += add;
+            }
+            if (lane == kWave - 1) sums[wave] = after;
+            __syncthreads();
+            int base = after - sum;
+            for (int w = 0; w < wave; w++) base += sums[w];
+#pragma unroll
+            for (int i = 0; i < 4; i++) flat[i] = (uint16_t)(base + local[i]);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < ITEMS; k++)
+                pairs[counts[(pair[k].x >> shift) & mask][wave] + rank[k]] = pair[k];
+            __syncthreads();
+        }
+    }
+};
+
 // The end of the row order for up to kBlockThreads * ITEMS rows, by one workgroup: the sort of the
 // keys, the deal of the long rows and, with `segments`, the list of their pieces.  Nine launches of
 // the general path (sort 4-6, flags, scan 2, deal) in one: each of those takes 3-5 us here whatever
-// it moves.  5 000 rows: 32 -> 15 us.
-constexpr int kBlockThreads = 1024;
+// it moves.  5 000 rows: 25 us (32 us with the library's sort of a block, about 45 us in nine launches);
+// what is left is the issue rate of one compute unit.
 template <int ITEMS>
 __global__ __launch_bounds__(kBlockThreads) void order_block_kernel(const uint32_t *__restrict__ keys,
                                                                     const int32_t *__restrict__ row_ptr,
@@ -162,43 +230,67 @@ __global__ __launch_bounds__(kBlockThreads) void order_block_kernel(const uint32
                                                                     int32_t *__restrict__ order, int row_cap,
                                                                     int row_piece, int max_segments,
                                                                     int32_t *__restrict__ segments) {
-    using Sort = hipcub::BlockRadixSort<uint32_t, kBlockThreads, ITEMS, int32_t>;
-    using Scan = hipcub::BlockScan<int, kBlockThreads>;
-    __shared__ union {
-        typename Sort::TempStorage sort;
-        typename Scan::TempStorage scan;
-    } temp;
-    uint32_t key[ITEMS];
-    int32_t row[ITEMS];
-    const int first = (int)threadIdx.x * ITEMS;
+    extern __shared__ __attribute__((aligned(16))) unsigned char order_lds[];
+    BlockSort<ITEMS> &sorter = *reinterpret_cast<BlockSort<ITEMS> *>(order_lds);
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
         // (the sort is stable: the entries past the last row stay behind every row of the same key)
-        key[k] = first + k < num_nodes ? keys[first + k] : ~0u;
-        row[k] = first + k < num_nodes ? first + k : 0;
+        const int i = k * kBlockThreads + threadIdx.x;
+        sorter.pairs[i] = make_uint2(i < num_nodes ? keys[i] : ~0u, i < num_nodes ? i : 0);
     }
-    Sort(temp.sort).Sort(key, row, 0, key_bits);
     __syncthreads();
+    sorter.sort(key_bits);
     const int64_t live = row_ptr[num_nodes];
-    int begin[ITEMS], end[ITEMS], flag[ITEMS], rank[ITEMS], num_long;
+    // a wave's entries: 64 consecutive ones per k; long rows are counted with ballots
+    int row[ITEMS], begin[ITEMS], end[ITEMS], rank[ITEMS], longs = 0;
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
+        row[k] = (int)sorter.pairs[(wave * ITEMS + k) * kWave + lane].y;
         begin[k] = row_ptr[row[k]];
         end[k] = row_ptr[row[k] + 1];
     }
-#pragma unroll
-    for (int k = 0; k < ITEMS; k++)
-        flag[k] = first + k < num_nodes && (int64_t)(end[k] - begin[k]) * num_nodes > 2 * live ? 1 : 0;
-    Scan(temp.scan).InclusiveSum(flag, rank, num_long);
+    bool flag[ITEMS];
 #pragma unroll
     for (int k = 0; k < ITEMS; k++) {
-        if (first + k >= num_nodes) continue;
-        const int64_t at = num_long == 0 ? first + k : dealt_position(first + k, flag[k] != 0, rank[k], num_long,
-                                                                      num_nodes);
+        const int i = (wave * ITEMS + k) * kWave + lane;
+        flag[k] = i < num_nodes && (int64_t)(end[k] - begin[k]) * num_nodes > 2 * live;
+        const unsigned long long mask = __ballot(flag[k]);
+        rank[k] = longs + __popcll(mask & ((2ull << lane) - 1ull));
+        longs += __popcll(mask);
+    }
+    if (lane == 0) sorter.sums[wave] = longs;
+    __syncthreads();
+    int before = 0, num_long = 0;
+    for (int w = 0; w < BlockSort<ITEMS>::WAVES; w++) {
+        if (w < wave) before += sorter.sums[w];
+        num_long += sorter.sums[w];
+    }
+#pragma unroll
+    for (int k = 0; k < ITEMS; k++) {
+        const int i = (wave * ITEMS + k) * kWave + lane;
+        if (i >= num_nodes) continue;
+        const int64_t at = num_long == 0 ? i : dealt_position(i, flag[k], before + rank[k], num_long, num_nodes);
         order[at] = row[k];
         if (segments != nullptr)
             list_row_pieces(row[k], begin[k], end[k], row_cap, row_piece, max_segments, segments);
     }
+}
+template <int ITEMS>
+int launch_order_block(const uint32_t *keys, const int32_t *row_ptr, int num_nodes, int key_bits, int32_t *order,
+                       int row_cap, int row_piece, int max_segments, int32_t *segments, hipStream_t stream) {
+    constexpr size_t lds = sizeof(BlockSort<ITEMS>);
+    static_assert(lds <= 160 * 1024, "LDS of a workgroup");
+    auto kernel = order_block_kernel<ITEMS>;
+    if (lds > 64 * 1024) {
+        const int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                                 "hipFuncSetAttribute(order_block)");
+        if (rc) return rc;
+    }
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kBlockThreads), lds, stream, keys, row_ptr, num_nodes, key_bits, order,
+                       row_cap, row_piece, max_segments, segments);
+    return check_hip(hipGetLastError(), "locality_order (one workgroup)");
 }
 
 size_t align_up(size_t v, size_t a = 256) { return (v + a - 1) / a * a; }
@@ -438,22 +530,29 @@ __global__ void tile_count_kernel(const int32_t *__restrict__ row_order, const i
     packed[t + 1] = tile_count(row_order, row_ptr, num_nodes, tile_rows, max_work_edges, t);
 }
 
-// The three lists of one tile, by one wave: the tile's positions (its rows in tile order, each
+// The three lists of one tile, by WPT waves: the tile's positions (its rows in tile order, each
 // row's positions ascending) are keyed by (sender, position), padding senders after the live
-// ones, and sorted in LDS with a bitonic network when the tile has at most kTileSortLimit of
-// them.  Longer tiles (hub rows) are not sorted by sender, only split into live positions first
+// ones.  A tile of at most kTileSortLimit positions is listed in the order of the keys: they are all
+// different, so a position's place is the number of smaller keys, which every lane counts for its
+// positions over the keys in LDS (all lanes read the same one).  Sorted with a bitonic network
+// by one wave instead, the 28 dependent steps of a tile of 120 positions were the kernel's time (150k
+// edges in tiles of four rows: 18 -> 14 us).
+// Longer tiles (hub rows) are not sorted by sender, only split into live positions first
 // and padding positions last, which is all the kernel needs for correctness (it sums runs of
 // equal senders wherever they occur); a hub's senders are mostly distinct anyway.
 // The entries past the last row (padding positions that belong to no tile) are filled by all
 // threads of the grid before they turn to their tiles.
 constexpr int kTileSortLimit = 512;
+template <int WPT>
 __global__ __launch_bounds__(256) void tile_lists_kernel(
     const int32_t *__restrict__ other, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ perm,
     const int32_t *__restrict__ row_order, const uint64_t *__restrict__ packed, int num_nodes, int64_t num_edges,
     int tile_rows, int num_tiles, int32_t *__restrict__ t_sender, int32_t *__restrict__ t_edge,
     int32_t *__restrict__ t_local) {
-    __shared__ uint64_t keys_all[4][kTileSortLimit];
-    __shared__ uint16_t local_all[4][kTileSortLimit];
+    static_assert(WPT == 1 || WPT == 4, "a wave or the workgroup per tile");
+    constexpr int TILES = 4 / WPT, LANES = kWave * WPT;
+    __shared__ __attribute__((aligned(16))) uint64_t keys_all[TILES][kTileSortLimit];
+    __shared__ uint16_t local_all[TILES][kTileSortLimit];
     {
         const int64_t stride = (int64_t)gridDim.x * blockDim.x;
         for (int64_t i = (int64_t)row_ptr[num_nodes] + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -461,19 +560,25 @@ __global__ __launch_bounds__(256) void tile_lists_kernel(
             t_sender[i] = -1; t_edge[i] = 0; t_local[i] = 0;
         }
     }
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const int t = blockIdx.x * 4 + wave;
-    if (t >= num_tiles) return;
-    uint64_t *keys = keys_all[wave];
-    uint16_t *locals = local_all[wave];
+    const int tile = threadIdx.x / LANES, lane = threadIdx.x % kWave, at_lane = threadIdx.x % LANES;
+    const int t = blockIdx.x * TILES + tile;
+    if (t >= num_tiles) return;  // (with WPT 4: the whole workgroup, also below)
+    uint64_t *keys = keys_all[tile];
+    uint16_t *locals = local_all[tile];
     const int begin = tile_start(packed[t]), m = tile_start(packed[t + 1]) - begin;
     if (m == 0) return;
     const int first = t * tile_rows;
     const int rows = num_nodes - first < tile_rows ? num_nodes - first : tile_rows;
     if (m <= kTileSortLimit) {
-        // up to 64 rows: a lane per row reads where it lies, then the positions are taken 64 at a time
-        // across the rows (row after row, each row's three dependent loads were the kernel's time)
+        auto put = [&](int q, int pos, int row) {
+            const int snd = other[pos];
+            const uint64_t sk = (unsigned)snd < (unsigned)num_nodes ? (uint64_t)snd : (uint64_t)num_nodes;
+            // (sender, position) orders the list; the row the position came from travels beside it
+            keys[q] = (sk << 32) | (uint64_t)(uint32_t)pos;
+            locals[q] = (uint16_t)row;
+        };
         if (rows <= kWave) {
+            // a lane per row reads where it lies, then the positions are taken across the rows
             int b = 0, d = 0;
             if (lane < rows) {
                 const int r = row_order ? row_order[first + lane] : first + lane;
@@ -486,67 +591,59 @@ __global__ __launch_bounds__(256) void tile_lists_kernel(
                 const int add = __shfl_up(after, off, kWave);
                 if (lane >= off) after += add;
             }
-            for (int q0 = 0; q0 < m; q0 += kWave) {
-                const int q = q0 + lane;
+            for (int q0 = 0; q0 < m; q0 += LANES) {
+                const int q = q0 + at_lane;
                 int row = 0, pos = 0;
                 for (int i = 0; i < rows; i++) {
                     const int stop = __builtin_amdgcn_readlane(after, i), len = __builtin_amdgcn_readlane(d, i);
                     const int start = __builtin_amdgcn_readlane(b, i);
                     if (q < stop && q >= stop - len) { row = i; pos = start + q - (stop - len); }
                 }
-                if (q >= m) continue;
-                const int snd = other[pos];
-                const uint64_t sk = (unsigned)snd < (unsigned)num_nodes ? (uint64_t)snd : (uint64_t)num_nodes;
-                // (sender, position) orders the list; the row the position came from travels beside it
-                keys[q] = (sk << 32) | (uint64_t)(uint32_t)pos;
-                locals[q] = (uint16_t)row;
+                if (q < m) put(q, pos, row);
+            }
+        } else {
+            for (int i = 0, filled = 0; i < rows; i++) {
+                const int r = row_order ? row_order[first + i] : first + i;
+                const int b = row_ptr[r], d = row_ptr[r + 1] - b;
+                for (int q = at_lane; q < d; q += LANES) put(filled + q, b + q, i);
+                filled += d;
             }
         }
-        int filled = 0;
-        for (int i = 0; i < (rows <= kWave ? 0 : rows); i++) {
-            const int r = row_order ? row_order[first + i] : first + i;
-            const int b = row_ptr[r], d = row_ptr[r + 1] - b;
-            for (int q = lane; q < d; q += 64) {
-                const int snd = other[b + q];
-                const uint64_t sk = (unsigned)snd < (unsigned)num_nodes ? (uint64_t)snd : (uint64_t)num_nodes;
-                keys[filled + q] = (sk << 32) | (uint64_t)(uint32_t)(b + q);
-                locals[filled + q] = (uint16_t)i;
-            }
-            filled += d;
+        constexpr int PER = kTileSortLimit / LANES;  // positions of a lane
+        for (int q = m + at_lane; q < (m + LANES - 1) / LANES * LANES; q += LANES) keys[q] = ~0ull;  // above every key
+        if (WPT == 1) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
         }
-        int padded = 64;
-        while (padded < m) padded *= 2;
-        for (int q = m + lane; q < padded; q += 64) { keys[q] = ~0ull; locals[q] = 0; }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        for (int k = 2; k <= padded; k *= 2) {
-            for (int j = k / 2; j > 0; j /= 2) {
-                // a lane per pair (q, q | j): q is the pair's number with a zero bit put in at j
-                for (int pr = lane; pr < padded / 2; pr += 64) {
-                    const int q = ((pr & ~(j - 1)) << 1) | (pr & (j - 1));
-                    const int partner = q | j;
-                    const uint64_t a = keys[q], c = keys[partner];
-                    const bool ascending = (q & k) == 0;
-                    if ((a > c) == ascending) {
-                        keys[q] = c; keys[partner] = a;
-                        const uint16_t la = locals[q];
-                        locals[q] = locals[partner]; locals[partner] = la;
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                __builtin_amdgcn_wave_barrier();
+        uint64_t mine[PER];
+        int place[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            place[k] = 0;
+            mine[k] = k * LANES < m ? keys[k * LANES + at_lane] : ~0ull;
+        }
+        for (int j = 0; j < m; j += 2) {  // (an odd m: entry m was written, LANES is even)
+            const ulonglong2 pair = *reinterpret_cast<const ulonglong2 *>(keys + j);
+#pragma unroll
+            for (int k = 0; k < PER; k++) {
+                if (k * LANES >= m) continue;
+                place[k] += (pair.x < mine[k] ? 1 : 0) + (pair.y < mine[k] ? 1 : 0);
             }
         }
-        for (int q = lane; q < m; q += 64) {
-            const uint64_t key = keys[q];
-            const int pos = (int)(uint32_t)key;
-            const uint64_t sk = key >> 32;
-            t_sender[begin + q] = sk == (uint64_t)num_nodes ? -1 : (int32_t)sk;
-            t_edge[begin + q] = perm ? perm[pos] : pos;
-            t_local[begin + q] = locals[q];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            if (k * LANES + at_lane >= m) continue;
+            const int slot = begin + place[k], pos = (int)(uint32_t)mine[k];
+            const uint64_t sk = mine[k] >> 32;
+            t_sender[slot] = sk == (uint64_t)num_nodes ? -1 : (int32_t)sk;
+            t_edge[slot] = perm ? perm[pos] : pos;
+            t_local[slot] = locals[k * LANES + at_lane];
         }
         return;
     }
+    if (at_lane >= kWave) return;  // the rest is one wave's
     // a long tile: live positions in tile order, then the padding positions
     int at = begin;
     for (int pass = 0; pass < 2; pass++) {
@@ -1032,23 +1129,25 @@ int locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nod
     const unsigned label_grid = (unsigned)(((int64_t)num_nodes * kLabelLanes + 255) / 256);
     const bool two_levels = rounds == 2 && 2 * label_bits <= 32;
     if (two_levels) {
-        // the two levels in one sort: same order as the two stable sorts below, half the passes
         hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
                            static_cast<const int32_t *>(nullptr), lab_b, nullptr, nullptr, 0);
         const bool one_block = num_nodes <= 8 * kBlockThreads;
         hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
                            lab_b, lab_a, keys_in, one_block ? nullptr : order, label_bits);
         if (one_block) {
-            auto kernel = num_nodes <= kBlockThreads       ? order_block_kernel<1>
-                          : num_nodes <= 2 * kBlockThreads ? order_block_kernel<2>
-                          : num_nodes <= 4 * kBlockThreads ? order_block_kernel<4>
-                                                           : order_block_kernel<8>;
-            hipLaunchKernelGGL(kernel, dim3(1), dim3(kBlockThreads), 0, stream, keys_in, row_ptr, num_nodes,
-                               2 * label_bits, order, pieces.cap, pieces.piece, pieces.max_segments, pieces.segments);
-            return check_hip(hipGetLastError(), "locality_order (one workgroup)");
+            // (the kernel's time is the instructions of one compute unit, for padded entries too)
+            using Launch = int (*)(const uint32_t *, const int32_t *, int, int, int32_t *, int, int, int, int32_t *,
+                                   hipStream_t);
+            static const Launch launches[8] = {launch_order_block<1>, launch_order_block<2>, launch_order_block<3>,
+                                               launch_order_block<4>, launch_order_block<5>, launch_order_block<6>,
+                                               launch_order_block<7>, launch_order_block<8>};
+            const Launch launch = launches[(num_nodes - 1) / kBlockThreads];
+            return launch(keys_in, row_ptr, num_nodes, 2 * label_bits, order, pieces.cap, pieces.piece,
+                          pieces.max_segments, pieces.segments, stream);
         }
         rc = check_hip(hipGetLastError(), "locality_order sweeps");
         if (rc) return rc;
+        // the two levels in one sort: same order as the two stable sorts below, half the passes
         size_t temp_bytes = sort_bytes;
         rc = check_hip(hipcub::DeviceRadixSort::SortPairs(sort_temp, temp_bytes, keys_in, keys_out, order, order_tmp,
                                                           (int)num_nodes, 0, 2 * label_bits, stream),
@@ -1245,8 +1344,11 @@ int e3j_amd_tile_schedule_build(const int32_t *other, const int32_t *row_ptr, co
     }
     rc = check_hip(hipGetLastError(), "tile schedule work");
     if (rc || num_edges == 0) return rc;
-    // the lists: one wave per tile sorts its positions by sender in LDS
-    hipLaunchKernelGGL(tile_lists_kernel, dim3((unsigned)((num_tiles + 3) / 4)), dim3(256), 0, stream, other, row_ptr,
+    // the lists: a workgroup per tile where a tile is longer than a wave (each of its threads then counts the
+    // keys below one or two), a wave per tile where it is not
+    const bool wide = num_edges > 64ll * num_tiles;
+    hipLaunchKernelGGL(wide ? tile_lists_kernel<4> : tile_lists_kernel<1>,
+                       dim3((unsigned)(wide ? num_tiles : (num_tiles + 3) / 4)), dim3(256), 0, stream, other, row_ptr,
                        edge_perm, row_order, packed, num_nodes, num_edges, tile_rows, num_tiles, t_sender, t_edge,
                        t_local);
     return check_hip(hipGetLastError(), "tile schedule lists");
