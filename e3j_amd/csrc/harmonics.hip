@@ -171,9 +171,10 @@ __device__ __forceinline__ float cos_pi<float>(float v) { return cospif(v); }
 template <>
 __device__ __forceinline__ double cos_pi<double>(double v) { return cospi(v); }
 
-// basis[n] and, if kGrad, dbasis[n] / dr, n = 0 .. num_basis - 1, at distance r > 0
-template <typename T, bool kGrad>
-__device__ __forceinline__ void radial_basis(T r, T cutoff, int num_basis, T *basis, T *dbasis) {
+// basis[n] and, if kGrad, dbasis[n] / dr, n = 0 .. num_basis - 1, at distance r > 0; zeros from there to NB
+// (the arrays are indexed by constants, else they would lie in scratch memory)
+template <typename T, bool kGrad, int NB>
+__device__ __forceinline__ void radial_basis(T r, T cutoff, int num_basis, T (&basis)[NB], T (&dbasis)[NB]) {
     const T t = r / cutoff;
     const T tc = t < T(1) ? t : T(1);
     const T t2 = tc * tc, t3 = t2 * tc;
@@ -181,7 +182,11 @@ __device__ __forceinline__ void radial_basis(T r, T cutoff, int num_basis, T *ba
     const T denv = t < T(1) ? (T(-30) * t2 + T(60) * t3 - T(30) * t2 * t2) / cutoff : T(0);
     const T pref = sqrt(T(2) / cutoff);
     const T inv_r = T(1) / r;
-    for (int n = 0; n < num_basis; n++) {
+#pragma unroll
+    for (int n = 0; n < NB; n++) {
+        basis[n] = T(0);
+        if (kGrad) dbasis[n] = T(0);
+        if (n >= num_basis) continue;
         const T k = T(n + 1);
         const T sn = sin_pi<T>(k * t);
         const T b = pref * sn * inv_r;
@@ -209,105 +214,191 @@ __device__ __forceinline__ bool edge_vector(const T *__restrict__ pos, const int
     return true;
 }
 
-template <typename T, int L>
-__global__ void edge_features_fwd_kernel(const T *__restrict__ pos, const int32_t *__restrict__ sender,
-                                         const int32_t *__restrict__ receiver, const T *__restrict__ shift,
-                                         const T *__restrict__ w1, EdgeFeatureSizes sz, Factors fac,
-                                         T *__restrict__ y, T *__restrict__ basis_out, T *__restrict__ h) {
-    constexpr int NOUT = (L + 1) * (L + 1);
+// Both kernels take 64 edges per workgroup of one wave.  Directions, harmonics and the radial basis are a
+// lane's own edge; every row that is wider than a lane (harmonics, hidden layers and their cotangents) crosses
+// LDS, so that the memory sees whole lines.  With a lane reading and writing its edge's rows itself, an
+// access touched 64 lines and three times the rows' bytes were written (180k edges, l <= 3, two layers of 32:
+// forward 76 us and backward 151 us; now 24 and 72).
+constexpr int kEdgeLanes = kWave;
+constexpr int kHiddenStep = 32;  // hidden units whose cotangents are staged at a time
+
+// w1[n * hidden + j] for n below num_basis, 0 for the rest of NB
+template <typename T, int NB>
+__device__ __forceinline__ void hidden_column(const T *w, int num_basis, int hidden, int j, T (&col)[NB]) {
+#pragma unroll
+    for (int n = 0; n < NB; n++) col[n] = n < num_basis ? w[n * hidden + j] : T(0);
+}
+
+template <typename T, int L, int NB>
+__global__ __launch_bounds__(kEdgeLanes) void edge_features_fwd_kernel(
+    const T *__restrict__ pos, const int32_t *__restrict__ sender, const int32_t *__restrict__ receiver,
+    const T *__restrict__ shift, const T *__restrict__ w1, EdgeFeatureSizes sz, Factors fac, T *__restrict__ y,
+    T *__restrict__ basis_out, T *__restrict__ h) {
+    constexpr int NOUT = (L + 1) * (L + 1), PITCH = NOUT | 1;
+    __shared__ __attribute__((aligned(16))) T lds_basis[kEdgeLanes][NB];
+    __shared__ T lds_y[kEdgeLanes * PITCH];
     const T cutoff = (T)sz.cutoff;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < sz.num_edges; e += stride) {
-        int a, b;
-        T v[3];
-        T *yrow = y + e * NOUT;
-        const bool live = edge_vector(pos, sender, receiver, shift, e, sz.num_nodes, a, b, v);
-        const T r = live ? sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) : T(0);
-        if (!(r > T(0))) {  // padding edge, or two atoms on one point: no direction, no features
-            for (int i = 0; i < NOUT; i++) yrow[i] = T(0);
-            if (basis_out) for (int n = 0; n < sz.num_basis; n++) basis_out[e * sz.num_basis + n] = T(0);
-            if (h) for (int l = 0; l < sz.layers; l++)
-                for (int j = 0; j < sz.hidden; j++) h[((int64_t)l * sz.num_edges + e) * sz.hidden + j] = T(0);
-            continue;
+    const int lane = threadIdx.x;
+    for (int64_t e0 = (int64_t)blockIdx.x * kEdgeLanes; e0 < sz.num_edges; e0 += (int64_t)gridDim.x * kEdgeLanes) {
+        const int64_t e = e0 + lane;
+        const int count = (int)min((int64_t)kEdgeLanes, sz.num_edges - e0);
+        T basis[NB], unused[NB];
+        {
+            int a, b;
+            T v[3];
+            const bool live = lane < count && edge_vector(pos, sender, receiver, shift, e, sz.num_nodes, a, b, v);
+            const T r = live ? sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) : T(0);
+            if (r > T(0)) {
+                const T inv = T(1) / r;
+                harmonics<L, T>(v[0] * inv, v[1] * inv, v[2] * inv, fac,
+                                [&](int index, T value) { lds_y[lane * PITCH + index] = value; });
+                radial_basis<T, false, NB>(r, cutoff, sz.num_basis, basis, unused);
+            } else {  // padding edge, or two atoms on one point: no direction, no features
+                for (int i = 0; i < NOUT; i++) lds_y[lane * PITCH + i] = T(0);
+#pragma unroll
+                for (int n = 0; n < NB; n++) basis[n] = T(0);
+            }
         }
-        const T inv = T(1) / r;
-        harmonics<L, T>(v[0] * inv, v[1] * inv, v[2] * inv, fac, [&](int index, T value) { yrow[index] = value; });
-        T basis[kMaxBasis];
-        radial_basis<T, false>(r, cutoff, sz.num_basis, basis, nullptr);
-        if (basis_out) for (int n = 0; n < sz.num_basis; n++) basis_out[e * sz.num_basis + n] = basis[n];
+#pragma unroll
+        for (int n = 0; n < NB; n++) lds_basis[lane][n] = basis[n];
+        __syncthreads();
+        for (int i = lane; i < count * NOUT; i += kEdgeLanes) y[e0 * NOUT + i] = lds_y[i / NOUT * PITCH + i % NOUT];
+        if (basis_out)
+            for (int i = lane; i < count * sz.num_basis; i += kEdgeLanes)
+                basis_out[e0 * sz.num_basis + i] = lds_basis[i / sz.num_basis][i % sz.num_basis];
         if (h) {
+            // a lane keeps its unit's weights where the units of an edge divide the wave, or fill whole waves
+            const int units = sz.hidden;
+            const bool side_by_side = units < kEdgeLanes;  // several edges at a time
+            const int edges = side_by_side ? kEdgeLanes / units : 1;
             for (int l = 0; l < sz.layers; l++) {
-                const T *w = w1 + (int64_t)l * sz.num_basis * sz.hidden;
-                T *hrow = h + ((int64_t)l * sz.num_edges + e) * sz.hidden;
-                for (int j = 0; j < sz.hidden; j++) {
-                    T pre = T(0);
-                    for (int n = 0; n < sz.num_basis; n++) pre += basis[n] * w[n * sz.hidden + j];
-                    hrow[j] = pre * sigmoid(pre);
+                const T *w = w1 + (int64_t)l * sz.num_basis * units;
+                T *rows = h + ((int64_t)l * sz.num_edges + e0) * units;
+                for (int j0 = 0; j0 < units; j0 += kEdgeLanes) {
+                    const int j = side_by_side ? lane % units : j0 + lane, first = side_by_side ? lane / units : 0;
+                    if (j >= units || first >= edges) continue;  // (no barrier in here)
+                    T col[NB];
+                    hidden_column(w, sz.num_basis, units, j, col);
+                    for (int i = first; i < count; i += edges) {
+                        T pre = T(0);
+#pragma unroll
+                        for (int n = 0; n < NB; n++) pre += lds_basis[i][n] * col[n];
+                        rows[(int64_t)i * units + j] = pre * sigmoid(pre);
+                    }
                 }
             }
         }
+        __syncthreads();  // the rows in LDS are free for the next edges
     }
 }
 
 template <typename T>
 __device__ __forceinline__ void add_to(T *p, T v) { unsafeAtomicAdd(p, v); }
 
-template <typename T, int L>
-__global__ void edge_features_bwd_kernel(const T *__restrict__ pos, const int32_t *__restrict__ sender,
-                                         const int32_t *__restrict__ receiver, const T *__restrict__ shift,
-                                         const T *__restrict__ w1, const T *__restrict__ dy,
-                                         const T *__restrict__ dbasis_in, const T *__restrict__ dh,
-                                         EdgeFeatureSizes sz, Factors fac, T *__restrict__ dpos) {
-    constexpr int NOUT = (L + 1) * (L + 1);
+template <typename T, int L, int NB>
+__global__ __launch_bounds__(kEdgeLanes) void edge_features_bwd_kernel(
+    const T *__restrict__ pos, const int32_t *__restrict__ sender, const int32_t *__restrict__ receiver,
+    const T *__restrict__ shift, const T *__restrict__ w1, const T *__restrict__ dy,
+    const T *__restrict__ dbasis_in, const T *__restrict__ dh, EdgeFeatureSizes sz, Factors fac,
+    T *__restrict__ dpos) {
+    constexpr int NOUT = (L + 1) * (L + 1), PITCH = NOUT | 1, STEP = kHiddenStep + 1;
+    constexpr int STAGE = kEdgeLanes * (PITCH > STEP ? PITCH : STEP);
+    __shared__ T stage[STAGE];
+    __shared__ T force[kEdgeLanes * 3];
+    __shared__ int ends[2][kEdgeLanes];
     const T cutoff = (T)sz.cutoff;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < sz.num_edges; e += stride) {
-        int a, b;
-        T v[3];
-        if (!edge_vector(pos, sender, receiver, shift, e, sz.num_nodes, a, b, v)) continue;
+    const int lane = threadIdx.x;
+    for (int64_t e0 = (int64_t)blockIdx.x * kEdgeLanes; e0 < sz.num_edges; e0 += (int64_t)gridDim.x * kEdgeLanes) {
+        const int64_t e = e0 + lane;
+        const int count = (int)min((int64_t)kEdgeLanes, sz.num_edges - e0);
+        int a = -1, b = -1;
+        T v[3] = {T(0), T(0), T(0)};
+        bool live = lane < count && edge_vector(pos, sender, receiver, shift, e, sz.num_nodes, a, b, v);
         const T r = sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-        if (!(r > T(0))) continue;
-        const T inv = T(1) / r;
+        live = live && r > T(0);
+        const T inv = live ? T(1) / r : T(0);
         const T u[3] = {v[0] * inv, v[1] * inv, v[2] * inv};
         T g[3] = {T(0), T(0), T(0)};
         if (dy) {  // through the harmonics of the direction: (g - u (u . g)) / r
+            for (int i = lane; i < count * NOUT; i += kEdgeLanes) stage[i / NOUT * PITCH + i % NOUT] = dy[e0 * NOUT + i];
+            __syncthreads();
             const Dual<T> dx{u[0], {T(1), T(0), T(0)}}, dyy{u[1], {T(0), T(1), T(0)}}, dz{u[2], {T(0), T(0), T(1)}};
-            const T *drow = dy + e * NOUT;
-            harmonics<L, T>(dx, dyy, dz, fac, [&](int index, const Dual<T> &value) {
-                const T w = drow[index];
-                g[0] += w * value.g[0];
-                g[1] += w * value.g[1];
-                g[2] += w * value.g[2];
-            });
+            if (live)
+                harmonics<L, T>(dx, dyy, dz, fac, [&](int index, const Dual<T> &value) {
+                    const T w = stage[lane * PITCH + index];
+                    g[0] += w * value.g[0];
+                    g[1] += w * value.g[1];
+                    g[2] += w * value.g[2];
+                });
             const T dot = u[0] * g[0] + u[1] * g[1] + u[2] * g[2];
 #pragma unroll
             for (int d = 0; d < 3; d++) g[d] = (g[d] - u[d] * dot) * inv;
+            __syncthreads();
         }
         // through the length: the radial basis and the hidden layers fed by it
-        T basis[kMaxBasis], dbdr[kMaxBasis], db[kMaxBasis];
-        radial_basis<T, true>(r, cutoff, sz.num_basis, basis, dbdr);
-        for (int n = 0; n < sz.num_basis; n++) db[n] = dbasis_in ? dbasis_in[e * sz.num_basis + n] : T(0);
+        T basis[NB], dbdr[NB], db[NB];
+        if (live) {
+            radial_basis<T, true, NB>(r, cutoff, sz.num_basis, basis, dbdr);
+        } else {
+#pragma unroll
+            for (int n = 0; n < NB; n++) basis[n] = dbdr[n] = T(0);
+        }
+#pragma unroll
+        for (int n = 0; n < NB; n++)
+            db[n] = dbasis_in && live && n < sz.num_basis ? dbasis_in[e * sz.num_basis + n] : T(0);
         if (dh) {
             for (int l = 0; l < sz.layers; l++) {
                 const T *w = w1 + (int64_t)l * sz.num_basis * sz.hidden;
-                const T *drow = dh + ((int64_t)l * sz.num_edges + e) * sz.hidden;
-                for (int j = 0; j < sz.hidden; j++) {
-                    T pre = T(0);
-                    for (int n = 0; n < sz.num_basis; n++) pre += basis[n] * w[n * sz.hidden + j];
-                    const T sg = sigmoid(pre);
-                    const T dpre = drow[j] * sg * (T(1) + pre * (T(1) - sg));
-                    for (int n = 0; n < sz.num_basis; n++) db[n] += dpre * w[n * sz.hidden + j];
+                const T *rows = dh + ((int64_t)l * sz.num_edges + e0) * sz.hidden;
+                for (int j0 = 0; j0 < sz.hidden; j0 += kHiddenStep) {
+                    const int units = min(kHiddenStep, sz.hidden - j0);
+                    if (units == kHiddenStep) {
+                        for (int i = lane; i < count * kHiddenStep; i += kEdgeLanes)
+                            stage[i / kHiddenStep * STEP + i % kHiddenStep] =
+                                rows[(int64_t)(i / kHiddenStep) * sz.hidden + j0 + i % kHiddenStep];
+                    } else {
+                        for (int i = lane; i < count * units; i += kEdgeLanes)
+                            stage[i / units * STEP + i % units] = rows[(int64_t)(i / units) * sz.hidden + j0 + i % units];
+                    }
+                    __syncthreads();
+#pragma unroll 4
+                    for (int j = 0; j < units; j++) {
+                        T col[NB];  // (the same for every lane)
+                        hidden_column(w, sz.num_basis, sz.hidden, j0 + j, col);
+                        T pre = T(0);
+#pragma unroll
+                        for (int n = 0; n < NB; n++) pre += basis[n] * col[n];
+                        const T sg = sigmoid(pre);
+                        const T dpre = (lane < count ? stage[lane * STEP + j] : T(0)) * sg * (T(1) + pre * (T(1) - sg));
+#pragma unroll
+                        for (int n = 0; n < NB; n++) db[n] += dpre * col[n];
+                    }
+                    __syncthreads();
                 }
             }
         }
         T dr = T(0);
-        for (int n = 0; n < sz.num_basis; n++) dr += db[n] * dbdr[n];
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-            const T total = g[d] + dr * u[d];
-            add_to(dpos + 3 * (int64_t)a + d, total);
-            add_to(dpos + 3 * (int64_t)b + d, -total);
+        for (int n = 0; n < NB; n++) dr += db[n] * dbdr[n];
+        // Float atomics retire per request, and a request covers the lanes that fall into one line: the three
+        // components of a node lie in neighbouring lanes, and consecutive edges of one receiver (sorted edges)
+        // are added up first.
+#pragma unroll
+        for (int d = 0; d < 3; d++) force[3 * lane + d] = g[d] + dr * u[d];
+        ends[0][lane] = live ? a : -1;
+        ends[1][lane] = live ? b : -1;
+        __syncthreads();
+#pragma unroll
+        for (int i = lane; i < 3 * kEdgeLanes; i += kEdgeLanes) {
+            const int k = i / 3, d = i % 3, node = ends[0][k], to = ends[1][k];
+            if (node >= 0) add_to(dpos + 3 * (int64_t)node + d, force[i]);
+            if (to >= 0 && (k == 0 || ends[1][k - 1] != to)) {
+                T sum = T(0);
+                for (int m = k; m < kEdgeLanes && ends[1][m] == to; m++) sum += force[3 * m + d];
+                add_to(dpos + 3 * (int64_t)to + d, -sum);
+            }
         }
+        __syncthreads();
     }
 }
 
@@ -381,19 +472,20 @@ int run(bool backward, const void *vec, const void *dout, int64_t num, int32_t l
     return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": unsupported value dtype");
 }
 
-template <typename T, int L>
+// NB: room for the radial basis (8 in registers without unused entries, or the largest size)
+template <typename T, int L, int NB>
 int launch_edge_features(bool backward, const void *pos, const int32_t *sender, const int32_t *receiver,
                          const void *shift, const void *w1, const void *a0, const void *a1, const void *a2,
                          const EdgeFeatureSizes &sz, const Factors &fac, void *r0, void *r1, void *r2,
                          hipStream_t stream) {
-    const unsigned blocks = (unsigned)std::min<int64_t>((sz.num_edges + 255) / 256, 1 << 20);
+    const unsigned blocks = (unsigned)std::min<int64_t>((sz.num_edges + kEdgeLanes - 1) / kEdgeLanes, 1 << 20);
     if (backward)
-        hipLaunchKernelGGL((edge_features_bwd_kernel<T, L>), dim3(blocks), dim3(256), 0, stream,
+        hipLaunchKernelGGL((edge_features_bwd_kernel<T, L, NB>), dim3(blocks), dim3(kEdgeLanes), 0, stream,
                            static_cast<const T *>(pos), sender, receiver, static_cast<const T *>(shift),
                            static_cast<const T *>(w1), static_cast<const T *>(a0), static_cast<const T *>(a1),
                            static_cast<const T *>(a2), sz, fac, static_cast<T *>(r0));
     else
-        hipLaunchKernelGGL((edge_features_fwd_kernel<T, L>), dim3(blocks), dim3(256), 0, stream,
+        hipLaunchKernelGGL((edge_features_fwd_kernel<T, L, NB>), dim3(blocks), dim3(kEdgeLanes), 0, stream,
                            static_cast<const T *>(pos), sender, receiver, static_cast<const T *>(shift),
                            static_cast<const T *>(w1), sz, fac, static_cast<T *>(r0), static_cast<T *>(r1),
                            static_cast<T *>(r2));
@@ -405,13 +497,20 @@ int dispatch_edge_features(int l_max, bool backward, const void *pos, const int3
                            const int32_t *receiver, const void *shift, const void *w1, const void *a0,
                            const void *a1, const void *a2, const EdgeFeatureSizes &sz, const Factors &fac,
                            void *r0, void *r1, void *r2, hipStream_t stream) {
-#define E3J_EDGE_CASE(L) \
-    case L: return launch_edge_features<T, L>(backward, pos, sender, receiver, shift, w1, a0, a1, a2, sz, fac, r0, r1, r2, stream)
+#define E3J_EDGE_ARGS backward, pos, sender, receiver, shift, w1, a0, a1, a2, sz, fac, r0, r1, r2, stream
+#define E3J_EDGE_CASE(L)                                                                  \
+    return sz.num_basis <= 8 ? launch_edge_features<T, L, 8>(E3J_EDGE_ARGS)               \
+                             : launch_edge_features<T, L, kMaxBasis>(E3J_EDGE_ARGS)
     switch (l_max) {
-        E3J_EDGE_CASE(0); E3J_EDGE_CASE(1); E3J_EDGE_CASE(2); E3J_EDGE_CASE(3); E3J_EDGE_CASE(4); E3J_EDGE_CASE(5);
-        default: return launch_edge_features<T, 6>(backward, pos, sender, receiver, shift, w1, a0, a1, a2, sz, fac,
-                                                   r0, r1, r2, stream);
+        case 0: E3J_EDGE_CASE(0);
+        case 1: E3J_EDGE_CASE(1);
+        case 2: E3J_EDGE_CASE(2);
+        case 3: E3J_EDGE_CASE(3);
+        case 4: E3J_EDGE_CASE(4);
+        case 5: E3J_EDGE_CASE(5);
+        default: E3J_EDGE_CASE(6);
     }
+#undef E3J_EDGE_ARGS
 #undef E3J_EDGE_CASE
 }
 
