@@ -59,16 +59,22 @@ int launch(const void *src, void *dst, int64_t num_nodes, int32_t rows, int32_t 
 // The mixing itself in one launch (float32, 64 or 128 channels): no regrouped copies, no library
 // calls.  A wave takes 32 nodes and one output row (degree l, component m) and runs
 // v_mfma_f32_32x32x2_f32 with the nodes as rows: lane t holds, for node t % 32, the 32 consecutive
-// channels 32 (t / 32) .. + 31 of a source row (one contiguous 128-byte read per lane: whole
-// lines of the (N, Z, K) array), and step s of the product takes channel 32 (t / 32) + s from
+// channels 32 (t / 32) .. + 31 of a source row (the row of a node is read by sixteen lanes side by
+// side and turned through LDS; with a lane reading its own 128 bytes every access touched 64 lines,
+// which the first-level cache does not hold until the next one), and step s of the product takes channel 32 (t / 32) + s from
 // every lane, which is the layout of the instruction's first operand when its two summed
 // indices are read as "channel s of the lower / of the upper half"; the second operand is the
-// matching row of the weight, 32 consecutive output channels per half wave (served by the
-// caches: a degree's weights are at most 7 x 16 KB at 64 channels).  Forward: the products of
+// matching row of the weight, 32 consecutive output channels per half wave.  The waves of a block
+// work on one output row and share its weights through LDS, 64 summed channels at a time
+// (with every wave reading them from the caches a chunk's 64 loads and its products took turns).
+// 6 000 nodes, 64 channels, 99 rows to 16: 85 -> 60 us
+// each way; the products alone take 32 us at the float32 rate of the matrix cores, the stream 35 us.  Forward: the products of
 // the mul copies of the degree accumulate into one output row.  Backward (weights transposed by
 // the caller): the cotangent row is read once and gives one product per copy.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMixDegrees = 8;
+constexpr int kMixWaves = 4;  // waves per block, 32 nodes each, on one output row
 struct MixShape {
     int32_t degrees;
     int32_t mul[kMixDegrees], dim[kMixDegrees];
@@ -80,11 +86,16 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
                                                           MixShape shape, int32_t rows_plain, int32_t rows_mixed) {
     constexpr int KC = K / 64, KT = K / 32;   // chunks of 64 summed channels, tiles of 32 output channels
     const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-    const int64_t item = (int64_t)blockIdx.x * blockDim.y + threadIdx.y;
-    const int64_t tiles = (num_nodes + 31) / 32;
-    if (item >= tiles * rows_mixed) return;  // (uniform per wave)
-    const int64_t tile = item / rows_mixed;
-    const int xr = (int)(item % rows_mixed);
+    constexpr int THREADS = kWave * kMixWaves, PIECES = 64 * K / 4 / THREADS;
+    constexpr int HALF = 32 * K + 32;  // (the halves of a wave read rows 32 apart: the pad puts them on other banks)
+    constexpr int PITCH = 64 + 4;              // (16-byte reads of 64 rows side by side spread over the banks)
+    __shared__ __attribute__((aligned(16))) float weights[2 * HALF];
+    __shared__ __attribute__((aligned(16))) float rows[kMixWaves][32 * PITCH];
+    const int tid = threadIdx.y * kWave + lane;
+    // (the waves of a block take neighbouring tiles of one output row; tiles past the last one run along)
+    const int64_t row_blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves);
+    const int64_t tile = (int64_t)blockIdx.x % row_blocks * kMixWaves + threadIdx.y;
+    const int xr = (int)(blockIdx.x / row_blocks);
     // the degree and component of mixed row xr, the first plain row and the first weight of the degree
     int l = 0, zbase = 0, xbase = 0;
     int64_t wbase = 0;
@@ -95,17 +106,30 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
         l++;
     }
     const int m = xr - xbase, mul = shape.mul[l], dim = shape.dim[l];
-    const int64_t node = tile * 32 + r;
-    const int64_t node_read = node < num_nodes ? node : num_nodes - 1;  // (lanes past the end read the last node)
-    // plain rows (N, rows_plain, K): the convolution's output / its cotangent; mixed rows (N, rows_mixed, K)
-    const float *plain_in = src + node_read * ((int64_t)rows_plain * K) + 32 * h;
-    const float *mixed_in = src + (node_read * rows_mixed + xr) * (int64_t)K + 32 * h;
-    auto load_row = [&](const float *p, float (&a)[32]) {
+    // 64 channels of a row of the wave's 32 nodes, from `first` (row of node 0) on: read in whole lines,
+    // sixteen lanes a node, and turned through LDS into the operand a lane supplies
+    auto fetch_rows = [&](const float *first, int64_t node_stride, f32x4 (&piece)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int64_t n = tile * 32 + 4 * i + lane / 16;  // (past the end: the last node)
+            piece[i] = *reinterpret_cast<const f32x4 *>(first + (n < num_nodes ? n : num_nodes - 1) * node_stride +
+                                                        lane % 16 * 4);
+        }
+    };
+    auto turn_rows = [&](const f32x4 (&piece)[8], float (&a)[32]) {
+        float *mine = rows[threadIdx.y];
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            *reinterpret_cast<f32x4 *>(mine + (4 * i + lane / 16) * PITCH + lane % 16 * 4) = piece[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int q = 0; q < 8; q++) {
-            const float4 v = *reinterpret_cast<const float4 *>(p + 4 * q);
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + r * PITCH + 32 * h + 4 * q);
             a[4 * q] = v.x; a[4 * q + 1] = v.y; a[4 * q + 2] = v.z; a[4 * q + 3] = v.w;
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     };
     auto store_tile = [&](const f32x16 (&acc)[KT], float *row0, int64_t node_stride) {
         // register v of lane t: node 8 (v / 4) + 4 (t / 32) + v % 4 of the tile, output channel t % 32 of tile ct
@@ -120,57 +144,79 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
     };
     f32x16 acc[KT];
     const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    // One chunk of 64 summed channels: the weight rows of a block of steps are read together (a
-    // read next to each product would leave the matrix unit waiting for it), then the products run.
-    constexpr int SB = K == 64 ? 32 : 16;  // steps per block: SB * KT weight registers
-    auto chunk = [&](const float (&a)[32], const float *wk) {
+    // One chunk of 64 summed channels: its weight rows lie in LDS for the waves of the block, those of
+    // the next chunk are on their way while the products of this one run.
+    const float *wl = w + wbase;
+    const int chunks = mul * KC;
+    f32x4 staged[PIECES];
+    auto fetch = [&](int q) {
 #pragma unroll
-        for (int s0 = 0; s0 < 32; s0 += SB) {
-            float b[SB][KT];
+        for (int i = 0; i < PIECES; i++)
+            staged[i] = *reinterpret_cast<const f32x4 *>(wl + (int64_t)q * (64 * K) + (i * THREADS + tid) * 4);
+    };
+    auto commit = [&]() {
 #pragma unroll
-            for (int s = 0; s < SB; s++) {
-#pragma unroll
-                for (int ct = 0; ct < KT; ct++) b[s][ct] = wk[(int64_t)(s0 + s) * K + ct * 32];
-            }
-            asm volatile("" ::: "memory");  // (the reads above are issued before the products below)
-#pragma unroll
-            for (int s = 0; s < SB; s++) {
-#pragma unroll
-                for (int ct = 0; ct < KT; ct++)
-                    acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s0 + s], b[s][ct], acc[ct], 0, 0, 0);
-            }
+        for (int i = 0; i < PIECES; i++) {
+            const int at = (i * THREADS + tid) * 4;
+            *reinterpret_cast<f32x4 *>(&weights[at + (at >= 32 * K ? 32 : 0)]) = staged[i];
         }
     };
+    auto products = [&](const float (&a)[32]) {
+        const float *wk = &weights[h * HALF + r];
+#pragma unroll
+        for (int s = 0; s < 32; s++) {
+#pragma unroll
+            for (int ct = 0; ct < KT; ct++)
+                acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], wk[s * K + ct * 32], acc[ct], 0, 0, 0);
+        }
+    };
+    // after the products of a chunk: its weights make room for those of the next
+    auto next_chunk = [&](int q) {
+        __syncthreads();
+        if (q < chunks) commit();
+        __syncthreads();
+    };
+    fetch(0);
+    commit();
+    const int64_t plain_stride = (int64_t)rows_plain * K, mixed_stride = (int64_t)rows_mixed * K;
+    f32x4 piece[8];
     if (!kTranspose) {
 #pragma unroll
         for (int ct = 0; ct < KT; ct++) acc[ct] = zero;
-        // (u, chunk) pairs in one sequence, the source row of the next pair read while the products of
-        // the one at hand run
-        const int pairs = mul * KC;
-        float a[32], ahead[32];
-        load_row(plain_in + (int64_t)(zbase + m) * K, a);
-        for (int q = 0; q < pairs; q++) {
-            const int u = q / KC, kc = q % KC;
-            if (q + 1 < pairs) {
-                const int un = (q + 1) / KC, kn = (q + 1) % KC;
-                load_row(plain_in + (int64_t)(zbase + un * dim + m) * K + kn * 64, ahead);
+        // the source row of the next chunk is read while the products of the one at hand run
+        auto row_of = [&](int q) { return src + (int64_t)(zbase + q / KC * dim + m) * K + q % KC * 64; };
+        fetch_rows(row_of(0), plain_stride, piece);
+        __syncthreads();
+        for (int q = 0; q < chunks; q++) {
+            float a[32];
+            turn_rows(piece, a);
+            if (q + 1 < chunks) {
+                fetch(q + 1);
+                fetch_rows(row_of(q + 1), plain_stride, piece);
             }
-            chunk(a, w + wbase + (int64_t)u * K * K + (int64_t)(kc * 64 + 32 * h) * K + r);
-#pragma unroll
-            for (int s = 0; s < 32; s++) a[s] = ahead[s];
+            products(a);
+            next_chunk(q + 1);
         }
-        store_tile(acc, dst + (int64_t)xr * K, (int64_t)rows_mixed * K);
+        store_tile(acc, dst + (int64_t)xr * K, mixed_stride);
     } else {
         float a[KC][32];
 #pragma unroll
-        for (int kc = 0; kc < KC; kc++) load_row(mixed_in + kc * 64, a[kc]);
+        for (int kc = 0; kc < KC; kc++) {
+            fetch_rows(src + (int64_t)xr * K + kc * 64, mixed_stride, piece);
+            turn_rows(piece, a[kc]);
+        }
+        __syncthreads();
         for (int u = 0; u < mul; u++) {
-            const float *wu = w + wbase + (int64_t)u * K * K;  // (transposed: [output channel c of the mixing][k])
 #pragma unroll
             for (int ct = 0; ct < KT; ct++) acc[ct] = zero;
 #pragma unroll
-            for (int kc = 0; kc < KC; kc++) chunk(a[kc], wu + (int64_t)(kc * 64 + 32 * h) * K + r);
-            store_tile(acc, dst + (int64_t)(zbase + u * dim + m) * K, (int64_t)rows_plain * K);
+            for (int kc = 0; kc < KC; kc++) {
+                const int q = u * KC + kc;
+                if (q + 1 < chunks) fetch(q + 1);
+                products(a[kc]);
+                next_chunk(q + 1);
+            }
+            store_tile(acc, dst + (int64_t)(zbase + u * dim + m) * K, plain_stride);
         }
     }
 }
@@ -178,15 +224,13 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
 template <int K>
 int launch_mix(const float *src, float *dst, const float *w, int64_t num_nodes, const MixShape &shape,
                int rows_plain, int rows_mixed, bool transpose, hipStream_t stream) {
-    constexpr int kWavesPerBlock = 4;
-    const int64_t items = (num_nodes + 31) / 32 * rows_mixed;
-    const int64_t blocks = (items + kWavesPerBlock - 1) / kWavesPerBlock;
+    const int64_t blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves) * rows_mixed;
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: too many nodes for one launch");
     if (transpose)
-        hipLaunchKernelGGL((channel_mix_kernel<K, true>), dim3((unsigned)blocks), dim3(kWave, kWavesPerBlock), 0, stream,
+        hipLaunchKernelGGL((channel_mix_kernel<K, true>), dim3((unsigned)blocks), dim3(kWave, kMixWaves), 0, stream,
                            src, dst, w, num_nodes, shape, rows_plain, rows_mixed);
     else
-        hipLaunchKernelGGL((channel_mix_kernel<K, false>), dim3((unsigned)blocks), dim3(kWave, kWavesPerBlock), 0, stream,
+        hipLaunchKernelGGL((channel_mix_kernel<K, false>), dim3((unsigned)blocks), dim3(kWave, kMixWaves), 0, stream,
                            src, dst, w, num_nodes, shape, rows_plain, rows_mixed);
     return check_hip(hipGetLastError(), "channel_mix launch");
 }
