@@ -64,6 +64,8 @@ LAUNCH = {
 #: parts of the float64 kernels: (forward, backward).  A double takes the registers of two channels
 #: of a float kernel, so these are the splits the two-channel float kernels use.
 F64_SPLIT = (3, 4)
+#: float64 backward over tiles of receivers: (waves per block, resident waves per SIMD, receivers per tile)
+F64_TILE = (4, 1, 4)
 #: float16 kernels (values held as half, computed in float): (channels per lane, parts forward,
 #: parts backward) by whether the channel count is a multiple of 128; the splits of the float
 #: kernels with as many channels per lane
@@ -651,6 +653,10 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
                                 for ln in lines]
         out += [f"template __global__ void unrolled_fwd_f64_kernel<{channels}, 4, {part_names[F64_SPLIT[0]]}>("] + as_f64(fwd_args)
         out += [f"template __global__ void unrolled_bwd_f64_kernel<{channels}, 4, {part_names[F64_SPLIT[1]]}>("] + as_f64(bwd_args)
+        out += [f"template __global__ void unrolled_bwd_tile_f64_kernel<{channels}, {F64_TILE[0]}, {F64_TILE[1]}, "
+                f"{part_names[F64_SPLIT[1]]}>("]
+        out += [ln.replace("float *", "double *").replace("int, float, unsigned);", "int, unsigned, F64Coefs);")
+                for ln in tile_args]
     if lead:
         for wpb, zs in lead["fwd"]:
             out += [f"template __global__ void unrolled_fwd_leading_kernel<{channels}, {wpb}, {part_names[zs]}>("] + fwd_args
@@ -706,6 +712,15 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
                 "                       const int32_t *perm, double *dx, double *dy, double *ds, hipStream_t stream) {",
                 f"    return launch_unrolled_bwd_f64<{channels}, 4, {t.Y}, {t.X}, {part_names[F64_SPLIT[1]]}>(",
                 "        p, x, y, s, dm, sender, row_ptr, perm, dx, dy, ds, stream);",
+                "}",
+                "static int run_bwd_tiled_f64(const e3j_amd_conv_params &p, const double *x, const double *y,",
+                "                             const double *s, const double *dm, const int32_t *sender,",
+                "                             const int32_t *row_ptr, const int32_t *perm,",
+                "                             const e3j_amd_tile_schedule &schedule, double *dx, double *dy, double *ds,",
+                "                             hipStream_t stream) {",
+                f"    return launch_unrolled_bwd_tile_f64<{channels}, {F64_TILE[0]}, {F64_TILE[1]}, "
+                f"{part_names[F64_SPLIT[1]]}>(",
+                "        p, x, y, s, dm, sender, row_ptr, perm, schedule, dx, dy, ds, stream);",
                 "}", ""]
     out += ["static int run_fwd" + fwd_sig[0]] + fwd_sig[1:]
     out += [ln.replace("VARIANT", "tuning().fwd_variant.load(std::memory_order_relaxed)") for ln in switch(
@@ -755,6 +770,8 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
             f"    {t.X}, {t.Y}, {t.Z}, {t.S}, {len(t.val)}, {channels}, E3J_AMD_LAYOUT_TRAILING, kVal, kIdx,",
             f"    &run_fwd, &run_bwd, {tiled}, &run_bwd_sender,",
             f"    {len(t.classes)}, kClass, &run_fwd_f64, &run_bwd_f64," if f64 else "    0, nullptr, nullptr, nullptr,",
+            f"    &run_bwd_tiled_f64, tile_row_bytes<1, {part_names[F64_SPLIT[1]]}>((int)sizeof(double)), {F64_TILE[2]},"
+            if f64 else "    nullptr, 0, 0,",
             "    &run_fwd_f16, &run_bwd_f16," if f16 else "    nullptr, nullptr,",
             "    &run_second_dm, &run_second_tile," if tile else "    nullptr, nullptr,",
             "};", ""]

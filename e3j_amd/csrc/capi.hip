@@ -532,15 +532,25 @@ int32_t e3j_amd_tile_rows_default(int32_t sig) {
     return want < 1 ? 1 : want > limit ? limit : want;
 }
 
-int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, const void *y,
-                                  const void *s, const void *dm, const int32_t *sender,
-                                  const int32_t *receiver_ptr, const int32_t *edge_perm,
-                                  const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
-                                  void *stream_) {
-    const char *op = "convolution_bwd_tiled";
+int32_t e3j_amd_tile_rows_f64(int32_t sig) {
+    if (sig < 0 || sig >= num_signatures()) return 0;
+    const Signature &sg = signature(sig);
+    return sg.bwd_tiled_f64 != nullptr && sg.tile_row_bytes_f64 > 0 ? (int32_t)(160 * 1024 / sg.tile_row_bytes_f64) : 0;
+}
+
+int32_t e3j_amd_tile_rows_default_f64(int32_t sig) {
+    const int32_t limit = e3j_amd_tile_rows_f64(sig);
+    // (at most half the LDS of a compute unit: with one workgroup there, nothing hides its loads)
+    return limit <= 0 ? 0 : std::max(1, std::min(signature(sig).tile_rows_f64, limit / 2));
+}
+
+namespace {
+int run_tiled(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s, const void *dm,
+              const int32_t *sender, const int32_t *receiver_ptr, const int32_t *edge_perm,
+              const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds, hipStream_t stream, bool f64) {
+    const char *op = f64 ? "convolution_bwd_tiled_f64" : "convolution_bwd_tiled";
     int rc = validate(p, op);
     if (rc) return rc;
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
     if (p->num_nodes == 0 && p->num_edges == 0) return E3J_AMD_OK;
     if (missing(x, p->num_nodes) || missing(dm, p->num_nodes) || missing(dx, p->num_nodes) ||
         receiver_ptr == nullptr || missing(sender, p->num_edges) || missing(y, p->num_edges) ||
@@ -548,22 +558,53 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
         schedule == nullptr)
         return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": null operand");
     if (p->num_nodes == 0) return E3J_AMD_OK;
-    if (p->signature < 0 || p->val_dtype != E3J_AMD_F32 || signature(p->signature).bwd_tiled == nullptr)
+    if (f64 && (p->signature < 0 || p->val_dtype != E3J_AMD_F64 || signature(p->signature).bwd_tiled_f64 == nullptr))
+        return set_error(E3J_AMD_UNIMPLEMENTED,
+                         std::string(op) + ": needs a float64 compile-time-unrolled kernel of the trailing layout; "
+                                           "e3j_amd_convolution_bwd_receiver serves the other cases");
+    if (!f64 && (p->signature < 0 || p->val_dtype != E3J_AMD_F32 || signature(p->signature).bwd_tiled == nullptr))
         return set_error(E3J_AMD_UNIMPLEMENTED,
                          std::string(op) + ": needs a float32 compile-time-unrolled kernel of the trailing layout "
                                            "with at least 64 channels; e3j_amd_convolution_bwd_receiver "
                                            "serves the other cases");
-    if (!aligned16({x, s, dm, dx, ds}))
+    if (!f64 && !aligned16({x, s, dm, dx, ds}))  // (rows of doubles are moved element by element)
         return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": operands must be 16-byte aligned");
     if (schedule->num_work < 0 || (schedule->num_work > 0 && schedule->work == nullptr) ||
         missing(schedule->sender, p->num_edges) || missing(schedule->edge, p->num_edges) ||
         missing(schedule->local, p->num_edges))
         return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": incomplete schedule");
+    if (f64) {
+        rc = signature(p->signature).bwd_tiled_f64(*p, static_cast<const double *>(x), static_cast<const double *>(y),
+                                                   static_cast<const double *>(s), static_cast<const double *>(dm),
+                                                   sender, receiver_ptr, edge_perm, *schedule,
+                                                   static_cast<double *>(dx), static_cast<double *>(dy),
+                                                   static_cast<double *>(ds), stream);
+        return finish(p, stream, rc, op);
+    }
     rc = signature(p->signature).bwd_tiled(*p, static_cast<const float *>(x), static_cast<const float *>(y),
                                            static_cast<const float *>(s), static_cast<const float *>(dm),
                                            sender, receiver_ptr, edge_perm, *schedule, static_cast<float *>(dx),
                                            static_cast<float *>(dy), static_cast<float *>(ds), stream);
     return finish(p, stream, rc, op);
+}
+}  // namespace
+
+int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, const void *y,
+                                  const void *s, const void *dm, const int32_t *sender,
+                                  const int32_t *receiver_ptr, const int32_t *edge_perm,
+                                  const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
+                                  void *stream) {
+    return run_tiled(p, x, y, s, dm, sender, receiver_ptr, edge_perm, schedule, dx, dy, ds,
+                     static_cast<hipStream_t>(stream), false);
+}
+
+int e3j_amd_convolution_bwd_tiled_f64(const e3j_amd_conv_params *p, const void *x, const void *y,
+                                      const void *s, const void *dm, const int32_t *sender,
+                                      const int32_t *receiver_ptr, const int32_t *edge_perm,
+                                      const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
+                                      void *stream) {
+    return run_tiled(p, x, y, s, dm, sender, receiver_ptr, edge_perm, schedule, dx, dy, ds,
+                     static_cast<hipStream_t>(stream), true);
 }
 
 int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s,

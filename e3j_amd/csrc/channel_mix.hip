@@ -61,16 +61,16 @@ int launch(const void *src, void *dst, int64_t num_nodes, int32_t rows, int32_t 
 // v_mfma_f32_32x32x2_f32 with the nodes as rows: lane t holds, for node t % 32, the 32 consecutive
 // channels 32 (t / 32) .. + 31 of a source row (the row of a node is read by sixteen lanes side by
 // side and turned through LDS; with a lane reading its own 128 bytes every access touched 64 lines,
-// which the first-level cache does not hold until the next one), and step s of the product takes channel 32 (t / 32) + s from
-// every lane, which is the layout of the instruction's first operand when its two summed
-// indices are read as "channel s of the lower / of the upper half"; the second operand is the
-// matching row of the weight, 32 consecutive output channels per half wave.  The waves of a block
-// work on one output row and share its weights through LDS, 64 summed channels at a time
-// (with every wave reading them from the caches a chunk's 64 loads and its products took turns).
-// 6 000 nodes, 64 channels, 99 rows to 16: 85 -> 60 us
-// each way; the products alone take 32 us at the float32 rate of the matrix cores, the stream 35 us.  Forward: the products of
-// the mul copies of the degree accumulate into one output row.  Backward (weights transposed by
-// the caller): the cotangent row is read once and gives one product per copy.
+// which the first-level cache does not hold until the next one), and step s of the product takes
+// channel 32 (t / 32) + s from every lane, which is the layout of the instruction's first operand when
+// its two summed indices are read as "channel s of the lower / of the upper half"; the second operand is
+// the matching row of the weight, 32 consecutive output channels per half wave.  The waves of a block
+// work on one output row and share its weights through LDS, 64 summed channels at a time (with every
+// wave reading them from the caches a chunk's 64 loads and its products took turns).
+// 6 000 nodes, 64 channels, 99 rows to 16: 85 -> 60 us each way; the products alone take 32 us at the
+// float32 rate of the matrix cores, the stream 35 us.  Forward: the products of the mul copies of the
+// degree accumulate into one output row.  Backward (weights transposed by the caller): the cotangent row
+// is read once and gives one product per copy.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMixDegrees = 8;

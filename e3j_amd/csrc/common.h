@@ -201,6 +201,12 @@ struct Signature {
     int (*bwd_f64)(const e3j_amd_conv_params &p, const double *x, const double *y, const double *s,
                    const double *dm, const int32_t *sender, const int32_t *receiver_ptr,
                    const int32_t *edge_perm, double *dx, double *dy, double *ds, hipStream_t stream);
+    // its backward over tiles of receivers, the LDS bytes of a tile row, receivers per tile by default
+    int (*bwd_tiled_f64)(const e3j_amd_conv_params &p, const double *x, const double *y, const double *s,
+                         const double *dm, const int32_t *sender, const int32_t *receiver_ptr,
+                         const int32_t *edge_perm, const e3j_amd_tile_schedule &schedule, double *dx, double *dy,
+                         double *ds, hipStream_t stream);
+    int32_t tile_row_bytes_f64, tile_rows_f64;
     // float16 kernels (trailing layout, receiver rows; nullptr: none): values held as half, the float
     // kernels' arithmetic, literals and scale factor
     int (*fwd_f16)(const e3j_amd_conv_params &p, const half_t *x, const half_t *y, const half_t *s,

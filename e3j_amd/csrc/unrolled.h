@@ -194,24 +194,41 @@ __device__ __forceinline__ void store_stream<4>(float *p, const Vec<4> &a) {
 // Backward: the C channels of a lane lie a wave apart (lane, lane + 64, ...), so each of the C
 // accesses of a wave is one coalesced 256-byte piece of a row and every float atomic request
 // carries 16 values (atomics retire per 64-byte request, whatever it holds).
-template <int C>
-__device__ __forceinline__ Vec<C> load_apart(const float *p) {
-    Vec<C> r;
+template <int C, typename T>
+__device__ __forceinline__ Vec<C, T> load_apart(const T *p) {
+    Vec<C, T> r;
 #pragma unroll
     for (int t = 0; t < C; t++) r.v[t] = p[t * kWave];
     return r;
 }
-template <int C>
-__device__ __forceinline__ Vec<C> load_apart_stream(const float *p) {
-    Vec<C> r;
+template <int C, typename T>
+__device__ __forceinline__ Vec<C, T> load_apart_stream(const T *p) {
+    Vec<C, T> r;
 #pragma unroll
     for (int t = 0; t < C; t++) r.v[t] = __builtin_nontemporal_load(p + t * kWave);
     return r;
 }
-template <int C>
-__device__ __forceinline__ void store_apart_stream(float *p, const Vec<C> &a) {
+template <int C, typename T>
+__device__ __forceinline__ void store_apart_stream(T *p, const Vec<C, T> &a) {
 #pragma unroll
     for (int t = 0; t < C; t++) __builtin_nontemporal_store(a.v[t], p + t * kWave);
+}
+// a lane's values side by side in LDS
+template <int C>
+__device__ __forceinline__ Vec<C> load_lds(const float *p) { return load_vec<C>(p); }
+template <int C>
+__device__ __forceinline__ Vec<C, double> load_lds(const double *p) {
+    Vec<C, double> r;
+#pragma unroll
+    for (int t = 0; t < C; t++) r.v[t] = p[t];
+    return r;
+}
+template <int C>
+__device__ __forceinline__ void store_lds(float *p, const Vec<C> &a) { store_vec<C>(p, a); }
+template <int C>
+__device__ __forceinline__ void store_lds(double *p, const Vec<C, double> &a) {
+#pragma unroll
+    for (int t = 0; t < C; t++) p[t] = a.v[t];
 }
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -239,7 +256,17 @@ __device__ __forceinline__ float flip_sign(float v, unsigned flip, int k) {
     return __uint_as_float(__float_as_uint(v) ^ (((flip >> k) & 1u) << 31));
 }
 
+__device__ __forceinline__ double flip_sign(double v, unsigned flip, int k) {
+    if (k >= 32) return v;
+    const unsigned long long bit = (unsigned long long)((flip >> k) & 1u) << 63;
+    return __longlong_as_double((long long)((unsigned long long)__double_as_longlong(v) ^ bit));
+}
+
 __device__ __forceinline__ float to_vgpr(float v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+__device__ __forceinline__ double to_vgpr(double v) {
     asm volatile("" : "+v"(v));
     return v;
 }
@@ -603,12 +630,12 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_fwd_kernel(
 
 // Where the generated arithmetic puts the ds value of path L (trailing layout: straight
 // into the edge's row of ds).
-template <int CPL, int K>
+template <int CPL, int K, typename T = float>
 struct DsRows {
-    float *row;
+    T *row;
     bool active;
     template <int L>
-    __device__ __forceinline__ void put(const Vec<CPL> &v) const {
+    __device__ __forceinline__ void put(const Vec<CPL, T> &v) const {
         if (active) store_apart_stream<CPL>(row + L * K, v);
     }
 };
@@ -906,27 +933,28 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_bwd_sender_kernel(
 // are written as in the kernel above.  One barrier per block (after the tile is staged).
 
 // The dm rows of one receiver of the tile as the generated arithmetic indexes them.
-template <int CPL>
+template <int CPL, typename T = float>
 struct DmTile {
-    const float *row;  // LDS: this lane's CPL values of the receiver's first staged row
-    __device__ __forceinline__ Vec<CPL> operator[](int i) const {
-        return load_vec<CPL>(row + i * (kWave * CPL));
+    const T *row;  // LDS: this lane's CPL values of the receiver's first staged row
+    __device__ __forceinline__ Vec<CPL, T> operator[](int i) const {
+        return load_lds<CPL>(row + i * (kWave * CPL));
     }
 };
 
-template <typename Part, int K, int CPL, bool kAtomicDy>
+// (T = double, with the coefficient classes `cf`: the float64 form, one channel per lane)
+template <typename Part, int K, int CPL, bool kAtomicDy, typename T>
 __device__ __forceinline__ void unrolled_bwd_tile_part(
-    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ s,
-    const float *__restrict__ dm, const int32_t *__restrict__ t_sender,
+    const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ s,
+    const T *__restrict__ dm, const int32_t *__restrict__ t_sender,
     const int32_t *__restrict__ t_edge, const int32_t *__restrict__ t_local,
-    const int32_t *__restrict__ row_order, float *__restrict__ dx, float *__restrict__ dy,
-    float *__restrict__ ds, int num_nodes, float scale, unsigned y_flip, int tile, int tile_rows,
-    int begin, int end, int slice, float *tile_lds) {
+    const int32_t *__restrict__ row_order, T *__restrict__ dx, T *__restrict__ dy,
+    T *__restrict__ ds, int num_nodes, T scale, unsigned y_flip, int tile, int tile_rows,
+    int begin, int end, int slice, T *tile_lds, const double *cf) {
     constexpr int NX = Part::NX, NS = Part::NS, NZ = Part::NZ, Y = Part::Y;
     constexpr int X = Part::X, S = Part::S, Z = Part::Z;
-    using V = Vec<CPL>;
+    using V = Vec<CPL, T>;
     using SL = Slice<K, CPL>;
-    using Red = WaveReduceBlocks<Y, kWave>;
+    using Red = WaveReduceBlocks<Y, kWave, T>;
     constexpr int WIDTH = SL::WIDTH;
     static_assert(SL::SUB == 1, "the tile kernel takes whole waves of channels");
     static_assert(CPL == 1 || SL::FULL, "several channels per lane need whole slices");
@@ -951,7 +979,7 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
     while (hi > lo && !((unsigned)load_uniform(t_sender + hi - 1) < (unsigned)num_nodes)) hi--;
 
     V xc[NX], xn[NX], sn[NS], acc[NX];
-    float yn[Y];
+    T yn[Y];
     bool valid_n = false, newx_n = false;
     int snd_n = 0, loc_n = 0;
     int64_t ee_n = 0;
@@ -976,12 +1004,12 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
         loc_n = loc_a;
         newx_n = valid_n && snd != held;
         if (newx_n) {
-            const float *xr = x + (int64_t)snd * (X * K) + c0;
+            const T *xr = x + (int64_t)snd * (X * K) + c0;
 #pragma unroll
             for (int j = 0; j < NX; j++) xn[j] = load_apart<CPL>(xr + Part::kX[j] * K);
         }
-        const float *sr = s + ee_n * (int64_t)(S * K) + c0;
-        const float *yr = y + ee_n * Y;
+        const T *sr = s + ee_n * (int64_t)(S * K) + c0;
+        const T *yr = y + ee_n * Y;
 #pragma unroll
         for (int l = 0; l < NS; l++) sn[l] = load_apart_stream<CPL>(sr + Part::kS[l] * K);
 #pragma unroll
@@ -989,7 +1017,7 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
     };
     auto flush = [&](int snd) {
         if (!active) return;
-        float *dxr = dx + (int64_t)snd * (X * K) + c0;
+        T *dxr = dx + (int64_t)snd * (X * K) + c0;
 #pragma unroll
         for (int j = 0; j < NX; j++) {
 #pragma unroll
@@ -1010,14 +1038,14 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
         const int rows = num_nodes - first < tile_rows ? num_nodes - first : tile_rows;
         for (int t = wave; t < rows; t += nw) {
             const int r = row_order ? row_order[first + t] : first + t;
-            const float *zr = dm + (int64_t)r * (Z * K) + c0;
-            float *dst = tile_lds + t * (NZ * WIDTH) + lane * CPL;
+            const T *zr = dm + (int64_t)r * (Z * K) + c0;
+            T *dst = tile_lds + t * (NZ * WIDTH) + lane * CPL;
             V v[NZ];
 #pragma unroll
             for (int i = 0; i < NZ; i++) v[i] = load_apart_stream<CPL>(zr + Part::kZ[i] * K);
 #pragma unroll
             for (int i = 0; i < NZ; i++)  // idle lanes must add nothing to dy
-                store_vec<CPL>(dst + i * WIDTH, active ? vmul(v[i], scale) : vzero<CPL>());
+                store_lds<CPL>(dst + i * WIDTH, active ? vmul(v[i], scale) : vzero<CPL, T>());
         }
     }
     __syncthreads();
@@ -1026,7 +1054,7 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
 
     for (int pos = lo; pos < hi; pos++) {
         V sc[NS];
-        float yc[Y];
+        T yc[Y];
         if (newx_n) {
 #pragma unroll
             for (int j = 0; j < NX; j++) xc[j] = xn[j];
@@ -1049,16 +1077,19 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
             if (run >= 0) flush(run);
             run = snd;
 #pragma unroll
-            for (int j = 0; j < NX; j++) acc[j] = vzero<CPL>();
+            for (int j = 0; j < NX; j++) acc[j] = vzero<CPL, T>();
         }
-        float dye[Red::P];
-        const DsRows<CPL, K> ds_rows{ds + ee * (int64_t)(S * K) + c0, active};
-        const DmTile<CPL> dm_rows{tile_lds + loc * (NZ * WIDTH) + lane * CPL};
-        Part::template edge_bwd<CPL, true, true>(xc, yc, sc, dm_rows, acc, dye, ds_rows);  // adds to the run's sums
+        T dye[Red::P];
+        const DsRows<CPL, K, T> ds_rows{ds + ee * (int64_t)(S * K) + c0, active};
+        const DmTile<CPL, T> dm_rows{tile_lds + loc * (NZ * WIDTH) + lane * CPL};
+        if constexpr (std::is_same<T, double>::value)  // adds to the run's sums
+            Part::template edge_bwd_f64<true, true>(xc, yc, sc, dm_rows, acc, dye, ds_rows, cf);
+        else
+            Part::template edge_bwd<CPL, true, true>(xc, yc, sc, dm_rows, acc, dye, ds_rows);
 #pragma unroll
-        for (int k = Y; k < Red::P; k++) dye[k] = 0.f;
-        Red::run(dye, lane, [&](int k, float sum) {
-            const float total = flip_sign(sum, y_flip, k);
+        for (int k = Y; k < Red::P; k++) dye[k] = T(0);
+        Red::run(dye, lane, [&](int k, T sum) {
+            const T total = flip_sign(sum, y_flip, k);
             if (!kAtomicDy) dy[ee * Y + k] = total;
             else unsafeAtomicAdd(dy + ee * Y + k, total);  // dy zero-filled by the launcher
         });
@@ -1066,40 +1097,34 @@ __device__ __forceinline__ void unrolled_bwd_tile_part(
     if (run >= 0) flush(run);
 }
 
-template <int K, int CPL, bool A, int I>
-__device__ __forceinline__ void dispatch_bwd_tile(int, const float *, const float *, const float *,
-                                                  const float *, const int32_t *, const int32_t *,
-                                                  const int32_t *, const int32_t *, float *, float *,
-                                                  float *, int, float, unsigned, int, int, int, int, int,
-                                                  float *) {}
-template <int K, int CPL, bool A, int I, typename Part, typename... Rest>
-__device__ __forceinline__ void dispatch_bwd_tile(int part, const float *x, const float *y, const float *s,
-                                                  const float *dm, const int32_t *t_sender,
-                                                  const int32_t *t_edge, const int32_t *t_local,
-                                                  const int32_t *row_order, float *dx, float *dy,
-                                                  float *ds, int num_nodes, float scale, unsigned y_flip,
-                                                  int tile, int tile_rows, int begin, int end, int slice,
-                                                  float *tile_lds) {
+template <int K, int CPL, bool A, int I, typename T>
+__device__ __forceinline__ void dispatch_bwd_tile(int, const T *, const T *, const T *, const T *, const int32_t *,
+                                                  const int32_t *, const int32_t *, const int32_t *, T *, T *, T *,
+                                                  int, same_t<T>, unsigned, int, int, int, int, int, T *,
+                                                  const double *) {}
+template <int K, int CPL, bool A, int I, typename Part, typename... Rest, typename T>
+__device__ __forceinline__ void dispatch_bwd_tile(int part, const T *x, const T *y, const T *s, const T *dm,
+                                                  const int32_t *t_sender, const int32_t *t_edge,
+                                                  const int32_t *t_local, const int32_t *row_order, T *dx, T *dy,
+                                                  T *ds, int num_nodes, same_t<T> scale, unsigned y_flip, int tile,
+                                                  int tile_rows, int begin, int end, int slice, T *tile_lds,
+                                                  const double *cf) {
     if (part == I)
         unrolled_bwd_tile_part<Part, K, CPL, A>(x, y, s, dm, t_sender, t_edge, t_local, row_order, dx, dy,
                                                 ds, num_nodes, scale, y_flip, tile, tile_rows, begin, end,
-                                                slice, tile_lds);
+                                                slice, tile_lds, cf);
     else
         dispatch_bwd_tile<K, CPL, A, I + 1, Rest...>(part, x, y, s, dm, t_sender, t_edge, t_local,
                                                      row_order, dx, dy, ds, num_nodes, scale, y_flip,
-                                                     tile, tile_rows, begin, end, slice, tile_lds);
+                                                     tile, tile_rows, begin, end, slice, tile_lds, cf);
 }
 
 // One block per (work item, channel slice, part); a work item is a piece of one tile's edge list.
-template <int K, int CPL, int WPB, int MINW, typename... Parts>
-__global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_bwd_tile_kernel(
-    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ s,
-    const float *__restrict__ dm, const int32_t *__restrict__ work,
-    const int32_t *__restrict__ t_sender, const int32_t *__restrict__ t_edge,
-    const int32_t *__restrict__ t_local, const int32_t *__restrict__ row_order,
-    float *__restrict__ dx, float *__restrict__ dy, float *__restrict__ ds, int num_nodes,
-    int tile_rows, int num_work, float scale, unsigned y_flip) {
-    extern __shared__ __attribute__((aligned(16))) float tile_lds[];
+template <int K, int CPL, typename... Parts, typename T>
+__device__ __forceinline__ void unrolled_bwd_tile_block(
+    const T *x, const T *y, const T *s, const T *dm, const int32_t *work, const int32_t *t_sender,
+    const int32_t *t_edge, const int32_t *t_local, const int32_t *row_order, T *dx, T *dy, T *ds, int num_nodes,
+    int tile_rows, int num_work, same_t<T> scale, unsigned y_flip, T *tile_lds, const double *cf) {
     constexpr int NP = sizeof...(Parts);
     constexpr int CW = Slice<K, CPL>::COUNT;
     constexpr bool kAtomicDy = NP * CW > 1;  // several waves add into one dy row
@@ -1118,7 +1143,19 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_bwd_tile_kernel(
     if (begin >= end) return;  // unused descriptor or a tile without edges (uniform over the block)
     dispatch_bwd_tile<K, CPL, kAtomicDy, 0, Parts...>(part, x, y, s, dm, t_sender, t_edge, t_local,
                                                       row_order, dx, dy, ds, num_nodes, scale, y_flip,
-                                                      tile, tile_rows, begin, end, slice, tile_lds);
+                                                      tile, tile_rows, begin, end, slice, tile_lds, cf);
+}
+template <int K, int CPL, int WPB, int MINW, typename... Parts>
+__global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_bwd_tile_kernel(
+    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ s,
+    const float *__restrict__ dm, const int32_t *__restrict__ work,
+    const int32_t *__restrict__ t_sender, const int32_t *__restrict__ t_edge,
+    const int32_t *__restrict__ t_local, const int32_t *__restrict__ row_order,
+    float *__restrict__ dx, float *__restrict__ dy, float *__restrict__ ds, int num_nodes,
+    int tile_rows, int num_work, float scale, unsigned y_flip) {
+    extern __shared__ __attribute__((aligned(16))) float tile_lds[];
+    unrolled_bwd_tile_block<K, CPL, Parts...>(x, y, s, dm, work, t_sender, t_edge, t_local, row_order, dx, dy, ds,
+                                              num_nodes, tile_rows, num_work, scale, y_flip, tile_lds, nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1719,8 +1756,8 @@ constexpr size_t kMaxTileLds = 160 * 1024;  // LDS of a CU, all of which one blo
 
 // LDS bytes per receiver of a tile (the part with the most dm rows decides).
 template <int CPL, typename... Parts>
-constexpr int tile_row_bytes() {
-    return max_of({Parts::NZ...}) * kWave * CPL * (int)sizeof(float);
+constexpr int tile_row_bytes(int value_bytes = (int)sizeof(float)) {
+    return max_of({Parts::NZ...}) * kWave * CPL * value_bytes;
 }
 
 template <int K, int CPL, int WPB, int MINW, int Y, int X, typename... Parts>

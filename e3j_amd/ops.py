@@ -566,13 +566,17 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
     if (group_receiver and not ordered and y.shape[0] > 0 and p.layout == _lib.LAYOUT_TRAILING and aligned
             and x.dtype == torch.float32):
         tile_rows = _tile_rows(p.signature)
+    if (group_receiver and x.dtype == torch.float64 and p.num_x >= TILE_F64_ROWS
+            and p.num_edges * p.num_x * p.channels >= TILE_F64_VALUES):
+        tile_rows = _tile_rows(p.signature, f64=True)
     with on_device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
         if tile_rows >= 1:
             if prepared is None:
                 prepared = PreparedGraph(other, row_ptr, perm, order, n)
             schedule = prepared.schedule(tile_rows)
-            _lib.check(lib.e3j_amd_convolution_bwd_tiled(
+            fn = lib.e3j_amd_convolution_bwd_tiled_f64 if x.dtype == torch.float64 else lib.e3j_amd_convolution_bwd_tiled
+            _lib.check(fn(
                 ctypes.byref(p), x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), other.data_ptr(),
                 row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
                 ctypes.byref(schedule.struct), dx.data_ptr(), dy.data_ptr(), ds.data_ptr(), _stream(x.device)))
@@ -623,13 +627,24 @@ def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph
     return grads
 
 
-def _tile_rows(signature: int) -> int:
+#: A float64 backward runs over tiles where the atomics they save are worth the schedule's two launches: from this
+#: many values added to dx (edges x num_x x channels; l <= 3 at 64 channels, forward + VJP: 6k edges 169 -> 181 us with
+#: tiles, 15k edges 306 -> 277, 240k edges 3 176 -> 2 687), and with more than four rows of x, below which dx is a small
+#: part of the stream (480k edges, four rows 1 381 -> 1 395 us, one row 760 -> 793).
+TILE_F64_VALUES = 1 << 23
+TILE_F64_ROWS = 5
+
+
+def _tile_rows(signature: int, f64: bool = False) -> int:
     """Receivers per tile of the tiled backward for a compiled signature under the current
     configuration; 0: the one-wave-per-receiver backward runs."""
     want = int(config().tile_rows)
     if signature < 0 or want == 0:
         return 0
     lib = _lib.load()
+    if f64:
+        return (int(lib.e3j_amd_tile_rows_default_f64(signature)) if want < 0
+                else min(want, int(lib.e3j_amd_tile_rows_f64(signature))))
     if want < 0:
         return int(lib.e3j_amd_tile_rows_default(signature))
     return min(want, int(lib.e3j_amd_tile_rows(signature)))

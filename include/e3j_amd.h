@@ -254,6 +254,17 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
                                   const int32_t *receiver_ptr, const int32_t *edge_perm,
                                   const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
                                   void *stream);
+/* The same for float64 operands (p->val_dtype E3J_AMD_F64 with a signature and coef_classes; any
+ * alignment of doubles); `tile_rows` of its schedule: at most e3j_amd_tile_rows_f64(signature), 0 where
+ * the signature has no such kernel (E3J_AMD_UNIMPLEMENTED). */
+int32_t e3j_amd_tile_rows_f64(int32_t signature);
+int32_t e3j_amd_tile_rows_default_f64(int32_t signature);
+int e3j_amd_convolution_bwd_tiled_f64(const e3j_amd_conv_params *p, const void *x, const void *y,
+                                      const void *s, const void *dm, const int32_t *sender,
+                                      const int32_t *receiver_ptr, const int32_t *edge_perm,
+                                      const e3j_amd_tile_schedule *schedule,
+                                      void *dx, void *dy, void *ds, void *stream);
+
 
 /* Second-order backward: the VJP of the backward, for losses on its results (forces).  With
  * L(x, y, s) = <dm, convolution(x, y, s)> and the cotangents ddx, ddy, dds of (dx, dy, ds), the gradients
