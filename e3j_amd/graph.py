@@ -165,10 +165,10 @@ def row_piece_for(num_edges: int, row_floats: int, row_piece: int = ROW_PIECE) -
 
 
 class RowSegments:
-    """The pieces of long rows for the second call of the forward pass
+    """The pieces of long rows of the forward pass
     (`e3j_amd_row_segments_build`).  `count`: pieces to launch, the bound `num_edges // row_piece`
     (the list's own count, which the kernel reads on the device, is never read back: the
-    surplus workgroups of the second call leave at once, which costs less than a wait).
+    surplus workgroups leave at once, which costs less than a wait).
     `partials(num_out, channels)`: the scratch of the fixed-order sums (`e3j_amd_conv_params.partials`)."""
 
     def __init__(self, row_ptr: torch.Tensor | None, num_nodes: int, num_edges: int, row_cap: int,

@@ -335,7 +335,7 @@ class PreparedGraph:
 
 
     def segments(self, row_cap: int, row_piece: int = ROW_PIECE) -> RowSegments:
-        """The pieces of the rows longer than `row_cap` (second call of the forward pass), of
+        """The pieces of the rows longer than `row_cap` (of the forward pass), of
         `row_piece` positions each."""
         key = (int(row_cap), int(row_piece))
         hit = self._segments.get(key)
