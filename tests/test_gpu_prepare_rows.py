@@ -95,6 +95,22 @@ def test_against_numpy(n, e, kind, form):
     assert len(set(starts.tolist())) == len(starts)      # the pieces of a row are adjacent
 
 
+@pytest.mark.parametrize("n,e", [(16000, 16384), (9000, 16384), (40, 16384), (20000, 1000)])
+def test_out_of_order_keys_of_one_workgroup(n, e):
+    """Keys out of order in the route of one workgroup: its first pass writes row pointers that the count
+    replaces, from other waves.  The first pass's stores have to have arrived by then (the kernel's fence),
+    or one of them overwrites a count."""
+    rng = np.random.default_rng(n)
+    dev = lambda a: torch.from_numpy(a.astype(np.int32)).cuda()  # noqa: E731
+    for _ in range(20):
+        key = rng.integers(0, n, e)
+        key[rng.random(e) < 0.1] = DUMMY
+        other = rng.integers(0, n, e)
+        ptr, oth, _, _, _ = prepare_rows(dev(key), dev(other), n, True, 0)
+        np.testing.assert_array_equal(ptr.cpu().numpy(), _rows(key, n))
+        np.testing.assert_array_equal(oth.cpu().numpy(), other)
+
+
 @pytest.mark.parametrize("n,tile_rows", [(1, 2), (4096, 1), (4097, 1), (8193, 2), (700, 8), (300, 65)])
 def test_schedule_work_and_lists(n, tile_rows):
     e, max_work = 6 * n + 600, 64
