@@ -243,11 +243,13 @@ __global__ __launch_bounds__(kEdgeLanes) void edge_features_fwd_kernel(
         const int64_t e = e0 + lane;
         const int count = (int)min((int64_t)kEdgeLanes, sz.num_edges - e0);
         T basis[NB], unused[NB];
+        unsigned long long live_edges;  // bit per lane; the others have zeros whatever the weights hold
         {
             int a, b;
             T v[3];
             const bool live = lane < count && edge_vector(pos, sender, receiver, shift, e, sz.num_nodes, a, b, v);
             const T r = live ? sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) : T(0);
+            live_edges = __ballot(r > T(0));
             if (r > T(0)) {
                 const T inv = T(1) / r;
                 harmonics<L, T>(v[0] * inv, v[1] * inv, v[2] * inv, fac,
@@ -283,7 +285,7 @@ __global__ __launch_bounds__(kEdgeLanes) void edge_features_fwd_kernel(
                         T pre = T(0);
 #pragma unroll
                         for (int n = 0; n < NB; n++) pre += lds_basis[i][n] * col[n];
-                        rows[(int64_t)i * units + j] = pre * sigmoid(pre);
+                        rows[(int64_t)i * units + j] = (live_edges >> i) & 1ull ? pre * sigmoid(pre) : T(0);
                     }
                 }
             }
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(kEdgeLanes) void edge_features_bwd_kernel(
         }
         T dr = T(0);
 #pragma unroll
-        for (int n = 0; n < NB; n++) dr += db[n] * dbdr[n];
+        for (int n = 0; n < NB; n++) dr += n < sz.num_basis ? db[n] * dbdr[n] : T(0);
         // Float atomics retire per request, and a request covers the lanes that fall into one line: the three
         // components of a node lie in neighbouring lanes, and consecutive edges of one receiver (sorted edges)
         // are added up first.

@@ -76,6 +76,33 @@ def test_edge_features_on_an_empty_edge_list_and_errors():
         edge_features(pos, none, none, None, torch.rand(1, 17, 4, device="cuda"), 3, 5.0)
 
 
+@pytest.mark.parametrize("hidden", [24, 32, 100])
+def test_edges_without_a_direction_stay_zero_for_any_weights(hidden):
+    """Padding edges and edges of zero length have exact zeros in h, also where the weights have
+    overflowed; edges beside them are not touched."""
+    pos, snd, rcv, sh, w1 = _problem(11, n=50, edges=300, hidden=hidden)
+    dead = (snd >= 50) | (rcv >= 50) | (np.arange(300) == 7)
+    w1[0, 2, 5], w1[1, 0, 0], w1[1, 1, 3] = np.inf, -np.inf, np.nan
+    args = [_dev(a, torch.float32) for a in (snd, rcv, sh, w1)]
+    y, h = edge_features(_dev(pos, torch.float32), *args, 3, 5.0)
+    h, y = h.cpu().numpy(), y.cpu().numpy()
+    assert dead.sum() > 4 and not h[:, dead].any() and not y[dead].any()     # (NaN would count as set)
+    finite = np.isfinite(w1).all(1)                                          # hidden units with finite weights
+    assert all(np.isfinite(h[layer][:, finite[layer]]).all() for layer in range(2))
+
+
+def test_an_infinite_cotangent_with_few_basis_functions_is_not_a_nan():
+    """The places behind the last basis function take no part: an infinite cotangent of a hidden unit gives
+    infinite forces along the edge, as the product with the one basis function that there is."""
+    pos = torch.tensor([[0.0, 0.0, 0.0], [1.0, 0.7, -0.4], [4.0, 4.0, 4.0]], device="cuda", requires_grad=True)
+    snd, rcv = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([0, 2], [1, 1]))
+    y, h = edge_features(pos, snd, rcv, None, torch.full((1, 1, 4), 0.5, device="cuda"), 1, 5.0)
+    dh = torch.zeros_like(h)
+    dh[0, 0, 2] = float("inf")
+    (g,) = torch.autograd.grad(h, pos, dh)
+    assert torch.isinf(g[:2]).all() and torch.isfinite(g[2]).all()
+
+
 @pytest.mark.parametrize("dtype,K", [(torch.float32, 64), (torch.float32, 128), (torch.float32, 32),
                                      (torch.float64, 64)])
 def test_channel_mix_matches_the_oracle(dtype, K):
