@@ -773,7 +773,8 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
             f"    &run_bwd_tiled_f64, tile_row_bytes<1, {part_names[F64_SPLIT[1]]}>((int)sizeof(double)), {F64_TILE[2]},"
             if f64 else "    nullptr, 0, 0,",
             "    &run_fwd_f16, &run_bwd_f16," if f16 else "    nullptr, nullptr,",
-            "    &run_second_dm, &run_second_tile," if tile else "    nullptr, nullptr,",
+            f"    &run_second_dm, &run_second_tile, tile_row_bytes<{second_tile[0]}, {part_names[second_tile[2]]}>()," if tile
+            else "    nullptr, nullptr, 0,",
             "};", ""]
     if lead:
         out += ["static int run_fwd_leading" + fwd_sig[0]] + fwd_sig[1:]

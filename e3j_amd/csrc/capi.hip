@@ -544,6 +544,12 @@ int32_t e3j_amd_tile_rows_default_f64(int32_t sig) {
     return limit <= 0 ? 0 : std::max(1, std::min(signature(sig).tile_rows_f64, limit / 2));
 }
 
+int32_t e3j_amd_tile_rows_second(int32_t sig) {
+    if (sig < 0 || sig >= num_signatures()) return 0;
+    const Signature &sg = signature(sig);
+    return sg.second_tile != nullptr && sg.second_row_bytes > 0 ? (int32_t)(160 * 1024 / sg.second_row_bytes) : 0;
+}
+
 namespace {
 int run_tiled(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s, const void *dm,
               const int32_t *sender, const int32_t *receiver_ptr, const int32_t *edge_perm,
@@ -635,6 +641,10 @@ int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, con
         missing(schedule->sender, p->num_edges) || missing(schedule->edge, p->num_edges) ||
         missing(schedule->local, p->num_edges))
         return set_error(E3J_AMD_INVALID_ARGUMENT, std::string(op) + ": incomplete schedule");
+    if (schedule->tile_rows < 1 || schedule->tile_rows > e3j_amd_tile_rows_second(p->signature))
+        return set_error(E3J_AMD_INVALID_ARGUMENT,
+                         std::string(op) + ": the schedule's tiles hold more receivers than fit the LDS "
+                                           "(e3j_amd_tile_rows_second gives the limit)");
     if (p->row_cap < 0 || p->max_segments < 0 || p->row_piece < 0 || p->row_piece > p->row_cap ||
         (p->segments != nullptr && (p->row_cap == 0 || p->partials == nullptr ||
                                     reinterpret_cast<uintptr_t>(p->partials) % 16 != 0)))

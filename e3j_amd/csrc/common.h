@@ -222,6 +222,7 @@ struct Signature {
     int (*second_tile)(const e3j_amd_conv_params &p, const SecondOperands &a, const int32_t *sender,
                        const int32_t *receiver_ptr, const int32_t *edge_perm, const e3j_amd_tile_schedule &schedule,
                        float *dx, float *dy, float *ds, hipStream_t stream);
+    int32_t second_row_bytes;  // the LDS bytes its tiles take per row (its own shape, whatever variant bwd_tiled runs)
 };
 // the coefficient classes of a float64 launch, passed to the kernel by value
 constexpr int kF64Classes = E3J_AMD_F64_CLASSES;

@@ -358,10 +358,6 @@ int launch_second_tile(const e3j_amd_conv_params &p, const SecondOperands &a, co
                        float *dy, float *ds, hipStream_t stream) {
     constexpr int64_t PER_WORK = (int64_t)Slice<K, CPL>::COUNT * sizeof...(Parts);
     const size_t lds = (size_t)tile_row_bytes<CPL, Parts...>() * (size_t)sch.tile_rows;
-    if (sch.tile_rows < 1 || lds > kMaxTileLds)
-        return set_error(E3J_AMD_INVALID_ARGUMENT,
-                         "convolution_bwd_bwd: the schedule's tiles hold more receivers than fit the LDS "
-                         "(e3j_amd_tile_rows gives the limit)");
     int rc = launch_bwd_targets(p, sender, row_ptr, perm, dx, dy, ds, PER_WORK > 1, stream);
     if (rc) return rc;
     const int64_t blocks = padded_grid((int64_t)sch.num_work * PER_WORK);

@@ -596,7 +596,9 @@ def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph
     if (meta.layout != Layout.TRAILING_CHANNELS or meta.ordering == GraphOrdering.SENDER or y.shape[0] == 0
             or x.dtype != torch.float32 or config().deterministic):
         return None
-    tile_rows = _tile_rows(meta.table.signature(*_shape(meta, x, y, s), meta.layout)[0])
+    sig = meta.table.signature(*_shape(meta, x, y, s), meta.layout)[0]
+    # (the second-order kernel has one shape, the first-order limit is the selected variant's)
+    tile_rows = min(_tile_rows(sig), int(_lib.load().e3j_amd_tile_rows_second(sig)))
     if tile_rows < 1:
         return None
     x, y, s, dm, ddx, ddy, dds = (t.contiguous() for t in (x, y, s, dm, ddx, ddy, dds))

@@ -271,10 +271,12 @@ int e3j_amd_convolution_bwd_tiled_f64(const e3j_amd_conv_params *p, const void *
  * of <ddx, dx> + <ddy, dy> + <dds, ds> with respect to x, y, s and dm (src/e3j/ops/convolution.py:535-562
  * composes them from three calls of each first-order operator; here two kernels compute all terms of an
  * edge at once).  Needs a float32 signature of the trailing layout with at least 64 channels
- * (e3j_amd_tile_rows(signature) > 0, else E3J_AMD_UNIMPLEMENTED), 16-byte aligned operands and the schedule
- * of e3j_amd_convolution_bwd_tiled.  grad_x is summed with float atomics, grad_dm in a fixed order.
+ * (e3j_amd_tile_rows_second(signature) > 0, else E3J_AMD_UNIMPLEMENTED), 16-byte aligned operands and the
+ * schedule of e3j_amd_convolution_bwd_tiled with `tile_rows` of at most e3j_amd_tile_rows_second(signature)
+ * (else E3J_AMD_INVALID_ARGUMENT; its kernel has one shape, so the limit can lie below e3j_amd_tile_rows).  grad_x is summed with float atomics, grad_dm in a fixed order.
  * Long rows: p->row_cap, row_piece, segments and partials as for the forward pass, all in this one
  * call (segments without partials: E3J_AMD_INVALID_ARGUMENT). */
+int32_t e3j_amd_tile_rows_second(int32_t signature);
 int e3j_amd_convolution_bwd_bwd(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s,
                                 const void *dm, const void *ddx, const void *ddy, const void *dds,
                                 const int32_t *sender, const int32_t *receiver_ptr,

@@ -171,6 +171,40 @@ def test_null_params_and_backward_errors():
     assert "do not match signature" in lib.e3j_amd_last_error().decode()
 
 
+def test_second_order_backward_refusals():
+    """What `e3j_amd_convolution_bwd_bwd` refuses, all of it before anything is launched."""
+    lib = _lib.load()
+    names = [lib.e3j_amd_signature_name(i).decode() for i in range(lib.e3j_amd_num_signatures())]
+    sig = next(i for i, n in enumerate(names) if n.startswith("l3_l3_to_l3_k64") and lib.e3j_amd_tile_rows_second(i) > 0)
+    limit = lib.e3j_amd_tile_rows_second(sig)
+    assert lib.e3j_amd_tile_rows_second(-1) == 0 and lib.e3j_amd_tile_rows_second(len(names)) == 0
+    assert lib.e3j_amd_tile_rows_second(next(i for i, n in enumerate(names) if "_k32" in n)) == 0
+    irreps = "0e+1o+2e+3o"
+    num_coef = len(Convolution((irreps, irreps), irreps, graph_ordering="RECEIVER").coef.val)
+    dims = dict(num_x=16, num_y=16, num_out=99, num_scalars=23, channels=64, val_dtype=_lib.F32, num_nodes=4, num_edges=8)
+
+    def call(schedule=None, operands=None, **kw):
+        p = _params(**{**dims, "num_coef": num_coef, "signature": sig, **kw})
+        sch = schedule or _lib.TileSchedule(tile_rows=limit, num_work=1, work=64, sender=64, edge=64, local=64)
+        ptr = [C.c_void_p(v) for v in (operands or [64] * 7)] + [C.c_void_p(64), C.c_void_p(64), None]
+        code = lib.e3j_amd_convolution_bwd_bwd(C.byref(p), *ptr, C.byref(sch), *([C.c_void_p(64)] * 4), None)
+        return code, lib.e3j_amd_last_error().decode()
+
+    for tile_rows in (0, limit + 1):
+        code, message = call(_lib.TileSchedule(tile_rows=tile_rows, num_work=1, work=64, sender=64, edge=64, local=64))
+        assert code == _lib.INVALID_ARGUMENT and "e3j_amd_tile_rows_second" in message
+    code, message = call(_lib.TileSchedule(tile_rows=limit, num_work=1, work=64, sender=64, edge=64, local=None))
+    assert code == _lib.INVALID_ARGUMENT and "incomplete schedule" in message
+    code, message = call(row_cap=64, row_piece=64, max_segments=1, segments=64)          # pieces without partials
+    assert code == _lib.INVALID_ARGUMENT and "partials" in message
+    code, message = call(operands=[64, 64, 64, 64, 68, 64, 64])                          # ddx off its alignment
+    assert code == _lib.INVALID_ARGUMENT and "16-byte aligned" in message
+    code, message = call(operands=[64, 64, 64, 64, None, 64, 64])
+    assert code == _lib.INVALID_ARGUMENT and "null operand" in message
+    code, message = call(signature=-1)
+    assert code == _lib.UNIMPLEMENTED and "float32" in message
+
+
 def test_empty_problem_is_a_no_op():
     lib = _lib.load()
     p = _params(num_nodes=0, num_edges=0)

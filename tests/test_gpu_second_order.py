@@ -2,11 +2,13 @@
 each gradient is a sum of two or three first-order results, so the reference and the magnitude of its
 terms are sums of the oracle's (the rounding allowance of `helpers.assert_parity` applies to the sum)."""
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from e3j_amd import ops
+from e3j_amd import _lib, config, ops
 from e3j_amd.codegen.gen_conv import BUILTIN_SIGNATURES
 from e3j_amd.convolution import Convolution
 from tests import helpers as H
@@ -44,8 +46,8 @@ CASES = [(sig, kind) for sig in BUILTIN_SIGNATURES if sig[4] >= 64
          for kind in (("single", "hub") if sig[4] == 256 else ("single", "hub", "padding", "shuffled"))]
 
 
-@pytest.mark.parametrize("sig,kind", CASES, ids=[f"{s[0]}-{k}" for s, k in CASES])
-def test_second_order_matches_oracle(sig, kind, monkeypatch):
+def _compare_with_oracle(sig, kind, monkeypatch):
+    """Second derivatives through autograd, which must come from one call of the library."""
     name, xi, yi, oi, channels = sig
     rng = np.random.default_rng(channels + len(kind))
     module = Convolution((xi, yi), oi, graph_ordering="NONE" if kind == "shuffled" else "RECEIVER")
@@ -58,13 +60,13 @@ def test_second_order_matches_oracle(sig, kind, monkeypatch):
     dev = {k: torch.from_numpy(v.copy()).cuda() for k, v in dict(x=x, y=y, s=s, dm=dm, x2=x2, y2=y2, s2=s2).items()}
     for k in ("y", "s", "y2", "s2"):           # padding edges hold anything
         dev[k][torch.from_numpy(pad)] = float("nan")
-    calls = []
-    monkeypatch.setattr(ops, "_raw_second", lambda *a, f=ops._raw_second: calls.append(1) or f(*a))
+    results = []
+    monkeypatch.setattr(ops, "_raw_second", lambda *a, f=ops._raw_second: results.append(f(*a)) or results[-1])
     leaves = [dev[k].requires_grad_(True) for k in ("x", "y", "s", "dm")]
     out = module(*leaves[:3], torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda())
     first = torch.autograd.grad(out, leaves[:3], leaves[3], create_graph=True)
     got = torch.autograd.grad(first, leaves, [dev["x2"], dev["y2"], dev["s2"]])
-    assert calls
+    assert len(results) == 1 and results[0] is not None     # (None: the first-order operators composed them)
     live = ~pad
     idx = np.asarray(module.coef.idx, dtype=np.int64)
     val, mix = np.asarray(module.coef.val, dtype=np.float32), module._mix.mix_indices
@@ -84,3 +86,28 @@ def test_second_order_matches_oracle(sig, kind, monkeypatch):
             ("dm", g[3], sum(t[0] for t in f), sum(t[1] for t in f))):
         H.assert_parity(result, ref, mag, f"{name} {kind} gradient of {name_}")
     assert not g[1][pad].any() and not g[2][pad].any()
+
+
+@pytest.mark.parametrize("sig,kind", CASES, ids=[f"{s[0]}-{k}" for s, k in CASES])
+def test_second_order_matches_oracle(sig, kind, monkeypatch):
+    _compare_with_oracle(sig, kind, monkeypatch)
+
+
+@pytest.mark.parametrize("channels,variant", [(64, 1), (128, 4)])
+def test_tiles_that_only_the_first_order_backward_can_hold(channels, variant, monkeypatch):
+    """A first-order launch variant whose tiles take less LDS a row allows more rows than the second-order
+    kernel holds: `config(tile_rows=...)` is cut to what each of them takes."""
+    sig = next(s for s in BUILTIN_SIGNATURES if s[0] == f"l3_l3_to_l3_k{channels}")
+    lib = _lib.load()
+    lib.e3j_amd_set_launch_variant.argtypes = [ctypes.c_int32, ctypes.c_int32]
+    lib.e3j_amd_set_launch_variant.restype = None
+    lib.e3j_amd_set_launch_variant(0, variant)
+    try:
+        ids = [i for i in range(lib.e3j_amd_num_signatures())
+               if lib.e3j_amd_signature_name(i).decode().startswith(sig[0]) and lib.e3j_amd_tile_rows_second(i) > 0]
+        rows, least = lib.e3j_amd_tile_rows(ids[0]), lib.e3j_amd_tile_rows_second(ids[0])
+        assert rows > least >= 1
+        with config.use(tile_rows=rows):
+            _compare_with_oracle(sig, "hub", monkeypatch)
+    finally:
+        lib.e3j_amd_set_launch_variant(0, 0)
