@@ -75,7 +75,8 @@ F16_SHAPE = {True: (2, 2, 3), False: (1, 1, 3)}
 #: the schedule of the first `bwd_tile` variant.  120k edges at 128 channels / 240k at 64, l <= 3: rows at
 #: one channel per lane in 3 parts 0.71 / 0.70 ms (2 parts 0.72 / 0.78, unsplit 1.06 at 64, two channels
 #: per lane 0.78); tiles at 128 with two channels per lane 1.22 ms, with one 1.24, at 64 1.22 (8 waves per
-#: block and two resident per SIMD 1.50).
+#: block and two resident per SIMD 1.50).  The bounds are those of the built-in tables (at 64 channels the l <= 3
+#: tiles just miss theirs: 168 registers and 4 spilled); larger tables get more registers (`second_shapes`).
 SECOND_DM = {64: (1, 4, 3, 3), 128: (1, 4, 3, 3), 256: (1, 4, 3, 3)}
 SECOND_TILE = {64: (1, 4, 3, 3), 128: (2, 4, 3, 2), 256: (2, 8, 3, 2)}
 #: the float64 kernels take one coefficient per class of equal magnitude as a kernel argument
@@ -557,6 +558,31 @@ def plugin_launch(channels: int):
     return trailing, leading
 
 
+def second_shapes(t: "Table", channels: int):
+    """Launch shapes of the second-order kernels (rows, tiles) of a table.
+
+    What a lane holds of a part: the operands of two edges, the sums and the y rows.  Beyond the registers
+    that the bound of the built-in tables leaves (168 at three waves per SIMD, 256 at two) the kernels
+    spill inside the edge loop, which costs more than the waves hide: x, y, out l <= 4 at 64 channels, 75k
+    edges, forward to second derivatives: 10.2 ms under the bound of three waves (477 registers spilled), 4.0
+    of two, 3.6 of one, 5.1 composed from the first-order operators; y and out l <= 4 with x l <= 3 4.3, 2.0,
+    2.0 and 3.6; at 128 channels, with one in the place of two waves for the tiles, 11.3 -> 5.7 and 3.7 -> 2.4.
+    Tables of a fifth fewer values than the lines drawn here are not faster with fewer waves
+    (x l <= 3 and y l <= 4 at 128 channels: 1.47 ms with two, 1.57 with one).
+    """
+    # (a run-time table at another multiple of 64 channels takes the shapes of 64 or 128 channels)
+    key = channels if channels in SECOND_DM else 128 if channels % 128 == 0 else 64
+    dm, tile = SECOND_DM[key], SECOND_TILE[key]
+    held = max(len(p.zi) + 4 * (len(p.xj) + len(p.sl)) + 2 * t.Y for p in split_parts(t, dm[2]))
+    waves = 3 if held <= 136 else 2 if held <= 220 else 1
+    dm = (*dm[:3], min(dm[3], waves))
+    if tile[0] == 1:
+        tile = (*tile[:3], min(tile[3], waves))
+    elif max(2 * (5 * len(p.xj) + 4 * len(p.sl)) + 3 * t.Y for p in split_parts(t, tile[2])) > 220:
+        tile = (tile[0], 4, tile[2], 1)   # (eight waves a block would need two per SIMD)
+    return dm, tile
+
+
 def supports(t: "Table", channels: int) -> bool:
     """Whether the kernel templates can take this table (register-resident dy sums, bit masks)."""
     return t.Y <= 64 and t.X <= 64 and t.S <= 64 and t.Z <= 255 and channels >= 1
@@ -590,9 +616,7 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
     # float64 kernels: trailing layout, whole waves of channels, few enough coefficient classes
     f64 = channels % 64 == 0 and 0 < len(t.classes) <= F64_MAX_CLASSES
     f16 = channels % 64 == 0   # float16 kernels: trailing layout, whole waves of channels
-    # (a run-time table at another multiple of 64 channels takes the tiles of 64 or 128 channels)
-    second_key = channels if channels in SECOND_DM else 128 if channels % 128 == 0 else 64
-    second_dm, second_tile = (SECOND_DM[second_key], SECOND_TILE[second_key]) if tile else (None, None)
+    second_dm, second_tile = second_shapes(t, channels) if tile else (None, None)
     second_splits = {second_dm[2], second_tile[2]} if tile else set()
     splits = sorted({v[2] for v in launch["fwd"] + launch["bwd"] + tile} | second_splits |
                     ({v[1] for v in lead["fwd"] + lead["bwd"]} if lead else set()) |

@@ -111,3 +111,16 @@ def test_tiles_that_only_the_first_order_backward_can_hold(channels, variant, mo
             _compare_with_oracle(sig, "hub", monkeypatch)
     finally:
         lib.e3j_amd_set_launch_variant(0, 0)
+
+
+#: tables the library is not built for: shapes of 64 channels at 192, and fewer waves per SIMD for the larger
+#: tables (`second_shapes`: two in both kernels; two and one)
+RUN_TIME = [("0e+1o+2e", "0e+1o+2e", "0e+1o+2e", 64), ("0e+1o+2e", "0e+1o+2e", "0e+1o+2e", 192),
+            ("0e+1o+2e", "0e+1o+2e+3o+4e", "0e+1o+2e+3o+4e", 64),
+            ("0e+1o+2e+3o+4e", "0e+1o+2e+3o+4e", "0e+1o+2e", 128)]
+
+
+@pytest.mark.parametrize("xi,yi,oi,channels", RUN_TIME)
+def test_run_time_compiled_tables(xi, yi, oi, channels, monkeypatch):
+    with config.use(jit=True):
+        _compare_with_oracle(("run-time table", xi, yi, oi, channels), "hub", monkeypatch)

@@ -420,3 +420,26 @@ def test_build_reads_the_assembly_for_dpp_operands_written_too_late():
         v_fmac_f32_dpp v32, v3, v16 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf
     """
     assert len(dpp_read_hazards(pair)) == 1
+
+
+def test_second_order_shapes_leave_large_tables_the_registers_they_need():
+    """The occupancy bounds of the second-order kernels are those of the built-in tables; a table whose
+    lanes hold more gets fewer waves per SIMD (spills inside the edge loop made them slower than the
+    first-order operators they replace)."""
+    from e3j_amd.codegen import gen_conv as G
+
+    def shapes(x, y, out, channels):
+        m = Convolution((x, y), out, graph_ordering="RECEIVER")
+        c = Coef4D.unpack(m._packed_coef("float32"), np.float32)
+        return G.second_shapes(G.Table(c.val, c.idx.astype(np.int64), m.source[0].dim, m.source[1].dim,
+                                       m.params.num_out, m.params.num_scalars), channels)
+
+    for name, x, y, out, counts in G.BUILTIN_TABLES:
+        for k in counts:
+            if k >= 64:
+                assert shapes(x, y, out, k) == (G.SECOND_DM[k], G.SECOND_TILE[k]), name
+    l2, l3, l4 = "0e+1o+2e", "0e+1o+2e+3o", "0e+1o+2e+3o+4e"
+    assert shapes(l2, l2, l2, 192) == (G.SECOND_DM[64], G.SECOND_TILE[64])
+    assert [s[3] for s in shapes(l3, l4, l4, 64)] == [2, 2] and [s[3] for s in shapes(l4, l4, l4, 64)] == [1, 1]
+    assert [s[3] for s in shapes(l3, l4, l3, 128)] == [2, 2] and [s[3] for s in shapes(l4, l4, l2, 128)] == [2, 1]
+    assert shapes(l4, l4, l2, 256)[1] == (2, 4, 3, 1) and shapes(l3, l4, l3, 256)[1] == G.SECOND_TILE[256]
