@@ -293,10 +293,13 @@ class PreparedGraph:
     built from do not change.  It remembers the stream it was prepared on and makes any other
     stream that uses it wait for the preparation.  The scratch rows of the forward's long-row sums
     belong to the handle: calls that share a handle must not overlap on different streams.
+    `kept`: it serves further calls (`prepare_graph`, the graph cache), so that a schedule built for it pays
+    over several backwards; False: prepared by an operator call for itself.
     """
 
-    def __init__(self, other, row_ptr, perm, order, num_nodes: int, ordering=None):
+    def __init__(self, other, row_ptr, perm, order, num_nodes: int, ordering=None, kept: bool = False):
         self.other, self.row_ptr, self.perm, self.order = other, row_ptr, perm, order
+        self.kept = kept
         self.num_nodes = int(num_nodes)
         self.ordering = ordering
         self._schedules = {}
@@ -364,7 +367,7 @@ def prepare_graph(sender: torch.Tensor, receiver: torch.Tensor, num_nodes: int,
     ordering = GraphOrdering.parse(graph_ordering)
     if pair_rows is None:
         pair_rows = config().pair_rows in (True, "prepared")
-    return _prepare_graph(ordering, int(num_nodes), sender, receiver, pair=bool(pair_rows))
+    return _prepare_graph(ordering, int(num_nodes), sender, receiver, pair=bool(pair_rows), kept=True)
 
 
 def _check_graph(graph: PreparedGraph, meta: "_Meta", num_edges: int) -> None:
@@ -388,7 +391,7 @@ def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, bu
         return hit[2]
     if not build:
         return None
-    graph = _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver, pieces=pieces)
+    graph = _prepare_graph(meta.ordering, meta.num_nodes, sender, receiver, pieces=pieces, kept=True)
     if len(_GRAPH_CACHE) >= _GRAPH_CACHE_SIZE:
         _GRAPH_CACHE.pop(next(iter(_GRAPH_CACHE)))
 
@@ -405,9 +408,9 @@ UNORDERED_ROWS = 256
 
 
 def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiver: torch.Tensor,
-                   pair: bool | None = None, pieces=None) -> PreparedGraph:
+                   pair: bool | None = None, pieces=None, kept: bool = False) -> PreparedGraph:
     """`pieces`: the `(row_cap, row_piece)` of the forward pass this graph is prepared for, which then finds
-    its list of pieces already built."""
+    its list of pieces already built; `kept`: see `PreparedGraph`."""
     if ordering == GraphOrdering.SENDER:
         # aggregate over reversed edges; y parities are folded into the coefficients
         key, other = sender, receiver
@@ -421,7 +424,7 @@ def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiv
             pair = config().pair_rows is True
         if pair and n > 1 and config().locality_rounds > 0:
             order = pair_rows(other, row_ptr, n, order)
-        graph = PreparedGraph(other, row_ptr, perm, order, n, ordering)
+        graph = PreparedGraph(other, row_ptr, perm, order, n, ordering, kept)
         if segments is not None:
             graph._segments[pieces] = segments
         return graph
@@ -430,7 +433,7 @@ def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiv
         other, row_ptr, perm = other.contiguous(), csr_row_ptr(key, n), None
     else:
         perm, other, row_ptr = sort_edges(key, other, n)
-    return PreparedGraph(other, row_ptr, perm, _row_order(other, row_ptr, n, pair), n, ordering)
+    return PreparedGraph(other, row_ptr, perm, _row_order(other, row_ptr, n, pair), n, ordering, kept)
 
 
 def _row_pieces(meta: _Meta, x: torch.Tensor, num_edges: int):
@@ -566,8 +569,8 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
     if (group_receiver and not ordered and y.shape[0] > 0 and p.layout == _lib.LAYOUT_TRAILING and aligned
             and x.dtype == torch.float32):
         tile_rows = _tile_rows(p.signature)
-    if (group_receiver and x.dtype == torch.float64 and p.num_x >= TILE_F64_ROWS
-            and p.num_edges * p.num_x * p.channels >= TILE_F64_VALUES):
+    if (group_receiver and x.dtype == torch.float64
+            and _tiles_pay_f64(p.num_edges, p.num_x, p.num_scalars, p.channels, prepared is not None and prepared.kept)):
         tile_rows = _tile_rows(p.signature, f64=True)
     with on_device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
@@ -629,12 +632,31 @@ def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph
     return grads
 
 
-#: A float64 backward runs over tiles where the atomics they save are worth the schedule's two launches: from this
-#: many values added to dx (edges x num_x x channels; l <= 3 at 64 channels, forward + VJP: 6k edges 169 -> 181 us with
-#: tiles, 15k edges 306 -> 277, 240k edges 3 176 -> 2 687), and with more than four rows of x, below which dx is a small
-#: part of the stream (480k edges, four rows 1 381 -> 1 395 us, one row 760 -> 793).
-TILE_F64_VALUES = 1 << 23
+#: Values added to dx (edges x num_x x channels) from which a float64 backward runs over tiles, where the
+#: schedule serves several calls, and where it is built for the one call.
+TILE_F64_VALUES, TILE_F64_VALUES_ONE_CALL = 1 << 23, 3 << 23
 TILE_F64_ROWS = 5
+
+
+def _tiles_pay_f64(num_edges: int, num_x: int, num_scalars: int, channels: int, kept: bool) -> bool:
+    """Whether the dx atomics that tiles save a float64 backward are worth the schedule and the rows in LDS.
+
+    Forward and VJP, microseconds over tiles against one wave per receiver, radius graphs:
+    with a kept schedule x l <= 3 gains from 8.4 M values on (64 channels 204 to 221, 128 channels 202 to
+    213, 256 channels 205 to 212; at 134 M 1 436 to 1 705), x l <= 2 to l <= 2 from there (208 to 209;
+    1 180 to 1 359).  Built for one call the schedule costs 60 us of the host: 317 to 256 at 8.4 M,
+    319 to 266 at 17 M, 404 to 429 and 347 to 352 at 25 M.  A table with many paths per row of x moves
+    more radial weights for the same atomics: x l <= 2 to l <= 3 (17 paths for 9 rows) 311 to 289 at 17 M,
+    499 to 499 at 34 M, 1 711 to 1 713 at 134 M with a kept schedule, 552 to 526 at 34 M without.  Four rows of
+    x or fewer are a small part of the stream (480k edges, four rows 1 395 to 1 381, one row 793 to 760).
+    Rows of uneven length gain at all of these sizes (5 to 30 %).
+    """
+    if num_x < TILE_F64_ROWS:
+        return False
+    values = num_edges * num_x * channels
+    if 2 * num_scalars > 3 * num_x:
+        return kept and values >= 4 * TILE_F64_VALUES
+    return values >= (TILE_F64_VALUES if kept else TILE_F64_VALUES_ONE_CALL)
 
 
 def _tile_rows(signature: int, f64: bool = False) -> int:

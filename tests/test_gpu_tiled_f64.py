@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import e3j_amd
-from e3j_amd import _lib
+from e3j_amd import _lib, ops
 from e3j_amd.graph import TileSchedule, csr_row_ptr, sort_edges
 from e3j_amd.ops import _Table
 
@@ -72,3 +72,37 @@ def test_tiled_equals_receiver_rows(x_irreps, channels, kind, tile_rows, max_wor
     p.val_dtype = _lib.F32
     assert lib.e3j_amd_convolution_bwd_tiled_f64(ctypes.byref(p), *args, ctypes.byref(sch.struct), *out) \
         == _lib.UNIMPLEMENTED
+
+
+@pytest.mark.parametrize("x_irreps,out_irreps,channels,kept", [
+    ("0e+1o+2e+3o", "0e+1o+2e+3o", 128, True), ("0e+1o+2e", "0e+1o+2e", 64, True), ("0e+1o+2e", "0e+1o+2e", 64, False),
+    ("0e+1o+2e", "0e+1o+2e", 192, True)])
+def test_operator_above_the_threshold(x_irreps, out_irreps, channels, kept, monkeypatch):
+    """Through the operator, with a row order (paired for a handle), just above the size from which tiles run,
+    against the same call without them; 192 channels: a table compiled at run time."""
+    y_irreps = "0e+1o+2e" if channels == 192 else "0e+1o+2e+3o"
+    module = e3j_amd.Convolution((x_irreps, y_irreps), out_irreps, graph_ordering="RECEIVER",
+                                 layout="TRAILING_CHANNELS", avg_num_neighbors=30.0)
+    num_x, num_y, num_s = module.source[0].dim, module.source[1].dim, module.params.num_scalars
+    n, e = 400, (1 if kept else 3) * 2 ** 23 // (num_x * channels) + 64
+    gen = torch.Generator(device="cuda").manual_seed(channels)
+    rand = lambda *shape: torch.randn(shape, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    receiver = torch.randint(0, n - 9, (e,), device="cuda", generator=gen).sort().values.int()
+    sender = ((receiver + torch.randint(1, 40, (e,), device="cuda", generator=gen)) % n).int()
+    sender[::13] = 2 ** 31 - 1
+    x, y, s = (t.requires_grad_(True) for t in (rand(n, num_x, channels), rand(e, num_y), rand(e, num_s, channels)))
+    dm = rand(n, module.params.num_out, channels)
+    graph = ops.prepare_graph(sender, receiver, n) if kept else None
+    taken = []
+    monkeypatch.setattr(ops, "_tile_rows", lambda *a, f=ops._tile_rows, **k: taken.append((k, f(*a, **k))) or taken[-1][1])
+    results = []
+    for tile_rows in (-1, 0):
+        with e3j_amd.config.use(tile_rows=tile_rows, jit=channels == 192):
+            out = module(x, y, s, sender, receiver, graph=graph)
+            results.append((out.detach(), *torch.autograd.grad(out, (x, y, s), dm)))
+    assert taken[0][0] == {"f64": True} and taken[0][1] >= 1 and taken[1][1] == 0
+    (out, dx, dy, ds), (out0, dx0, dy0, ds0) = results
+    assert torch.equal(out, out0) and torch.equal(ds, ds0)
+    for a, b, terms in ((dx0, dx, e // n), (dy0, dy, 16)):
+        # sums of about `terms` values in another order: sqrt(terms) roundings of the largest result
+        assert float((a - b).abs().max()) <= 8 * terms ** 0.5 * 1.2e-16 * float(a.abs().max())

@@ -443,3 +443,16 @@ def test_second_order_shapes_leave_large_tables_the_registers_they_need():
     assert [s[3] for s in shapes(l3, l4, l4, 64)] == [2, 2] and [s[3] for s in shapes(l4, l4, l4, 64)] == [1, 1]
     assert [s[3] for s in shapes(l3, l4, l3, 128)] == [2, 2] and [s[3] for s in shapes(l4, l4, l2, 128)] == [2, 1]
     assert shapes(l4, l4, l2, 256)[1] == (2, 4, 3, 1) and shapes(l3, l4, l3, 256)[1] == G.SECOND_TILE[256]
+
+
+def test_float64_tiles_only_where_they_pay():
+    """Tiles of the float64 backward: from another size on where the schedule is built for one call, and not for
+    one call of a table with many paths per row of x."""
+    from e3j_amd.ops import _tiles_pay_f64 as pays
+    edges = 2 ** 23 // (16 * 64)
+    assert pays(edges, 16, 23, 64, True) and not pays(edges - 1, 16, 23, 64, True)       # x, out l <= 3
+    assert pays(3 * edges, 16, 23, 64, False) and not pays(3 * edges - 1, 16, 23, 64, False)
+    assert pays(edges // 2, 16, 23, 128, True) and pays(2 ** 23 // (9 * 64) + 1, 9, 13, 64, True)
+    many = 4 * 2 ** 23 // (9 * 128) + 1                                                  # x l <= 2 to out l <= 3
+    assert pays(many, 9, 17, 128, True) and not pays(many - 1, 9, 17, 128, True) and not pays(100 * many, 9, 17, 128, False)
+    assert not pays(10 ** 8, 4, 4, 64, True)                                             # few rows of x
