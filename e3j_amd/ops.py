@@ -27,7 +27,7 @@ from . import _lib
 from .coef import Coef4D
 from .graph import (RowSegments, TileSchedule, csr_row_ptr, fold_endpoints, locality_order,
                     on_device, pair_rows, prepare_rows, raw_stream, row_cap_for, row_piece_for, sort_edges, wrap_global_index, ROW_PIECE)
-from .options import GraphOrdering, Layout, config
+from .options import Config, GraphOrdering, Layout, config
 
 
 @dataclasses.dataclass
@@ -256,19 +256,39 @@ def _check_operands(x, y, s, sender, receiver):
         raise TypeError("x, y and s must share one dtype")
 
 
-def _row_order(other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: bool | None = None):
-    """Locality-aware processing order of the rows of a CSR, or None when switched off.
-    `pair`: also put rows with common senders side by side (None: only if `config().pair_rows` is
+#: An adjacency that one call prepares for itself keeps the index order up to this many rows and edges, unless
+#: `config(locality_rounds=...)` asks for another number of sweeps than the default: so few rows fit the
+#: compute units and one L2 in any order, the tiles of the backward lose few shared senders, and the order is
+#: three launches.  GPU time of forward and VJP without and with it, x, y, out l <= 3, microseconds: 128 rows of
+#: 19 edges 125 and 136 at 128 channels, 256 rows of 30 edges 174 and 188 (256 channels 241 and 250; l <= 2 at 64
+#: channels 94 and 108); on the host 10 us a call.  At 256 rows of 120 edges it is the other way round (525 and 486 at
+#: 128 channels), and a handle, whose order serves many calls, always has it (473 and 426 there).
+UNORDERED_ROWS, UNORDERED_EDGES = 256, 16384
+
+
+def _order_rounds(n: int, num_edges: int, kept: bool = False) -> int:
+    """Sweeps behind the row order of an adjacency (0: index order); `kept`: see `PreparedGraph`."""
+    rounds = int(config().locality_rounds)
+    if n < 2 or num_edges == 0 or rounds <= 0:
+        return 0
+    small = n <= UNORDERED_ROWS and num_edges <= UNORDERED_EDGES
+    return 0 if small and not kept and rounds == Config.locality_rounds else rounds
+
+
+def _paired(order, other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: bool | None):
+    """`order` with rows of common senders side by side if `pair` says so (None: only if `config().pair_rows` is
     True; the handles of `prepare_graph` ask for it by default)."""
-    rounds = config().locality_rounds
-    if rounds <= 0 or n < 2 or other.numel() == 0:
-        return None
-    order = locality_order(other, row_ptr, n, rounds)
     if pair is None:
         pair = config().pair_rows is True
-    if pair:
+    if pair and n > 1 and other.numel() > 0 and config().locality_rounds > 0:
         order = pair_rows(other, row_ptr, n, order)
     return order
+
+
+def _row_order(other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: bool | None = None):
+    """Processing order of the rows of a CSR that one call prepares for itself, None for the index order."""
+    rounds = _order_rounds(n, int(other.numel()))
+    return _paired(locality_order(other, row_ptr, n, rounds) if rounds > 0 else None, other, row_ptr, n, pair)
 
 
 #: Opt-in (`config(graph_cache=True)`): adjacencies prepared for the index tensors seen last, keyed by
@@ -402,11 +422,6 @@ def _forward_graph(meta: _Meta, sender: torch.Tensor, receiver: torch.Tensor, bu
     return graph
 
 
-#: rows up to which the index order stays: every row then has a compute unit of its own, and whatever
-#: the rows share fits one L2 (256 rows of 16 x 128 floats: 2 MB)
-UNORDERED_ROWS = 256
-
-
 def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiver: torch.Tensor,
                    pair: bool | None = None, pieces=None, kept: bool = False) -> PreparedGraph:
     """`pieces`: the `(row_cap, row_piece)` of the forward pass this graph is prepared for, which then finds
@@ -417,14 +432,10 @@ def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiv
     else:
         key, other = receiver, sender
     if n >= 1 and 0 < key.numel() == other.numel():
-        rounds = config().locality_rounds if n > UNORDERED_ROWS else 0
+        rounds = _order_rounds(n, int(key.numel()), kept)
         row_ptr, other, perm, order, segments = prepare_rows(
             key, other, n, ordering != GraphOrdering.NONE, rounds, pieces)
-        if pair is None:
-            pair = config().pair_rows is True
-        if pair and n > 1 and config().locality_rounds > 0:
-            order = pair_rows(other, row_ptr, n, order)
-        graph = PreparedGraph(other, row_ptr, perm, order, n, ordering, kept)
+        graph = PreparedGraph(other, row_ptr, perm, _paired(order, other, row_ptr, n, pair), n, ordering, kept)
         if segments is not None:
             graph._segments[pieces] = segments
         return graph

@@ -97,7 +97,9 @@ class Config:
     #: atomic-free backward for `dx` (bit-reproducible, slower).
     deterministic: bool = False
     #: sweeps of label propagation behind the locality-aware row order of the kernels
-    #: (0 = rows are processed in index order).
+    #: (0 = rows are processed in index order).  At the default, an adjacency that an operator call prepares
+    #: for itself stays in index order up to 256 rows and 16 384 edges, where the order costs more than it
+    #: gives; any other number, and the handles of `prepare_graph`, order the rows of graphs of any size.
     locality_rounds: int = 2
     #: keep the adjacencies prepared for the index tensors seen last and reuse them when the same
     #: tensors (identity and in-place version) come again.  Off by default: a buffer rewritten behind

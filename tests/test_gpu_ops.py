@@ -63,6 +63,53 @@ def test_row_order_does_not_change_results():
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
+@pytest.mark.parametrize("n,edges", [(200, 3000), (300, 4000), (8300, 20000)])
+def test_a_row_order_leaves_the_forward_bits(n, edges):
+    """Orders of each route (a few rows, rows sorted by one workgroup, the library's sort), prepared by the
+    call and by a handle: not the identity, and the same forward bits as the index order."""
+    from e3j_amd import ops
+    p = _problem(12, N=n, E=edges, K=32)
+    args = [dev(p[k]) for k in ("x", "y", "s")]
+    snd, rcv = dev(p["snd"]), dev(p["rcv"])
+    with e3j_amd.config.use(locality_rounds=0):
+        base = convolution(p["coef"], *args, snd, rcv, p["params"])
+        assert ops.prepare_graph(snd, rcv, n).order is None
+    for rounds in (1, 2, 4):
+        with e3j_amd.config.use(locality_rounds=rounds):
+            call = ops._prepare_graph(e3j_amd.GraphOrdering.RECEIVER, n, snd, rcv)
+            handle = ops.prepare_graph(snd, rcv, n)
+            for graph in (call, handle):
+                if graph is call and n <= ops.UNORDERED_ROWS and rounds == 2:
+                    assert graph.order is None         # the rule of small graphs: at the default only
+                    continue
+                order = graph.order.long().sort()
+                assert torch.equal(order.values, torch.arange(n, device="cuda"))
+                assert not torch.equal(order.indices, order.values)
+            assert torch.equal(base, convolution(p["coef"], *args, snd, rcv, p["params"]))
+            assert torch.equal(base, convolution(p["coef"], *args, snd, rcv, p["params"], graph=handle))
+
+
+def test_small_graphs_keep_the_index_order_on_every_path(monkeypatch):
+    """The rule of small graphs is the same for the operator, a direct backward and one of SENDER rows, and ends
+    with the edges, not only with the rows."""
+    from e3j_amd import ops
+    made = []
+    real_order, real_prepare = ops.locality_order, ops.prepare_rows
+    monkeypatch.setattr(ops, "locality_order", lambda *a: made.append("order") or real_order(*a))
+    monkeypatch.setattr(ops, "prepare_rows", lambda *a: made.append(f"rounds {a[4]}") or real_prepare(*a))
+    for n, edges, rounds, ordered in ((200, 3000, 2, False), (200, 3000, 3, True), (200, 16385, 2, True), (257, 3000, 2, True)):
+        p = _problem(13, N=n, E=edges, K=32)
+        args = [dev(p[k]) for k in ("x", "y", "s")]
+        snd, rcv, dm = dev(p["snd"]), dev(p["rcv"]), dev(p["dm"])
+        with e3j_amd.config.use(locality_rounds=rounds):
+            made.clear()
+            convolution(p["coef"], *args, snd, rcv, p["params"])
+            assert made == [f"rounds {rounds if ordered else 0}"]
+            made.clear()
+            convolution_bwd(p["coef"], *args, snd, rcv, dm, p["params"])
+            assert made == (["order"] if ordered else [])
+
+
 def test_convolution_bwd_direct_and_deterministic_bits():
     p = _problem(2, N=64, E=2000, K=32)
     args = [dev(p[k]) for k in ("x", "y", "s")]
