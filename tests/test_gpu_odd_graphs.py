@@ -9,6 +9,7 @@ import torch
 
 import e3j_amd
 from e3j_amd import DUMMY_INDEX, Convolution
+from e3j_amd.ops import prepare_graph
 from tests import helpers as H
 
 pytestmark = pytest.mark.gpu
@@ -32,6 +33,15 @@ def _degrees(rng, kind, n):
     if kind == 3:
         return rng.poisson(8, n)
     return rng.integers(0, 2, n)
+
+
+def _handle(case, sender, receiver, n, ordering):
+    """Half of the cases (5 to 9, 15 to 19, ...) run with a prepared handle: its rows have a paired locality order
+    whatever the size, where a small graph prepared by the call itself keeps the index order."""
+    graph = prepare_graph(sender, receiver, n, ordering) if case // 5 % 2 else None
+    if graph is not None and n > 1 and sender.numel() > 0:
+        assert graph.order is not None
+    return graph
 
 
 @pytest.mark.parametrize("case", range(50))
@@ -67,10 +77,11 @@ def test_odd_graph(case):
 
     coef = m._packed_coef("float32")
     args = (dev(put(x)), dev(y), dev(put(s)), dev(snd), dev(rcv))
-    out = e3j_amd.convolution(coef, *args, m.params, ordering, layout=layout)
-    atomics = e3j_amd.convolution_bwd(coef, *args, dev(put(dm)), m.params, ordering, layout=layout)
+    graph = _handle(case, *args[3:], N, ordering)
+    out = e3j_amd.convolution(coef, *args, m.params, ordering, layout=layout, graph=graph)
+    atomics = e3j_amd.convolution_bwd(coef, *args, dev(put(dm)), m.params, ordering, layout=layout, graph=graph)
     with e3j_amd.config.use(deterministic=True):
-        ordered = e3j_amd.convolution_bwd(coef, *args, dev(put(dm)), m.params, ordering, layout=layout)
+        ordered = e3j_amd.convolution_bwd(coef, *args, dev(put(dm)), m.params, ordering, layout=layout, graph=graph)
     idx = np.asarray(m.coef.idx, dtype=np.int64)[:, :3]
     val, mix = np.asarray(m.coef.val, dtype=np.float32), m._mix.mix_indices
     ref, mag = H.forward_reference(idx, val, mix, x, y, s, snd, rcv, Z)
@@ -118,8 +129,10 @@ def test_odd_graph_in_float64_and_float16(case, dtype):
 
     coef = m._packed_coef(dtype)
     args = (dev(x), dev(y_dev), dev(s_dev), dev(snd), dev(rcv))
-    out = e3j_amd.convolution(coef, *args, m.params, ordering, layout="TRAILING_CHANNELS")
-    dx, dy, ds = e3j_amd.convolution_bwd(coef, *args, dev(dm), m.params, ordering, layout="TRAILING_CHANNELS")
+    graph = _handle(case, *args[3:], N, ordering)
+    out = e3j_amd.convolution(coef, *args, m.params, ordering, layout="TRAILING_CHANNELS", graph=graph)
+    dx, dy, ds = e3j_amd.convolution_bwd(coef, *args, dev(dm), m.params, ordering, layout="TRAILING_CHANNELS",
+                                         graph=graph)
     torch.cuda.synchronize()
     idx = np.asarray(m.coef.idx, dtype=np.int64)[:, :3]
     val = np.asarray(m.coef.val).astype(np_dtype).astype(np.float64)

@@ -27,6 +27,10 @@ def _graph(rng, kind):
         n = 37
         degree = rng.integers(0, 9, size=n)    # some rows are empty
         degree[5] = 300
+    elif kind == "many":                       # past the rows that keep their index order; a hub, empty rows
+        n = 300
+        degree = rng.integers(0, 4, size=n)
+        degree[7] = 200
     else:                                      # rows of 63, 64, 65 positions; padding edges; the last tile is short
         n = 13
         degree = np.array([63, 64, 65, 0, 1, 2, 7, 8, 9, 0, 30, 31, 4])
@@ -46,8 +50,9 @@ CASES = [(sig, kind) for sig in BUILTIN_SIGNATURES if sig[4] >= 64
          for kind in (("single", "hub") if sig[4] == 256 else ("single", "hub", "padding", "shuffled"))]
 
 
-def _compare_with_oracle(sig, kind, monkeypatch):
-    """Second derivatives through autograd, which must come from one call of the library."""
+def _compare_with_oracle(sig, kind, monkeypatch, handle=False, ordered=False):
+    """Second derivatives through autograd, which must come from one call of the library.  `handle`: the
+    adjacency from `prepare_graph`; `ordered`: the rows then have an order."""
     name, xi, yi, oi, channels = sig
     rng = np.random.default_rng(channels + len(kind))
     module = Convolution((xi, yi), oi, graph_ordering="NONE" if kind == "shuffled" else "RECEIVER")
@@ -63,10 +68,17 @@ def _compare_with_oracle(sig, kind, monkeypatch):
     results = []
     monkeypatch.setattr(ops, "_raw_second", lambda *a, f=ops._raw_second: results.append(f(*a)) or results[-1])
     leaves = [dev[k].requires_grad_(True) for k in ("x", "y", "s", "dm")]
-    out = module(*leaves[:3], torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda())
+    index = torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda()
+    graph = ops.prepare_graph(*index, n, module.graph_ordering) if handle else None
+    orders = []
+    monkeypatch.setattr(ops, "_fill_params",
+                        lambda *a, f=ops._fill_params, **k: orders.append(k.get("row_order")) or f(*a, **k))
+    out = module(*leaves[:3], *index, graph=graph)
     first = torch.autograd.grad(out, leaves[:3], leaves[3], create_graph=True)
     got = torch.autograd.grad(first, leaves, [dev["x2"], dev["y2"], dev["s2"]])
     assert len(results) == 1 and results[0] is not None     # (None: the first-order operators composed them)
+    if ordered:                                # of forward, backward and second-order backward
+        assert len(orders) == 3 and not any(torch.equal(o.cpu(), torch.arange(n).int()) for o in orders)
     live = ~pad
     idx = np.asarray(module.coef.idx, dtype=np.int64)
     val, mix = np.asarray(module.coef.val, dtype=np.float32), module._mix.mix_indices
@@ -111,6 +123,19 @@ def test_tiles_that_only_the_first_order_backward_can_hold(channels, variant, mo
             _compare_with_oracle(sig, "hub", monkeypatch)
     finally:
         lib.e3j_amd_set_launch_variant(0, 0)
+
+
+ORDERED = [(f"{table}_k{k}", kind, handle) for table, k in (("l3_l3_to_l3", 64), ("l3_l3_to_l3", 128), ("l2_l3_to_l2", 64))
+           for kind, handle in (("many", False), ("hub", True), ("padding", True), ("shuffled", True))]
+ORDERED += [("l3_l3_to_l3_k256", "hub", True), ("l0_l3_to_l3_k64", "many", False)]
+
+
+@pytest.mark.parametrize("name,kind,handle", ORDERED)
+def test_rows_with_an_order(name, kind, handle, monkeypatch):
+    """Rows and tiles in a locality order: prepared by the call (more rows than keep their index order) and by a
+    handle, which pairs rows too."""
+    sig = next(s for s in BUILTIN_SIGNATURES if s[0] == name)
+    _compare_with_oracle(sig, kind, monkeypatch, handle, ordered=True)
 
 
 #: tables the library is not built for: shapes of 64 channels at 192, and fewer waves per SIMD for the larger

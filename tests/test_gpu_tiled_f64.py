@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("x_irreps,channels", [("0e+1o+2e+3o", 64), ("0e+1o+2e", 128), ("0e", 64)])
-@pytest.mark.parametrize("kind,tile_rows,max_work", [("even", 1, 256), ("even", 4, 256), ("hub", 3, 7), ("sorted", -1, 64),
+@pytest.mark.parametrize("kind,tile_rows,max_work", [("even", 1, 256), ("even", 4, 256), ("hub", 3, 7), ("sorted", -1, 64), ("ordered", 4, 64),
                                                      ("one", 2, 256)])
 def test_tiled_equals_receiver_rows(x_irreps, channels, kind, tile_rows, max_work):
     n, e = (1, 9) if kind == "one" else (90, 1500)
@@ -45,11 +45,13 @@ def test_tiled_equals_receiver_rows(x_irreps, channels, kind, tile_rows, max_wor
     lib = _lib.load()
     limit = int(lib.e3j_amd_tile_rows_f64(sig))
     assert sig >= 0 and limit >= 1 and 1 <= lib.e3j_amd_tile_rows_default_f64(sig) <= limit
-    sch = TileSchedule(other, ptr, perm, None, n, limit if tile_rows < 0 else min(tile_rows, limit), max_work)
+    order = torch.randperm(n, device="cuda", generator=gen).int() if kind == "ordered" else None
+    sch = TileSchedule(other, ptr, perm, order, n, limit if tile_rows < 0 else min(tile_rows, limit), max_work)
     p = _lib.ConvParams(num_nodes=n, num_edges=e, num_coef=table.num_coef, num_x=dims[0], num_y=dims[1],
                         num_out=dims[2], num_scalars=dims[3], channels=channels, layout=_lib.LAYOUT_TRAILING,
                         val_dtype=_lib.F64, coef_idx_bytes=table.idx_bytes, signature=sig, coef_scale=1.0,
-                        coef_classes=ctypes.cast(classes, ctypes.c_void_p).value)
+                        coef_classes=ctypes.cast(classes, ctypes.c_void_p).value,
+                        row_order=order.data_ptr() if order is not None else None)
     pairs = []
     for tiled in (False, True):
         grads = [torch.full_like(t, float("nan")) for t in (x, y, s)]
