@@ -607,8 +607,9 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
 def _raw_second(meta: _Meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph=None):
     """Gradients of `<ddx, dx> + <ddy, dy> + <dds, ds>` with respect to `(x, y, s, dm)` in one call of the
     library, or None where it has no kernel for that (the first-order operators then compose them)."""
+    # (fixed_order_rows off asks for no scratch rows, and these kernels sum shared rows in no other way)
     if (meta.layout != Layout.TRAILING_CHANNELS or meta.ordering == GraphOrdering.SENDER or y.shape[0] == 0
-            or x.dtype != torch.float32 or config().deterministic):
+            or x.dtype != torch.float32 or config().deterministic or not config().fixed_order_rows):
         return None
     sig = meta.table.signature(*_shape(meta, x, y, s), meta.layout)[0]
     # (the second-order kernel has one shape, the first-order limit is the selected variant's)

@@ -138,6 +138,30 @@ def test_rows_with_an_order(name, kind, handle, monkeypatch):
     _compare_with_oracle(sig, kind, monkeypatch, handle, ordered=True)
 
 
+def test_no_scratch_rows_without_the_fixed_order(monkeypatch):
+    """`config(fixed_order_rows=False)` promises no scratch rows: the second derivatives are then composed from the
+    first-order operators, which add the pieces of long rows with atomics."""
+    n, snd, rcv = _graph(np.random.default_rng(3), "hub")
+    module = Convolution(("0e+1o", "0e+1o+2e"), "0e+1o+2e", graph_ordering="RECEIVER")
+    rand = lambda *shape: torch.randn(shape, device="cuda")  # noqa: E731
+    dims = module.source[0].dim, module.source[1].dim, module.params.num_scalars, module.target.dim
+    leaves = [t.requires_grad_(True) for t in (rand(n, dims[0], 64), rand(len(snd), dims[1]), rand(len(snd), dims[2], 64),
+                                               rand(n, dims[3], 64))]
+    second = [rand(*t.shape) for t in leaves[:3]]
+    index = torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda()
+    results = []
+    for fixed in (False, True):
+        graph = ops.prepare_graph(*index, n)
+        with config.use(fixed_order_rows=fixed):
+            out = module(*leaves[:3], *index, graph=graph)
+            first = torch.autograd.grad(out, leaves[:3], leaves[3], create_graph=True)
+            results.append(torch.autograd.grad(first, leaves, second))
+        assert any(s._partials for s in graph._segments.values()) == fixed
+    for a, b in zip(*results):
+        # sums of at most 300 terms in another order, twice: sqrt(300) roundings of the largest value
+        assert float((a - b).abs().max()) <= 2 * 300 ** 0.5 * 1.2e-7 * float(b.abs().max())
+
+
 #: tables the library is not built for: shapes of 64 channels at 192, and fewer waves per SIMD for the larger
 #: tables (`second_shapes`: two in both kernels; two and one)
 RUN_TIME = [("0e+1o+2e", "0e+1o+2e", "0e+1o+2e", 64), ("0e+1o+2e", "0e+1o+2e", "0e+1o+2e", 192),
