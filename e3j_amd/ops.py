@@ -4,9 +4,10 @@ Same signatures, argument meaning and errors as the reference's primitives
 (`src/e3j/ops/convolution.py:106-116,334-345`), with tensors in GPU memory
 and the HIP library of this package behind them instead of the CUDA `e3j_ops`
 binding.  `convolution` is differentiable in `(x, y, s)` to any reverse-mode
-order: its backward is `convolution_bwd`, whose own backward is expressed with
-three `convolution` and three `convolution_bwd` calls
-(`src/e3j/ops/convolution.py:535-562`).
+order: its backward is `convolution_bwd`, whose own backward is one call of the
+library where no further derivative is recorded (`_raw_second`: float32, trailing
+layout, at least 64 channels, not SENDER rows) and is otherwise expressed with three
+`convolution` and three `convolution_bwd` calls (`src/e3j/ops/convolution.py:535-562`).
 
 Extensions over the reference's operator: a `layout` keyword (the reference's
 fused kernel is trailing-channels only), any channel count (no power-of-two
@@ -256,23 +257,24 @@ def _check_operands(x, y, s, sender, receiver):
         raise TypeError("x, y and s must share one dtype")
 
 
-#: An adjacency that one call prepares for itself keeps the index order up to this many rows and edges, unless
-#: `config(locality_rounds=...)` asks for another number of sweeps than the default: so few rows fit the
-#: compute units and one L2 in any order, the tiles of the backward lose few shared senders, and the order is
-#: three launches.  GPU time of forward and VJP without and with it, x, y, out l <= 3, microseconds: 128 rows of
-#: 19 edges 125 and 136 at 128 channels, 256 rows of 30 edges 174 and 188 (256 channels 241 and 250; l <= 2 at 64
-#: channels 94 and 108); on the host 10 us a call.  At 256 rows of 120 edges it is the other way round (525 and 486 at
-#: 128 channels), and a handle, whose order serves many calls, always has it (473 and 426 there).
-UNORDERED_ROWS, UNORDERED_EDGES = 256, 16384
+#: Graphs of up to this many rows keep the index order, unless `config(locality_rounds=...)` asks for another
+#: number of sweeps than the default: so few rows fit the compute units and one L2 in any order, the tiles of
+#: the backward lose few shared senders, and the order is three launches (10 us a call on the host).  GPU time of
+#: forward and VJP without and with it, microseconds, the graph prepared by the call, 256 rows: of 30 edges, x, y, out
+#: l <= 3 at 128 channels 174 and 188 (256 channels 241 and 250; l <= 2 at 64 channels 94 and 108); of 200 edges
+#: with hub rows 763 and 813 (1 336 and 1 380; 397 and 428); all rows joined with all 800 and 825 (1 392 and 1 412; 422
+#: and 451).  On a handle, whose order is made once, the two are within 4 % of each other (149 and 151; 705 and 703;
+#: 758 and 760), except that hub rows side by side share a compute unit (194 rows, x l <= 2 to l <= 3 at 128
+#: channels, to the second derivatives: 606 and 659).
+UNORDERED_ROWS = 256
 
 
-def _order_rounds(n: int, num_edges: int, kept: bool = False) -> int:
-    """Sweeps behind the row order of an adjacency (0: index order); `kept`: see `PreparedGraph`."""
+def _order_rounds(n: int, num_edges: int) -> int:
+    """Sweeps behind the row order of an adjacency (0: index order)."""
     rounds = int(config().locality_rounds)
     if n < 2 or num_edges == 0 or rounds <= 0:
         return 0
-    small = n <= UNORDERED_ROWS and num_edges <= UNORDERED_EDGES
-    return 0 if small and not kept and rounds == Config.locality_rounds else rounds
+    return 0 if n <= UNORDERED_ROWS and rounds == Config.locality_rounds else rounds
 
 
 def _paired(order, other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: bool | None):
@@ -286,7 +288,7 @@ def _paired(order, other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: boo
 
 
 def _row_order(other: torch.Tensor, row_ptr: torch.Tensor, n: int, pair: bool | None = None):
-    """Processing order of the rows of a CSR that one call prepares for itself, None for the index order."""
+    """Processing order of the rows of a CSR, None for the index order."""
     rounds = _order_rounds(n, int(other.numel()))
     return _paired(locality_order(other, row_ptr, n, rounds) if rounds > 0 else None, other, row_ptr, n, pair)
 
@@ -432,7 +434,7 @@ def _prepare_graph(ordering: GraphOrdering, n: int, sender: torch.Tensor, receiv
     else:
         key, other = receiver, sender
     if n >= 1 and 0 < key.numel() == other.numel():
-        rounds = _order_rounds(n, int(key.numel()), kept)
+        rounds = _order_rounds(n, int(key.numel()))
         row_ptr, other, perm, order, segments = prepare_rows(
             key, other, n, ordering != GraphOrdering.NONE, rounds, pieces)
         graph = PreparedGraph(other, row_ptr, perm, _paired(order, other, row_ptr, n, pair), n, ordering, kept)

@@ -97,9 +97,8 @@ class Config:
     #: atomic-free backward for `dx` (bit-reproducible, slower).
     deterministic: bool = False
     #: sweeps of label propagation behind the locality-aware row order of the kernels
-    #: (0 = rows are processed in index order).  At the default, an adjacency that an operator call prepares
-    #: for itself stays in index order up to 256 rows and 16 384 edges, where the order costs more than it
-    #: gives; any other number, and the handles of `prepare_graph`, order the rows of graphs of any size.
+    #: (0 = rows are processed in index order).  At the default, graphs of up to 256 rows stay in index
+    #: order, where the order costs more than it gives; any other number orders graphs of any size.
     locality_rounds: int = 2
     #: keep the adjacencies prepared for the index tensors seen last and reuse them when the same
     #: tensors (identity and in-place version) come again.  Off by default: a buffer rewritten behind
@@ -118,13 +117,13 @@ class Config:
     #: serves many calls; True: also for the adjacency an operator call prepares for itself; False: never
     pair_rows: object = "prepared"
     #: positions of a row one wave of the forward pass sums; longer rows are shared between waves
-    #: (their sums then come from float atomics).  -1: twice the mean row length, at least 64;
+    #: (`fixed_order_rows` says how their pieces are added).  -1: twice the mean row length, at least 64;
     #: 0: never share a row.
     row_cap: int = -1
     #: add the pieces of a shared row to its output row in a fixed order (a scratch row per piece,
     #: up to 256 MB per prepared graph; the forward then gives the same bits in every run, as the
     #: reference's does); off: the pieces are added with float atomics (no scratch, and about 0.1 ms
-    #: less for a hub of 50 000 edges)
+    #: less for a hub of 50 000 edges) and second derivatives are composed from the first-order operators
     fixed_order_rows: bool = True
     #: compile unrolled kernels at run time for coefficient tables the library was not built
     #: for (needs hipcc; about half a minute per new table, cached on disk); off: such tables

@@ -36,10 +36,13 @@ def _degrees(rng, kind, n):
 
 
 def _handle(case, sender, receiver, n, ordering):
-    """Half of the cases (5 to 9, 15 to 19, ...) run with a prepared handle: its rows have a paired locality order
-    whatever the size, where a small graph prepared by the call itself keeps the index order."""
-    graph = prepare_graph(sender, receiver, n, ordering) if case // 5 % 2 else None
-    if graph is not None and n > 1 and sender.numel() > 0:
+    """Half of the cases (5 to 9, 15 to 19, ...) run with a prepared handle, whose rows have a locality order
+    and are paired: asked for, since graphs as small as these keep the index order at the default."""
+    if case // 5 % 2 == 0:
+        return None
+    with e3j_amd.config.use(locality_rounds=1 + case % 3):
+        graph = prepare_graph(sender, receiver, n, ordering)
+    if n > 1 and sender.numel() > 0:
         assert graph.order is not None
     return graph
 

@@ -69,7 +69,8 @@ def _compare_with_oracle(sig, kind, monkeypatch, handle=False, ordered=False):
     monkeypatch.setattr(ops, "_raw_second", lambda *a, f=ops._raw_second: results.append(f(*a)) or results[-1])
     leaves = [dev[k].requires_grad_(True) for k in ("x", "y", "s", "dm")]
     index = torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda()
-    graph = ops.prepare_graph(*index, n, module.graph_ordering) if handle else None
+    with config.use(locality_rounds=1):        # (graphs as small as most of these keep the index order at 2)
+        graph = ops.prepare_graph(*index, n, module.graph_ordering) if handle else None
     orders = []
     monkeypatch.setattr(ops, "_fill_params",
                         lambda *a, f=ops._fill_params, **k: orders.append(k.get("row_order")) or f(*a, **k))
