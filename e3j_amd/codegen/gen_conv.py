@@ -64,7 +64,9 @@ LAUNCH = {
 #: parts of the float64 kernels: (forward, backward).  A double takes the registers of two channels
 #: of a float kernel, so these are the splits the two-channel float kernels use.
 F64_SPLIT = (3, 4)
-#: float64 backward over tiles of receivers: (waves per block, resident waves per SIMD, receivers per tile)
+#: float64 backward over tiles of receivers: (waves per block, resident waves per SIMD, receivers per tile);
+#: 150 to 185 registers, two waves per SIMD (the l <= 3 table also keeps 20 bytes of scratch at 64 and 128 channels,
+#: none of it spilled vector registers)
 F64_TILE = (4, 1, 4)
 #: float16 kernels (values held as half, computed in float): (channels per lane, parts forward,
 #: parts backward) by whether the channel count is a multiple of 128; the splits of the float

@@ -496,7 +496,8 @@ __global__ void live_keys_kernel(const int32_t *__restrict__ other, const int32_
 
 // ---- schedule of the backward over tiles of receivers ---------------------------------------
 // Tiles are `tile_rows` consecutive entries of the row order.  A scan of the tiles' position
-// counts places each tile's list; one wave per tile then writes the list, sorted by sender.
+// counts places each tile's list; one wave per tile, or a workgroup where the tiles are longer than a
+// wave, then writes the list, sorted by sender.
 
 __global__ void tile_rank_kernel(const int32_t *__restrict__ row_order, int num_nodes,
                                  int32_t *__restrict__ rank) {

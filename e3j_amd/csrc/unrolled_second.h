@@ -18,6 +18,8 @@
 // 120k edges, K = 128, l <= 3: 0.71 ms (rows; the two streams alone 0.60 ms at the rate of a copy) and
 // 1.22 ms (tiles; three streams, 0.90 ms) against 4.1 ms for the composed form (3 x 0.35 forward,
 // 3 x 0.73 backward, 0.9 of sums); forward, backward and second-order backward together 5.37 -> 3.11 ms.
+// (Every table with tiles takes them: at 64 to 256 channels, 30 to 6 000 nodes, even or hub rows, the built-in
+// tables take 0.51 to 0.72 of the composed form's time.)
 // Both are bound by their vector instructions (4 370 and 6 210 per edge and 128 channels) at two to three
 // waves per SIMD, the tile kernel next by the latency of its first loads per tile.
 #ifndef E3J_AMD_CSRC_UNROLLED_SECOND_H_
