@@ -460,9 +460,8 @@ __global__ __launch_bounds__(kBlockThreads) void rows_block_kernel(const int32_t
     if (segments != nullptr && threadIdx.x < 4) segments[threadIdx.x] = 0;
     const bool mine = rows_from_keys(key, other, nullptr, num_edges, num_nodes, other_out, row_ptr,
                                      threadIdx.x / kWave, kBlockThreads / kWave, threadIdx.x % kWave);
-    // the rows above have arrived before another wave clears them for the counts: the barrier below orders
-    // the waves, not their stores
-    __threadfence();
+    // the rows above are ordered before another wave of the workgroup clears them for the counts
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     if (__syncthreads_or(mine ? 1 : 0)) rows_by_count(key, num_edges, num_nodes, row_ptr);
     if (!list_pieces || segments == nullptr) return;
     __threadfence();

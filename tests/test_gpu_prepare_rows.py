@@ -98,8 +98,8 @@ def test_against_numpy(n, e, kind, form):
 @pytest.mark.parametrize("n,e", [(16000, 16384), (9000, 16384), (40, 16384), (20000, 1000)])
 def test_out_of_order_keys_of_one_workgroup(n, e):
     """Keys out of order in the route of one workgroup: its first pass writes row pointers that the count
-    replaces, from other waves.  The first pass's stores have to have arrived by then (the kernel's fence),
-    or one of them overwrites a count."""
+    replaces, from other waves.  The first pass's stores are ordered before that (the kernel's fence), or one of
+    them would overwrite a count."""
     rng = np.random.default_rng(n)
     dev = lambda a: torch.from_numpy(a.astype(np.int32)).cuda()  # noqa: E731
     for _ in range(20):
