@@ -139,6 +139,50 @@ def test_rows_with_an_order(name, kind, handle, monkeypatch):
     _compare_with_oracle(sig, kind, monkeypatch, handle, ordered=True)
 
 
+@pytest.mark.parametrize("handle", [False, True])
+def test_capture_and_replay(handle):
+    """Forward, backward and second-order backward (and the preparation of sorted rows) recorded into a graph: every
+    replay on rewritten operands equals the eager call."""
+    n, snd, rcv = _graph(np.random.default_rng(5), "many")
+    module = Convolution(("0e+1o+2e", "0e+1o+2e+3o"), "0e+1o+2e", graph_ordering="RECEIVER")
+    dims = module.source[0].dim, module.source[1].dim, module.params.num_scalars, module.target.dim
+    shapes = [(n, dims[0], 64), (len(snd), dims[1]), (len(snd), dims[2], 64), (n, dims[3], 64)]
+    operands = [torch.zeros(shape, device="cuda") for shape in (*shapes, *shapes[:3])]    # x, y, s, dm and the cotangents
+    x, y, s, dm = operands[:4]
+    index = torch.from_numpy(snd).cuda(), torch.from_numpy(rcv).cuda()
+    meta = ops._make_meta(module._packed_coef("float32"), x, y, s, module.params, module.graph_ordering, None, module.layout)
+    kept = ops.prepare_graph(*index, n) if handle else None
+
+    def passes():
+        graph = kept or ops._prepare_graph(meta.ordering, n, *index, pieces=ops._row_pieces(meta, x, len(snd)))
+        out = ops._raw_forward(meta, x, y, s, *index, graph)
+        first = ops._raw_backward(meta, x, y, s, dm, *index, graph)
+        return out, *first, *ops._raw_second(meta, *operands, *index, graph)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        passes()                                          # warm-up outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        recorded = passes()
+    for trial in range(4):
+        for t in operands:
+            t.copy_(torch.randn_like(t))
+        eager = passes()
+        for t in recorded:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for which, (a, b) in enumerate(zip(recorded, eager)):
+            if which in (0, 3, 6, 7):                     # out, ds, and the second-order ds and dm: fixed orders
+                assert torch.equal(a, b), (trial, which)
+            else:                                         # atomics: equal up to summation order
+                assert float((a - b).abs().max()) <= 2e-5 * float(b.abs().max()), (trial, which)
+
+
 def test_no_scratch_rows_without_the_fixed_order(monkeypatch):
     """`config(fixed_order_rows=False)` promises no scratch rows: the second derivatives are then composed from the
     first-order operators, which add the pieces of long rows with atomics."""
