@@ -273,6 +273,7 @@ __global__ __launch_bounds__(kEdgeLanes) void edge_features_fwd_kernel(
             const int units = sz.hidden;
             const bool side_by_side = units < kEdgeLanes;  // several edges at a time
             const int edges = side_by_side ? kEdgeLanes / units : 1;
+            const bool some_dead = __popcll(live_edges) != count;  // (of the wave: one branch past the mask)
             for (int l = 0; l < sz.layers; l++) {
                 const T *w = w1 + (int64_t)l * sz.num_basis * units;
                 T *rows = h + ((int64_t)l * sz.num_edges + e0) * units;
@@ -285,7 +286,9 @@ __global__ __launch_bounds__(kEdgeLanes) void edge_features_fwd_kernel(
                         T pre = T(0);
 #pragma unroll
                         for (int n = 0; n < NB; n++) pre += lds_basis[i][n] * col[n];
-                        rows[(int64_t)i * units + j] = (live_edges >> i) & 1ull ? pre * sigmoid(pre) : T(0);
+                        T value = pre * sigmoid(pre);
+                        if (some_dead) value = (live_edges >> i) & 1ull ? value : T(0);
+                        rows[(int64_t)i * units + j] = value;
                     }
                 }
             }
