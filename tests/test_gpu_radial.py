@@ -97,3 +97,63 @@ def test_input_gradient_matches_the_float64_product(inner, edges, n):
     pick[torch.arange(edges), (torch.arange(edges) * 7) % n] = 1.0
     (picked,) = torch.autograd.grad(radial_linear(h, wi), (h,), pick)
     assert torch.equal(picked, wi.t()[(torch.arange(edges, device="cuda") * 7) % n])
+
+
+@pytest.mark.parametrize("inner", [64, 128])
+@pytest.mark.parametrize("edges,n", [(63, 64), (65, 32), (300, 2944), (3000, 544)])
+@pytest.mark.parametrize("largest", ["first", "last", "anywhere"])
+def test_scales_of_the_split_products_follow_the_terms(inner, edges, n, largest):
+    """Operands whose magnitude differs by up to 2^40 from row to row and along the sums: every result
+    within float32 rounding of its own sum of magnitudes (2^-24 a term for the split operands and for the
+    sums, as for operands of one size; terms below 2^-13 of the largest are held to 2^-37 of it, n 2^-37 < 2^-24)."""
+    g = torch.Generator(device="cuda").manual_seed(inner + edges + n)
+
+    def spread(count):
+        e = torch.linspace(-20, 20, count, device="cuda").round()
+        if largest == "first":
+            e = e.flip(0)
+        if largest == "anywhere":
+            e = e[torch.randperm(count, device="cuda", generator=g)]
+        return torch.exp2(e)
+
+    h = (torch.randn(edges, inner, device="cuda", generator=g) * spread(edges)[:, None]
+         * spread(inner)[None]).requires_grad_(True)
+    w = (torch.randn(inner, n, device="cuda", generator=g) * spread(n)[None]).requires_grad_(True)
+    ds = torch.randn(edges, n, device="cuda", generator=g) * spread(edges)[:, None] * spread(n)[None]
+    ds[edges // 2] = 0.0
+    s = radial_linear(h, w)
+    dh, dw = torch.autograd.grad(s, (h, w), ds)
+    hd, wd, dd = h.detach().double(), w.detach().double(), ds.double()
+    for got, a, b, terms in ((s.detach(), hd, wd, inner), (dh, dd, wd.t().contiguous(), n),
+                             (dw, hd.t().contiguous(), dd, edges)):
+        bound = (8 + terms ** 0.5) * 2.0 ** -24 * (a.abs() @ b.abs())
+        assert bool(((got.double() - a @ b).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("inner", [8, 32, 64, 128])
+@pytest.mark.parametrize("edges,n", [(5, 2944), (256, 992), (70000, 64)])
+def test_forward_over_ranges_of_columns(inner, edges, n):
+    """Few edges: blocks share the columns; many: each takes all of them."""
+    g = torch.Generator(device="cuda").manual_seed(inner + edges)
+    h = torch.randn(edges, inner, device="cuda", generator=g)
+    w = torch.randn(inner, n, device="cuda", generator=g)
+    want = h.double() @ w.double()
+    bound = 8 * 2.0 ** -24 * (h.double().abs() @ w.double().abs())
+    assert bool(((radial_linear(h, w).double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_value_that_is_no_number_stays_in_its_row_and_column(bad):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    h = torch.randn(300, 64, device="cuda", generator=g)
+    w = torch.randn(64, 96, device="cuda", generator=g)
+    ds = torch.randn(300, 96, device="cuda", generator=g)
+    h[7, 5], ds[200, 40] = bad, bad
+    h.requires_grad_(True)
+    w.requires_grad_(True)
+    s = radial_linear(h, w)
+    dh, dw = torch.autograd.grad(s, (h, w), ds)
+    rows = lambda t: torch.nonzero(~t.isfinite().all(1)).flatten().tolist()   # noqa: E731
+    assert rows(s) == [7] and rows(dh) == [200]
+    assert rows(dw[:, torch.arange(96, device="cuda") != 40]) == [5]
+    assert not bool(dw[:, 40].isfinite().any())
