@@ -103,6 +103,31 @@ def _compile_one(src: str, extra: list[str]) -> str:
     return obj
 
 
+#: the native host side of the operators (`native.py`): plain C++ against torch, no device code
+HOST_SOURCE = os.path.join(CSRC, "host", "operators.cpp")
+HOST_PATH = os.path.join(HERE, "lib", "_operators.so")
+
+
+def build_host() -> str:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    # (__HIP_PLATFORM_AMD__, USE_ROCM: what the HIP and torch headers ask of a host compiler)
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{path}" for path in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
+           f"-isystem{sysconfig.get_paths()['include']}", HOST_SOURCE, "-o", HOST_PATH + ".tmp", f"-L{lib_dir}",
+           "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-lc10", "-lc10_hip"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {HOST_SOURCE}:\n{' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
+    return HOST_PATH
+
+
 def sources() -> list[str]:
     return sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(GENERATED, "*.hip")))
 
@@ -121,7 +146,9 @@ def build(regenerate: bool = True, jobs: int | None = None, verbose: bool = True
     if verbose:
         print(f"[e3j_amd.build] compiling {len(srcs)} sources for {ARCH} with {jobs} jobs", flush=True)
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        host = pool.submit(build_host)
         objs = list(pool.map(lambda s: _compile_one(s, extra), srcs))
+        host.result()
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", LIB_PATH + ".tmp", *objs]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:

@@ -16,6 +16,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
+from . import native
 from .coef import Coef4D, resolve_val_dtype
 from .graph import GraphCSR
 from .ops import ConvolutionParams, convolution
@@ -52,6 +53,10 @@ class Convolution:
         self._mix = mix
         self._coef = None
         self._packed = {}
+        self._plans, self._plan_sets = None, {}   # plans of the native call by settings and kind of operand
+
+    def __getstate__(self):   # (plans hold device memory and are made again on use)
+        return {**self.__dict__, "_plans": None, "_plan_sets": {}}
 
     @property
     def coef(self) -> Coef4D:
@@ -110,5 +115,8 @@ class Convolution:
         if node_mask is not None:
             senders, receivers = GraphCSR.mask_edges(senders, receivers, node_mask)
         if self.config.convolution == ConvolutionImpl.FUSED_HIP:
+            out = native.call(self, node_features, edge_features, edge_scalars, senders, receivers, graph)
+            if out is not None:
+                return out
             return self._fused_eval(node_features, edge_features, edge_scalars, senders, receivers, graph)
         raise RuntimeError("Unknown convolution implementation.")

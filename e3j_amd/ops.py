@@ -326,6 +326,7 @@ class PreparedGraph:
         self.ordering = ordering
         self._schedules = {}
         self._segments = {}
+        self._native = {}
         self._mark()
 
     def _mark(self):
@@ -368,6 +369,35 @@ class PreparedGraph:
             self.ready()
             hit = self._segments[key] = RowSegments(self.row_ptr, self.num_nodes, self.num_edges, *key)
             self._mark()
+        return hit
+
+    def adopt_segments(self, buffer: torch.Tensor, row_cap: int, row_piece: int) -> None:
+        """Take a list of pieces that was built with the adjacency."""
+        pieces = RowSegments(None, self.num_nodes, self.num_edges, row_cap, row_piece)
+        pieces.buffer = buffer
+        self._segments[(int(row_cap), int(row_piece))] = pieces
+
+    def native(self, plan, module, x: torch.Tensor, cfg: Config):
+        """The arrays of this adjacency for the native calls of a plan (`native.py`), None if they are not of
+        the plain kind."""
+        arrays = (self.other, self.row_ptr, self.perm, self.order)
+        hit, seen = self._native.get(plan, (None, ()))
+        if hit is None or any(a is not b for a, b in zip(arrays, seen)):
+            from . import native
+            if any(t.dtype != torch.int32 or not t.is_contiguous() or t.device != x.device
+                   for t in arrays if t is not None):
+                return None
+            want = None
+            if module.layout == Layout.TRAILING_CHANNELS and x.dtype == torch.float32 and self.num_edges > 0:
+                want = _pieces_for(self.num_nodes, self.num_edges, int(module.target.dim) * int(x.shape[2]), cfg)
+            pieces = self.segments(*want) if want is not None else None
+            listed = pieces is not None and pieces.count > 0
+            hit = native.load().adjacency(
+                self.num_nodes, *arrays, pieces is not None,
+                pieces.row_cap if pieces is not None else 0, pieces.row_piece if pieces is not None else 0,
+                pieces.count if pieces is not None else 0, pieces.buffer if listed else None,
+                pieces.partials(int(module.target.dim), int(x.shape[2])) if listed else None)
+            self._native[plan] = hit, arrays
         return hit
 
 
@@ -457,12 +487,15 @@ def _row_pieces(meta: _Meta, x: torch.Tensor, num_edges: int):
     if (meta.layout != Layout.TRAILING_CHANNELS or x.dtype != torch.float32 or num_edges == 0
             or (cfg.deterministic and not fixed_order)):
         return None
+    return _pieces_for(x.shape[0], num_edges, int(meta.params.num_out) * int(x.shape[2]), cfg)
+
+
+def _pieces_for(num_nodes: int, num_edges: int, row_floats: int, cfg: Config):
     want = int(cfg.row_cap)
-    cap = row_cap_for(x.shape[0], num_edges) if want < 0 else want
+    cap = row_cap_for(num_nodes, num_edges) if want < 0 else want
     if cap <= 0:
         return None
-    row_floats = int(meta.params.num_out) * int(x.shape[2])
-    return cap, row_piece_for(num_edges, row_floats) if fixed_order else ROW_PIECE
+    return cap, row_piece_for(num_edges, row_floats) if cfg.fixed_order_rows else ROW_PIECE
 
 
 def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Tensor:
@@ -665,12 +698,17 @@ def _tiles_pay_f64(num_edges: int, num_x: int, num_scalars: int, channels: int, 
     x or fewer are a small part of the stream (480k edges, four rows 1 395 to 1 381, one row 793 to 760).
     Rows of uneven length gain at all of these sizes (5 to 30 %).
     """
+    least = tile_values_f64(num_x, num_scalars, kept)
+    return least is not None and num_edges * num_x * channels >= least
+
+
+def tile_values_f64(num_x: int, num_scalars: int, kept: bool) -> int | None:
+    """Values added to dx from which `_tiles_pay_f64` says yes, None: never."""
     if num_x < TILE_F64_ROWS:
-        return False
-    values = num_edges * num_x * channels
+        return None
     if 2 * num_scalars > 3 * num_x:
-        return kept and values >= 4 * TILE_F64_VALUES
-    return values >= (TILE_F64_VALUES if kept else TILE_F64_VALUES_ONE_CALL)
+        return 4 * TILE_F64_VALUES if kept else None
+    return TILE_F64_VALUES if kept else TILE_F64_VALUES_ONE_CALL
 
 
 def _tile_rows(signature: int, f64: bool = False) -> int:
