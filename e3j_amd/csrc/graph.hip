@@ -54,7 +54,7 @@ __global__ void gather_kernel(const int32_t *__restrict__ src, const int32_t *__
 // A row is read up to kLabelRowCap positions: the labels only steer which rows run together,
 // and a thread that walked a hub's whole row would outlast the rest of the sweep many times.
 constexpr int kLabelRowCap = 128;
-constexpr int kLabelLanes = 4;  // lanes that share a row (its gathers then run four at a time)
+constexpr int kLabelLanes = 16;  // lanes that share a row (its gathers then run sixteen at a time)
 __global__ void min_label_kernel(const int32_t *__restrict__ other,
                                  const int32_t *__restrict__ row_ptr, int num_nodes,
                                  const int32_t *__restrict__ cur, int32_t *__restrict__ next,
@@ -479,6 +479,120 @@ __global__ void sort_input_kernel(const int32_t *__restrict__ key, int64_t num_e
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < num_edges; i += stride) {
         keys[i] = min(wrap_node(key[i], num_nodes), num_nodes);
         positions[i] = (int32_t)i;
+    }
+}
+
+// Stable sort of edge positions by key for up to kSortChunk * kSortChunks edges of fewer than 2^16 nodes, in two passes
+// of at most eight bits, a count and a scatter each: four launches, where the library's sort takes
+// eight and the launch that writes its keys a ninth (150k edges, 5 000 nodes: 58 us -> 20; 3-5 us a launch whatever
+// it moves).  A workgroup takes kSortChunk consecutive edges; the scatter of each adds up for itself how
+// many edges of a smaller digit, or of the same one in an earlier chunk, there are.
+constexpr int kSortItems = 4, kSortChunk = kBlockThreads * kSortItems, kSortChunks = 64, kSortDigits = 256;
+
+// `key` from the endpoints (`reduce`: as sort_input_kernel makes it) or from the pass before
+__device__ __forceinline__ unsigned sort_key(const int32_t *key, int64_t i, int num_nodes, bool reduce) {
+    return (unsigned)(reduce ? min(wrap_node(key[i], num_nodes), num_nodes) : key[i]);
+}
+__global__ __launch_bounds__(kBlockThreads) void edge_digits_kernel(const int32_t *__restrict__ key, int64_t num_edges,
+                                                                    int num_nodes, bool reduce, int shift, unsigned mask,
+                                                                    int32_t *__restrict__ digits) {
+    __shared__ int count[kSortDigits];
+    if (threadIdx.x < kSortDigits) count[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSortItems; k++) {
+        const int64_t i = (int64_t)blockIdx.x * kSortChunk + k * kBlockThreads + threadIdx.x;
+        if (i < num_edges) atomicAdd(&count[sort_key(key, i, num_nodes, reduce) >> shift & mask], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < kSortDigits) digits[blockIdx.x * kSortDigits + threadIdx.x] = count[threadIdx.x];
+}
+// `from`: position a key came from (null: its own)
+__global__ __launch_bounds__(kBlockThreads) void edge_scatter_kernel(
+    const int32_t *__restrict__ key, const int32_t *__restrict__ from, int64_t num_edges, int num_nodes, bool reduce,
+    int shift, int step, const int32_t *__restrict__ digits, int32_t *__restrict__ key_out, int32_t *__restrict__ from_out) {
+    constexpr int WAVES = kBlockThreads / kWave, PARTS = kBlockThreads / kSortDigits;
+    __shared__ uint16_t counts[kSortDigits][WAVES];  // edges of a digit in a wave, then in the waves before it
+    __shared__ int before[PARTS][kSortDigits], all[PARTS][kSortDigits], sums[kSortDigits / kWave];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    const unsigned mask = (1u << step) - 1;
+    {   // a quarter of the chunks each: edges of a digit in all of them and in those before this one
+        const int digit = tid % kSortDigits, part = tid / kSortDigits, chunks = gridDim.x;
+        int mine = 0, total = 0;
+        for (int c = part; c < chunks; c += PARTS) {
+            const int v = digits[c * kSortDigits + digit];
+            total += v;
+            if (c < (int)blockIdx.x) mine += v;
+        }
+        before[part][digit] = mine;
+        all[part][digit] = total;
+    }
+    for (int i = lane; i < kSortDigits; i += kWave) counts[i][wave] = 0;
+    unsigned item[kSortItems];
+    int rank[kSortItems], source[kSortItems];
+    const int64_t first = (int64_t)blockIdx.x * kSortChunk + wave * (kSortItems * kWave);
+#pragma unroll
+    for (int k = 0; k < kSortItems; k++) {
+        const int64_t i = first + k * kWave + lane;
+        item[k] = i < num_edges ? sort_key(key, i, num_nodes, reduce) : 0u;
+        source[k] = i < num_edges ? (from != nullptr ? from[i] : (int)i) : 0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int k = 0; k < kSortItems; k++) {  // (as in BlockSort: lanes of equal digits find each other with ballots)
+        const bool inside = first + k * kWave + lane < num_edges;
+        const unsigned digit = item[k] >> shift & mask;
+        unsigned long long same = __ballot(inside);
+#pragma unroll
+        for (int bit = 0; bit < 8; bit++) {
+            if (bit == step) break;
+            const unsigned long long set = __ballot((digit >> bit) & 1u);
+            same &= (digit >> bit) & 1u ? set : ~set;
+        }
+        const int earlier = counts[digit][wave];
+        rank[k] = earlier + __popcll(same & ((1ull << lane) - 1ull));
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (inside && (same >> lane) == 1ull) counts[digit][wave] = (uint16_t)(rank[k] + 1);  // the last of its digit
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    int start = 0, total = 0;
+    if (tid < kSortDigits) {
+#pragma unroll
+        for (int p = 0; p < PARTS; p++) {
+            start += before[p][tid];
+            total += all[p][tid];
+        }
+        int sum = 0;
+        for (int w = 0; w < WAVES; w++) {
+            const int c = counts[tid][w];
+            counts[tid][w] = (uint16_t)sum;
+            sum += c;
+        }
+        int after = total;  // edges of this digit and of smaller ones
+#pragma unroll
+        for (int off = 1; off < kWave; off *= 2) {
+            const int add = __shfl_up(after, off, kWave);
+            if (lane >= off) after += add;
+        }
+        if (lane == kWave - 1) sums[wave] = after;
+        start += after - total;
+    }
+    __syncthreads();
+    if (tid < kSortDigits) {
+        for (int w = 0; w < wave; w++) start += sums[w];
+        before[0][tid] = start;  // where the chunk's edges of the digit begin
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSortItems; k++) {
+        if (first + k * kWave + lane >= num_edges) continue;
+        const unsigned digit = item[k] >> shift & mask;
+        const int to = before[0][digit] + counts[digit][wave] + rank[k];
+        key_out[to] = (int32_t)item[k];
+        from_out[to] = source[k];
     }
 }
 
@@ -1214,12 +1328,17 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
 namespace {
 struct PrepareWorkspace {
     size_t order, sort_temp, sort_bytes, keys_in, keys_out, positions, unsorted, total;
+    // the sort of this file: keys of two eight-bit digits, chunks whose counts a workgroup reads by itself
+    static bool own_sort(int32_t num_nodes, int64_t num_edges) {
+        return num_nodes < (1 << 16) && num_edges <= (int64_t)kSortChunk * kSortChunks;
+    }
     PrepareWorkspace(int32_t num_nodes, int64_t num_edges, bool sorted) {
         size_t at = 0;
         auto take = [&](size_t bytes) { const size_t here = at; at += align_up(bytes); return here; };
         order = take(e3j_amd_order_workspace_bytes(num_nodes));
         unsorted = take(sizeof(int32_t) * kMaxRowsBlocks);
-        sort_bytes = sorted ? 0 : sort_temp_bytes(num_edges);
+        sort_bytes = sorted ? 0 : own_sort(num_nodes, num_edges) ? sizeof(int32_t) * kSortChunks * kSortDigits
+                                                                 : sort_temp_bytes(num_edges);
         sort_temp = take(sort_bytes);
         const size_t list = sorted ? 0 : sizeof(int32_t) * (size_t)num_edges;
         keys_in = take(list);
@@ -1257,17 +1376,33 @@ int e3j_amd_prepare_rows(const int32_t *key, const int32_t *other, int64_t num_e
         int32_t *keys_in = reinterpret_cast<int32_t *>(ws + w.keys_in);
         int32_t *keys_out = reinterpret_cast<int32_t *>(ws + w.keys_out);
         int32_t *positions = reinterpret_cast<int32_t *>(ws + w.positions);
-        hipLaunchKernelGGL(sort_input_kernel, dim3(grid_for(num_edges)), dim3(256), 0, stream, key, num_edges,
-                           num_nodes, keys_in, positions);
-        rc = check_hip(hipGetLastError(), "prepare_rows keys");
-        if (rc) return rc;
         int bits = 1;  // the keys reach num_nodes
         while (bits < 32 && ((int64_t)1 << bits) <= (int64_t)num_nodes) bits++;
-        size_t temp_bytes = w.sort_bytes;
-        rc = check_hip(hipcub::DeviceRadixSort::SortPairs(
-                           ws + w.sort_temp, temp_bytes, reinterpret_cast<const uint32_t *>(keys_in),
-                           reinterpret_cast<uint32_t *>(keys_out), positions, perm, (int)num_edges, 0, bits, stream),
-                       "prepare_rows sort");
+        if (PrepareWorkspace::own_sort(num_nodes, num_edges)) {
+            int32_t *digits = reinterpret_cast<int32_t *>(ws + w.sort_temp);
+            const dim3 chunks((unsigned)((num_edges + kSortChunk - 1) / kSortChunk)), threads(kBlockThreads);
+            const int low = (bits + 1) / 2, high = bits - low > 0 ? bits - low : 1;
+            const int32_t *here = nullptr;
+            hipLaunchKernelGGL(edge_digits_kernel, chunks, threads, 0, stream, key, num_edges, num_nodes, true, 0,
+                               (1u << low) - 1, digits);
+            hipLaunchKernelGGL(edge_scatter_kernel, chunks, threads, 0, stream, key, here, num_edges, num_nodes, true, 0,
+                               low, digits, keys_in, positions);
+            hipLaunchKernelGGL(edge_digits_kernel, chunks, threads, 0, stream, keys_in, num_edges, num_nodes, false, low,
+                               (1u << high) - 1, digits);
+            hipLaunchKernelGGL(edge_scatter_kernel, chunks, threads, 0, stream, keys_in, positions, num_edges, num_nodes,
+                               false, low, high, digits, keys_out, perm);
+            rc = check_hip(hipGetLastError(), "prepare_rows sort");
+        } else {
+            hipLaunchKernelGGL(sort_input_kernel, dim3(grid_for(num_edges)), dim3(256), 0, stream, key, num_edges,
+                               num_nodes, keys_in, positions);
+            rc = check_hip(hipGetLastError(), "prepare_rows keys");
+            if (rc) return rc;
+            size_t temp_bytes = w.sort_bytes;
+            rc = check_hip(hipcub::DeviceRadixSort::SortPairs(
+                               ws + w.sort_temp, temp_bytes, reinterpret_cast<const uint32_t *>(keys_in),
+                               reinterpret_cast<uint32_t *>(keys_out), positions, perm, (int)num_edges, 0, bits, stream),
+                           "prepare_rows sort");
+        }
         if (rc) return rc;
         hipLaunchKernelGGL(rows_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, keys_out, other, perm, num_edges,
                            num_nodes, other_out, row_ptr, static_cast<int32_t *>(nullptr), segments);

@@ -139,3 +139,23 @@ def test_schedule_work_and_lists(n, tile_rows):
         np.testing.assert_array_equal(edge[pos], pos[by])
         row = np.searchsorted(ptr, pos[by], side="right") - 1
         np.testing.assert_array_equal(local[pos], row - t * tile_rows)
+
+
+@pytest.mark.parametrize("n,e,kind", [
+    (1, 5, "even"), (2, 4095, "hub"), (3, 4096, "even"), (255, 4097, "even"), (256, 8192, "hub"), (8191, 12289, "hub"),
+    (65535, 70001, "even"), (65536, 70001, "even"), (4999, 262144, "hub"), (4999, 262145, "even"), (40000, 262143, "even"),
+])
+def test_edge_sort_against_numpy(n, e, kind):
+    """Unsorted edges at the sizes where the sort changes: digits of the keys, chunks of 4 096 edges, 64 of
+    them, 2^16 nodes; ids of another shard and keys that are sorted already among them."""
+    key, other = _graph(n, e, kind, n + e)
+    shuffle = np.random.default_rng(e).permutation(e)
+    dev = lambda a: torch.from_numpy(a.astype(np.int32)).cuda()  # noqa: E731
+    for k, o in ((key[shuffle], other[shuffle]), (key, other)):
+        shifted = np.where(k == DUMMY, k, k - 2 * n)
+        ptr, oth, perm, order, _ = prepare_rows(dev(shifted), dev(o), n, False, 0, None)
+        want = np.argsort(k, kind="stable")
+        np.testing.assert_array_equal(perm.cpu().numpy(), want)
+        np.testing.assert_array_equal(ptr.cpu().numpy(), _rows(k, n))
+        np.testing.assert_array_equal(oth.cpu().numpy(), o[want])
+        assert order is None
