@@ -142,6 +142,8 @@ SYMBOLS = {
     "e3j_amd_tile_schedule_build": (ctypes.c_int, [_P] * 4 + [ctypes.c_int32, ctypes.c_int64, ctypes.c_int32,
                                                               ctypes.c_int32] + [_P] * 6),
     "e3j_amd_convolution_bwd_tiled": (ctypes.c_int, [_PARAMS] + [_P] * 7 + [ctypes.POINTER(TileSchedule)] + [_P] * 4),
+    "e3j_amd_convolution_bwd_tiled_edges": (ctypes.c_int,
+                                            [_PARAMS] + [_P] * 7 + [ctypes.POINTER(TileSchedule)] + [_P] * 3),
     "e3j_amd_convolution_bwd_tiled_f64": (ctypes.c_int, [_PARAMS] + [_P] * 7 + [ctypes.POINTER(TileSchedule)] + [_P] * 4),
     "e3j_amd_tile_rows_second": (ctypes.c_int32, [ctypes.c_int32]),
     "e3j_amd_tile_rows_f64": (ctypes.c_int32, [ctypes.c_int32]),

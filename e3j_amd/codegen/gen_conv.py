@@ -301,6 +301,7 @@ def emit_edge_bwd(p: Part, f64: bool = False) -> list[str]:
     """
     t = p.t
     V, R = ("Vec<1, double>", "double") if f64 else ("Vec<C>", "float")
+    only = "" if f64 else "if (kDx) "
     if f64:
         lines = ["    // the float64 form of edge_bwd: one double per lane, coefficients from `cf`",
                  "    template <bool kAcc = false, bool kPin = false, typename Dm, typename DsSink>",
@@ -313,7 +314,8 @@ def emit_edge_bwd(p: Part, f64: bool = False) -> list[str]:
                  "    // `dm`: anything indexable by the part's local output row (registers or LDS).",
                  "    // kAcc: dx holds running sums the edge's contributions are added to (else it is overwritten).",
                  "    // kPin: each row's dx sums are computed where the row is (see `pin`); for dm rows read from LDS.",
-                 "    template <int C, bool kAcc = false, bool kPin = false, typename Dm, typename DsSink>",
+                 "    // kDx: off, dx is left alone (and the row's sums towards dy and ds are what is pinned).",
+                 "    template <int C, bool kAcc = false, bool kPin = false, bool kDx = true, typename Dm, typename DsSink>",
                  "    __device__ static __forceinline__ void edge_bwd(const Vec<C> *x, const float *y,",
                  "                                                     const Vec<C> *s, const Dm &dm,",
                  "                                                     Vec<C> *dx, float *dy, const DsSink &ds) {"]
@@ -338,9 +340,9 @@ def emit_edge_bwd(p: Part, f64: bool = False) -> list[str]:
                     lines.append(f"                const {R} w{j} = {expr};")
                     expr = f"w{j}"
                 if j in dx_init:
-                    lines.append(f"                dx[{xj}] = vfma(g, {expr}, dx[{xj}]);")
+                    lines.append(f"                {only}dx[{xj}] = vfma(g, {expr}, dx[{xj}]);")
                 else:
-                    lines.append(f"                dx[{xj}] = kAcc ? vfma(g, {expr}, dx[{xj}]) : vmul(g, {expr});")
+                    lines.append(f"                {only}dx[{xj}] = kAcc ? vfma(g, {expr}, dx[{xj}]) : vmul(g, {expr});")
                     dx_init.add(j)
                 lines.append(f"                {{ const {V} pr = vmulv(dmi, x[{xj}]);")
                 for c, k in terms:
@@ -351,7 +353,10 @@ def emit_edge_bwd(p: Part, f64: bool = False) -> list[str]:
                         a_init.add(k)
                 lines.append("                }")
             lines.append("            }")
-            lines.append("            if (kPin) { " + " ".join(f"pin(dx[{p.xj[j]}]);" for j in cols) + " }")
+            lines.append(f"            if (kPin{'' if f64 else ' && kDx'}) {{ " + " ".join(f"pin(dx[{p.xj[j]}]);" for j in cols) + " }")
+            if not f64:
+                touched = sorted({k for terms in cols.values() for _, k in terms})
+                lines.append("            if (kPin && !kDx) { " + " ".join(f"pin(a{k});" for k in touched) + " }")
         first = True
         for k in ks:
             if first:
@@ -652,8 +657,9 @@ def emit_table_source(t: "Table", name: str, desc: str, channels: int, symbols, 
                  "    int, int, int, float, unsigned);"]
     for v in tile:
         cpl, wpb, zs, minw = (*v, 1)[:4]
-        out += [f"template __global__ void unrolled_bwd_tile_kernel<{channels}, {cpl}, {wpb}, {minw}, "
-                f"{part_names[zs]}>("] + tile_args
+        for with_dx in ("true", "false"):
+            out += [f"template __global__ void unrolled_bwd_tile_kernel<{channels}, {cpl}, {wpb}, {minw}, {with_dx}, "
+                    f"{part_names[zs]}>("] + tile_args
     second_args = ["    const float *, const float *, const float *, const float *, const float *, const float *,"]
     if tile:
         cpl, wpb, zs, minw = second_dm

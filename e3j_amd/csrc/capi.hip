@@ -553,12 +553,13 @@ int32_t e3j_amd_tile_rows_second(int32_t sig) {
 namespace {
 int run_tiled(const e3j_amd_conv_params *p, const void *x, const void *y, const void *s, const void *dm,
               const int32_t *sender, const int32_t *receiver_ptr, const int32_t *edge_perm,
-              const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds, hipStream_t stream, bool f64) {
-    const char *op = f64 ? "convolution_bwd_tiled_f64" : "convolution_bwd_tiled";
+              const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds, hipStream_t stream, bool f64,
+              bool edges_only = false) {
+    const char *op = f64 ? "convolution_bwd_tiled_f64" : edges_only ? "convolution_bwd_tiled_edges" : "convolution_bwd_tiled";
     int rc = validate(p, op);
     if (rc) return rc;
     if (p->num_nodes == 0 && p->num_edges == 0) return E3J_AMD_OK;
-    if (missing(x, p->num_nodes) || missing(dm, p->num_nodes) || missing(dx, p->num_nodes) ||
+    if (missing(x, p->num_nodes) || missing(dm, p->num_nodes) || (!edges_only && missing(dx, p->num_nodes)) ||
         receiver_ptr == nullptr || missing(sender, p->num_edges) || missing(y, p->num_edges) ||
         missing(s, p->num_edges) || missing(dy, p->num_edges) || missing(ds, p->num_edges) ||
         schedule == nullptr)
@@ -602,6 +603,14 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
                                   void *stream) {
     return run_tiled(p, x, y, s, dm, sender, receiver_ptr, edge_perm, schedule, dx, dy, ds,
                      static_cast<hipStream_t>(stream), false);
+}
+
+int e3j_amd_convolution_bwd_tiled_edges(const e3j_amd_conv_params *p, const void *x, const void *y,
+                                        const void *s, const void *dm, const int32_t *sender,
+                                        const int32_t *receiver_ptr, const int32_t *edge_perm,
+                                        const e3j_amd_tile_schedule *schedule, void *dy, void *ds, void *stream) {
+    return run_tiled(p, x, y, s, dm, sender, receiver_ptr, edge_perm, schedule, nullptr, dy, ds,
+                     static_cast<hipStream_t>(stream), false, true);
 }
 
 int e3j_amd_convolution_bwd_tiled_f64(const e3j_amd_conv_params *p, const void *x, const void *y,

@@ -449,7 +449,7 @@ int zero_padding(const e3j_amd_conv_params &p, const int32_t *other, const int32
 template <typename Val>
 int bwd_targets(const e3j_amd_conv_params &p, const int32_t *other, const int32_t *row_ptr, const int32_t *perm,
                 Val *dx, Val *dy, Val *ds, bool shared_dy, hipStream_t stream) {
-    const ZeroRun dx_run(dx, sizeof(Val) * (size_t)p.num_nodes * p.num_x * p.channels);
+    const ZeroRun dx_run(dx, dx != nullptr ? sizeof(Val) * (size_t)p.num_nodes * p.num_x * p.channels : 0);
     const ZeroRun dy_run(dy, shared_dy ? sizeof(Val) * (size_t)p.num_edges * p.num_y : 0);
     const int64_t items = std::max<int64_t>({(int64_t)dx_run.pieces, (int64_t)dy_run.pieces, p.num_edges, 1});
     hipLaunchKernelGGL(bwd_targets_kernel<Val>, dim3((unsigned)std::min<int64_t>((items + 255) / 256, 4096)),

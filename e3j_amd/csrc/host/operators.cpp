@@ -45,6 +45,7 @@ struct Library {
     decltype(&e3j_amd_convolution_fwd_whole) fwd_whole = nullptr;
     decltype(&e3j_amd_convolution_bwd_receiver) bwd_receiver = nullptr;
     decltype(&e3j_amd_convolution_bwd_tiled) bwd_tiled = nullptr;
+    decltype(&e3j_amd_convolution_bwd_tiled_edges) bwd_tiled_edges = nullptr;
     decltype(&e3j_amd_convolution_bwd_tiled_f64) bwd_tiled_f64 = nullptr;
     decltype(&e3j_amd_tile_schedule_num_work) tile_schedule_num_work = nullptr;
     decltype(&e3j_amd_tile_schedule_workspace_bytes) tile_schedule_workspace_bytes = nullptr;
@@ -289,15 +290,16 @@ py::object python_graph(Call &call) {  // with the interpreter's lock held
 
 // The Python operators' backward: for derivatives of derivatives, under transforms, and wherever something is unusual
 // or failed (the call is then made again there and raises what it raises).
-variable_list python_backward(Call &call, const at::Tensor &x, const at::Tensor &y, const at::Tensor &s, const at::Tensor &dm) {
+variable_list python_backward(Call &call, const at::Tensor &x, const at::Tensor &y, const at::Tensor &s, const at::Tensor &dm,
+                              bool need_dx) {
     if (!call.handle) {
         std::lock_guard<std::mutex> guard(call.graph->lock);
         call.graph->wait_on(current_stream(call.plan->device));
     }
     py::gil_scoped_acquire gil;
     try {
-        const py::tuple r = call.plan->fallback.get()(x, y, s, dm, call.sender, call.receiver, python_graph(call));
-        return {r[0].cast<at::Tensor>(), r[1].cast<at::Tensor>(), r[2].cast<at::Tensor>()};
+        const py::tuple r = call.plan->fallback.get()(x, y, s, dm, call.sender, call.receiver, python_graph(call), need_dx);
+        return {r[0].is_none() ? at::Tensor() : r[0].cast<at::Tensor>(), r[1].cast<at::Tensor>(), r[2].cast<at::Tensor>()};
     } catch (py::error_already_set &e) {
         e.restore();
         python_error error;
@@ -325,13 +327,14 @@ struct Convolution : torch::autograd::Function<Convolution> {
                                                              : std::vector<int64_t>{g.num_nodes, plan.params.channels, plan.params.num_out};
         at::Tensor dm = cotangents[0].defined() ? cotangents[0] : at::zeros(out_shape, on(plan.device, plan.type));
         variable_list grads;
-        if (c10::GradMode::is_enabled() || !plain_context() || !native(plan, g, *call, x, y, s, dm, out_shape, grads))
-            grads = python_backward(*call, x, y, s, dm);
+        if (c10::GradMode::is_enabled() || !plain_context() || !native(plan, g, *call, x, y, s, dm, out_shape, ctx->needs_input_grad(0), grads))
+            grads = python_backward(*call, x, y, s, dm, ctx->needs_input_grad(0));
         return {grads[0], grads[1], grads[2], at::Tensor()};
     }
 
     static bool native(const Plan &plan, Adjacency &g, const Call &call, const at::Tensor &x, const at::Tensor &y,
-                       const at::Tensor &s, const at::Tensor &dm_in, const std::vector<int64_t> &out_shape, variable_list &grads) {
+                       const at::Tensor &s, const at::Tensor &dm_in, const std::vector<int64_t> &out_shape, bool need_dx,
+                       variable_list &grads) {
         // (saved tensors may come back changed from hooks)
         if (!plan.operands(x, y, s) || x.size(0) != g.num_nodes || y.size(0) != g.num_edges || dm_in.sizes() != out_shape) return false;
         const at::Tensor dm = dm_in.contiguous();
@@ -351,10 +354,16 @@ struct Convolution : torch::autograd::Function<Convolution> {
                 schedule = g.schedule;
             }
         }
-        const at::Tensor dx = at::empty(x.sizes(), x.options()), dy = at::empty(y.sizes(), y.options()), ds = at::empty(s.sizes(), s.options());
+        // dx is left out where nobody asks for it (unrolled_bwd_tile_part has the figures)
+        const bool edges_only = tiles && plan.type == at::kFloat && !need_dx;
+        const at::Tensor dx = edges_only ? at::Tensor() : at::empty(x.sizes(), x.options());
+        const at::Tensor dy = at::empty(y.sizes(), y.options()), ds = at::empty(s.sizes(), s.options());
         const e3j_amd_conv_params p = plan.with(g);
         int rc;
-        if (tiles) {
+        if (edges_only) {
+            rc = lib.bwd_tiled_edges(&p, x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), g.other, g.row_ptr, g.perm,
+                                     &schedule, dy.data_ptr(), ds.data_ptr(), raw_stream(plan.device));
+        } else if (tiles) {
             const auto run = plan.type == at::kDouble ? lib.bwd_tiled_f64 : lib.bwd_tiled;
             rc = run(&p, x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), g.other, g.row_ptr, g.perm, &schedule,
                      dx.data_ptr(), dy.data_ptr(), ds.data_ptr(), raw_stream(plan.device));
@@ -469,6 +478,7 @@ PYBIND11_MODULE(_operators, m) {
         take(d, "e3j_amd_convolution_fwd_whole", lib.fwd_whole);
         take(d, "e3j_amd_convolution_bwd_receiver", lib.bwd_receiver);
         take(d, "e3j_amd_convolution_bwd_tiled", lib.bwd_tiled);
+        take(d, "e3j_amd_convolution_bwd_tiled_edges", lib.bwd_tiled_edges);
         take(d, "e3j_amd_convolution_bwd_tiled_f64", lib.bwd_tiled_f64);
         take(d, "e3j_amd_tile_schedule_num_work", lib.tile_schedule_num_work);
         take(d, "e3j_amd_tile_schedule_workspace_bytes", lib.tile_schedule_workspace_bytes);

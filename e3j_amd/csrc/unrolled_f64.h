@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kWave *WPB, MINW) void unrolled_bwd_tile_f64_kernel
     double *__restrict__ dx, double *__restrict__ dy, double *__restrict__ ds, int num_nodes, int tile_rows,
     int num_work, unsigned y_flip, F64Coefs coefs) {
     extern __shared__ __attribute__((aligned(16))) double tile_lds_f64[];
-    unrolled_bwd_tile_block<K, 1, Parts...>(x, y, s, dm, work, t_sender, t_edge, t_local, row_order, dx, dy, ds,
+    unrolled_bwd_tile_block<K, 1, true, Parts...>(x, y, s, dm, work, t_sender, t_edge, t_local, row_order, dx, dy, ds,
                                             num_nodes, tile_rows, num_work, 1.0, y_flip, tile_lds_f64, coefs.v);
 }
 

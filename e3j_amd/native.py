@@ -23,7 +23,8 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_ope
 
 _BOUND = ("e3j_amd_prepare_rows", "e3j_amd_prepare_rows_workspace_bytes", "e3j_amd_row_segments_max",
           "e3j_amd_row_partials_bytes", "e3j_amd_convolution_fwd", "e3j_amd_convolution_fwd_whole",
-          "e3j_amd_convolution_bwd_receiver", "e3j_amd_convolution_bwd_tiled", "e3j_amd_convolution_bwd_tiled_f64",
+          "e3j_amd_convolution_bwd_receiver", "e3j_amd_convolution_bwd_tiled",
+          "e3j_amd_convolution_bwd_tiled_edges", "e3j_amd_convolution_bwd_tiled_f64",
           "e3j_amd_tile_schedule_num_work", "e3j_amd_tile_schedule_workspace_bytes", "e3j_amd_tile_schedule_build")
 _module = None
 
@@ -78,9 +79,9 @@ def _plan(module, x: torch.Tensor, cfg: Config):
         tile_rows = ops._tile_rows(sig, f64=True)
         values, values_kept = (ops.tile_values_f64(dims[0], dims[3], kept) or _NEVER for kept in (False, True))
 
-    def fallback(x, y, s, dm, sender, receiver, graph):
+    def fallback(x, y, s, dm, sender, receiver, graph, need_dx):
         meta = ops._make_meta(coef, x, y, s, params, ordering, None, layout)
-        return ops._apply_bwd(x, y, s, dm, sender, receiver, meta, graph)
+        return ops._backward(x, y, s, dm, sender, receiver, meta, graph, need_dx)
 
     def make_graph(other, row_ptr, perm, order, num_nodes, segments, row_cap, row_piece):
         graph = ops.PreparedGraph(other, row_ptr, perm, order, num_nodes, ordering)

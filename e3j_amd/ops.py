@@ -541,11 +541,12 @@ def _raw_forward(meta: _Meta, x, y, s, sender, receiver, graph=None) -> torch.Te
     return out
 
 
-def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
-    """`graph`: the forward's `(other, row_ptr, perm, row_order)` when it can be reused."""
+def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None, need_dx=True):
+    """`graph`: the forward's `(other, row_ptr, perm, row_order)` when it can be reused.  Without `need_dx` the
+    kernels that have a form without dx return None for it."""
     x, y, s, dm = x.contiguous(), y.contiguous(), s.contiguous(), dm.contiguous()
     n = meta.num_nodes
-    dx, dy, ds = torch.empty_like(x), torch.empty_like(y), torch.empty_like(s)
+    dx, dy, ds = torch.empty_like(x) if need_dx else None, torch.empty_like(y), torch.empty_like(s)
     lib = _lib.load()
     table = meta.table
     has_kernel = table.signature(*_shape(meta, x, y, s), meta.layout)[0] >= 0
@@ -568,7 +569,7 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
     channels = _shape(meta, x, y, s)[1]
     sender_kernel = (deterministic and has_kernel and meta.layout == Layout.TRAILING_CHANNELS and channels <= 128
                      and x.dtype == torch.float32
-                     and all(t.data_ptr() % 16 == 0 for t in (x, y, s, dm, dx, dy, ds)))
+                     and all(t.data_ptr() % 16 == 0 for t in (x, y, s, dm, dy, ds)))
     sender_rows = meta.ordering == GraphOrdering.SENDER and (not has_kernel or sender_kernel)
     resort = meta.ordering in (GraphOrdering.NONE, GraphOrdering.SENDER) and not sender_rows
     ordered = deterministic and has_kernel and not sender_kernel
@@ -605,30 +606,30 @@ def _raw_backward(meta: _Meta, x, y, s, dm, sender, receiver, graph=None):
             group_receiver, other, row_ptr, perm = True, sender_l.contiguous(), csr_row_ptr(receiver_l, n), None
         order = (graph[3] if graph is not None and forward_rows else _row_order(other, row_ptr, n))
     p, table = _fill_params(meta, x, y, s, table, use_signature=group_receiver or sender_kernel, row_order=order)
-    args = (ctypes.byref(p), table.device(x.device).data_ptr(), x.data_ptr(), y.data_ptr(),
-            s.data_ptr(), dm.data_ptr(), other.data_ptr(), row_ptr.data_ptr(),
-            perm.data_ptr() if perm is not None else None,
-            dx.data_ptr(), dy.data_ptr(), ds.data_ptr())
     # tiles of receivers whose dm rows fit the LDS of a workgroup: dx summed per (tile, sender)
     tile_rows = 0
-    aligned = all(t.data_ptr() % 16 == 0 for t in (x, y, s, dm, dx, dy, ds))  # what the unrolled kernels take
+    aligned = all(t.data_ptr() % 16 == 0 for t in (x, y, s, dm, dy, ds))  # what the unrolled kernels take
     if (group_receiver and not ordered and y.shape[0] > 0 and p.layout == _lib.LAYOUT_TRAILING and aligned
             and x.dtype == torch.float32):
         tile_rows = _tile_rows(p.signature)
     if (group_receiver and x.dtype == torch.float64
             and _tiles_pay_f64(p.num_edges, p.num_x, p.num_scalars, p.channels, prepared is not None and prepared.kept)):
         tile_rows = _tile_rows(p.signature, f64=True)
+    if dx is None and (tile_rows < 1 or x.dtype != torch.float32):
+        dx = torch.empty_like(x)
+    operands = (x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), other.data_ptr(), row_ptr.data_ptr(),
+                perm.data_ptr() if perm is not None else None)
+    results = (*([] if dx is None else [dx.data_ptr()]), dy.data_ptr(), ds.data_ptr())
+    args = (ctypes.byref(p), table.device(x.device).data_ptr(), *operands, *results)
     with on_device(x.device):
         plan = _table_plan(p, table, x.device)  # noqa: F841 (kept alive until the call is enqueued)
         if tile_rows >= 1:
             if prepared is None:
                 prepared = PreparedGraph(other, row_ptr, perm, order, n)
             schedule = prepared.schedule(tile_rows)
-            fn = lib.e3j_amd_convolution_bwd_tiled_f64 if x.dtype == torch.float64 else lib.e3j_amd_convolution_bwd_tiled
-            _lib.check(fn(
-                ctypes.byref(p), x.data_ptr(), y.data_ptr(), s.data_ptr(), dm.data_ptr(), other.data_ptr(),
-                row_ptr.data_ptr(), perm.data_ptr() if perm is not None else None,
-                ctypes.byref(schedule.struct), dx.data_ptr(), dy.data_ptr(), ds.data_ptr(), _stream(x.device)))
+            fn = (lib.e3j_amd_convolution_bwd_tiled_edges if dx is None else
+                  lib.e3j_amd_convolution_bwd_tiled_f64 if x.dtype == torch.float64 else lib.e3j_amd_convolution_bwd_tiled)
+            _lib.check(fn(ctypes.byref(p), *operands, ctypes.byref(schedule.struct), *results, _stream(x.device)))
         elif ordered:
             nbytes = int(lib.e3j_amd_convolution_bwd_ordered_workspace_bytes(ctypes.byref(p)))
             workspace = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
@@ -790,7 +791,7 @@ class _Convolution(torch.autograd.Function):
     def backward(ctx, dm):
         x, y, s = ctx.saved_tensors
         sender, receiver = ctx.index
-        dx, dy, ds = _apply_bwd(x, y, s, dm, sender, receiver, ctx.meta, ctx.graph)
+        dx, dy, ds = _backward(x, y, s, dm, sender, receiver, ctx.meta, ctx.graph, ctx.needs_input_grad[0])
         return dx, dy, ds, None, None, None, None
 
     @staticmethod
@@ -893,6 +894,15 @@ def _apply_fwd(*args):
 
 def _apply_bwd(*args):
     return (_ConvolutionBwd if _under_transform() else _PlainConvolutionBwd).apply(*args)
+
+
+def _backward(x, y, s, dm, sender, receiver, meta, graph, need_dx):
+    """`(dx, dy, ds)` of a backward pass; dx may be None where nobody asks for it and nothing is recorded."""
+    if need_dx or torch.is_grad_enabled() or _under_transform():
+        return _apply_bwd(x, y, s, dm, sender, receiver, meta, graph)
+    if graph is None:
+        graph = _forward_graph(meta, sender, receiver, build=False)
+    return _raw_backward(meta, x, y, s, dm, sender, receiver, graph, need_dx=False)
 
 
 def _make_meta(coef, x, y, s, params, graph_ordering, y_parity, layout) -> _Meta:

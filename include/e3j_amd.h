@@ -254,6 +254,12 @@ int e3j_amd_convolution_bwd_tiled(const e3j_amd_conv_params *p, const void *x, c
                                   const int32_t *receiver_ptr, const int32_t *edge_perm,
                                   const e3j_amd_tile_schedule *schedule, void *dx, void *dy, void *ds,
                                   void *stream);
+/* The same without dx, for an x that needs no gradient (the first layer of a model): the same dy and ds,
+ * the same limits; dx's sums, its clearing and its atomics are left out. */
+int e3j_amd_convolution_bwd_tiled_edges(const e3j_amd_conv_params *p, const void *x, const void *y,
+                                        const void *s, const void *dm, const int32_t *sender,
+                                        const int32_t *receiver_ptr, const int32_t *edge_perm,
+                                        const e3j_amd_tile_schedule *schedule, void *dy, void *ds, void *stream);
 /* The same for float64 operands (p->val_dtype E3J_AMD_F64 with a signature and coef_classes; any
  * alignment of doubles); `tile_rows` of its schedule: at most e3j_amd_tile_rows_f64(signature), 0 where
  * the signature has no such kernel (E3J_AMD_UNIMPLEMENTED). */
