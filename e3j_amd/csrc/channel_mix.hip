@@ -11,6 +11,9 @@
 // The backward pass uses the same kernel in the other direction, so the cotangent rows are
 // written once (no zero fill, no additions of per-degree slices).
 #include "common.h"
+#include "split_half.h"
+
+#include <type_traits>
 
 namespace e3j_amd {
 namespace {
@@ -58,46 +61,87 @@ int launch(const void *src, void *dst, int64_t num_nodes, int32_t rows, int32_t 
 // ---------------------------------------------------------------------------
 // The mixing itself in one launch (float32, 64 or 128 channels): no regrouped copies, no library
 // calls.  A wave takes 32 nodes and one output row (degree l, component m) and runs
-// v_mfma_f32_32x32x2_f32 with the nodes as rows: lane t holds, for node t % 32, the 32 consecutive
-// channels 32 (t / 32) .. + 31 of a source row (the row of a node is read by sixteen lanes side by
-// side and turned through LDS; with a lane reading its own 128 bytes every access touched 64 lines,
-// which the first-level cache does not hold until the next one), and step s of the product takes
-// channel 32 (t / 32) + s from every lane, which is the layout of the instruction's first operand when
-// its two summed indices are read as "channel s of the lower / of the upper half"; the second operand is
-// the matching row of the weight, 32 consecutive output channels per half wave.  The waves of a block
-// work on one output row and share its weights through LDS, 64 summed channels at a time (with every
-// wave reading them from the caches a chunk's 64 loads and its products took turns).
-// 6 000 nodes, 64 channels, 99 rows to 16: 85 -> 60 us each way; the products alone take 32 us at the
-// float32 rate of the matrix cores, the stream 35 us.  At 128 channels a block takes 68 KB of LDS (two blocks a
-// compute unit) and up to 240 registers: 6 000 nodes 287 -> 227 us forward and 282 -> 237 backward, 20 000 nodes
-// 846 -> 568 and 935 -> 587, 200 nodes 122 -> 72 and 120 -> 71; the products alone take 128 us at 6 000.  Forward: the products of the mul copies of the
-// degree accumulate into one output row.  Backward (weights transposed by the caller): the cotangent row
-// is read once and gives one product per copy.
+// v_mfma_f32_32x32x16_f16 with the nodes as rows on operands split two ways (see split_half.h): lane t holds, for
+// node t % 32, the 32 consecutive channels 32 (t / 32) .. + 31 of a source row (the row of a node is read by
+// sixteen lanes side by side and turned through LDS; with a lane reading its own 128 bytes every access touched 64
+// lines, which the first-level cache does not hold until the next one), and step s of the product takes
+// channels 32 (t / 32) + 8 s .. + 7 from every lane; the second operand is the matching piece of a weight column.
+// The waves of a block work on one output row and share its weights through LDS, 64 summed channels (a chunk) at a
+// time, each wave splitting a fourth of the columns.  A scale belongs to the row of a node or to a column of the
+// weights within a chunk; the sums of a chunk are scaled back and added in float32.  A chunk with an infinity, a NaN or
+// values near the ends of the range (found by the exponent of its scale) runs on v_mfma_f32_32x32x2_f32 from memory.
+// Forward: the products of the mul copies of the degree accumulate into one output row.  Backward (weights
+// transposed by the caller): the cotangent row is read once and gives one product per copy.
+// At 128 channels a block of the backward makes 64 output channels: the operand of both chunks of a row stays in
+// registers (with the sums of 128 channels beside it they spilled, and a spill waits for every load in flight: 168 us
+// for 114 below), and the cotangent rows that are read twice are few.  A forward block makes all: with 64 the source
+// rows are read and split twice (130 -> 165 us, though 200 nodes 52 -> 42).
+// Bound by the stream and, in a block's chain of chunks, by latency: 99 rows to 16, 6 000 nodes, 64 channels: 57 -> 47 us
+// forward and 63 -> 39 backward where float32 products took 32 and the stream takes 35; 128 channels 222 -> 130 and
+// 231 -> 114 (stream 70), 20 000 nodes 577 -> 376 and 584 -> 364, 200 nodes 66 -> 52 and 68 -> 27 (64 channels
+// there: 21 -> 22 and 22 -> 15).  Error against float64 over normal values, rms: 0.35 to 0.8 times that of float32
+// products (fewer additions).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMixDegrees = 8;
 constexpr int kMixWaves = 4;  // waves per block, 32 nodes each, on one output row
+constexpr int kMixExponents = 90;  // a scale outside 2^-90 .. 2^90 (no number, or next to the ends of the range) is not used
 struct MixShape {
     int32_t degrees;
     int32_t mul[kMixDegrees], dim[kMixDegrees];
 };
 
+// the exponent of the scale of terms with largest value m, 0 without terms
+__device__ __forceinline__ int mix_exponent(float m) { return m == 0.f ? 0 : scale_exponent(m); }
+__device__ __forceinline__ bool odd_exponent(int k) { return k < -kMixExponents || k > kMixExponents; }
+
+// the largest of the values of the lanes t, t + EVERY, t + 2 EVERY .. (modulo the wave) in each of them
+template <int EVERY>
+__device__ __forceinline__ float largest_over(float m) {
+    auto rotated = [](float v, auto control) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(control)::value, 0xf, 0xf, false));
+    };
+    if (EVERY <= 4) m = fmaxf(m, rotated(m, std::integral_constant<int, 0x124>{}));  // by 4, by 8 of sixteen lanes
+    if (EVERY <= 8) m = fmaxf(m, rotated(m, std::integral_constant<int, 0x128>{}));
+    if (EVERY <= 16) {
+        const auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+        m = fmaxf(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
+    }
+    const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    return fmaxf(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
+}
+
 template <int K, bool kTranspose>
-__global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restrict__ src, float *__restrict__ dst,
-                                                          const float *__restrict__ w, int64_t num_nodes,
-                                                          MixShape shape, int32_t rows_plain, int32_t rows_mixed) {
-    constexpr int KC = K / 64, KT = K / 32;   // chunks of 64 summed channels, tiles of 32 output channels
-    const int lane = threadIdx.x, r = lane & 31, h = lane >> 5;
-    constexpr int THREADS = kWave * kMixWaves, PIECES = 64 * K / 4 / THREADS;
-    constexpr int HALF = 32 * K + 32;  // (the halves of a wave read rows 32 apart: the pad puts them on other banks)
+__global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
+    const float *__restrict__ src, float *__restrict__ dst, const float *__restrict__ w, int64_t num_nodes,
+    MixShape shape, int32_t rows_plain, int32_t rows_mixed) {
+    // chunks of 64 summed channels, output channels of a block, tiles of 32 of them
+    constexpr int KC = K / 64, KO = kTranspose ? 64 : K, KT = KO / 32;
+    const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y), r = lane & 31, h = lane >> 5;
+    constexpr int ROWS = KO / 16;              // weights: a thread stages ROWS rows of four columns,
+    constexpr int GROUPS = KO / kMixWaves / 4;  //   GROUPS lanes side by side the columns of their wave
+    constexpr bool kTight = K == 64 && !kTranspose;  // (a spilled register waits for every load in flight)
+    constexpr int WEIGHT_PITCH = 64 + 8;       // halves a column (16-byte reads of 32 columns spread over the banks)
     constexpr int PITCH = 64 + 4;              // (16-byte reads of 64 rows side by side spread over the banks)
-    __shared__ __attribute__((aligned(16))) float weights[2 * HALF];
+    __shared__ __attribute__((aligned(16))) _Float16 weights[2][KO * WEIGHT_PITCH];
     __shared__ __attribute__((aligned(16))) float rows[kMixWaves][32 * PITCH];
-    const int tid = threadIdx.y * kWave + lane;
+    __shared__ __attribute__((aligned(16))) float row_scale[kMixWaves][KC][32];  // 2^-k of rows and columns
+    __shared__ float col_scale[KO];
+    __shared__ int odd_weights;                // set for good by a chunk with a scale that is not used
     // (the waves of a block take neighbouring tiles of one output row; tiles past the last one run along)
     const int64_t row_blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves);
-    const int64_t tile = (int64_t)blockIdx.x % row_blocks * kMixWaves + threadIdx.y;
-    const int xr = (int)(blockIdx.x / row_blocks);
+    const int64_t block = blockIdx.x / (K / KO);
+    const int64_t tile = block % row_blocks * kMixWaves + wave;
+    const int xr = (int)(block / row_blocks), out0 = blockIdx.x % (K / KO) * KO;
+    // first node of the tile and how many it has (none or fewer: tiles past the last one)
+    const int64_t node0 = tile * 32;
+    const int nodes = (int)(num_nodes - node0 < 0 ? 0 : num_nodes - node0 < 32 ? num_nodes - node0 : 32);
+    // `count` values of a row of each of the tile's nodes, as a buffer: loads past the last node are zeros, stores
+    // past it are dropped, an address is one register
+    auto tile_rows = [&](const float *first, uint32_t node_stride, int count) {
+        const uint32_t bytes = nodes > 0 ? ((uint32_t)(nodes - 1) * node_stride + count) * 4u : 0u;
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(first) + node0 * node_stride, 0, bytes, 0x00020000);
+    };
     // the degree and component of mixed row xr, the first plain row and the first weight of the degree
     int l = 0, zbase = 0, xbase = 0;
     int64_t wbase = 0;
@@ -110,77 +154,171 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
     const int m = xr - xbase, mul = shape.mul[l], dim = shape.dim[l];
     // 64 channels of a row of the wave's 32 nodes, from `first` (row of node 0) on: read in whole lines,
     // sixteen lanes a node, and turned through LDS into the operand a lane supplies
-    auto fetch_rows = [&](const float *first, int64_t node_stride, f32x4 (&piece)[8]) {
+    auto fetch_rows = [&](const float *first, uint32_t node_stride, f32x4 (&piece)[8]) {
+        const auto buffer = tile_rows(first, node_stride, 64);
+        uint32_t at = (lane / 16 * node_stride + lane % 16 * 4) * 4u;
+        asm volatile("" : "+v"(at));  // (the eight addresses are made where they are used, not kept)
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int64_t n = tile * 32 + 4 * i + lane / 16;  // (past the end: the last node)
-            piece[i] = *reinterpret_cast<const f32x4 *>(first + (n < num_nodes ? n : num_nodes - 1) * node_stride +
-                                                        lane % 16 * 4);
-        }
+        for (int i = 0; i < 8; i++)
+            piece[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                buffer, at + 16 * i * node_stride, 0, 0));
     };
-    auto turn_rows = [&](const f32x4 (&piece)[8], float (&a)[32]) {
-        float *mine = rows[threadIdx.y];
+    // returns whether a row has a scale that is not used
+    auto turn_rows = [&](const f32x4 (&piece)[8], Split2 (&a)[4], float (&scales)[32]) {
+        float *mine = rows[wave];
 #pragma unroll
         for (int i = 0; i < 8; i++)
             *reinterpret_cast<f32x4 *>(mine + (4 * i + lane / 16) * PITCH + lane % 16 * 4) = piece[i];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        float x[4][8];
+        float most = 0.f;
 #pragma unroll
-        for (int q = 0; q < 8; q++) {
-            const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + r * PITCH + 32 * h + 4 * q);
-            a[4 * q] = v.x; a[4 * q + 1] = v.y; a[4 * q + 2] = v.z; a[4 * q + 3] = v.w;
+        for (int q = 0; q < 4; q++) {
+#pragma unroll
+            for (int j = 0; j < 8; j += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + r * PITCH + 32 * h + 8 * q + j);
+                x[q][j] = v.x; x[q][j + 1] = v.y; x[q][j + 2] = v.z; x[q][j + 3] = v.w;
+            }
+            most = fmaxf(most, max_abs(x[q]));
         }
+        const int k = mix_exponent(largest_over<32>(most));
+#pragma unroll
+        for (int q = 0; q < 4; q++) a[q] = split2(x[q], pow2(k));
+        if (h == 0) scales[r] = pow2(-k);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        return __any(odd_exponent(k)) != 0;
     };
-    auto store_tile = [&](const f32x16 (&acc)[KT], float *row0, int64_t node_stride) {
+    auto store_tile = [&](const f32x16 (&acc)[KT], float *row0, uint32_t node_stride) {
+        const auto buffer = tile_rows(row0 + out0, node_stride, KO);
         // register v of lane t: node 8 (v / 4) + 4 (t / 32) + v % 4 of the tile, output channel t % 32 of tile ct
 #pragma unroll
-        for (int ct = 0; ct < KT; ct++) {
+        for (int v = 0; v < 16; v++) {
+            const uint32_t at = ((8 * (v / 4) + 4 * h + v % 4) * node_stride + r) * 4u;
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int64_t n = tile * 32 + 8 * (v / 4) + 4 * h + v % 4;
-                if (n < num_nodes) row0[n * node_stride + ct * 32 + r] = acc[ct][v];
-            }
+            for (int ct = 0; ct < KT; ct++)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[ct][v]), buffer, at + ct * 128, 0, 0);
         }
     };
     f32x16 acc[KT];
     const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // One chunk of 64 summed channels: its weight rows lie in LDS for the waves of the block, those of
     // the next chunk are on their way while the products of this one run.
-    const float *wl = w + wbase;
+    const float *wl = w + wbase + out0;
     const int chunks = mul * KC;
-    f32x4 staged[PIECES];
+    const int col0 = wave * (KO / kMixWaves) + lane % GROUPS * 4, k0 = lane / GROUPS * ROWS;
+    f32x4 staged[ROWS];
     auto fetch = [&](int q) {
+        const auto buffer = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(wl) + (int64_t)q * (64 * K), 0,
+                                                              (63 * K + KO) * 4, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < PIECES; i++)
-            staged[i] = *reinterpret_cast<const f32x4 *>(wl + (int64_t)q * (64 * K) + (i * THREADS + tid) * 4);
+        for (int i = 0; i < ROWS; i++)
+            staged[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                buffer, ((k0 + i) * K + col0) * 4, 0, 0));
     };
-    auto commit = [&]() {
+    typedef _Float16 Halves __attribute__((ext_vector_type(ROWS)));
+    struct Weights {
+        Halves term[2][4];
+        int exponent[4];
+    };
+    auto split_weights = [&]() {
+        Weights out;
 #pragma unroll
-        for (int i = 0; i < PIECES; i++) {
-            const int at = (i * THREADS + tid) * 4;
-            *reinterpret_cast<f32x4 *>(&weights[at + (at >= 32 * K ? 32 : 0)]) = staged[i];
+        for (int c = 0; c < 4; c++) {
+            float most = 0.f;
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) most = fmaxf(most, fabsf(staged[i][c]));
+            out.exponent[c] = mix_exponent(largest_over<GROUPS>(most));
+            const float scale = pow2(out.exponent[c]);
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) {  // see split2
+                out.term[0][c][i] = (_Float16)(staged[i][c] * scale);
+                out.term[1][c][i] = (_Float16)__builtin_fmaf(staged[i][c], scale, -(float)out.term[0][c][i]);
+            }
+        }
+        return out;
+    };
+    auto commit = [&](const Weights &split) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                *reinterpret_cast<Halves *>(&weights[u][(col0 + c) * WEIGHT_PITCH + k0]) = split.term[u][c];
+            if (lane / GROUPS == 0) col_scale[col0 + c] = pow2(-split.exponent[c]);
+            if (odd_exponent(split.exponent[c])) odd_weights = 1;
         }
     };
-    auto products = [&](const float (&a)[32]) {
-        const float *wk = &weights[h * HALF + r];
+    // `first`, node_stride: the source rows of the chunk, `q`: the chunk of weights
+    auto products = [&](const Split2 (&a)[4], const float (&scales)[32], bool odd, const float *first,
+                        uint32_t node_stride, int q) {
+        if (odd || odd_weights != 0) {
+            const auto buffer = tile_rows(first, node_stride, 64);
+            const float *wk = wl + ((int64_t)q * 64 + 32 * h) * K + r;
+#pragma unroll 1
+            for (int s = 0; s < 32; s++) {
+                const float x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    buffer, (r * node_stride + 32 * h + s) * 4u, 0, 0));
 #pragma unroll
-        for (int s = 0; s < 32; s++) {
+                for (int ct = 0; ct < KT; ct++)
+                    acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, wk[s * K + ct * 32], acc[ct], 0, 0, 0);
+            }
+            return;
+        }
+        constexpr int TILES = kTight ? 1 : 2;
 #pragma unroll
-            for (int ct = 0; ct < KT; ct++)
-                acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], wk[s * K + ct * 32], acc[ct], 0, 0, 0);
+        for (int c0 = 0; c0 < KT; c0 += TILES) {
+            f32x16 d[TILES];
+#pragma unroll
+            for (int i = 0; i < TILES; i++) d[i] = zero;
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                f16x8 b[TILES][2];
+#pragma unroll
+                for (int i = 0; i < TILES; i++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        b[i][u] = *reinterpret_cast<const f16x8 *>(
+                            &weights[u][((c0 + i) * 32 + r) * WEIGHT_PITCH + 32 * h + 8 * s]);
+#pragma unroll
+                for (int u = 0; u < 3; u++)
+#pragma unroll
+                    for (int i = 0; i < TILES; i++)
+                        d[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s].term[kPairs[u][0]], b[i][kPairs[u][1]], d[i], 0, 0, 0);
+                if (kTight || s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+            }
+            // (two operands of a tile of columns or four scales at a time in registers)
+            float col[TILES];
+#pragma unroll
+            for (int i = 0; i < TILES; i++) col[i] = col_scale[(c0 + i) * 32 + r];
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                if (v % 4 == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+#pragma unroll
+                for (int i = 0; i < TILES; i++)
+                    acc[c0 + i][v] = __builtin_fmaf(d[i][v] * scales[8 * (v / 4) + 4 * h + v % 4], col[i], acc[c0 + i][v]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     // after the products of a chunk: its weights make room for those of the next
     auto next_chunk = [&](int q) {
-        __syncthreads();
-        if (q < chunks) commit();
+        if (q < chunks) {
+            const Weights split = split_weights();
+            __builtin_amdgcn_sched_barrier(0);
+            __syncthreads();
+            commit(split);
+        }
         __syncthreads();
     };
+    if (lane + wave == 0) odd_weights = 0;
     fetch(0);
-    commit();
-    const int64_t plain_stride = (int64_t)rows_plain * K, mixed_stride = (int64_t)rows_mixed * K;
+    __syncthreads();
+    commit(split_weights());
+    const uint32_t plain_stride = (uint32_t)rows_plain * K, mixed_stride = (uint32_t)rows_mixed * K;
     f32x4 piece[8];
     if (!kTranspose) {
 #pragma unroll
@@ -190,22 +328,25 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
         fetch_rows(row_of(0), plain_stride, piece);
         __syncthreads();
         for (int q = 0; q < chunks; q++) {
-            float a[32];
-            turn_rows(piece, a);
+            Split2 a[4];
+            const bool odd = turn_rows(piece, a, row_scale[wave][0]);
+            __builtin_amdgcn_sched_barrier(0);
             if (q + 1 < chunks) {
                 fetch(q + 1);
                 fetch_rows(row_of(q + 1), plain_stride, piece);
             }
-            products(a);
+            products(a, row_scale[wave][0], odd, row_of(q), plain_stride, q);
             next_chunk(q + 1);
         }
         store_tile(acc, dst + (int64_t)xr * K, mixed_stride);
     } else {
-        float a[KC][32];
+        Split2 a[KC][4];
+        bool odd[KC];
 #pragma unroll
         for (int kc = 0; kc < KC; kc++) {
             fetch_rows(src + (int64_t)xr * K + kc * 64, mixed_stride, piece);
-            turn_rows(piece, a[kc]);
+            odd[kc] = turn_rows(piece, a[kc], row_scale[wave][kc]);
+            __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
         for (int u = 0; u < mul; u++) {
@@ -215,7 +356,7 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
             for (int kc = 0; kc < KC; kc++) {
                 const int q = u * KC + kc;
                 if (q + 1 < chunks) fetch(q + 1);
-                products(a[kc]);
+                products(a[kc], row_scale[wave][kc], odd[kc], src + (int64_t)xr * K + kc * 64, mixed_stride, q);
                 next_chunk(q + 1);
             }
             store_tile(acc, dst + (int64_t)(zbase + u * dim + m) * K, plain_stride);
@@ -226,7 +367,7 @@ __global__ __launch_bounds__(256) void channel_mix_kernel(const float *__restric
 template <int K>
 int launch_mix(const float *src, float *dst, const float *w, int64_t num_nodes, const MixShape &shape,
                int rows_plain, int rows_mixed, bool transpose, hipStream_t stream) {
-    const int64_t blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves) * rows_mixed;
+    const int64_t blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves) * rows_mixed * (transpose ? K / 64 : 1);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: too many nodes for one launch");
     if (transpose)
         hipLaunchKernelGGL((channel_mix_kernel<K, true>), dim3((unsigned)blocks), dim3(kWave, kMixWaves), 0, stream,
@@ -252,17 +393,21 @@ extern "C" int e3j_amd_channel_mix(const void *src, void *dst, const void *weigh
     MixShape shape;
     shape.degrees = num_degrees;
     int rows_plain = 0, rows_mixed = 0;
+    int64_t total_rows = 0;
     for (int l = 0; l < kMixDegrees; l++) {
         shape.mul[l] = l < num_degrees ? mul[l] : 0;
         shape.dim[l] = l < num_degrees ? dim[l] : 0;
         if (l < num_degrees && (mul[l] < 1 || dim[l] < 1))
             return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: multiplicities and dimensions must be >= 1");
         rows_plain += shape.mul[l] * shape.dim[l];
+        total_rows += (int64_t)shape.mul[l] * shape.dim[l];
         rows_mixed += shape.dim[l];
     }
     if (num_nodes == 0) return E3J_AMD_OK;
     if (src == nullptr || dst == nullptr || weights == nullptr)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: null operand");
+    if (total_rows * channels > (int64_t)1 << 25)  // (the rows of 32 nodes are addressed with 32 bits)
+        return set_error(E3J_AMD_UNIMPLEMENTED, "channel_mix: more than 2^25 values per node");
     if (reinterpret_cast<uintptr_t>(src) % 16 != 0 || reinterpret_cast<uintptr_t>(dst) % 16 != 0 ||
         reinterpret_cast<uintptr_t>(weights) % 16 != 0)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: operands must be 16-byte aligned");

@@ -15,6 +15,7 @@
 #include <initializer_list>
 
 #include "common.h"
+#include "split_half.h"
 
 namespace e3j_amd {
 namespace {
@@ -105,46 +106,10 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_kernel(
 
 // Inner sizes of 64 and more: at the float32 rate of the matrix cores (64 flop per cycle and
 // SIMD) the products themselves would take longer than the stream, so they run at the half-precision
-// rate (16 times that) on operands scaled by powers of two into its range and split two ways:
-// x 2^k = hi + lo, 11 bits each and lo signed, so that 2^-24 of x or less is lost, and
-// x y = hi hi + (hi lo + lo hi) + O(2^-24 x y): three products, exact each, summed in float32, at 3/16 of the
-// cost of a float32 product.  A scale belongs to a row or a column of the result, i.e. it is one number
-// for all terms of a sum: its largest term lies in [2^12, 2^15], and what another one loses at the lower end
-// of the range is 2^-37 of the largest or less.  Three bfloat16 parts, whose range needs no scales, took six
+// rate on operands split two ways (see split_half.h).  A scale belongs to a row or a column of the result, i.e. it
+// is one number for all terms of a sum.  Three bfloat16 parts, whose range needs no scales, took six
 // products: with these the error against float64 is 0.6 to 0.9 times as large (fewer additions), 250k edges,
 // H = 64, n = 2 944: forward 690 -> 620 us, dh 700 -> 570, dW 790 -> 540.
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-constexpr int kScaleTop = 125;         // the largest exponent of a scale; also that of a sum without terms
-constexpr float kScaledMax = 32768.f;  // a scaled term above this asks for a smaller scale
-
-struct Split2 {
-    f16x8 term[2];
-};
-__device__ __forceinline__ float pow2(int k) { return __uint_as_float((uint32_t)(k + 127) << 23); }
-// the exponent that takes a largest term of m to [2^12, 2^13)
-__device__ __forceinline__ int scale_exponent(float m) {
-    const int k = 139 - (int)((__float_as_uint(m) >> 23) & 255u);
-    return k < kScaleTop ? k : kScaleTop;
-}
-__device__ __forceinline__ Split2 split2(const float (&x)[8], float scale) {
-    Split2 out;
-#pragma unroll
-    for (int m = 0; m < 8; m++) {
-        const _Float16 hi = (_Float16)(x[m] * scale);
-        out.term[0][m] = hi;
-        out.term[1][m] = (_Float16)__builtin_fmaf(x[m], scale, -(float)hi);
-    }
-    return out;
-}
-__device__ __forceinline__ float max_abs(const float (&x)[8]) {
-    float m = fabsf(x[0]);
-#pragma unroll
-    for (int i = 1; i < 8; i++) m = fmaxf(m, fabsf(x[i]));
-    return m;
-}
-// the partial products, smallest first
-constexpr int kPairs[3][2] = {{0, 1}, {1, 0}, {0, 0}};
 
 // One 32x32x16 product takes sixteen inner indices; a lane (g, c) supplies eight of them for
 // row (A) or column (B) c: block q of the inner dimension gives it the indices 16 q + 8 g + m.
