@@ -91,12 +91,10 @@ class ChannelMix:
 
     def _fused(self, src: torch.Tensor, transpose: bool):
         """The mixing (or its transpose) in one launch of the library's matrix-core kernel, or None
-        where that kernel does not apply (it takes float32 at 64 or 128 channels, up to 8 degrees and 2^25 values
-        per node)."""
+        where that kernel does not apply (it takes float32 at 64 or 128 channels, up to 8 degrees)."""
         import ctypes
         K = self.channels
-        if (src.dtype != torch.float32 or K not in (64, 128) or len(self.blocks) > 8 or src.data_ptr() % 16
-                or self.rows_in * K > 1 << 25):
+        if src.dtype != torch.float32 or K not in (64, 128) or len(self.blocks) > 8 or src.data_ptr() % 16:
             return None
         key = ("fused", transpose, src.device)
         w = self._device.get(key)

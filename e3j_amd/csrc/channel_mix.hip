@@ -114,7 +114,7 @@ __device__ __forceinline__ float largest_over(float m) {
 template <int K, bool kTranspose>
 __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
     const float *__restrict__ src, float *__restrict__ dst, const float *__restrict__ w, int64_t num_nodes,
-    MixShape shape, int32_t rows_plain, int32_t rows_mixed) {
+    MixShape shape, uint32_t plain_stride, uint32_t mixed_stride) {
     // chunks of 64 summed channels, output channels of a block, tiles of 32 of them
     constexpr int KC = K / 64, KO = kTranspose ? 64 : K, KT = KO / 32;
     const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y), r = lane & 31, h = lane >> 5;
@@ -318,7 +318,6 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
     fetch(0);
     __syncthreads();
     commit(split_weights());
-    const uint32_t plain_stride = (uint32_t)rows_plain * K, mixed_stride = (uint32_t)rows_mixed * K;
     f32x4 piece[8];
     if (!kTranspose) {
 #pragma unroll
@@ -369,12 +368,23 @@ int launch_mix(const float *src, float *dst, const float *w, int64_t num_nodes, 
                int rows_plain, int rows_mixed, bool transpose, hipStream_t stream) {
     const int64_t blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves) * rows_mixed * (transpose ? K / 64 : 1);
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: too many nodes for one launch");
+    const int64_t plain = (int64_t)rows_plain * K, mixed = (int64_t)rows_mixed * K;
+    if (num_nodes > 1 && std::max(plain, mixed) > (int64_t)1 << 25) {  // (the nodes of a tile are 32 bits of bytes apart)
+        for (int64_t n = 0; n < num_nodes; n++) {
+            int rc = launch_mix<K>(src + n * (transpose ? mixed : plain), dst + n * (transpose ? plain : mixed), w, 1, shape,
+                                   rows_plain, rows_mixed, transpose, stream);
+            if (rc) return rc;
+        }
+        return E3J_AMD_OK;
+    }
+    // (of one node no stride is used but to tell the nodes that are not there: one row apart will do)
+    const uint32_t plain_stride = num_nodes > 1 ? (uint32_t)plain : K, mixed_stride = num_nodes > 1 ? (uint32_t)mixed : K;
     if (transpose)
         hipLaunchKernelGGL((channel_mix_kernel<K, true>), dim3((unsigned)blocks), dim3(kWave, kMixWaves), 0, stream,
-                           src, dst, w, num_nodes, shape, rows_plain, rows_mixed);
+                           src, dst, w, num_nodes, shape, plain_stride, mixed_stride);
     else
         hipLaunchKernelGGL((channel_mix_kernel<K, false>), dim3((unsigned)blocks), dim3(kWave, kMixWaves), 0, stream,
-                           src, dst, w, num_nodes, shape, rows_plain, rows_mixed);
+                           src, dst, w, num_nodes, shape, plain_stride, mixed_stride);
     return check_hip(hipGetLastError(), "channel_mix launch");
 }
 
@@ -393,21 +403,17 @@ extern "C" int e3j_amd_channel_mix(const void *src, void *dst, const void *weigh
     MixShape shape;
     shape.degrees = num_degrees;
     int rows_plain = 0, rows_mixed = 0;
-    int64_t total_rows = 0;
     for (int l = 0; l < kMixDegrees; l++) {
         shape.mul[l] = l < num_degrees ? mul[l] : 0;
         shape.dim[l] = l < num_degrees ? dim[l] : 0;
         if (l < num_degrees && (mul[l] < 1 || dim[l] < 1))
             return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: multiplicities and dimensions must be >= 1");
         rows_plain += shape.mul[l] * shape.dim[l];
-        total_rows += (int64_t)shape.mul[l] * shape.dim[l];
         rows_mixed += shape.dim[l];
     }
     if (num_nodes == 0) return E3J_AMD_OK;
     if (src == nullptr || dst == nullptr || weights == nullptr)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: null operand");
-    if (total_rows * channels > (int64_t)1 << 25)  // (the rows of 32 nodes are addressed with 32 bits)
-        return set_error(E3J_AMD_UNIMPLEMENTED, "channel_mix: more than 2^25 values per node");
     if (reinterpret_cast<uintptr_t>(src) % 16 != 0 || reinterpret_cast<uintptr_t>(dst) % 16 != 0 ||
         reinterpret_cast<uintptr_t>(weights) % 16 != 0)
         return set_error(E3J_AMD_INVALID_ARGUMENT, "channel_mix: operands must be 16-byte aligned");

@@ -92,3 +92,21 @@ def test_the_ends_of_the_range(K):
     out, weights = out / np.abs(out).max() * 2.0 ** 127, [weights[0] / np.abs(weights[0]).max() * 2.0 ** -120]
     x = _run(out, blocks, K, weights)
     assert _bound(x, E.channel_mix(out, blocks, weights), E.channel_mix(np.abs(out), blocks, [np.abs(weights[0])])).all()
+
+
+def test_nodes_too_far_apart_for_one_launch():
+    """More than 2^25 values a node: a launch a node."""
+    K, n, dim = 64, 2, (1 << 25) // 64 + 1
+    w = np.random.default_rng(3).normal(size=(1, K, K)).astype(np.float32)
+    mixer = ChannelMix([(1, dim)], K, [w])
+    g = torch.Generator(device="cuda").manual_seed(0)
+    out = torch.randn(n, dim, K, device="cuda", generator=g, requires_grad=True)
+    x = mixer(out)
+    dx = torch.randn(x.shape, device="cuda", generator=g)
+    (grad,) = torch.autograd.grad(x, out, dx)
+    weights = torch.as_tensor(w[0], device="cuda")
+    # the bound of `_bound` with the largest sum of magnitudes there is, for the products of torch as well
+    for got, a, b in ((x.detach(), out.detach(), weights), (grad, dx, weights.t().contiguous())):
+        want = (a.view(-1, K) @ b).view_as(got)
+        size = float(a.abs().max()) * float(b.abs().sum(0).max())
+        assert float((got - want).abs().max()) <= 2 * 66 * 2.0 ** -24 * size
