@@ -11,11 +11,10 @@
 // B agree: product j of a lane half takes the inner index g * (inner / 2) + j, so the operands of a
 // lane are contiguous in memory.
 
-#include <algorithm>
 #include <initializer_list>
 
 #include "common.h"
-#include "split_half.h"
+#include "split_bf16.h"
 
 namespace e3j_amd {
 namespace {
@@ -29,7 +28,7 @@ constexpr int kWaves = 4;        // waves per block
 // s = h W.  A block takes kWaves * R * 32 consecutive edges, keeps their rows of h in registers
 // as A operands and walks the columns of W in tiles of 32 that all its waves share through LDS
 // (double buffered: the next tile is fetched while the current one is multiplied).  Few edges leave
-// the chip empty: blockIdx.y then stands for a range of `per_range` column tiles (`column_ranges`).
+// the chip empty: blockIdx.y then stands for a range of `per_range` column tiles (`column_range`).
 template <int H, int R>
 __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_kernel(
     const float *__restrict__ h, const float *__restrict__ w, float *__restrict__ s, int64_t num_edges, int n,
@@ -105,141 +104,100 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_kernel(
 }
 
 // Inner sizes of 64 and more: at the float32 rate of the matrix cores (64 flop per cycle and
-// SIMD) the products themselves would take longer than the stream, so they run at the half-precision
-// rate on operands split two ways (see split_half.h).  A scale belongs to a row or a column of the result, i.e. it
-// is one number for all terms of a sum.  Three bfloat16 parts, whose range needs no scales, took six
-// products: with these the error against float64 is 0.6 to 0.9 times as large (fewer additions), 250k edges,
-// H = 64, n = 2 944: forward 690 -> 620 us, dh 700 -> 570, dW 790 -> 540.
+// SIMD) the products themselves would take longer than the stream, so they run at the bfloat16
+// rate on operands split three ways (see split_bf16.h).
 
 // One 32x32x16 product takes sixteen inner indices; a lane (g, c) supplies eight of them for
 // row (A) or column (B) c: block q of the inner dimension gives it the indices 16 q + 8 g + m.
-// The scale of a row of h is found once, that of a column of W while its tile is on its way.
 template <int H, int R>
-__global__ __launch_bounds__(kWave * kWaves, 2) void radial_linear_fwd_split_kernel(
+__global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_split_kernel(
     const float *__restrict__ h, const float *__restrict__ w, float *__restrict__ s, int64_t num_edges, int n,
     int per_range) {
     constexpr int Q = H / 16;                         // inner blocks
     constexpr int SLOTS = 2 * Q * kTile;              // (q, g, c) operand slots of a W tile: 8 values each
-    constexpr int PER_THREAD = SLOTS / (kWave * kWaves);
-    static_assert(H % 16 == 0 && SLOTS % (kWave * kWaves) == 0, "whole inner blocks, whole rounds of slots");
-    __shared__ __attribute__((aligned(16))) f16x8 tile[2][2][SLOTS];
-    __shared__ uint32_t largest[4][kTile];            // largest weight of a column, by tile modulo 4
-    __shared__ int row_exp[kWaves][R * kTile];
+    constexpr int PER_THREAD = (SLOTS + kWave * kWaves - 1) / (kWave * kWaves);
+    static_assert(H % 16 == 0, "whole inner blocks");
+    __shared__ __attribute__((aligned(16))) bf16x8 tile[2][3][SLOTS];
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int g = lane / kTile, c = lane % kTile;
     const int64_t e0 = ((int64_t)blockIdx.x * kWaves + wave) * (kTile * R);
 
-    Split2 a[R][Q];
+    Split3 a[R][Q];
 #pragma unroll
     for (int r = 0; r < R; r++) {
         int64_t row = e0 + r * kTile + c;
         if (row >= num_edges) row = num_edges - 1;  // rows past the end are computed and not stored
-        float x[Q][8], m = 0.f;
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const f32x4 *p = reinterpret_cast<const f32x4 *>(h + row * H + q * 16 + g * 8);
             const f32x4 v0 = __builtin_nontemporal_load(p), v1 = __builtin_nontemporal_load(p + 1);
-            const float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-#pragma unroll
-            for (int i = 0; i < 8; i++) x[q][i] = v[i];
-            m = fmaxf(m, max_abs(x[q]));
+            const float x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+            a[r][q] = split3(x);
         }
-        const int k = scale_exponent(fmaxf(m, __shfl_xor(m, kTile, kWave)));
-        if (g == 0) row_exp[wave][r * kTile + c] = k;
-#pragma unroll
-        for (int q = 0; q < Q; q++) a[r][q] = split2(x[q], pow2(k));
     }
 
     // a thread stages whole operand slots: eight consecutive inner indices of one column
-    float now[PER_THREAD][8], next[PER_THREAD][8];
-    const int first = blockIdx.y * per_range, tiles = min(n / kTile, first + per_range);
-    auto fetch = [&](int t, float (&x)[PER_THREAD][8]) {  // (past the last tile: the last one again)
+    float staged[PER_THREAD][8];
+    auto fetch = [&](int t) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; i++) {
             const int slot = i * kWave * kWaves + tid;
-            const float *col = w + (int64_t)((slot / kTile) * 8) * n + min(t, tiles - 1) * kTile + c;
+            if (SLOTS % (kWave * kWaves) == 0 || slot < SLOTS) {
+                const float *col = w + (int64_t)((slot / kTile) * 8) * n + t * kTile + slot % kTile;
 #pragma unroll
-            for (int m = 0; m < 8; m++) x[i][m] = col[(int64_t)m * n];
+                for (int m = 0; m < 8; m++) staged[i][m] = col[(int64_t)m * n];
+            }
         }
     };
-    auto note = [&](int t, const float (&x)[PER_THREAD][8]) {
-        float m = max_abs(x[0]);
-#pragma unroll
-        for (int i = 1; i < PER_THREAD; i++) m = fmaxf(m, max_abs(x[i]));
-        atomicMax(&largest[t & 3][c], __float_as_uint(m));
-    };
-    auto column_exponent = [&](int t) { return scale_exponent(__uint_as_float(largest[t & 3][c])); };
-    auto commit = [&](int t, const float (&x)[PER_THREAD][8]) {
-        const float scale = pow2(column_exponent(t));
+    auto commit = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; i++) {
-            const Split2 parts = split2(x[i], scale);
+            const int slot = i * kWave * kWaves + tid;
+            if (SLOTS % (kWave * kWaves) == 0 || slot < SLOTS) {
+                const Split3 parts = split3(staged[i]);
 #pragma unroll
-            for (int p = 0; p < 2; p++) tile[t & 1][p][i * kWave * kWaves + tid] = parts.term[p];
+                for (int t = 0; t < 3; t++) tile[buf][t][slot] = parts.term[t];
+            }
         }
     };
-    if (tid < 4 * kTile) (&largest[0][0])[tid] = 0u;
-    fetch(first, now);
-    fetch(first + 1, next);
-    __syncthreads();
-    int row_k[R][16];
-#pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) row_k[r][v] = row_exp[wave][r * kTile + 8 * (v / 4) + 4 * g + v % 4];
-    note(first, now);
-    note(first + 1, next);
-    __syncthreads();
-    commit(first, now);
-#pragma unroll
-    for (int i = 0; i < PER_THREAD; i++)
-#pragma unroll
-        for (int m = 0; m < 8; m++) now[i][m] = next[i][m];
-    fetch(first + 2, next);
+    const int first = blockIdx.y * per_range, tiles = min(n / kTile, first + per_range);
+    fetch(first);
+    commit(first & 1);
     __syncthreads();
     for (int t = first; t < tiles; t++) {
-        // (of the four sets of column maxima: tile t's is read, t + 1's complete, t + 2's collected, t + 3's cleared)
+        if (t + 1 < tiles) fetch(t + 1);
         f32x16 d[R];
 #pragma unroll
         for (int r = 0; r < R; r++) d[r] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < Q; q++) {
-            f16x8 b[2];
+            bf16x8 b[3];
 #pragma unroll
-            for (int tb = 0; tb < 2; tb++) b[tb] = tile[t & 1][tb][(q * 2 + g) * kTile + c];
+            for (int tb = 0; tb < 3; tb++) b[tb] = tile[t & 1][tb][(q * 2 + g) * kTile + c];
 #pragma unroll
-            for (int u = 0; u < 3; u++) {
+            for (int u = 0; u < 6; u++) {
 #pragma unroll
                 for (int r = 0; r < R; r++)
-                    d[r] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[r][q].term[kPairs[u][0]], b[kPairs[u][1]], d[r], 0, 0, 0);
+                    d[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r][q].term[kPairs[u][0]], b[kPairs[u][1]], d[r], 0, 0, 0);
             }
         }
-        const int col_k = column_exponent(t);
-        commit(t + 1, now);
-        note(t + 2, next);
-        if (tid < kTile) largest[(t + 3) & 3][tid] = 0u;
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; i++)
-#pragma unroll
-            for (int m = 0; m < 8; m++) now[i][m] = next[i][m];
-        fetch(t + 3, next);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             float *out = s + (e0 + r * kTile + 4 * g) * n + t * kTile + c;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const int row = 8 * (v / 4) + v % 4;
-                if (e0 + r * kTile + 4 * g + row < num_edges)
-                    __builtin_nontemporal_store(__builtin_ldexpf(d[r][v], -(row_k[r][v] + col_k)), out + (int64_t)row * n);
+                if (e0 + r * kTile + 4 * g + row < num_edges) __builtin_nontemporal_store(d[r][v], out + (int64_t)row * n);
             }
         }
+        if (t + 1 < tiles) commit((t + 1) & 1);
         __syncthreads();
     }
 }
 
 // Column tiles per block: all of them where the edges alone make a block per compute unit, else ranges of them so
 // that there are about as many (4 099 edges, H = 64, n = 992: 60 -> 11 us; 2 000 edges, H = 128, n = 2 048: 104 -> 13; two
-// or four blocks per unit: 11 and 15, 14 and 18, since every range reads h again).
+// blocks per unit: 11 and 13, and 12 000 edges, n = 992: 20 -> 24).
 int column_range(int64_t blocks, int tiles) {
     const int64_t ranges = std::min<int64_t>(tiles, std::max<int64_t>(1, 256 / blocks));
     return (int)((tiles + ranges - 1) / ranges);
@@ -379,26 +337,24 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_bwd_weight_kerne
     }
 }
 
-// The same from inner size 64 on, at the half-precision rate with both operands split two ways (see
-// split2): h when a chunk is staged (an operand slot = eight consecutive edges of one row of dW; a
-// scale per row, agreed on by the block), ds in registers as it arrives (a scale per column, the lane's own).
+// The same from inner size 64 on, at the bfloat16 rate with both operands split three ways (see
+// split_bf16.h): h when a chunk is staged (an operand slot = eight consecutive edges of one
+// row of dW), ds in registers as it arrives.
 // Two blocks of ds are on their way while a third is multiplied: they are read through buffer descriptors, which
-// take one 32-bit offset a load instead of a 64-bit address and a bound (208 -> 241 registers with twice the loads
-// in flight; the loads alone 790 -> 690 us).  kWide: rows too long for 32-bit offsets.
+// take one 32-bit offset a load instead of a 64-bit address and a bound (250k edges, H = 64, n = 2 944: 800 -> 640 us;
+// H = 128, n = 1 472: 750 -> 595).  kWide: rows too long for 32-bit offsets.
 template <int H, bool kWide>
 __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linear_bwd_weight_split_kernel(
     const float *__restrict__ h, const float *__restrict__ ds, float *__restrict__ partial, int64_t num_edges,
     int n, int groups) {
     constexpr int RT = H / kTile;                // row tiles of dW
-    constexpr int CHUNK = H >= 128 ? 32 : 64, Q = CHUNK / 16;  // edges per step; inner blocks of 16 edges
+    constexpr int CHUNK = 64, Q = CHUNK / 16;    // edges per step; inner blocks of 16 edges
     constexpr int SLOTS = 2 * Q * H;             // (q, g, row) operand slots of a chunk of h
     constexpr int PER_THREAD = SLOTS / (kWave * kWaves);
     constexpr int AHEAD = 2;                     // blocks of ds on their way
     static_assert(H % kTile == 0 && SLOTS % (kWave * kWaves) == 0, "whole tiles, whole rounds of slots");
-    static_assert(kWave * kWaves % H == 0, "a thread stages one row of dW");
-    __shared__ __attribute__((aligned(16))) f16x8 rows[2][2][SLOTS];
-    __shared__ uint32_t largest[2][H];           // largest terms that asked for a smaller scale, by chunk parity
-    __shared__ int exponent[H], asked[2];
+    static_assert(Q % AHEAD == 0, "a block of ds has one place among those on their way");
+    __shared__ __attribute__((aligned(16))) bf16x8 rows[2][3][SLOTS];
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int g = lane / kTile, c = lane % kTile;
     const int slabs = (n + kSlab - 1) / kSlab;
@@ -419,54 +375,29 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
     for (int t = 0; t < kColTiles; t++) col_ok[t] = col0 + t * kTile < n;
 
     // slot (q, g, row): h[e0 + 16 q + 8 g + m][row], m < 8; edges past the range read as zeros
-    const int row = tid % H;
-    int row_exp = kScaleTop;                     // exponent of the scale of this thread's row
-    auto fetch = [&](int64_t e0, float (&x)[PER_THREAD][8]) {
+    float staged[PER_THREAD][8];
+    auto fetch = [&](int64_t e0) {
         const int64_t left = last - e0;
         const uint32_t bytes = left <= 0 ? 0u : (uint32_t)((left < CHUNK ? left : CHUNK) * H) * 4u;
         const __amdgpu_buffer_rsrc_t range =
             __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(h + (left > 0 ? e0 : (int64_t)0) * H), 0, bytes, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < PER_THREAD; i++)
+        for (int i = 0; i < PER_THREAD; i++) {
+            const int slot = i * kWave * kWaves + tid;
 #pragma unroll
             for (int m = 0; m < 8; m++)
-                x[i][m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    range, (((i * kWave * kWaves + tid) / H) * 8 * H + row) * 4 + m * H * 4, 0, 0));
-    };
-    auto ask = [&](const float (&x)[PER_THREAD][8], int parity, int chunk) {
-        float m = max_abs(x[0]);
-#pragma unroll
-        for (int i = 1; i < PER_THREAD; i++) m = fmaxf(m, max_abs(x[i]));
-        if (m * pow2(row_exp) > kScaledMax) {
-            atomicMax(&largest[parity][row], __float_as_uint(m));
-            asked[parity] = chunk;
+                staged[i][m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    range, (slot / H * 8 * H + slot % H) * 4 + m * H * 4, 0, 0));
         }
     };
-    for (int i = tid; i < H; i += kWave * kWaves) {
-        largest[0][i] = largest[1][i] = 0u;
-        exponent[i] = kScaleTop;
-    }
-    if (tid < 2) asked[tid] = -1;
-    __syncthreads();
-    // after the products of a chunk: the scales that the next chunk asked for, and the sums so far with them
-    auto rescale = [&](int parity) {
-        row_exp = min(row_exp, scale_exponent(__uint_as_float(largest[parity][row])));
+    auto commit = [&](int buf) {
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
+        for (int i = 0; i < PER_THREAD; i++) {
+            const Split3 parts = split3(staged[i]);
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int at = rt * kTile + 8 * (v / 4) + 4 * g + v % 4;
-                const int by = min(0, scale_exponent(__uint_as_float(largest[parity][at])) - exponent[at]);
-#pragma unroll
-                for (int t = 0; t < kColTiles; t++) d[t][rt][v] = __builtin_ldexpf(d[t][rt][v], by);
-            }
+            for (int t = 0; t < 3; t++) rows[buf][t][i * kWave * kWaves + tid] = parts.term[t];
         }
-        __syncthreads();
-        for (int i = tid; i < H; i += kWave * kWaves)
-            exponent[i] = min(exponent[i], scale_exponent(__uint_as_float(largest[parity][i])));
-        __syncthreads();
     };
-
     // the eight ds values of a lane for the block of 16 edges at `e`: a range of the array that ends with the
     // edges of this block, past which a buffer load reads zeros (columns past the last one read the next
     // row's or zeros, and are not stored)
@@ -495,71 +426,40 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
             for (int t = 0; t < kColTiles; t++)  // (2: non-temporal)
                 x[t][m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(range, at[m] + t * kTile * 4, 0, 2));
     };
-    int col_exp[kColTiles];
-#pragma unroll
-    for (int t = 0; t < kColTiles; t++) col_exp[t] = kScaleTop;
-
-    float staged[2][PER_THREAD][8];
-    fetch(first, staged[0]);
-    ask(staged[0], 1, 0);
-    __syncthreads();
-    rescale(1);
-    fetch(first + CHUNK, staged[1]);
+    fetch(first);
+    commit(0);
 #pragma unroll
     for (int u = 0; u < AHEAD; u++) load_ds(first + u * 16, xn[u]);
-    int chunk = 0;
-    for (int64_t e0 = first; e0 < last; e0 += CHUNK, chunk++) {
-        const int buf = chunk & 1;
-        {
-            const float scale = pow2(row_exp);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t e0 = first; e0 < last; e0 += CHUNK, buf ^= 1) {
+        fetch(e0 + CHUNK);
+#pragma unroll 1
+        for (int q0 = 0; q0 < Q; q0 += AHEAD) {  // (not unrolled further: the split operands of a block fill the registers)
 #pragma unroll
-            for (int i = 0; i < PER_THREAD; i++) {
-                const Split2 parts = split2(staged[0][i], scale);
+            for (int u = 0; u < AHEAD; u++) {
+                const int q = q0 + u;
+                Split3 b[kColTiles];
 #pragma unroll
-                for (int t = 0; t < 2; t++) rows[buf][t][i * kWave * kWaves + tid] = parts.term[t];
+                for (int t = 0; t < kColTiles; t++) b[t] = split3(xn[u][t]);
+                load_ds(e0 + (q + AHEAD) * 16, xn[u]);
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++) {
+                    bf16x8 a[3];
+#pragma unroll
+                    for (int ta = 0; ta < 3; ta++) a[ta] = rows[buf][ta][(q * 2 + g) * H + rt * kTile + c];
+#pragma unroll
+                    for (int p = 0; p < 6; p++) {
+#pragma unroll
+                        for (int t = 0; t < kColTiles; t++)
+                            d[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kPairs[p][0]], b[t].term[kPairs[p][1]],
+                                                                               d[t][rt], 0, 0, 0);
+                    }
+                }
             }
         }
-        ask(staged[1], buf, chunk);
-#pragma unroll
-        for (int i = 0; i < PER_THREAD; i++)
-#pragma unroll
-            for (int m = 0; m < 8; m++) staged[0][i][m] = staged[1][i][m];
-        fetch(e0 + 2 * CHUNK, staged[1]);
+        commit(buf ^ 1);
         __syncthreads();
-        const bool smaller = asked[buf] == chunk;
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            float (&x)[kColTiles][8] = xn[q % AHEAD];
-            Split2 b[kColTiles];
-#pragma unroll
-            for (int t = 0; t < kColTiles; t++) {
-                const float m = max_abs(x[t]);
-                if (__any(m * pow2(col_exp[t]) > kScaledMax)) {
-                    const int now = min(col_exp[t], scale_exponent(fmaxf(m, __shfl_xor(m, kTile, kWave))));
-#pragma unroll
-                    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-                        for (int v = 0; v < 16; v++) d[t][rt][v] = __builtin_ldexpf(d[t][rt][v], now - col_exp[t]);
-                    col_exp[t] = now;
-                }
-                b[t] = split2(x[t], pow2(col_exp[t]));
-            }
-            load_ds(e0 + (q + AHEAD) * 16, x);
-#pragma unroll
-            for (int rt = 0; rt < RT; rt++) {
-                f16x8 a[2];
-#pragma unroll
-                for (int ta = 0; ta < 2; ta++) a[ta] = rows[buf][ta][(q * 2 + g) * H + rt * kTile + c];
-#pragma unroll
-                for (int u = 0; u < 3; u++) {
-#pragma unroll
-                    for (int t = 0; t < kColTiles; t++)
-                        d[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[kPairs[u][0]], b[t].term[kPairs[u][1]],
-                                                                          d[t][rt], 0, 0, 0);
-                }
-            }
-        }
-        if (smaller) rescale(buf);
     }
 #pragma unroll
     for (int t = 0; t < kColTiles; t++) {
@@ -568,10 +468,7 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int r = rt * kTile + 8 * (v / 4) + 4 * g + v % 4;
-                out[(int64_t)r * n] = __builtin_ldexpf(d[t][rt][v], -(exponent[r] + col_exp[t]));
-            }
+            for (int v = 0; v < 16; v++) out[(int64_t)(rt * kTile + 8 * (v / 4) + 4 * g + v % 4) * n] = d[t][rt][v];
         }
     }
 }
@@ -628,17 +525,18 @@ int launch_bwd_weight(const float *h, const float *ds, float *dw, float *partial
 // dh (E, H) = ds W^T for inner sizes of 64 and more, with W^T passed as wt (n, H).  The
 // contraction runs along the rows of ds, so a lane (which stands for an edge in the operand
 // layout) would read its own row; instead a wave loads its tile of 32 R edges x 32 n the coalesced
-// way (a row piece of 128 bytes per 8 lanes), splits it two ways (see split2; a scale per edge) and writes
-// the parts to its private piece of LDS in operand order, from where every lane fetches its slots with 16-byte
-// reads.  The rows of wt of the same 32 n, one contiguous block, are split (a scale per column of dh, agreed on
-// by the block) and shared by the waves of the block, one barrier a step.  ds is read once, two steps ahead.
+// way (a row piece of 128 bytes per 8 lanes), splits it three ways and writes the parts to its private piece of LDS
+// in operand order, from where every lane fetches its slots with 16-byte reads.  The rows of wt of the same 32 n,
+// one contiguous block, are split and shared by the waves of the block, one barrier a step.  ds is read once,
+// two steps ahead: 250k edges, H = 64, n = 2 944: 690 us, H = 128, n = 1 472: 590 (eight waves a block: 585, but 2 000
+// edges, n = 2 048, 147 instead of 105).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-template <int H, int R, int W, int CHUNK>
-__global__ __launch_bounds__(kWave * W, 8 / W) void radial_linear_bwd_input_split_kernel(
+template <int H, int R>
+__global__ __launch_bounds__(kWave * kWaves, 2) void radial_linear_bwd_input_split_kernel(
     const float *__restrict__ ds, const float *__restrict__ wt, float *__restrict__ dh, int64_t num_edges, int n) {
     constexpr int CT = H / kTile;                 // column tiles of dh
-    constexpr int Q = CHUNK / 16;                 // inner blocks of 16 of a step of CHUNK n
+    constexpr int CHUNK = 32, Q = CHUNK / 16;     // n per step; inner blocks of 16
     constexpr int ROWS = R * kTile;               // edges of a wave
     constexpr int A_BLOCK = ROWS + 2;             // operand slots of one (q, g): an edge each, and a pad
     constexpr int LANES = CHUNK / 4, EDGES = kWave / LANES;  // lanes side by side on an edge, edges of a piece
@@ -646,16 +544,13 @@ __global__ __launch_bounds__(kWave * W, 8 / W) void radial_linear_bwd_input_spli
     constexpr int A_PIECES = ROWS * CHUNK / 4 / kWave;  // 16-byte pieces of the tile per lane
     constexpr int AHEAD = 2;                      // chunks of ds on their way
     constexpr int B_SLOTS = 2 * Q * H;            // (q, g, column) operand slots of the wt chunk
-    constexpr int B_PER_THREAD = B_SLOTS / (kWave * W);
-    static_assert(B_SLOTS % (kWave * W) == 0 && kWave * W % H == 0, "a thread stages one column of dh");
-    __shared__ __attribute__((aligned(16))) f16x8 a_tile[W][2][A_SLOTS];
-    __shared__ __attribute__((aligned(16))) f16x8 b_tile[2][2][B_SLOTS];
-    __shared__ int row_by[W][ROWS];          // by what power of two the scale of an edge changed
-    __shared__ uint32_t largest[2][H];            // largest terms that asked for a smaller scale, by chunk parity
-    __shared__ int asked[2];
+    constexpr int B_PER_THREAD = B_SLOTS / (kWave * kWaves);
+    static_assert(B_SLOTS % (kWave * kWaves) == 0, "whole rounds of slots");
+    __shared__ __attribute__((aligned(16))) bf16x8 a_tile[kWaves][3][A_SLOTS];
+    __shared__ __attribute__((aligned(16))) bf16x8 b_tile[2][3][B_SLOTS];
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
     const int g = lane / kTile, c = lane % kTile;
-    const int64_t e0 = ((int64_t)blockIdx.x * W + wave) * ROWS;
+    const int64_t e0 = ((int64_t)blockIdx.x * kWaves + wave) * ROWS;
 
     // a lane moves A_PIECES pieces of 16 bytes of the tile: piece p = 64 i + lane is n-quad p % LANES of edge p / LANES
     const float *src[A_PIECES];
@@ -674,15 +569,8 @@ __global__ __launch_bounds__(kWave * W, 8 / W) void radial_linear_bwd_input_spli
 #pragma unroll
         for (int ct = 0; ct < CT; ct++)
             d[r][ct] = f32x16{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    int row_exp[A_PIECES], col_exp[CT];           // exponents of the scales: of the edges of a lane's pieces,
-    int stage_exp = kScaleTop;                    // of the columns a lane holds, of the column a thread stages
-#pragma unroll
-    for (int i = 0; i < A_PIECES; i++) row_exp[i] = kScaleTop;
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) col_exp[ct] = kScaleTop;
-
     f32x4 a[AHEAD][A_PIECES];
-    float b_now[B_PER_THREAD][8], b_next[B_PER_THREAD][8];
+    float b_next[B_PER_THREAD][8];
     const int chunks = n / CHUNK;
     // (loads past the last chunk read it again: with every load issued on every path the waits count exactly)
     auto fetch_a = [&](int t, f32x4 (&x)[A_PIECES]) {
@@ -690,132 +578,59 @@ __global__ __launch_bounds__(kWave * W, 8 / W) void radial_linear_bwd_input_spli
 #pragma unroll
         for (int i = 0; i < A_PIECES; i++) x[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src[i] + at));
     };
-    auto fetch_b = [&](int t, float (&x)[B_PER_THREAD][8]) {  // slot (q, g, column): wt[32 t + 16 q + 8 g + m][column]
+    auto fetch_b = [&](int t) {  // slot (q, g, column): wt[32 t + 16 q + 8 g + m][column]
 #pragma unroll
         for (int i = 0; i < B_PER_THREAD; i++) {
-            const int slot = i * kWave * W + tid;
+            const int slot = i * kWave * kWaves + tid;
             const float *col = wt + ((int64_t)min(t, chunks - 1) * CHUNK + (slot / H) * 8) * H + slot % H;
 #pragma unroll
-            for (int m = 0; m < 8; m++) x[i][m] = col[m * H];
+            for (int m = 0; m < 8; m++) b_next[i][m] = col[m * H];
         }
     };
-    auto ask = [&](const float (&x)[B_PER_THREAD][8], int parity, int chunk) {
-        float m = max_abs(x[0]);
-#pragma unroll
-        for (int i = 1; i < B_PER_THREAD; i++) m = fmaxf(m, max_abs(x[i]));
-        if (m * pow2(stage_exp) > kScaledMax) {
-            atomicMax(&largest[parity][tid % H], __float_as_uint(m));
-            asked[parity] = chunk;
-        }
-    };
-    // the scales of the columns that the next chunk asked for, and the sums so far with them
-    auto rescale_columns = [&](int parity) {
-        stage_exp = min(stage_exp, scale_exponent(__uint_as_float(largest[parity][tid % H])));
-#pragma unroll
-        for (int ct = 0; ct < CT; ct++) {
-            const int now = min(col_exp[ct], scale_exponent(__uint_as_float(largest[parity][ct * kTile + c])));
-#pragma unroll
-            for (int r = 0; r < R; r++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) d[r][ct][v] = __builtin_ldexpf(d[r][ct][v], now - col_exp[ct]);
-            col_exp[ct] = now;
-        }
-    };
-    auto wave_fence = [] {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    };
-    auto largest_of = [](const f32x4 &x) { return fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))); };
-    // the same for the edges of the wave, before their terms are split
-    auto rescale_rows = [&](const f32x4 (&x)[A_PIECES]) {
-#pragma unroll
-        for (int i = 0; i < A_PIECES; i++) {
-            float m = largest_of(x[i]);
-#pragma unroll
-            for (int off = 1; off < LANES; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, kWave));  // the lanes of an edge
-            const int now = m * pow2(row_exp[i]) > kScaledMax ? min(row_exp[i], scale_exponent(m)) : row_exp[i];
-            if (quad == 0) row_by[wave][i * EDGES + lane / LANES] = now - row_exp[i];
-            row_exp[i] = now;
-        }
-        wave_fence();
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int by = row_by[wave][r * kTile + 8 * (v / 4) + 4 * g + v % 4];
-#pragma unroll
-                for (int ct = 0; ct < CT; ct++) d[r][ct][v] = __builtin_ldexpf(d[r][ct][v], by);
-            }
-        }
-        wave_fence();
-    };
-
-    for (int i = tid; i < H; i += kWave * W) largest[0][i] = largest[1][i] = 0u;
-    if (tid < 2) asked[tid] = -1;
-    __syncthreads();
-    fetch_b(0, b_now);
-    ask(b_now, 1, 0);
-    __syncthreads();
-    rescale_columns(1);
-    fetch_b(1, b_next);
+    fetch_b(0);
 #pragma unroll
     for (int u = 0; u < AHEAD; u++) fetch_a(u, a[u]);
     auto step = [&](int t, f32x4 (&x)[A_PIECES]) {
         const int buf = t & 1;
-        float most = 0.f;
-#pragma unroll
-        for (int i = 0; i < A_PIECES; i++) most = fmaxf(most, largest_of(x[i]) * pow2(row_exp[i]));
-        if (__any(most > kScaledMax)) rescale_rows(x);
-        u32x2 *halves[2] = {reinterpret_cast<u32x2 *>(a_tile[wave][0]), reinterpret_cast<u32x2 *>(a_tile[wave][1])};
+        u32x2 *halves[3] = {reinterpret_cast<u32x2 *>(a_tile[wave][0]), reinterpret_cast<u32x2 *>(a_tile[wave][1]),
+                            reinterpret_cast<u32x2 *>(a_tile[wave][2])};
 #pragma unroll
         for (int i = 0; i < A_PIECES; i++) {
-            const float v[4] = {x[i].x, x[i].y, x[i].z, x[i].w}, scale = pow2(row_exp[i]);
-            f16x4 hi, lo;
+            float rest[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
 #pragma unroll
-            for (int m = 0; m < 4; m++) {  // see split2
-                hi[m] = (_Float16)(v[m] * scale);
-                lo[m] = (_Float16)__builtin_fmaf(v[m], scale, -(float)hi[m]);
-            }
-            halves[0][half_slot + i * EDGES * 2] = __builtin_bit_cast(u32x2, hi);
-            halves[1][half_slot + i * EDGES * 2] = __builtin_bit_cast(u32x2, lo);
+            for (int p = 0; p < 3; p++)  // see split3
+                halves[p][half_slot + i * EDGES * 2] = u32x2{take_upper(rest[0], rest[1]), take_upper(rest[2], rest[3])};
         }
         fetch_a(t + AHEAD, x);
 #pragma unroll
         for (int i = 0; i < B_PER_THREAD; i++) {
-            const Split2 parts = split2(b_now[i], pow2(stage_exp));
+            const Split3 parts = split3(b_next[i]);
 #pragma unroll
-            for (int p = 0; p < 2; p++) b_tile[buf][p][i * kWave * W + tid] = parts.term[p];
+            for (int p = 0; p < 3; p++) b_tile[buf][p][i * kWave * kWaves + tid] = parts.term[p];
         }
-        ask(b_next, buf, t);
-#pragma unroll
-        for (int i = 0; i < B_PER_THREAD; i++)
-#pragma unroll
-            for (int m = 0; m < 8; m++) b_now[i][m] = b_next[i][m];
-        fetch_b(t + 2, b_next);
+        fetch_b(t + 1);
         __syncthreads();  // (one barrier a chunk: the shared rows of wt are double buffered)
-        const bool smaller = asked[buf] == t;
 #pragma unroll
         for (int q = 0; q < Q; q++) {
-            f16x8 p[R][2];
+            bf16x8 p[R][3];
 #pragma unroll
             for (int r = 0; r < R; r++)
 #pragma unroll
-                for (int ta = 0; ta < 2; ta++) p[r][ta] = a_tile[wave][ta][(q * 2 + g) * A_BLOCK + r * kTile + c];
+                for (int ta = 0; ta < 3; ta++) p[r][ta] = a_tile[wave][ta][(q * 2 + g) * A_BLOCK + r * kTile + c];
 #pragma unroll
             for (int ct = 0; ct < CT; ct++) {
-                f16x8 b[2];
+                bf16x8 b[3];
 #pragma unroll
-                for (int tb = 0; tb < 2; tb++) b[tb] = b_tile[buf][tb][(q * 2 + g) * H + ct * kTile + c];
+                for (int tb = 0; tb < 3; tb++) b[tb] = b_tile[buf][tb][(q * 2 + g) * H + ct * kTile + c];
 #pragma unroll
-                for (int u = 0; u < 3; u++) {
+                for (int u = 0; u < 6; u++) {
 #pragma unroll
                     for (int r = 0; r < R; r++)
-                        d[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(p[r][kPairs[u][0]], b[kPairs[u][1]], d[r][ct],
-                                                                          0, 0, 0);
+                        d[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[r][kPairs[u][0]], b[kPairs[u][1]], d[r][ct],
+                                                                           0, 0, 0);
                 }
             }
         }
-        if (smaller) rescale_columns(buf);
     };
     for (int t = 0;;) {
         step(t, a[0]);
@@ -823,35 +638,25 @@ __global__ __launch_bounds__(kWave * W, 8 / W) void radial_linear_bwd_input_spli
         step(t, a[1]);
         if (++t >= chunks) break;
     }
-    // the exponents of the edges, in the order of the accumulators
-#pragma unroll
-    for (int i = 0; i < A_PIECES; i++)
-        if (quad == 0) row_by[wave][i * EDGES + lane / LANES] = row_exp[i];
-    wave_fence();
 #pragma unroll
     for (int r = 0; r < R; r++) {
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int row = r * kTile + 8 * (v / 4) + 4 * g + v % 4;
-            const int by = -row_by[wave][row];
             if (e0 + row >= num_edges) continue;
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++)
-                dh[(e0 + row) * H + ct * kTile + c] = __builtin_ldexpf(d[r][ct][v], by - col_exp[ct]);
+            for (int ct = 0; ct < CT; ct++) dh[(e0 + row) * H + ct * kTile + c] = d[r][ct][v];
         }
     }
 }
 
 template <int H>
 int launch_bwd_input(const float *ds, const float *wt, float *dh, int64_t num_edges, int n, hipStream_t stream) {
-    // row tiles per wave and waves per block: 256 edges share the rows of wt either way (H = 128, n = 1 472: 440 us
-    // with four waves of one tile, 420 with eight; H = 64, n = 2 944: 570 with four waves of two tiles, 600 with eight
-    // of one and 64 columns a step, 640 with four of one)
-    constexpr int R = H >= 128 ? 1 : 2, W = H >= 128 ? 8 : 4;
-    const int64_t per_block = (int64_t)W * R * kTile;
+    constexpr int R = H >= 128 ? 1 : 2;  // row tiles per wave
+    const int64_t per_block = (int64_t)kWaves * R * kTile;
     const int64_t blocks = (num_edges + per_block - 1) / per_block;
     if (blocks > 0x7fffffffLL) return set_error(E3J_AMD_INVALID_ARGUMENT, "radial_linear_bwd_input: too many edges");
-    hipLaunchKernelGGL((radial_linear_bwd_input_split_kernel<H, R, W, 32>), dim3((unsigned)blocks), dim3(kWave * W), 0,
+    hipLaunchKernelGGL((radial_linear_bwd_input_split_kernel<H, R>), dim3((unsigned)blocks), dim3(kWave * kWaves), 0,
                        stream, ds, wt, dh, num_edges, n);
     return check_hip(hipGetLastError(), "radial_linear_bwd_input launch");
 }

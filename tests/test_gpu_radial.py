@@ -105,7 +105,7 @@ def test_input_gradient_matches_the_float64_product(inner, edges, n):
 def test_scales_of_the_split_products_follow_the_terms(inner, edges, n, largest):
     """Operands whose magnitude differs by up to 2^40 from row to row and along the sums: every result
     within float32 rounding of its own sum of magnitudes (2^-24 a term for the split operands and for the
-    sums, as for operands of one size; terms below 2^-13 of the largest are held to 2^-37 of it, n 2^-37 < 2^-24)."""
+    sums, as for operands of one size)."""
     g = torch.Generator(device="cuda").manual_seed(inner + edges + n)
 
     def spread(count):
@@ -128,6 +128,55 @@ def test_scales_of_the_split_products_follow_the_terms(inner, edges, n, largest)
                              (dw, hd.t().contiguous(), dd, edges)):
         bound = (8 + terms ** 0.5) * 2.0 ** -24 * (a.abs() @ b.abs())
         assert bool(((got.double() - a @ b).abs() <= bound).all())
+
+
+def _assert_products(h, w, ds):
+    """s, dh and dw within the bound of `test_scales_of_the_split_products_follow_the_terms`."""
+    h, w = h.requires_grad_(True), w.requires_grad_(True)
+    s = radial_linear(h, w)
+    dh, dw = torch.autograd.grad(s, (h, w), ds)
+    hd, wd, dd = h.detach().double(), w.detach().double(), ds.double()
+    for name, got, a, b, terms in (("s", s.detach(), hd, wd, h.shape[1]), ("dh", dh, dd, wd.t().contiguous(), w.shape[1]),
+                                   ("dw", dw, hd.t().contiguous(), dd, h.shape[0])):
+        over = (got.double() - a @ b).abs() / ((8 + terms ** 0.5) * 2.0 ** -24 * (a.abs() @ b.abs())).clamp_min(1e-300)
+        assert float(over.max()) <= 1.0, (name, float(over.max()))
+
+
+@pytest.mark.parametrize("inner", [64, 128])
+@pytest.mark.parametrize("edges,n", [(65, 32), (300, 2944), (3000, 544)])
+@pytest.mark.parametrize("bits", [8, 14, 20, 40])
+def test_spreads_that_oppose_each_other(inner, edges, n, bits):
+    """Along each of the three sums one operand grows where the other shrinks, so that all terms are of a size: a small
+    operand of a row is not lost beside a large one."""
+    g = torch.Generator(device="cuda").manual_seed(inner + edges + n + bits)
+
+    def spread(count):
+        return torch.exp2(torch.randint(-bits, bits + 1, (count,), device="cuda", generator=g).float())
+
+    over_edges, over_inner, over_n = spread(edges)[:, None], spread(inner), spread(n)[None]
+    h = torch.randn(edges, inner, device="cuda", generator=g) * over_edges * over_inner[None]
+    w = torch.randn(inner, n, device="cuda", generator=g) / over_inner[:, None] / over_n
+    _assert_products(h, w, torch.randn(edges, n, device="cuda", generator=g) * over_n / over_edges)
+
+
+@pytest.mark.parametrize("inner", [64, 128])
+@pytest.mark.parametrize("outlier", [1e8, 1e10, 1e15])
+def test_outliers_that_meet_zeros(inner, outlier):
+    """A masked edge whose hidden units hold anything, a unit whose weights are zeros, a column without weights, and
+    columns that pick one unit each: the other terms of their sums keep their digits."""
+    g = torch.Generator(device="cuda").manual_seed(inner)
+    h, w = torch.randn(300, inner, device="cuda", generator=g), torch.randn(inner, 544, device="cuda", generator=g)
+    ds = torch.randn(300, 544, device="cuda", generator=g)
+    h[17] *= outlier
+    ds[17] = 0.0
+    h[:, 9] *= outlier
+    w[9] = 0.0
+    ds[:, 40] *= outlier
+    w[:, 40] = 0.0
+    picks = torch.arange(64, 64 + 32, device="cuda")
+    w[:, picks] = 0.0
+    w[10 + torch.arange(32, device="cuda"), picks] = torch.randn(32, device="cuda", generator=g)
+    _assert_products(h, w, ds)
 
 
 @pytest.mark.parametrize("inner", [8, 32, 64, 128])
