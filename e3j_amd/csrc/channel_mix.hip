@@ -11,9 +11,7 @@
 // The backward pass uses the same kernel in the other direction, so the cotangent rows are
 // written once (no zero fill, no additions of per-degree slices).
 #include "common.h"
-#include "split_half.h"
-
-#include <type_traits>
+#include "split_bf16.h"
 
 namespace e3j_amd {
 namespace {
@@ -61,55 +59,33 @@ int launch(const void *src, void *dst, int64_t num_nodes, int32_t rows, int32_t 
 // ---------------------------------------------------------------------------
 // The mixing itself in one launch (float32, 64 or 128 channels): no regrouped copies, no library
 // calls.  A wave takes 32 nodes and one output row (degree l, component m) and runs
-// v_mfma_f32_32x32x16_f16 with the nodes as rows on operands split two ways (see split_half.h): lane t holds, for
+// v_mfma_f32_32x32x16_bf16 with the nodes as rows on operands split three ways (see split_bf16.h): lane t holds, for
 // node t % 32, the 32 consecutive channels 32 (t / 32) .. + 31 of a source row (the row of a node is read by
 // sixteen lanes side by side and turned through LDS; with a lane reading its own 128 bytes every access touched 64
 // lines, which the first-level cache does not hold until the next one), and step s of the product takes
 // channels 32 (t / 32) + 8 s .. + 7 from every lane; the second operand is the matching piece of a weight column.
 // The waves of a block work on one output row and share its weights through LDS, 64 summed channels (a chunk) at a
-// time, each wave splitting a fourth of the columns.  A scale belongs to the row of a node or to a column of the
-// weights within a chunk; the sums of a chunk are scaled back and added in float32.  A chunk with an infinity, a NaN or
-// values near the ends of the range (found by the exponent of its scale) runs on v_mfma_f32_32x32x2_f32 from memory.
+// time, each wave splitting a fourth of the columns.  A tile with a value that does not split (an infinity, a NaN, bits
+// below the smallest bfloat16) is summed again on v_mfma_f32_32x32x2_f32 from memory, behind everything else: as a
+// branch in each chunk it took the registers that the loads on their way need (200 bytes of scratch at 128 channels).
+// For the same reason the loads past the last chunk read it again instead of being left out.
 // Forward: the products of the mul copies of the degree accumulate into one output row.  Backward (weights
 // transposed by the caller): the cotangent row is read once and gives one product per copy.
 // At 128 channels a block of the backward makes 64 output channels: the operand of both chunks of a row stays in
-// registers (with the sums of 128 channels beside it they spilled, and a spill waits for every load in flight: 168 us
-// for 114 below), and the cotangent rows that are read twice are few.  A forward block makes all: with 64 the source
-// rows are read and split twice (130 -> 165 us, though 200 nodes 52 -> 42).
-// Bound by the stream and, in a block's chain of chunks, by latency: 99 rows to 16, 6 000 nodes, 64 channels: 57 -> 47 us
-// forward and 63 -> 39 backward where float32 products took 32 and the stream takes 35; 128 channels 222 -> 130 and
-// 231 -> 114 (stream 70), 20 000 nodes 577 -> 376 and 584 -> 364, 200 nodes 66 -> 52 and 68 -> 27 (64 channels
-// there: 21 -> 22 and 22 -> 15).  Error against float64 over normal values, rms: 0.35 to 0.8 times that of float32
+// registers, and the cotangent rows that are read twice are few.  A forward block makes all.
+// Bound by the stream and, in a block's chain of chunks, by latency: 99 rows to 16, 6 000 nodes, 64 channels: 55 -> 42 us
+// forward and 63 -> 38 backward where float32 products took 32 and the stream takes 35; 128 channels 225 -> 155 and
+// 231 -> 134 (stream 70), 20 000 nodes 569 -> 467 and 578 -> 427, 200 nodes 66 -> 62 and 68 -> 28 (64 channels
+// there: 21 -> 22 and 22 -> 16).  Error against float64 over normal values, rms: 0.76 to 0.85 times that of float32
 // products (fewer additions).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMixDegrees = 8;
 constexpr int kMixWaves = 4;  // waves per block, 32 nodes each, on one output row
-constexpr int kMixExponents = 90;  // a scale outside 2^-90 .. 2^90 (no number, or next to the ends of the range) is not used
 struct MixShape {
     int32_t degrees;
     int32_t mul[kMixDegrees], dim[kMixDegrees];
 };
-
-// the exponent of the scale of terms with largest value m, 0 without terms
-__device__ __forceinline__ int mix_exponent(float m) { return m == 0.f ? 0 : scale_exponent(m); }
-__device__ __forceinline__ bool odd_exponent(int k) { return k < -kMixExponents || k > kMixExponents; }
-
-// the largest of the values of the lanes t, t + EVERY, t + 2 EVERY .. (modulo the wave) in each of them
-template <int EVERY>
-__device__ __forceinline__ float largest_over(float m) {
-    auto rotated = [](float v, auto control) {
-        return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(control)::value, 0xf, 0xf, false));
-    };
-    if (EVERY <= 4) m = fmaxf(m, rotated(m, std::integral_constant<int, 0x124>{}));  // by 4, by 8 of sixteen lanes
-    if (EVERY <= 8) m = fmaxf(m, rotated(m, std::integral_constant<int, 0x128>{}));
-    if (EVERY <= 16) {
-        const auto pair = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-        m = fmaxf(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
-    }
-    const auto pair = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
-    return fmaxf(__uint_as_float(pair[0]), __uint_as_float(pair[1]));
-}
 
 template <int K, bool kTranspose>
 __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
@@ -120,14 +96,11 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
     const int lane = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(threadIdx.y), r = lane & 31, h = lane >> 5;
     constexpr int ROWS = KO / 16;              // weights: a thread stages ROWS rows of four columns,
     constexpr int GROUPS = KO / kMixWaves / 4;  //   GROUPS lanes side by side the columns of their wave
-    constexpr bool kTight = K == 64 && !kTranspose;  // (a spilled register waits for every load in flight)
-    constexpr int WEIGHT_PITCH = 64 + 8;       // halves a column (16-byte reads of 32 columns spread over the banks)
-    constexpr int PITCH = 64 + 4;              // (16-byte reads of 64 rows side by side spread over the banks)
-    __shared__ __attribute__((aligned(16))) _Float16 weights[2][KO * WEIGHT_PITCH];
+    constexpr int WEIGHT_PITCH = 64 + 8;       // bfloat16 values a column (16-byte reads of 32 columns spread over the banks)
+    constexpr int PITCH = 32 + 4;              // (16-byte reads of 64 rows side by side spread over the banks)
+    __shared__ __attribute__((aligned(16))) uint16_t weights[3][KO * WEIGHT_PITCH];
     __shared__ __attribute__((aligned(16))) float rows[kMixWaves][32 * PITCH];
-    __shared__ __attribute__((aligned(16))) float row_scale[kMixWaves][KC][32];  // 2^-k of rows and columns
-    __shared__ float col_scale[KO];
-    __shared__ int odd_weights;                // set for good by a chunk with a scale that is not used
+    __shared__ int odd_weights;                // set for good by a chunk whose weights do not split
     // (the waves of a block take neighbouring tiles of one output row; tiles past the last one run along)
     const int64_t row_blocks = (num_nodes + 32 * kMixWaves - 1) / (32 * kMixWaves);
     const int64_t block = blockIdx.x / (K / KO);
@@ -163,32 +136,34 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
             piece[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                 buffer, at + 16 * i * node_stride, 0, 0));
     };
-    // returns whether a row has a scale that is not used
-    auto turn_rows = [&](const f32x4 (&piece)[8], Split2 (&a)[4], float (&scales)[32]) {
+    // returns whether there is a value that does not split
+    auto turn_rows = [&](const f32x4 (&piece)[8], Split3 (&a)[4]) {
         float *mine = rows[wave];
+        uint32_t lost = 0;
 #pragma unroll
-        for (int i = 0; i < 8; i++)
-            *reinterpret_cast<f32x4 *>(mine + (4 * i + lane / 16) * PITCH + lane % 16 * 4) = piece[i];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        float x[4][8];
-        float most = 0.f;
+        for (int half = 0; half < 2; half++) {  // sixteen channels of each lane half at a time: 18 KB a block, not 35
+            if (lane / 4 % 2 == half) {
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-#pragma unroll
-            for (int j = 0; j < 8; j += 4) {
-                const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + r * PITCH + 32 * h + 8 * q + j);
-                x[q][j] = v.x; x[q][j + 1] = v.y; x[q][j + 2] = v.z; x[q][j + 3] = v.w;
+                for (int i = 0; i < 8; i++)
+                    *reinterpret_cast<f32x4 *>(mine + (4 * i + lane / 16) * PITCH + lane / 8 % 2 * 16 + lane % 4 * 4) = piece[i];
             }
-            most = fmaxf(most, max_abs(x[q]));
-        }
-        const int k = mix_exponent(largest_over<32>(most));
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-        for (int q = 0; q < 4; q++) a[q] = split2(x[q], pow2(k));
-        if (h == 0) scales[r] = pow2(-k);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        return __any(odd_exponent(k)) != 0;
+            for (int q = 0; q < 2; q++) {
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; j += 4) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + r * PITCH + 16 * h + 8 * q + j);
+                    x[j] = v.x; x[j + 1] = v.y; x[j + 2] = v.z; x[j + 3] = v.w;
+                }
+                a[2 * half + q] = split3_nearest(x, lost);
+                asm volatile("" : "+v"(lost));  // (one value is kept, not those that it was made of)
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+        return __any(lost != 0) != 0;
     };
     auto store_tile = [&](const f32x16 (&acc)[KT], float *row0, uint32_t node_stride) {
         const auto buffer = tile_rows(row0 + out0, node_stride, KO);
@@ -203,6 +178,10 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
     };
     f32x16 acc[KT];
     const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto clear = [&]() {
+#pragma unroll
+        for (int ct = 0; ct < KT; ct++) acc[ct] = zero;
+    };
     // One chunk of 64 summed channels: its weight rows lie in LDS for the waves of the block, those of
     // the next chunk are on their way while the products of this one run.
     const float *wl = w + wbase + out0;
@@ -217,91 +196,72 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
             staged[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                 buffer, ((k0 + i) * K + col0) * 4, 0, 0));
     };
-    typedef _Float16 Halves __attribute__((ext_vector_type(ROWS)));
+    typedef uint32_t Pairs __attribute__((ext_vector_type(ROWS / 2)));  // ROWS bfloat16 values
     struct Weights {
-        Halves term[2][4];
-        int exponent[4];
+        Pairs term[3][4];
+        uint32_t lost;
     };
     auto split_weights = [&]() {
         Weights out;
+        out.lost = 0;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            float most = 0.f;
+            float rest[ROWS];
 #pragma unroll
-            for (int i = 0; i < ROWS; i++) most = fmaxf(most, fabsf(staged[i][c]));
-            out.exponent[c] = mix_exponent(largest_over<GROUPS>(most));
-            const float scale = pow2(out.exponent[c]);
+            for (int i = 0; i < ROWS; i++) rest[i] = staged[i][c];
 #pragma unroll
-            for (int i = 0; i < ROWS; i++) {  // see split2
-                out.term[0][c][i] = (_Float16)(staged[i][c] * scale);
-                out.term[1][c][i] = (_Float16)__builtin_fmaf(staged[i][c], scale, -(float)out.term[0][c][i]);
-            }
+            for (int u = 0; u < 3; u++)
+#pragma unroll
+                for (int i = 0; i < ROWS; i += 2) out.term[u][c][i / 2] = take_nearest(rest[i], rest[i + 1]);  // see split3_nearest
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) out.lost |= __float_as_uint(rest[i]);
+            asm volatile("" : "+v"(out.lost));
+            __builtin_amdgcn_sched_barrier(0);
         }
         return out;
     };
     auto commit = [&](const Weights &split) {
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int u = 0; u < 2; u++)
-                *reinterpret_cast<Halves *>(&weights[u][(col0 + c) * WEIGHT_PITCH + k0]) = split.term[u][c];
-            if (lane / GROUPS == 0) col_scale[col0 + c] = pow2(-split.exponent[c]);
-            if (odd_exponent(split.exponent[c])) odd_weights = 1;
-        }
+            for (int u = 0; u < 3; u++)
+                *reinterpret_cast<Pairs *>(&weights[u][(col0 + c) * WEIGHT_PITCH + k0]) = split.term[u][c];
+        if (split.lost != 0) odd_weights = 1;
     };
-    // `first`, node_stride: the source rows of the chunk, `q`: the chunk of weights
-    auto products = [&](const Split2 (&a)[4], const float (&scales)[32], bool odd, const float *first,
-                        uint32_t node_stride, int q) {
-        if (odd || odd_weights != 0) {
-            const auto buffer = tile_rows(first, node_stride, 64);
-            const float *wk = wl + ((int64_t)q * 64 + 32 * h) * K + r;
-#pragma unroll 1
-            for (int s = 0; s < 32; s++) {
-                const float x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    buffer, (r * node_stride + 32 * h + s) * 4u, 0, 0));
-#pragma unroll
-                for (int ct = 0; ct < KT; ct++)
-                    acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, wk[s * K + ct * 32], acc[ct], 0, 0, 0);
-            }
-            return;
-        }
-        constexpr int TILES = kTight ? 1 : 2;
+    auto products = [&](const Split3 (&a)[4]) {
+        constexpr int TILES = 2;
 #pragma unroll
         for (int c0 = 0; c0 < KT; c0 += TILES) {
-            f32x16 d[TILES];
-#pragma unroll
-            for (int i = 0; i < TILES; i++) d[i] = zero;
 #pragma unroll
             for (int s = 0; s < 4; s++) {
-                f16x8 b[TILES][2];
+                bf16x8 b[TILES][3];
 #pragma unroll
                 for (int i = 0; i < TILES; i++)
 #pragma unroll
-                    for (int u = 0; u < 2; u++)
-                        b[i][u] = *reinterpret_cast<const f16x8 *>(
+                    for (int u = 0; u < 3; u++)
+                        b[i][u] = *reinterpret_cast<const bf16x8 *>(
                             &weights[u][((c0 + i) * 32 + r) * WEIGHT_PITCH + 32 * h + 8 * s]);
 #pragma unroll
-                for (int u = 0; u < 3; u++)
+                for (int u = 0; u < 6; u++)
 #pragma unroll
                     for (int i = 0; i < TILES; i++)
-                        d[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s].term[kPairs[u][0]], b[i][kPairs[u][1]], d[i], 0, 0, 0);
-                if (kTight || s % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                        acc[c0 + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s].term[kPairs[u][0]], b[i][kPairs[u][1]],
+                                                                              acc[c0 + i], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);  // (the operands of one step at a time in registers)
             }
-            // (two operands of a tile of columns or four scales at a time in registers)
-            float col[TILES];
+        }
+    };
+    // chunk `q` of the weights in float32; `first`, node_stride: its source rows
+    auto plain_products = [&](const float *first, uint32_t node_stride, int q) {
+        const auto buffer = tile_rows(first, node_stride, 64);
+        const float *wk = wl + ((int64_t)q * 64 + 32 * h) * K + r;
+#pragma unroll 1
+        for (int s = 0; s < 32; s++) {
+            const float x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                buffer, (r * node_stride + 32 * h + s) * 4u, 0, 0));
 #pragma unroll
-            for (int i = 0; i < TILES; i++) col[i] = col_scale[(c0 + i) * 32 + r];
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                if (v % 4 == 0) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-#pragma unroll
-                for (int i = 0; i < TILES; i++)
-                    acc[c0 + i][v] = __builtin_fmaf(d[i][v] * scales[8 * (v / 4) + 4 * h + v % 4], col[i], acc[c0 + i][v]);
-            }
-            __builtin_amdgcn_sched_barrier(0);
+            for (int ct = 0; ct < KT; ct++)
+                acc[ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, wk[s * K + ct * 32], acc[ct], 0, 0, 0);
         }
     };
     // after the products of a chunk: its weights make room for those of the next
@@ -320,45 +280,56 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
     commit(split_weights());
     f32x4 piece[8];
     if (!kTranspose) {
-#pragma unroll
-        for (int ct = 0; ct < KT; ct++) acc[ct] = zero;
+        clear();
         // the source row of the next chunk is read while the products of the one at hand run
         auto row_of = [&](int q) { return src + (int64_t)(zbase + q / KC * dim + m) * K + q % KC * 64; };
         fetch_rows(row_of(0), plain_stride, piece);
         __syncthreads();
+        bool odd = false;
         for (int q = 0; q < chunks; q++) {
-            Split2 a[4];
-            const bool odd = turn_rows(piece, a, row_scale[wave][0]);
+            Split3 a[4];
+            odd |= turn_rows(piece, a);
             __builtin_amdgcn_sched_barrier(0);
-            if (q + 1 < chunks) {
-                fetch(q + 1);
-                fetch_rows(row_of(q + 1), plain_stride, piece);
-            }
-            products(a, row_scale[wave][0], odd, row_of(q), plain_stride, q);
+            const int next = min(q + 1, chunks - 1);  // (past the last chunk: it again)
+            fetch(next);
+            fetch_rows(row_of(next), plain_stride, piece);
+            products(a);
             next_chunk(q + 1);
+        }
+        if (odd || odd_weights != 0) {
+            clear();
+            for (int q = 0; q < chunks; q++) plain_products(row_of(q), plain_stride, q);
         }
         store_tile(acc, dst + (int64_t)xr * K, mixed_stride);
     } else {
-        Split2 a[KC][4];
-        bool odd[KC];
+        Split3 a[KC][4];
+        bool odd = false;
 #pragma unroll
         for (int kc = 0; kc < KC; kc++) {
             fetch_rows(src + (int64_t)xr * K + kc * 64, mixed_stride, piece);
-            odd[kc] = turn_rows(piece, a[kc], row_scale[wave][kc]);
+            odd |= turn_rows(piece, a[kc]);
             __builtin_amdgcn_sched_barrier(0);
         }
         __syncthreads();
         for (int u = 0; u < mul; u++) {
-#pragma unroll
-            for (int ct = 0; ct < KT; ct++) acc[ct] = zero;
+            clear();
 #pragma unroll
             for (int kc = 0; kc < KC; kc++) {
                 const int q = u * KC + kc;
-                if (q + 1 < chunks) fetch(q + 1);
-                products(a[kc], row_scale[wave][kc], odd[kc], src + (int64_t)xr * K + kc * 64, mixed_stride, q);
+                fetch(min(q + 1, chunks - 1));
+                products(a[kc]);
                 next_chunk(q + 1);
             }
             store_tile(acc, dst + (int64_t)(zbase + u * dim + m) * K, plain_stride);
+        }
+        if (odd || odd_weights != 0) {
+            __threadfence();  // (these stores come after those)
+            for (int u = 0; u < mul; u++) {
+                clear();
+#pragma unroll 1
+                for (int kc = 0; kc < KC; kc++) plain_products(src + (int64_t)xr * K + kc * 64, mixed_stride, u * KC + kc);
+                store_tile(acc, dst + (int64_t)(zbase + u * dim + m) * K, plain_stride);
+            }
         }
     }
 }

@@ -40,6 +40,33 @@ __device__ __forceinline__ Split3 split3(const float (&x)[8]) {
     }
     return out;
 }
+// The same with every part rounded to the nearest bfloat16: what is left out of a product is then 2^-26 of it and of
+// either sign.  The last bits below the smallest bfloat16, infinities, NaN and what rounds to an infinity do not
+// split: `lost` is then not zero.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t take_nearest(float &x, float &y) {
+    const uint32_t both = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+    x -= __uint_as_float(both << 16);
+    y -= __uint_as_float(both & 0xffff0000u);
+    return both;
+}
+__device__ __forceinline__ Split3 split3_nearest(const float (&x)[8], uint32_t &lost) {
+    Split3 out;
+    float rest[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) rest[m] = x[m];
+#pragma unroll
+    for (int t = 0; t < 3; t++) {
+        u32x4 packed;
+#pragma unroll
+        for (int m = 0; m < 8; m += 2) packed[m / 2] = take_nearest(rest[m], rest[m + 1]);
+        out.term[t] = __builtin_bit_cast(bf16x8, packed);
+    }
+#pragma unroll
+    for (int m = 0; m < 8; m++) lost |= __float_as_uint(rest[m]);
+    return out;
+}
 // the partial products, smallest first
 constexpr int kPairs[6][2] = {{0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};
 

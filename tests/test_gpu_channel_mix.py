@@ -1,5 +1,5 @@
-"""`ChannelMix` in the matrix-core kernel: sums of products split two ways against float64, tile and chunk edges,
-scales that follow rows, columns and chunks, and values that are no numbers."""
+"""`ChannelMix` in the matrix-core kernel: sums of split products against float64, tile and chunk edges, values whose
+sizes differ from row to row, along the sums and against each other, and values that are no numbers."""
 
 import numpy as np
 import pytest
@@ -30,15 +30,16 @@ def _problem(n, blocks, K, seed=0):
 
 
 def _bound(got, want, sizes):
-    """Three in 2^24 of a term (2^-23 lost of a factor at most, the product of the low parts) and a rounding of 2^-24
-    per addition; `sizes`: the same sums of the terms' magnitudes, `terms` of them through at most 60 additions."""
+    """Six in 2^24 of a term (its six partial products are added in float32, what is left out is 2^-26 of it) and a
+    rounding of 2^-24 per addition; `sizes`: the same sums of the terms' magnitudes, `terms` of them through at most 60 additions."""
     return np.abs(got - want) <= (6 + 60) * 2.0 ** -24 * sizes
 
 
 @pytest.mark.parametrize("K", [64, 128])
 @pytest.mark.parametrize("n,blocks", [(1, [(1, 1)]), (31, [(2, 1), (1, 3)]), (33, [(1, 1), (3, 5)]), (127, [(1, 1)]),
                                       (129, [(4, 1), (7, 3)])])
-@pytest.mark.parametrize("scales", ["one", "rows", "columns", "chunks"])
+@pytest.mark.parametrize("scales", ["one", "rows", "columns", "chunks", "opposed 8", "opposed 14", "opposed 20",
+                                    "opposed 40"])
 def test_against_float64(K, n, blocks, scales):
     out, dx, weights = _problem(n, blocks, K)
     if scales == "rows":         # nodes 2^60 apart, and a node of zeros
@@ -52,11 +53,49 @@ def test_against_float64(K, n, blocks, scales):
         weights = [w * 2.0 ** (np.arange(w.shape[0]) * 12)[:, None, None] for w in weights]
         out[..., K // 2:] *= 2.0 ** 20
         dx[..., K // 2:] *= 2.0 ** -20
+    elif scales.startswith("opposed"):   # terms of a size, whose factors differ by orders of magnitude along both sums
+        rng, bits = np.random.default_rng(n), int(scales.split()[1])
+        plain, mixed = (2.0 ** rng.integers(-bits, bits + 1, K) for _ in range(2))
+        out, dx = out * plain, dx * mixed
+        weights = [w / plain[None, :, None] / mixed[None, None, :] for w in weights]
     x, g = _run(out, blocks, K, weights, dx)
     sizes = E.channel_mix(np.abs(out), blocks, [np.abs(w) for w in weights])
     assert _bound(x, E.channel_mix(out, blocks, weights), sizes).all()
     sizes = E.channel_mix_vjp(np.abs(dx), blocks, [np.abs(w) for w in weights])
     assert _bound(g, E.channel_mix_vjp(dx, blocks, weights), sizes).all()
+
+
+@pytest.mark.parametrize("K", [64, 128])
+def test_weights_that_pick_one_channel(K):
+    """One term a sum, beside channels of any size: the six partial products of that term, added in float32, and 2^-26
+    of it left out."""
+    blocks, n = [(1, 1), (1, 3)], 70
+    out, dx, weights = _problem(n, blocks, K)
+    out *= 2.0 ** np.random.default_rng(0).integers(-60, 61, K)
+    dx *= 2.0 ** np.random.default_rng(1).integers(-60, 61, K)
+    weights = [np.where(np.eye(K)[None] > 0, w, 0.0) for w in weights]
+    x, g = _run(out, blocks, K, weights, dx)
+    for got, want in ((x, E.channel_mix(out, blocks, weights)), (g, E.channel_mix_vjp(dx, blocks, weights))):
+        assert (np.abs(got - want) <= 6.25 * 2.0 ** -24 * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("small", ["row", "weights"])
+def test_operands_whose_last_bits_leave_the_range_of_a_part(K, small):
+    """Near 2^-120 the lowest of three bfloat16 parts would lie below the smallest bfloat16."""
+    blocks, n = [(2, 1)], 40
+    out, dx, weights = _problem(n, blocks, K)
+    if small == "row":
+        out[7, :, K // 2:] *= 2.0 ** -121
+        out[7, :, :K // 2], dx[7] = 0.0, dx[7] * 2.0 ** -120
+    else:
+        weights = [w * 2.0 ** -120 for w in weights]
+    out, dx, weights = (np.asarray(a, np.float32).astype(np.float64) for a in (out, dx, weights[0]))
+    x, g = _run(out, blocks, K, [weights], dx)
+    sizes = E.channel_mix(np.abs(out), blocks, [np.abs(weights)])
+    assert _bound(x, E.channel_mix(out, blocks, [weights]), sizes).all()
+    sizes = E.channel_mix_vjp(np.abs(dx), blocks, [np.abs(weights)])
+    assert _bound(g, E.channel_mix_vjp(dx, blocks, [weights]), sizes).all()
 
 
 @pytest.mark.parametrize("K", [64, 128])
