@@ -826,8 +826,8 @@ class _ConvolutionBwd(torch.autograd.Function):
         meta = ctx.meta
 
         graph = ctx.graph
-        if not torch.is_grad_enabled() and not _under_transform():
-            # nothing is recorded for a further derivative: all terms in one call where a kernel takes them
+        if not _followed():
+            # no further derivative of the results: all terms in one call where a kernel takes them
             grads = _raw_second(meta, x, y, s, dm, ddx, ddy, dds, sender, receiver, graph)
             if grads is not None:
                 return *grads, None, None, None, None
@@ -897,8 +897,8 @@ def _apply_bwd(*args):
 
 
 def _backward(x, y, s, dm, sender, receiver, meta, graph, need_dx):
-    """`(dx, dy, ds)` of a backward pass; dx may be None where nobody asks for it and nothing is recorded."""
-    if need_dx or torch.is_grad_enabled() or _under_transform():
+    """`(dx, dy, ds)` of a backward pass; dx may be None where nobody asks for it and nothing follows the call."""
+    if need_dx or _followed():
         return _apply_bwd(x, y, s, dm, sender, receiver, meta, graph)
     if graph is None:
         graph = _forward_graph(meta, sender, receiver, build=False)
@@ -922,6 +922,12 @@ def _make_meta(coef, x, y, s, params, graph_ordering, y_parity, layout) -> _Meta
 
 def _under_transform() -> bool:
     return torch._C._functorch.peek_interpreter_stack() is not None
+
+
+def _followed() -> bool:
+    """Whether something may follow the tensors of a call that only an autograd function shows them to: a recorded
+    graph, a `torch.func` transform, a level of forward-mode derivatives."""
+    return torch.is_grad_enabled() or _under_transform() or torch.autograd.forward_ad._current_level >= 0
 
 
 def _canonical(x, y, s, layout: Layout):
