@@ -52,6 +52,10 @@ struct Library {
     decltype(&e3j_amd_tile_schedule_build) tile_schedule_build = nullptr;
 } lib;
 
+// the number of the settings in force (`options.config.number`)
+const int64_t *settings_number = nullptr;
+int64_t settings_now() { return __atomic_load_n(settings_number, __ATOMIC_RELAXED); }
+
 // A Python object that may be dropped from any thread, with or without the interpreter's lock.
 class Held {
 public:
@@ -264,6 +268,7 @@ struct Call : torch::CustomClassHolder {
     std::shared_ptr<Plan> plan;
     std::shared_ptr<Adjacency> graph;
     at::Tensor sender, receiver;
+    int64_t settings = 0;               // of the forward call: its plan's
     Held handle;                        // the caller's `PreparedGraph`, if there is one
     std::optional<e3j_amd_tile_schedule> handle_schedule;  // its schedule, if it was built before the call
     Held schedule_owner;                // (the memory of that schedule)
@@ -288,7 +293,8 @@ py::object python_graph(Call &call) {  // with the interpreter's lock held
     return made;
 }
 
-// The Python operators' backward: for derivatives of derivatives, under transforms, and wherever something is unusual
+// The Python operators' backward: for derivatives of derivatives, under transforms, under other settings than the
+// forward call's (a backward follows the settings it runs under), and wherever something is unusual
 // or failed (the call is then made again there and raises what it raises).
 variable_list python_backward(Call &call, const at::Tensor &x, const at::Tensor &y, const at::Tensor &s, const at::Tensor &dm,
                               bool need_dx) {
@@ -327,7 +333,8 @@ struct Convolution : torch::autograd::Function<Convolution> {
                                                              : std::vector<int64_t>{g.num_nodes, plan.params.channels, plan.params.num_out};
         at::Tensor dm = cotangents[0].defined() ? cotangents[0] : at::zeros(out_shape, on(plan.device, plan.type));
         variable_list grads;
-        if (c10::GradMode::is_enabled() || !plain_context() || !native(plan, g, *call, x, y, s, dm, out_shape, ctx->needs_input_grad(0), grads))
+        const bool plain = !c10::GradMode::is_enabled() && settings_now() == call->settings && plain_context();
+        if (!plain || !native(plan, g, *call, x, y, s, dm, out_shape, ctx->needs_input_grad(0), grads))
             grads = python_backward(*call, x, y, s, dm, ctx->needs_input_grad(0));
         return {grads[0], grads[1], grads[2], at::Tensor()};
     }
@@ -384,10 +391,10 @@ bool is_tensor(const py::object &o) {
 }
 
 // One call of the operator; None where it is not the plain one.  `kept`: the adjacency of `handle`, both None
-// for a call that prepares its own.
+// for a call that prepares its own; `settings`: the number of those that `plan` is for.
 py::object call(const std::shared_ptr<Plan> &plan, const py::object &x_, const py::object &y_, const py::object &s_,
                 const py::object &sender_, const py::object &receiver_, const std::shared_ptr<Adjacency> &kept,
-                const py::object &handle, const py::object &schedule) {
+                const py::object &handle, const py::object &schedule, int64_t settings) {
     for (const py::object *o : {&x_, &y_, &s_, &sender_, &receiver_})
         if (!is_tensor(*o)) return py::none();
     const at::Tensor &x = THPVariable_Unpack(x_.ptr()), &y = THPVariable_Unpack(y_.ptr()), &s = THPVariable_Unpack(s_.ptr());
@@ -402,6 +409,7 @@ py::object call(const std::shared_ptr<Plan> &plan, const py::object &x_, const p
     c10::intrusive_ptr<Call> state;
     if (record) {
         state = c10::make_intrusive<Call>();
+        state->settings = settings;
         if (!handle.is_none()) state->handle.set(handle);
         if (!schedule.is_none()) {
             e3j_amd_tile_schedule t{};
@@ -469,7 +477,8 @@ void take(const py::dict &d, const char *name, F &slot) {
 }  // namespace
 
 PYBIND11_MODULE(_operators, m) {
-    m.def("bind", [](const py::dict &d) {
+    m.def("bind", [](const py::dict &d, uintptr_t number) {
+        settings_number = reinterpret_cast<const int64_t *>(number);
         take(d, "e3j_amd_prepare_rows", lib.prepare_rows);
         take(d, "e3j_amd_prepare_rows_workspace_bytes", lib.prepare_rows_workspace_bytes);
         take(d, "e3j_amd_row_segments_max", lib.row_segments_max);

@@ -39,7 +39,8 @@ def load():
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_operators", loader))
         loader.exec_module(module)
         lib = _lib.load()
-        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND})
+        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND},
+                    ctypes.addressof(config.number))
         _module = module
     return _module
 
@@ -101,7 +102,7 @@ def _plan(module, x: torch.Tensor, cfg: Config):
 
 def call(module, x, y, s, sender, receiver, graph):
     """`module`'s convolution of the operands, or None."""
-    cfg = config()
+    cfg, number = config.state
     plans = module._plans   # the settings seen last and their plans
     if plans is None or plans[0] is not cfg:
         sets = module._plan_sets
@@ -125,7 +126,7 @@ def call(module, x, y, s, sender, receiver, graph):
     if plan is False:
         return None
     if graph is None:
-        return _module.call(plan, x, y, s, sender, receiver, None, None, None)
+        return _module.call(plan, x, y, s, sender, receiver, None, None, None, number)
     if not isinstance(graph, ops.PreparedGraph) or graph.ordering != module.graph_ordering or not graph.kept:
         return None
     adjacency = graph.native(plan, module, x, cfg)
@@ -133,4 +134,4 @@ def call(module, x, y, s, sender, receiver, graph):
         return None
     schedule = graph._schedules.get(plan.tile_rows) if plan.tile_rows else None
     graph.ready()
-    return _module.call(plan, x, y, s, sender, receiver, adjacency, graph, schedule)
+    return _module.call(plan, x, y, s, sender, receiver, adjacency, graph, schedule, number)

@@ -10,7 +10,9 @@ library is missing.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import dataclasses
+import itertools
 import os
 from enum import Enum
 
@@ -135,7 +137,11 @@ class _ConfigHolder:
     """Mutable process-wide holder with `use(**kw)` scoping (`src/e3j/utils/config.py:107-216`)."""
 
     def __init__(self):
-        self._current = Config(
+        #: the number of the settings in force: every change of them counts on, the end of a `use` takes the number
+        #: from before it.  In memory of its own, where native code reads it without the interpreter.
+        self.number = ctypes.c_int64(0)
+        self._numbers = itertools.count(1)
+        self._enter(Config(
             debug_level=int(os.environ.get("E3J_AMD_DEBUG", "0")),
             deterministic=os.environ.get("E3J_AMD_DETERMINISTIC", "0") not in ("0", ""),
             locality_rounds=int(os.environ.get("E3J_AMD_LOCALITY_ROUNDS", "2")),
@@ -146,12 +152,17 @@ class _ConfigHolder:
                                                              "prepared"),
             graph_cache=os.environ.get("E3J_AMD_GRAPH_CACHE", "0") not in ("0", ""),
             jit=os.environ.get("E3J_AMD_JIT", "0") not in ("0", ""),
-        )
+        ))
+
+    def _enter(self, settings: Config, number: int | None = None):
+        #: the settings in force and their number
+        self.state = (settings, next(self._numbers) if number is None else number)
+        self.number.value = self.state[1]
 
     def __call__(self, **updates) -> Config:
         if updates:
-            self._current = self._coerce(updates)
-        return self._current
+            self._enter(self._coerce(updates))
+        return self.state[0]
 
     def _coerce(self, updates) -> Config:
         fields = {f.name for f in dataclasses.fields(Config)}
@@ -162,20 +173,20 @@ class _ConfigHolder:
             updates["layout"] = Layout.parse(updates["layout"])
         if "convolution" in updates:
             updates["convolution"] = Convolution.parse(updates["convolution"])
-        return dataclasses.replace(self._current, **updates)
+        return dataclasses.replace(self.state[0], **updates)
 
     @contextlib.contextmanager
     def use(self, **updates):
-        previous = self._current
-        self._current = self._coerce(updates)
+        previous = self.state
+        self._enter(self._coerce(updates))
         try:
-            yield self._current
+            yield self.state[0]
         finally:
-            self._current = previous
+            self._enter(*previous)
 
     def snapshot(self, config: Config | None = None) -> Config:
         """Modules freeze the settings they were built under."""
-        return self._current if config is None else config
+        return self.state[0] if config is None else config
 
 
 config = _ConfigHolder()

@@ -1,6 +1,7 @@
 """The native call of a module (`e3j_amd/native.py`) against the Python operators it stands in for: the same
 library calls, hence the same bits where the kernels have a fixed order, and the same derivatives, routes and errors."""
 
+import contextlib
 import copy
 import threading
 
@@ -8,7 +9,7 @@ import pytest
 import torch
 
 import e3j_amd
-from e3j_amd import native, ops
+from e3j_amd import _lib, native, ops
 from e3j_amd.options import config
 
 pytestmark = pytest.mark.gpu
@@ -198,6 +199,50 @@ def test_settings(monkeypatch, setting):
         torch.testing.assert_close(got[0], want[0], rtol=1e-5, atol=1e-5)
         got = (want[0], *got[1:])
     _same(got, want, torch.float32)
+
+
+class _Calls:
+    """The library with the names of the entries that the Python operators call on record."""
+
+    def __init__(self, lib):
+        self._lib, self.names = lib, []
+
+    def __getattr__(self, name):
+        if "convolution_bwd" in name:
+            self.names.append(name)
+        return getattr(self._lib, name)
+
+
+@pytest.mark.parametrize("prepared", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_settings_of_the_backward(monkeypatch, dtype, prepared):
+    """The backward follows the settings it runs under, not those of its forward call."""
+    m, xs, sender, receiver, dm = _operands(300, 64, dtype)
+    graph = ops.prepare_graph(sender, receiver, 300) if prepared else None
+    want = _grads(m, xs, sender, receiver, dm, graph)
+    native.load()
+    lib = _Calls(_lib.load())
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    routes = {}
+    for name, setting in (("deterministic", dict(deterministic=True)), ("tiles", dict(tile_rows=0)), ("same", None)):
+        runs = []
+        for _ in range(3):
+            out = m(*xs, sender, receiver, graph=graph)
+            with config.use(**setting) if setting else contextlib.nullcontext():
+                runs.append((out.detach(), *torch.autograd.grad(out, xs, dm)))
+            _same(runs[-1], want, dtype)
+        if name == "deterministic":
+            assert all(torch.equal(a, b) for r in runs[1:] for a, b in zip(r, runs[0]))
+        routes[name] = list(lib.names)
+        lib.names.clear()
+    assert len(routes["deterministic"]) == len(routes["tiles"]) == 3 and not routes["same"]
+    assert not any("tiled" in r for r in routes["deterministic"] + routes["tiles"])
+    # the other way about: a forward pass of its own settings, the backward under the usual ones
+    with config.use(tile_rows=0):
+        m(*xs, sender, receiver, graph=graph)
+        out = m(*xs, sender, receiver, graph=graph)
+    _same((out.detach(), *torch.autograd.grad(out, xs, dm)), want, dtype)
+    assert len(lib.names) == 1
 
 
 def test_streams_and_threads():
