@@ -404,7 +404,10 @@ py::object call(const std::shared_ptr<Plan> &plan, const py::object &x_, const p
     auto index = [&](const at::Tensor &t) {
         return t.device() == plan->device && t.scalar_type() == at::kInt && t.dim() == 1 && t.numel() == e && t.is_contiguous();
     };
-    if (kept ? kept->num_nodes != n || kept->num_edges != e : !index(sender) || !index(receiver)) return py::none();
+    // (a handle's call does not read the endpoints; the operators refuse those outside GPU memory all the same)
+    if (kept ? kept->num_nodes != n || kept->num_edges != e || !sender.is_cuda() || !receiver.is_cuda()
+             : !index(sender) || !index(receiver))
+        return py::none();
     const bool record = c10::GradMode::is_enabled() && (x.requires_grad() || y.requires_grad() || s.requires_grad());
     c10::intrusive_ptr<Call> state;
     if (record) {

@@ -245,6 +245,18 @@ def test_settings_of_the_backward(monkeypatch, dtype, prepared):
     assert len(lib.names) == 1
 
 
+def test_endpoints_beside_a_handle_are_refused_as_often_as_asked():
+    m, xs, sender, receiver, _ = _operands(40, 64)
+    graph = ops.prepare_graph(sender, receiver, 40)
+    for _ in range(3):
+        m(*xs, sender, receiver, graph=graph)
+        for snd, rcv in ((sender.cpu(), receiver), (sender, receiver.cpu())):
+            with pytest.raises(RuntimeError, match="GPU memory"):
+                m(*xs, snd, rcv, graph=graph)
+        with pytest.raises(TypeError, match="sender"):
+            m(*xs, None, receiver, graph=graph)
+
+
 def test_streams_and_threads():
     m, xs, sender, receiver, dm = _operands(400, 64)
     want = _grads(m, xs, sender, receiver, dm)
