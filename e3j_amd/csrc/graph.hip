@@ -50,38 +50,39 @@ __global__ void gather_kernel(const int32_t *__restrict__ src, const int32_t *__
 }
 
 // One sweep of minimum-label propagation over a CSR adjacency:
-// next[n] = min(cur[n], cur[m] for every m in row n).  One thread per row, no atomics.
+// next[n] = min(cur[n], cur[m] for every m in row n), no atomics.
 // A row is read up to kLabelRowCap positions: the labels only steer which rows run together,
 // and a thread that walked a hub's whole row would outlast the rest of the sweep many times.
 constexpr int kLabelRowCap = 128;
 constexpr int kLabelLanes = 16;  // lanes that share a row (its gathers then run sixteen at a time)
+constexpr int64_t kLabelBlocks = 1 << 22;  // (a launch has fewer than 2^32 threads: past 2^26 rows a thread takes several)
 __global__ void min_label_kernel(const int32_t *__restrict__ other,
                                  const int32_t *__restrict__ row_ptr, int num_nodes,
                                  const int32_t *__restrict__ cur, int32_t *__restrict__ next,
                                  uint32_t *__restrict__ keys, int32_t *__restrict__ vals, int bits) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = t / kLabelLanes, part = t % kLabelLanes;
-    const bool inside = n < num_nodes;  // (no early exit: the lanes of a group exchange below)
-    // cur == nullptr: every node still carries its own id (the first sweep)
-    int best = inside ? (cur ? cur[n] : n) : 0;
-    if (inside) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, lanes = (int64_t)num_nodes * kLabelLanes;
+    // (the lanes of a row go round together: they exchange below)
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < lanes; t += stride) {
+        const int n = (int)(t / kLabelLanes), part = (int)(t % kLabelLanes);
+        // cur == nullptr: every node still carries its own id (the first sweep)
+        int best = cur ? cur[n] : n;
         const int begin = row_ptr[n];
         const int end = min(row_ptr[n + 1], begin + kLabelRowCap);
         for (int e = begin + part; e < end; e += kLabelLanes) {
             const int m = other[e];
             if ((unsigned)m < (unsigned)num_nodes) best = min(best, cur ? cur[m] : m);
         }
-    }
 #pragma unroll
-    for (int off = 1; off < kLabelLanes; off *= 2) best = min(best, __shfl_xor(best, off, kWave));
-    if (!inside || part != 0) return;
-    if (keys == nullptr) {
-        next[n] = best;
-    } else {
-        // the last of two sweeps: key = (label after it, label before it); one sort lists the coarse
-        // clusters and, inside them, the fine ones
-        keys[n] = ((uint32_t)best << bits) | (uint32_t)cur[n];
-        if (vals != nullptr) vals[n] = n;
+        for (int off = 1; off < kLabelLanes; off *= 2) best = min(best, __shfl_xor(best, off, kWave));
+        if (part != 0) continue;
+        if (keys == nullptr) {
+            next[n] = best;
+        } else {
+            // the last of two sweeps: key = (label after it, label before it); one sort lists the coarse
+            // clusters and, inside them, the fine ones
+            keys[n] = ((uint32_t)best << bits) | (uint32_t)cur[n];
+            if (vals != nullptr) vals[n] = n;
+        }
     }
 }
 
@@ -1243,7 +1244,7 @@ int locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nod
     int done = 0;
     int label_bits = 1;  // labels are node ids: the sort passes stop at their highest bit
     while (label_bits < 32 && ((int64_t)1 << label_bits) < (int64_t)num_nodes) label_bits++;
-    const unsigned label_grid = (unsigned)(((int64_t)num_nodes * kLabelLanes + 255) / 256);
+    const unsigned label_grid = (unsigned)std::min<int64_t>(((int64_t)num_nodes * kLabelLanes + 255) / 256, kLabelBlocks);
     const bool two_levels = rounds == 2 && 2 * label_bits <= 32;
     if (two_levels) {
         hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from e3j_amd.graph import TileSchedule, prepare_rows
+from e3j_amd.graph import TileSchedule, locality_order, prepare_rows
 
 pytestmark = pytest.mark.gpu
 DUMMY = 2 ** 31 - 1
@@ -159,3 +159,22 @@ def test_edge_sort_against_numpy(n, e, kind):
         np.testing.assert_array_equal(ptr.cpu().numpy(), _rows(k, n))
         np.testing.assert_array_equal(oth.cpu().numpy(), o[want])
         assert order is None
+
+
+def test_row_order_of_more_rows_than_a_sweep_has_threads():
+    """2^27 rows and a few: sixteen lanes a row are more than 2^31, and threads take several rows."""
+    n = (1 << 27) + 9
+    other = torch.arange(n, dtype=torch.int32, device="cuda")
+    row_ptr = torch.arange(n + 1, dtype=torch.int32, device="cuda")
+    # (each row has itself for a neighbour, except three that belong to clusters at the front, one of them two hops away)
+    far = [n - 1, 1 << 27, (1 << 26) + 3]
+    other[far[0]], other[far[1]], other[far[2]] = 5, 100, n - 1
+    order = locality_order(other, row_ptr, n, 2)
+    del other, row_ptr
+    front = [*range(6), far[0], far[2], *range(6, 101), far[1]]   # (labels 5, 5 and 100 after two sweeps)
+    assert order[:len(front)].tolist() == front
+    rest = order[len(front):]
+    want = torch.arange(101, n, dtype=torch.int32, device="cuda")
+    keep = torch.ones(n - 101, dtype=torch.bool, device="cuda")
+    keep[torch.tensor([f - 101 for f in far], device="cuda")] = False
+    assert torch.equal(rest, want[keep])
