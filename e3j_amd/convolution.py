@@ -53,10 +53,13 @@ class Convolution:
         self._mix = mix
         self._coef = None
         self._packed = {}
-        self._plans, self._plan_sets = None, {}   # plans of the native call by settings and kind of operand
+
+    #: plans of the native call by settings and kind of operand, and those of the settings seen last; filled on use,
+    #: also in an object that was unpickled without them
+    _plans = _plan_sets = None
 
     def __getstate__(self):   # (plans hold device memory and are made again on use)
-        return {**self.__dict__, "_plans": None, "_plan_sets": {}}
+        return {k: v for k, v in self.__dict__.items() if k not in ("_plans", "_plan_sets")}
 
     @property
     def coef(self) -> Coef4D:

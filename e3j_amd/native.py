@@ -105,6 +105,8 @@ def call(module, x, y, s, sender, receiver, graph):
     cfg, number = config.state
     plans = module._plans   # the settings seen last and their plans
     if plans is None or plans[0] is not cfg:
+        if module._plan_sets is None:
+            module._plan_sets = {}
         sets = module._plan_sets
         if len(sets) >= 8 and cfg not in sets:
             sets.clear()

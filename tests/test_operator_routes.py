@@ -1,12 +1,13 @@
 """Which way an operator call takes, with the library stubbed: no GPU needed."""
 
+import pickle
 import types
 
 import pytest
 import torch
 from torch.autograd import forward_ad
 
-from e3j_amd import ops
+from e3j_amd import Convolution, ops
 
 
 def _blank(*like):
@@ -39,3 +40,21 @@ def test_a_second_derivative_drops_no_forward_mode_tangent(monkeypatch):
         assert len(ops._ConvolutionBwd.backward(ctx, x, y, s)) == 8
         with forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
             ops._ConvolutionBwd.backward(ctx, forward_ad.make_dual(x, torch.ones_like(x)), y, s)
+
+
+def test_a_module_pickled_without_plans_runs():
+    """As one was before modules kept plans of native calls; and plans do not travel with a module."""
+    module = Convolution(("0e+1o", "0e+1o"), "0e+1o", graph_ordering="RECEIVER")
+    state = {k: v for k, v in vars(module).items() if "plan" not in k}
+    old = pickle.loads(pickle.dumps(module))
+    vars(old).clear()
+    vars(old).update(state)
+    x, index = torch.zeros(2, 4, 8), torch.zeros(3, dtype=torch.int32)
+    operands = x, torch.zeros(3, 4), torch.zeros(3, module.params.num_scalars, 8), index, index
+    for m in (old, module):
+        for _ in range(3):
+            with pytest.raises(RuntimeError, match="GPU memory"):
+                m(*operands)
+    module._plan_sets, module._plans = {"settings": object}, ("settings", {})
+    twin = pickle.loads(pickle.dumps(module))
+    assert twin._plans is None and not twin._plan_sets and twin.params == module.params
