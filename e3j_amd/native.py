@@ -12,6 +12,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import warnings
 
 import torch
 
@@ -45,6 +46,23 @@ def load():
     return _module
 
 
+_missing = False
+
+
+def available():
+    """`load()`'s module; None, said once, where this tree holds none that loads (not built, or built against another
+    torch): the Python operators then make every call, by the same kernels."""
+    global _missing
+    if _module is None and not _missing:
+        try:
+            load()
+        except ImportError as e:
+            _missing = True
+            warnings.warn(f"e3j_amd: calls of small graphs are slower without the native host side ({e})",
+                          RuntimeWarning, stacklevel=2)
+    return _module
+
+
 #: no size reaches this: a route that is never taken
 _NEVER = 1 << 62
 
@@ -63,7 +81,7 @@ def _plan(module, x: torch.Tensor, cfg: Config):
     num_x, channels = (x.shape[1], x.shape[2]) if trailing else (x.shape[2], x.shape[1])
     dims = (int(num_x), int(module.source[1].dim), int(params.num_out), int(params.num_scalars))
     sig, scale, flip = table.signature(dims, int(channels), layout)
-    if sig < 0:
+    if sig < 0 or available() is None:
         return False
     f64 = x.dtype == torch.float64
     p = _lib.ConvParams(

@@ -2,12 +2,13 @@
 
 import pickle
 import types
+import warnings
 
 import pytest
 import torch
 from torch.autograd import forward_ad
 
-from e3j_amd import Convolution, ops
+from e3j_amd import Convolution, native, ops
 
 
 def _blank(*like):
@@ -58,3 +59,20 @@ def test_a_module_pickled_without_plans_runs():
     module._plan_sets, module._plans = {"settings": object}, ("settings", {})
     twin = pickle.loads(pickle.dumps(module))
     assert twin._plans is None and not twin._plan_sets and twin.params == module.params
+
+
+@pytest.mark.parametrize("there", [False, True])
+def test_a_tree_without_its_native_host_side_says_so_once(monkeypatch, tmp_path, there):
+    """Not built, or not a module that loads here."""
+    path = tmp_path / "_operators.so"
+    if there:
+        path.write_bytes(b"of another torch")
+    for name, value in (("LIB_PATH", str(path)), ("_module", None), ("_missing", False)):
+        monkeypatch.setattr(native, name, value)
+    with pytest.warns(RuntimeWarning, match="native host side"):
+        assert native.available() is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert native.available() is None
+    with pytest.raises(ImportError):
+        native.load()
