@@ -195,11 +195,16 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_split_kernel
     }
 }
 
-// Column tiles per block: all of them where the edges alone make a block per compute unit, else ranges of them so
-// that there are about as many (4 099 edges, H = 64, n = 992: 60 -> 11 us; 2 000 edges, H = 128, n = 2 048: 104 -> 13; two
-// blocks per unit: 11 and 13, and 12 000 edges, n = 992: 20 -> 24).
+// Column tiles per block: all of them where the edges alone make a block per compute unit (256), else ranges of them.
+// Up to 128 blocks as many ranges as stay within one block per unit (4 099 edges, H = 64, n = 992: 60 -> 11 us; 2 000
+// edges, H = 128, n = 2 048: 104 -> 13; rounded up instead, 12 000 edges, n = 992: 20 -> 24, some units then have two
+// blocks, every one of which reads its edges' h).  From 129 to 255, where one range leaves up to half of the units idle,
+// two from 24 tiles on (n = 2 944, H = 64, 33 000 edges 175 -> 137 us, 64 000 edges 200 -> 160; H = 32, 33 000 edges
+// 155 -> 128; n = 800, H = 64, 49 -> 46, 128, 45 -> 40); with fewer columns the second reading of h costs more (n = 416,
+// H = 64: 29 -> 32; n = 96: 11 -> 13).
 int column_range(int64_t blocks, int tiles) {
-    const int64_t ranges = std::min<int64_t>(tiles, std::max<int64_t>(1, 256 / blocks));
+    const int64_t most = blocks > 128 && blocks < 256 && tiles >= 24 ? 2 : std::max<int64_t>(1, 256 / blocks);
+    const int64_t ranges = std::min<int64_t>(tiles, most);
     return (int)((tiles + ranges - 1) / ranges);
 }
 

@@ -180,9 +180,9 @@ def test_outliers_that_meet_zeros(inner, outlier):
 
 
 @pytest.mark.parametrize("inner", [8, 32, 64, 128])
-@pytest.mark.parametrize("edges,n", [(5, 2944), (256, 992), (70000, 64)])
+@pytest.mark.parametrize("edges,n", [(5, 2944), (256, 992), (16400, 96), (33000, 736), (33000, 800), (65000, 768), (70000, 64)])
 def test_forward_over_ranges_of_columns(inner, edges, n):
-    """Few edges: blocks share the columns; many: each takes all of them."""
+    """Few edges: blocks share the columns, an odd number of tiles too; many: each takes all of them."""
     g = torch.Generator(device="cuda").manual_seed(inner + edges)
     h = torch.randn(edges, inner, device="cuda", generator=g)
     w = torch.randn(inner, n, device="cuda", generator=g)
