@@ -1,6 +1,7 @@
 """The tiled backward without dx (`e3j_amd_convolution_bwd_tiled_edges`): taken where x needs no gradient, and
 dy and ds are what the kernel with dx gives."""
 
+import contextlib
 import ctypes
 
 import numpy as np
@@ -9,6 +10,7 @@ import torch
 
 import e3j_amd
 from e3j_amd import _lib, native, ops
+from e3j_amd.options import config
 
 pytestmark = pytest.mark.gpu
 
@@ -23,6 +25,29 @@ class _Calls:
         if "convolution_bwd" in name:
             self.names.append(name)
         return getattr(self._lib, name)
+
+
+@contextlib.contextmanager
+def _native_calls():
+    """The names of the tiled backwards that native calls make, which go through a callback to the same entries."""
+    module, lib, names, keep = native.load(), _lib.load(), [], []
+    entries = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in native._BOUND}
+    watched = dict(entries)
+    for name in ("e3j_amd_convolution_bwd_tiled", "e3j_amd_convolution_bwd_tiled_edges"):
+        kind = ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * len(getattr(lib, name).argtypes))
+
+        def through(*args, name=name, entry=kind(entries[name])):
+            names.append(name)
+            return entry(*args)
+
+        keep.append(kind(through))
+        watched[name] = ctypes.cast(keep[-1], ctypes.c_void_p).value
+    number = ctypes.addressof(config.number)
+    module.bind(watched, number)
+    try:
+        yield names
+    finally:
+        module.bind(entries, number)
 
 
 def _operands(n, channels, degree, irreps="0e+1o+2e+3o", dtype=torch.float32, seed=0):
@@ -68,8 +93,8 @@ def test_same_edge_gradients(monkeypatch, n, degree, irreps, channels):
     def near(got, want):
         return float((got - want).abs().max()) <= 64 * 2.0 ** -24 * float(want.abs().max())
 
-    for attempt in range(3):   # (the Python operators, then native calls)
-        for handle in (None, graph):
+    def passes(handles):
+        for handle in handles:
             for operand, wanted in ((x, "ys"), (leaf, "ys"), (x, "s")):   # (x a leaf that nobody asks about, too)
                 got = edges(handle, operand, wanted)
                 assert near(got[-1], ds)
@@ -77,7 +102,18 @@ def test_same_edge_gradients(monkeypatch, n, degree, irreps, channels):
                     assert near(got[0], dy)
                     assert not got[0][sender >= n].any()
                 assert not got[-1][sender >= n].any()
-    assert lib.names.count("e3j_amd_convolution_bwd_tiled") == 0
+
+    form = "e3j_amd_convolution_bwd_tiled_edges"
+    with _native_calls() as names:
+        lib.names.clear()   # (asked for entries, not called)
+        passes((None, graph, None, graph))
+    # (the first backward of a handle makes its schedule, in Python)
+    assert lib.names == [form] and names == [form] * 11
+    lib.names.clear()
+    monkeypatch.setattr(native, "call", lambda *a: None)   # (the Python operators)
+    passes((None, graph))
+    # (a node in Python knows which operands want gradients, not which of them are asked for)
+    assert lib.names == [form, "e3j_amd_convolution_bwd_tiled", form] * 2
 
 
 def test_dx_is_there_when_it_is_asked_for():
