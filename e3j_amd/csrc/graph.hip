@@ -54,26 +54,27 @@ __global__ void gather_kernel(const int32_t *__restrict__ src, const int32_t *__
 // A row is read up to kLabelRowCap positions: the labels only steer which rows run together,
 // and a thread that walked a hub's whole row would outlast the rest of the sweep many times.
 constexpr int kLabelRowCap = 128;
-constexpr int kLabelLanes = 16;  // lanes that share a row (its gathers then run sixteen at a time)
-constexpr int64_t kLabelBlocks = 1 << 22;  // (a launch has fewer than 2^32 threads: past 2^26 rows a thread takes several)
+constexpr int64_t kLabelBlocks = 1 << 20;  // (a launch has fewer than 2^32 threads: past 2^26 rows a thread takes several)
+// kLanes: lanes that share a row (its gathers then run that many at a time), see sweep_labels
+template <int kLanes>
 __global__ void min_label_kernel(const int32_t *__restrict__ other,
                                  const int32_t *__restrict__ row_ptr, int num_nodes,
                                  const int32_t *__restrict__ cur, int32_t *__restrict__ next,
                                  uint32_t *__restrict__ keys, int32_t *__restrict__ vals, int bits) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x, lanes = (int64_t)num_nodes * kLabelLanes;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, lanes = (int64_t)num_nodes * kLanes;
     // (the lanes of a row go round together: they exchange below)
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < lanes; t += stride) {
-        const int n = (int)(t / kLabelLanes), part = (int)(t % kLabelLanes);
+        const int n = (int)(t / kLanes), part = (int)(t % kLanes);
         // cur == nullptr: every node still carries its own id (the first sweep)
         int best = cur ? cur[n] : n;
         const int begin = row_ptr[n];
         const int end = min(row_ptr[n + 1], begin + kLabelRowCap);
-        for (int e = begin + part; e < end; e += kLabelLanes) {
+        for (int e = begin + part; e < end; e += kLanes) {
             const int m = other[e];
             if ((unsigned)m < (unsigned)num_nodes) best = min(best, cur ? cur[m] : m);
         }
 #pragma unroll
-        for (int off = 1; off < kLabelLanes; off *= 2) best = min(best, __shfl_xor(best, off, kWave));
+        for (int off = 1; off < kLanes; off *= 2) best = min(best, __shfl_xor(best, off, kWave));
         if (part != 0) continue;
         if (keys == nullptr) {
             next[n] = best;
@@ -84,6 +85,18 @@ __global__ void min_label_kernel(const int32_t *__restrict__ other,
             if (vals != nullptr) vals[n] = n;
         }
     }
+}
+
+// Sixteen lanes a row up to 2^14 rows, where a hub's row is what a sweep waits for (5 000 rows of 30 with hubs among
+// them: two sweeps 17 -> 10 us); four from there on, where the rows fill the chip and lanes without a position cost
+// (the row order of 1M rows of 4 positions 324 us and 395 with sixteen, of 30 positions 394 and 421, of 100 000 rows of
+// 16 131 and 136; of 300 000 rows of 120 positions 377 and 346).
+void sweep_labels(const int32_t *other, const int32_t *row_ptr, int num_nodes, const int32_t *cur, int32_t *next,
+                  uint32_t *keys, int32_t *vals, int bits, hipStream_t stream) {
+    const bool few = num_nodes <= 1 << 14;
+    const int64_t blocks = std::min<int64_t>(((int64_t)num_nodes * (few ? 16 : 4) + 255) / 256, kLabelBlocks);
+    hipLaunchKernelGGL(few ? min_label_kernel<16> : min_label_kernel<4>, dim3((unsigned)blocks), dim3(256), 0, stream, other,
+                       row_ptr, num_nodes, cur, next, keys, vals, bits);
 }
 
 __global__ void copy_i32_kernel(const int32_t *__restrict__ src, int32_t *__restrict__ dst, int64_t n) {
@@ -1244,14 +1257,11 @@ int locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nod
     int done = 0;
     int label_bits = 1;  // labels are node ids: the sort passes stop at their highest bit
     while (label_bits < 32 && ((int64_t)1 << label_bits) < (int64_t)num_nodes) label_bits++;
-    const unsigned label_grid = (unsigned)std::min<int64_t>(((int64_t)num_nodes * kLabelLanes + 255) / 256, kLabelBlocks);
     const bool two_levels = rounds == 2 && 2 * label_bits <= 32;
     if (two_levels) {
-        hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
-                           static_cast<const int32_t *>(nullptr), lab_b, nullptr, nullptr, 0);
+        sweep_labels(other, row_ptr, num_nodes, nullptr, lab_b, nullptr, nullptr, 0, stream);
         const bool one_block = num_nodes <= 8 * kBlockThreads;
-        hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr, num_nodes,
-                           lab_b, lab_a, keys_in, one_block ? nullptr : order, label_bits);
+        sweep_labels(other, row_ptr, num_nodes, lab_b, lab_a, keys_in, one_block ? nullptr : order, label_bits, stream);
         if (one_block) {
             // (the kernel's time is the instructions of one compute unit, for padded entries too)
             using Launch = int (*)(const uint32_t *, const int32_t *, int, int, int32_t *, int, int, int, int32_t *,
@@ -1281,8 +1291,7 @@ int locality_order(const int32_t *other, const int32_t *row_ptr, int32_t num_nod
     }
     for (int level = 1; level <= rounds; level *= 2) {
         for (; done < level; done++) {
-            hipLaunchKernelGGL(min_label_kernel, dim3(label_grid), dim3(256), 0, stream, other, row_ptr,
-                               num_nodes, lab_a, lab_b, nullptr, nullptr, 0);
+            sweep_labels(other, row_ptr, num_nodes, lab_a, lab_b, nullptr, nullptr, 0, stream);
             int32_t *t = lab_a; lab_a = lab_b; lab_b = t;
         }
         hipLaunchKernelGGL(gather_kernel, dim3(ngrid), dim3(256), 0, stream, lab_a, order,

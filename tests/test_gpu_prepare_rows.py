@@ -161,8 +161,18 @@ def test_edge_sort_against_numpy(n, e, kind):
         assert order is None
 
 
+@pytest.mark.parametrize("kind", ["even", "hub"])
+@pytest.mark.parametrize("n", [16384, 16385])
+def test_row_order_either_side_of_four_lanes_a_row(n, kind):
+    key, other = _graph(n, 5 * n, kind, n)
+    dev = lambda a: torch.from_numpy(a.astype(np.int32)).cuda()  # noqa: E731
+    ptr = _rows(key, n)
+    order = locality_order(dev(other), dev(ptr), n, 2)
+    np.testing.assert_array_equal(order.cpu().numpy(), _order(other, ptr, n))
+
+
 def test_row_order_of_more_rows_than_a_sweep_has_threads():
-    """2^27 rows and a few: sixteen lanes a row are more than 2^31, and threads take several rows."""
+    """2^27 rows and a few: sixteen lanes a row would be more than 2^31, and threads take several rows."""
     n = (1 << 27) + 9
     other = torch.arange(n, dtype=torch.int32, device="cuda")
     row_ptr = torch.arange(n + 1, dtype=torch.int32, device="cuda")
