@@ -496,7 +496,7 @@ __global__ void sort_input_kernel(const int32_t *__restrict__ key, int64_t num_e
     }
 }
 
-// Stable sort of edge positions by key for up to kSortChunk * kSortChunks edges of fewer than 2^16 nodes, in two passes
+// Stable sort of edge positions by key for up to kSortChunk * kSortChunks edges of fewer than 2^16 nodes (`own_sort`), in two passes
 // of at most eight bits, a count and a scatter each: four launches, where the library's sort takes
 // eight and the launch that writes its keys a ninth (150k edges, 5 000 nodes: 58 us -> 20; 3-5 us a launch whatever
 // it moves).  A workgroup takes kSortChunk consecutive edges; the scatter of each adds up for itself how
@@ -1338,9 +1338,12 @@ int e3j_amd_locality_order(const int32_t *other, const int32_t *row_ptr, int32_t
 namespace {
 struct PrepareWorkspace {
     size_t order, sort_temp, sort_bytes, keys_in, keys_out, positions, unsorted, total;
-    // the sort of this file: keys of two eight-bit digits, chunks whose counts a workgroup reads by itself
+    // The sort of this file: keys of two eight-bit digits, and no more chunks than the counts of which a workgroup reads
+    // by itself.  It is the faster one up to there (CSR and sort: 60 000 rows, 262 144 edges 42 us for the library's
+    // 103; 5 000 rows, 150 000 edges 34 for 63; 4 500 edges 26 for 33; 2 000 edges 26 for 28); up to 1 024 edges
+    // the library sorts in one launch (500 edges: 20 us for 25).
     static bool own_sort(int32_t num_nodes, int64_t num_edges) {
-        return num_nodes < (1 << 16) && num_edges <= (int64_t)kSortChunk * kSortChunks;
+        return num_nodes < (1 << 16) && num_edges > 1024 && num_edges <= (int64_t)kSortChunk * kSortChunks;
     }
     PrepareWorkspace(int32_t num_nodes, int64_t num_edges, bool sorted) {
         size_t at = 0;

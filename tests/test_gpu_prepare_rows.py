@@ -142,11 +142,11 @@ def test_schedule_work_and_lists(n, tile_rows):
 
 
 @pytest.mark.parametrize("n,e,kind", [
-    (1, 5, "even"), (2, 4095, "hub"), (3, 4096, "even"), (255, 4097, "even"), (256, 8192, "hub"), (8191, 12289, "hub"),
+    (1, 5, "even"), (300, 1024, "hub"), (300, 1025, "hub"), (2, 4095, "hub"), (3, 4096, "even"), (255, 4097, "even"), (256, 8192, "hub"), (8191, 12289, "hub"),
     (65535, 70001, "even"), (65536, 70001, "even"), (4999, 262144, "hub"), (4999, 262145, "even"), (40000, 262143, "even"),
 ])
 def test_edge_sort_against_numpy(n, e, kind):
-    """Unsorted edges at the sizes where the sort changes: digits of the keys, chunks of 4 096 edges, 64 of
+    """Unsorted edges at the sizes where the sort changes: 1 024 edges, digits of the keys, chunks of 4 096 edges, 64 of
     them, 2^16 nodes; ids of another shard and keys that are sorted already among them."""
     key, other = _graph(n, e, kind, n + e)
     shuffle = np.random.default_rng(e).permutation(e)
