@@ -142,7 +142,10 @@ def call(module, x, y, s, sender, receiver, graph):
         plans[1][key] = True
         return None
     if plan is True:
-        plan = plans[1][key] = _plan(module, x, cfg)
+        plan = _plan(module, x, cfg)
+        if config.state[1] != number:   # (another thread changed the settings under it: the plan may be of both)
+            return None
+        plans[1][key] = plan
     if plan is False:
         return None
     if graph is None:

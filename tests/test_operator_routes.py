@@ -9,6 +9,7 @@ import torch
 from torch.autograd import forward_ad
 
 from e3j_amd import Convolution, native, ops
+from e3j_amd.options import config
 
 
 def _blank(*like):
@@ -76,3 +77,22 @@ def test_a_tree_without_its_native_host_side_says_so_once(monkeypatch, tmp_path,
         assert native.available() is None
     with pytest.raises(ImportError):
         native.load()
+
+
+def test_a_plan_made_while_the_settings_change_is_not_kept(monkeypatch):
+    module = Convolution(("0e+1o", "0e+1o"), "0e+1o", graph_ordering="RECEIVER")
+    x = torch.zeros(2, 4, 64)
+    key, cfg = (x.dtype, x.device, x.shape[1:], module.layout, module.graph_ordering), config()
+    module._plan_sets = {cfg: {key: True}}   # (a call of this kind was made)
+
+    def plan(*args):
+        config(tile_rows=0)   # another thread's
+        return object()
+
+    before = config.state
+    monkeypatch.setattr(native, "_plan", plan)
+    try:
+        assert native.call(module, x, None, None, None, None, None) is None
+    finally:
+        config._enter(*before)
+    assert module._plan_sets[cfg] == {key: True}
