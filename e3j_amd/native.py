@@ -72,7 +72,8 @@ def _plan(module, x: torch.Tensor, cfg: Config):
     ordering, layout = module.graph_ordering, module.layout
     if (x.device.type != "cuda" or x.dtype not in ops._VAL_DTYPES or ordering == GraphOrdering.SENDER
             or cfg.graph_cache or cfg.deterministic or not cfg.fixed_order_rows or cfg.debug_level
-            or cfg.pair_rows is True):
+            or cfg.pair_rows is True
+            or not all(-1 << 31 <= int(v) < 1 << 31 for v in (cfg.row_cap, cfg.locality_rounds, cfg.tile_rows))):
         return False
     code, val_np = ops._VAL_DTYPES[x.dtype]
     coef, params = module._packed_coef(val_np.__name__), module.params

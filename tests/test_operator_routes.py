@@ -9,7 +9,7 @@ import torch
 from torch.autograd import forward_ad
 
 from e3j_amd import Convolution, native, ops
-from e3j_amd.options import config
+from e3j_amd.options import Config, config
 
 
 def _blank(*like):
@@ -96,3 +96,10 @@ def test_a_plan_made_while_the_settings_change_is_not_kept(monkeypatch):
     finally:
         config._enter(*before)
     assert module._plan_sets[cfg] == {key: True}
+
+
+@pytest.mark.parametrize("setting", [dict(row_cap=10 ** 10), dict(locality_rounds=2 ** 31)])
+def test_settings_past_32_bits_are_left_to_the_python_operators(setting):
+    module = Convolution(("0e+1o+2e+3o", "0e+1o+2e+3o"), "0e+1o+2e+3o", graph_ordering="RECEIVER")
+    x = types.SimpleNamespace(dtype=torch.float32, device=torch.device("cuda", 0), shape=torch.Size((2, 16, 64)))
+    assert native._plan(module, x, Config(**setting)) is False
