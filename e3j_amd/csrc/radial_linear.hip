@@ -110,7 +110,7 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_kernel(
 // One 32x32x16 product takes sixteen inner indices; a lane (g, c) supplies eight of them for
 // row (A) or column (B) c: block q of the inner dimension gives it the indices 16 q + 8 g + m.
 template <int H, int R>
-__global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_split_kernel(
+__global__ __launch_bounds__(kWave * kWaves, 2) void radial_linear_fwd_split_kernel(
     const float *__restrict__ h, const float *__restrict__ w, float *__restrict__ s, int64_t num_edges, int n,
     int per_range) {
     constexpr int Q = H / 16;                         // inner blocks
@@ -175,11 +175,20 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_fwd_split_kernel
 #pragma unroll
             for (int tb = 0; tb < 3; tb++) b[tb] = tile[t & 1][tb][(q * 2 + g) * kTile + c];
 #pragma unroll
-            for (int u = 0; u < 6; u++) {
+            for (int u = 0; u < 5; u++) {
 #pragma unroll
                 for (int r = 0; r < R; r++)
                     d[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r][q].term[kPairs[u][0]], b[kPairs[u][1]], d[r], 0, 0, 0);
             }
+        }
+        // the products of the upper parts behind the small ones of all blocks: error of s, rms, H = 64 1.25e-7 -> 0.77e-7,
+        // H = 128 1.75e-7 -> 0.87e-7, at no time (the tile's upper parts are read twice from LDS)
+        if constexpr (H >= 128) __builtin_amdgcn_sched_barrier(0);  // (read ahead they take a wave per SIMD)
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const bf16x8 b = tile[t & 1][0][(q * 2 + g) * kTile + c];
+#pragma unroll
+            for (int r = 0; r < R; r++) d[r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[r][q].term[0], b, d[r], 0, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -348,6 +357,9 @@ __global__ __launch_bounds__(kWave * kWaves) void radial_linear_bwd_weight_kerne
 // Two blocks of ds are on their way while a third is multiplied: they are read through buffer descriptors, which
 // take one 32-bit offset a load instead of a 64-bit address and a bound (250k edges, H = 64, n = 2 944: 800 -> 640 us;
 // H = 128, n = 1 472: 750 -> 595).  kWide: rows too long for 32-bit offsets.
+// Every other range of the edges sums its part of dW with the sign turned (see split_bf16.h: error at 250k edges, rms,
+// 1.35e-6 -> 0.72e-6, mean of the errors 1.1e-6 -> 4e-10, 620 -> 630 us; sums of a block by itself would take 128
+// registers more at H = 128: 570 -> 720 us).
 template <int H, bool kWide>
 __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linear_bwd_weight_split_kernel(
     const float *__restrict__ h, const float *__restrict__ ds, float *__restrict__ partial, int64_t num_edges,
@@ -379,6 +391,7 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
 #pragma unroll
     for (int t = 0; t < kColTiles; t++) col_ok[t] = col0 + t * kTile < n;
 
+    const float sign = group & 1 ? -1.f : 1.f;
     // slot (q, g, row): h[e0 + 16 q + 8 g + m][row], m < 8; edges past the range read as zeros
     float staged[PER_THREAD][8];
     auto fetch = [&](int64_t e0) {
@@ -398,6 +411,8 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
     auto commit = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < PER_THREAD; i++) {
+#pragma unroll
+            for (int m = 0; m < 8; m++) staged[i][m] *= sign;
             const Split3 parts = split3(staged[i]);
 #pragma unroll
             for (int t = 0; t < 3; t++) rows[buf][t][i * kWave * kWaves + tid] = parts.term[t];
@@ -473,7 +488,7 @@ __global__ __launch_bounds__(kWave * kWaves, H >= 128 ? 1 : 2) void radial_linea
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) out[(int64_t)(rt * kTile + 8 * (v / 4) + 4 * g + v % 4) * n] = d[t][rt][v];
+            for (int v = 0; v < 16; v++) out[(int64_t)(rt * kTile + 8 * (v / 4) + 4 * g + v % 4) * n] = sign * d[t][rt][v];
         }
     }
 }
@@ -533,8 +548,9 @@ int launch_bwd_weight(const float *h, const float *ds, float *dw, float *partial
 // way (a row piece of 128 bytes per 8 lanes), splits it three ways and writes the parts to its private piece of LDS
 // in operand order, from where every lane fetches its slots with 16-byte reads.  The rows of wt of the same 32 n,
 // one contiguous block, are split and shared by the waves of the block, one barrier a step.  ds is read once,
-// two steps ahead: 250k edges, H = 64, n = 2 944: 690 us, H = 128, n = 1 472: 590 (eight waves a block: 585, but 2 000
-// edges, n = 2 048, 147 instead of 105).
+// two steps ahead: 250k edges, H = 64, n = 2 944: 700 us, H = 128, n = 1 472: 600 (eight waves a block are no faster, and
+// 2 000 edges, n = 2 048, take 147 instead of 105).  670 and 570 of it without a sum for each chunk, at an error of
+// 8.5e-7 and 5.9e-7, rms, where it is 2.0e-7 and 1.5e-7 now.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int H, int R>
@@ -616,24 +632,26 @@ __global__ __launch_bounds__(kWave * kWaves, 2) void radial_linear_bwd_input_spl
         fetch_b(t + 1);
         __syncthreads();  // (one barrier a chunk: the shared rows of wt are double buffered)
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-            bf16x8 p[R][3];
+        for (int ct = 0; ct < CT; ct++) {
+            bf16x8 b[Q][3];
 #pragma unroll
-            for (int r = 0; r < R; r++)
+            for (int q = 0; q < Q; q++)
 #pragma unroll
-                for (int ta = 0; ta < 3; ta++) p[r][ta] = a_tile[wave][ta][(q * 2 + g) * A_BLOCK + r * kTile + c];
+                for (int tb = 0; tb < 3; tb++) b[q][tb] = b_tile[buf][tb][(q * 2 + g) * H + ct * kTile + c];
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++) {
-                bf16x8 b[3];
+            for (int r = 0; r < R; r++) {
+                f32x16 chunk = {};  // (by itself, the small products first: see split_bf16.h)
+                bf16x8 p[Q][3];
 #pragma unroll
-                for (int tb = 0; tb < 3; tb++) b[tb] = b_tile[buf][tb][(q * 2 + g) * H + ct * kTile + c];
+                for (int q = 0; q < Q; q++)
 #pragma unroll
-                for (int u = 0; u < 6; u++) {
+                    for (int ta = 0; ta < 3; ta++) p[q][ta] = a_tile[wave][ta][(q * 2 + g) * A_BLOCK + r * kTile + c];
 #pragma unroll
-                    for (int r = 0; r < R; r++)
-                        d[r][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[r][kPairs[u][0]], b[kPairs[u][1]], d[r][ct],
-                                                                           0, 0, 0);
-                }
+                for (int u = 0; u < 6; u++)
+#pragma unroll
+                    for (int q = 0; q < Q; q++)
+                        chunk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(p[q][kPairs[u][0]], b[q][kPairs[u][1]], chunk, 0, 0, 0);
+                d[r][ct] += chunk;
             }
         }
     };

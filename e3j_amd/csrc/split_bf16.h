@@ -5,6 +5,12 @@
 // float32, i.e. about the accuracy of a float32 product at 6/16 of its cost.
 // (Two float16 parts with a scale for all terms of a sum take three products, but hold a term to 2^-37 of the largest
 // operand of its row however large its partner is: opposed spreads of 2^20 left no digit.)
+//
+// The errors of these sums lie to one side, downwards whatever the sign of the sum (measured, sums of 250 007 terms in 128
+// parts, normal values: mean -1.07e-6 of the sums' rms, also with all terms negated), and there are six additions a block
+// of sixteen terms.  So a stretch of a sum is taken by itself where the registers allow it, the small products first and
+// x1 y1 last, and added to the rest by a vector instruction, which rounds to nearest; or every other part is summed with
+// its sign turned, so that the errors cancel.
 #pragma once
 #include "common.h"
 

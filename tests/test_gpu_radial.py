@@ -179,6 +179,35 @@ def test_outliers_that_meet_zeros(inner, outlier):
     _assert_products(h, w, ds)
 
 
+@pytest.mark.parametrize("inner,n", [(64, 2944), (64, 96), (128, 1472), (128, 32)])
+def test_errors_of_sums_of_one_size(inner, n):
+    """Normal values: a sum of k parts of random sign, rounded (or cut off) after each, is 2^-24 sqrt((k + 1) / 2) off, rms,
+    beside the rounding of the parts; s adds the upper products of inner / 16 blocks, dh the sums of n / 32 chunks."""
+    g = torch.Generator(device="cuda").manual_seed(inner + n)
+    h, w = (torch.randn(*shape, device="cuda", generator=g).requires_grad_(True) for shape in ((3001, inner), (inner, n)))
+    s = radial_linear(h, w)
+    ds = torch.randn(*s.shape, device="cuda", generator=g)
+    (dh,) = torch.autograd.grad(s, h, ds)
+    h, w, s = h.detach().double(), w.detach().double(), s.detach()
+    for name, got, want, parts in (("s", s, h @ w, inner // 16), ("dh", dh, ds.double() @ w.t().contiguous(), n // 32)):
+        error = float(((got.double() - want).square().mean() / want.square().mean()).sqrt())
+        assert error <= 2.0 ** -24 * ((parts + 1) / 2 + 1) ** 0.5, (name, error)
+
+
+@pytest.mark.parametrize("inner", [64, 128])
+def test_errors_of_the_weight_gradient_have_no_sign(inner):
+    """Sums on the matrix cores err downwards: the errors of dW, which is a sum over all edges, do not all have that sign
+    (errors of either sign would have a mean of a hundredth of their rms over so many values)."""
+    edges, n = 100003, 512
+    g = torch.Generator(device="cuda").manual_seed(inner)
+    h = torch.nn.functional.silu(torch.randn(edges, inner, device="cuda", generator=g))
+    w = torch.randn(inner, n, device="cuda", generator=g).requires_grad_(True)
+    ds = torch.randn(edges, n, device="cuda", generator=g)
+    (dw,) = torch.autograd.grad(radial_linear(h, w), w, ds)
+    error = dw.double() - h.double().t().contiguous() @ ds.double()
+    assert abs(float(error.mean())) <= float(error.square().mean().sqrt()) / 8
+
+
 @pytest.mark.parametrize("inner", [8, 32, 64, 128])
 @pytest.mark.parametrize("edges,n", [(5, 2944), (256, 992), (16400, 96), (33000, 736), (33000, 800), (65000, 768), (70000, 64)])
 def test_forward_over_ranges_of_columns(inner, edges, n):
