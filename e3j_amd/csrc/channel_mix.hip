@@ -73,11 +73,12 @@ int launch(const void *src, void *dst, int64_t num_nodes, int32_t rows, int32_t 
 // transposed by the caller): the cotangent row is read once and gives one product per copy.
 // At 128 channels a block of the backward makes 64 output channels: the operand of both chunks of a row stays in
 // registers, and the cotangent rows that are read twice are few.  A forward block makes all.
-// Bound by the stream and, in a block's chain of chunks, by latency: 99 rows to 16, 6 000 nodes, 64 channels: 55 -> 42 us
-// forward and 63 -> 38 backward where float32 products took 32 and the stream takes 35; 128 channels 225 -> 155 and
-// 231 -> 134 (stream 70), 20 000 nodes 569 -> 467 and 578 -> 427, 200 nodes 66 -> 62 and 68 -> 28 (64 channels
-// there: 21 -> 22 and 22 -> 16).  Error against float64 over normal values, rms: 0.76 to 0.85 times that of float32
-// products (fewer additions).
+// A chunk is summed by itself (see split_bf16.h): error against float64 over normal values, rms, 64 channels 3.0e-7 -> 0.7e-7
+// forward and 1.1e-7 -> 0.5e-7 backward, 128 channels 4.3e-7 -> 0.8e-7 and 1.6e-7 -> 0.5e-7, for 2 to 5 % of the time.
+// Bound by the stream and, in a block's chain of chunks, by latency: 99 rows to 16, 6 000 nodes, 64 channels: 55 -> 44 us
+// forward and 63 -> 37 backward where float32 products took 32 and the stream takes 35; 128 channels 225 -> 156 and
+// 231 -> 127 (stream 70), 20 000 nodes 569 -> 459 and 578 -> 427, 200 nodes 66 -> 63 and 68 -> 29 (64 channels
+// there: 21 -> 21 and 22 -> 16).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kMixDegrees = 8;
@@ -232,23 +233,35 @@ __global__ __launch_bounds__(256, K == 64 ? 3 : 2) void channel_mix_kernel(
         constexpr int TILES = 2;
 #pragma unroll
         for (int c0 = 0; c0 < KT; c0 += TILES) {
+            f32x16 chunk[TILES];  // (summed by itself, the small products first: see split_bf16.h)
+#pragma unroll
+            for (int i = 0; i < TILES; i++) chunk[i] = zero;
+            auto piece_of = [&](int i, int u, int s) {
+                return *reinterpret_cast<const bf16x8 *>(&weights[u][((c0 + i) * 32 + r) * WEIGHT_PITCH + 32 * h + 8 * s]);
+            };
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 bf16x8 b[TILES][3];
 #pragma unroll
                 for (int i = 0; i < TILES; i++)
 #pragma unroll
-                    for (int u = 0; u < 3; u++)
-                        b[i][u] = *reinterpret_cast<const bf16x8 *>(
-                            &weights[u][((c0 + i) * 32 + r) * WEIGHT_PITCH + 32 * h + 8 * s]);
+                    for (int u = 0; u < 3; u++) b[i][u] = piece_of(i, u, s);
 #pragma unroll
-                for (int u = 0; u < 6; u++)
+                for (int u = 0; u < 5; u++)
 #pragma unroll
                     for (int i = 0; i < TILES; i++)
-                        acc[c0 + i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s].term[kPairs[u][0]], b[i][kPairs[u][1]],
-                                                                              acc[c0 + i], 0, 0, 0);
+                        chunk[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s].term[kPairs[u][0]], b[i][kPairs[u][1]],
+                                                                           chunk[i], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);  // (the operands of one step at a time in registers)
             }
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int i = 0; i < TILES; i++)
+                    chunk[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s].term[0], piece_of(i, 0, s), chunk[i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < TILES; i++) acc[c0 + i] += chunk[i];
         }
     };
     // chunk `q` of the weights in float32; `first`, node_stride: its source rows

@@ -66,6 +66,19 @@ def test_against_float64(K, n, blocks, scales):
 
 
 @pytest.mark.parametrize("K", [64, 128])
+@pytest.mark.parametrize("blocks", [[(1, 1)], [(9, 1)], [(4, 1), (2, 3)]])
+def test_errors_of_sums_of_one_size(K, blocks):
+    """Normal values: a sum of k parts of random sign, rounded (or cut off) after each, is 2^-24 sqrt((k + 1) / 2) off, rms,
+    beside the rounding of the parts; a part is a chunk of 64 channels."""
+    out, dx, weights = _problem(500, blocks, K)
+    x, g = _run(out, blocks, K, weights, dx)
+    for got, want, parts in ((x, E.channel_mix(out, blocks, weights), max(m for m, _ in blocks) * K // 64),
+                             (g, E.channel_mix_vjp(dx, blocks, weights), K // 64)):
+        error = np.sqrt(((got - want) ** 2).mean() / (want ** 2).mean())
+        assert error <= 2.0 ** -24 * np.sqrt((parts + 1) / 2 + 1), error
+
+
+@pytest.mark.parametrize("K", [64, 128])
 def test_weights_that_pick_one_channel(K):
     """One term a sum, beside channels of any size: the six partial products of that term, added in float32, and 2^-26
     of it left out."""
