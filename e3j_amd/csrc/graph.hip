@@ -496,8 +496,8 @@ __global__ void sort_input_kernel(const int32_t *__restrict__ key, int64_t num_e
     }
 }
 
-// Stable sort of edge positions by key for up to kSortChunk * kSortChunks edges of fewer than 2^16 nodes (`own_sort`), in two passes
-// of at most eight bits, a count and a scatter each: four launches, where the library's sort takes
+// Stable sort of edge positions by key for 1 025 to kSortChunk * kSortChunks edges of fewer than 2^16 nodes (`own_sort`), in
+// two passes of at most eight bits, a count and a scatter each: four launches, where the library's sort takes
 // eight and the launch that writes its keys a ninth (150k edges, 5 000 nodes: 58 us -> 20; 3-5 us a launch whatever
 // it moves).  A workgroup takes kSortChunk consecutive edges; the scatter of each adds up for itself how
 // many edges of a smaller digit, or of the same one in an earlier chunk, there are.

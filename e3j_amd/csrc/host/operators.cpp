@@ -8,7 +8,7 @@
 // launches the VJP without the interpreter.  1 000 atoms, forward and VJP: 150 to 250 us (as the host was busy) -> 95;
 // 21 atoms, forward: 69 -> 15 us, three launches of 2 to 7.
 //
-// It takes calls whose route is the plain one (the conditions of `Plan::takes` and of e3j_amd/native.py); every
+// It takes calls whose route is the plain one (the conditions of `call`, `Plan::operands` and e3j_amd/native.py); every
 // other call, every error and every derivative of a derivative goes to the Python operators, which stay the
 // only place where those are decided: the caller gets None, or the node calls `Plan::fallback`.
 
