@@ -548,9 +548,9 @@ int launch_bwd_weight(const float *h, const float *ds, float *dw, float *partial
 // way (a row piece of 128 bytes per 8 lanes), splits it three ways and writes the parts to its private piece of LDS
 // in operand order, from where every lane fetches its slots with 16-byte reads.  The rows of wt of the same 32 n,
 // one contiguous block, are split and shared by the waves of the block, one barrier a step.  ds is read once,
-// two steps ahead: 250k edges, H = 64, n = 2 944: 700 us (745 behind the forward pass), H = 128, n = 1 472: 600 (eight waves a block are no faster, and
-// 2 000 edges, n = 2 048, take 147 instead of 105).  670 and 570 of it without a sum for each chunk, at an error of
-// 8.5e-7 and 5.9e-7, rms, where it is 2.0e-7 and 1.5e-7 now.
+// two steps ahead: 250k edges, H = 64, n = 2 944: 700 us (745 behind the forward pass), H = 128, n = 1 472: 600 (eight
+// waves a block are no faster, and 2 000 edges, n = 2 048, take 147 instead of 105).  670 and 570 of it without a sum for
+// each chunk, at an error of 8.5e-7 and 5.9e-7, rms, where it is 2.0e-7 and 1.5e-7 now.
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int H, int R>
